@@ -185,14 +185,22 @@ def _ragged_lengths(B, T, seed):
 
 
 # ---- the calls -------------------------------------------------------------------------------------
-def _live(L, pages):
-    """The state of a layer that the calls have written: the rows in use, and the pages if any were packed."""
-    out = [L.Sink_Buffer_K[:, :, :L.Sink_Count], L.Sink_Buffer_V[:, :, :L.Sink_Count],
-           L.Q_Buffer_K[:, :, :L.Q_Buffer_Count_K], L.Q_Buffer_V[:, :, :L.Q_Buffer_Count_V],
-           L.Local_Buffer_V[:, :, :L.Local_Count_V]]
+def _state(L, pages):
+    """The state of a layer that the calls have written: its fp16 windows, and the pages if any were packed."""
+    out = [L.Sink_Buffer_K, L.Sink_Buffer_V, L.Q_Buffer_K, L.Q_Buffer_V, L.Local_Buffer_V]
     if pages:
         out += [L.KeyCache, L.KeyCache_metadata, L.ValueCache, L.ValueCache_metadata]
-    return [t for t in out if t.numel()]
+    return out
+
+
+def _state_after_chunk(L):
+    """The same after a chunk, with the Q-buffers up to their fill counts: rows past them are not state."""
+    out = [L.Sink_Buffer_K, L.Sink_Buffer_V, L.Local_Buffer_V, L.KeyCache, L.KeyCache_metadata, L.ValueCache,
+           L.ValueCache_metadata]
+    for rows, n in ((L.Q_Buffer_K, L.Q_Buffer_Count_K), (L.Q_Buffer_V, L.Q_Buffer_Count_V)):
+        if n:
+            out.append(rows[:, :, :n])
+    return out
 
 
 def run(state):
@@ -211,19 +219,19 @@ def run(state):
         for l in layers:
             cache.update(s.k[l], s.v[l], l)
             cache.quantize_prefill(l)
-        return {"state": [_live(L, True) for L in cache.kv_cache]}
+        return {"state": [_state(L, True) for L in cache.kv_cache]}
     if s.kind == "prompt":
         cache.restore_host_counters(s.empty)
         for l in layers:
             k, v = cache.update(s.k[l], s.v[l], l)
             outs.append(hf.kitty_attention(s.modules[l], s.q[l], k, v, None, scaling=s.scaling)[0])
-        return {"out": outs, "state": [_live(L, True) for L in cache.kv_cache]}
+        return {"out": outs, "state": [_state(L, True) for L in cache.kv_cache]}
     cache.restore_host_counters(s.held)
     if s.kind == "chunk":
         for l in layers:
             outs.append(kitty_prefill_attention(s.module, s.q[l], s.k[l], s.v[l], cache.kv_cache[l], s.scaling)[0])
             cache.append(s.k[l], s.v[l], l)
-        return {"out": outs, "state": [_live(L, True) for L in cache.kv_cache]}
+        return {"out": outs, "state": [_state_after_chunk(L) for L in cache.kv_cache]}
     if s.kind == "serve":
         for l in layers:
             L = cache.kv_cache[l]
@@ -239,7 +247,7 @@ def run(state):
         outs.append(kitty_attention_forward(s.module, s.q[l], cache.kv_cache[l], s.scaling)[0])
         cache.quantize_decode(l)
     packed = cache.kv_cache[0].PageCount_K != s.held[0][1]
-    return {"out": outs, "state": [_live(L, packed) for L in cache.kv_cache]}
+    return {"out": outs, "state": [_state(L, packed) for L in cache.kv_cache]}
 
 
 # ---- what a pass cannot do without -------------------------------------------------------------------
