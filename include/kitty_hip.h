@@ -286,6 +286,17 @@ int kitty_append_chunk(const kitty_kv_layer* layer, const void* k_new, const voi
                        int64_t stride_b, int64_t stride_h, int64_t stride_t, int B, int T, void* stream);
 
 /*
+ * One token per sequence with the layer's scalar counters (layer->counts; seq_counts must be NULL): the
+ * slice copies of KittyCache.update's decode branch (kitty.py:97-123) as one launch, for every supported
+ * head dimension.  k_new / v_new: fp16 [B,H_KV,1,D], D contiguous, byte strides of their own, 16-byte
+ * aligned.  Sink not full -> the sink rows; else K -> Q_Buffer_K[Q_Buffer_Count_K] and V -> the local
+ * ring, whose oldest row first moves to Q_Buffer_V when the ring is full.  The caller advances its
+ * counters by the same rules; full Q-buffers are rejected with KITTY_E_RANGE (the reference's asserts).
+ */
+int kitty_append_row(const kitty_kv_layer* layer, const void* k_new, const void* v_new, int64_t k_stride_b,
+                     int64_t k_stride_h, int64_t v_stride_b, int64_t v_stride_h, int B, void* stream);
+
+/*
  * Fake quantization of dense fp16 keys or values in place: replaces fake_quant_groupwise_lastdim of
  * the reference's accuracy simulator (src/kitty_sim/utils_quant.py:64-114) on the slices its cache
  * hands it (src/kitty_sim/kitty_simulate.py:196-252).  Arithmetic as that function evaluates on a GPU

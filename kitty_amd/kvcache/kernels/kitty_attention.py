@@ -7,6 +7,7 @@ SV kernel, each on a ``(B, H_KV)`` grid (:433-523).  Here one fused split-K kern
 packed pages once (QK^T, online softmax and PV per split of the sequence) and a merge kernel
 combines the splits; no score tensor exists.
 """
+import functools
 from typing import Optional
 
 import torch
@@ -16,6 +17,15 @@ from ... import _lib
 from ..utils_kv_per_layer import KVCache_Layer
 
 MAX_KV_GROUP = 16   # kitty_attention.py:418
+
+
+@functools.lru_cache(maxsize=4096)
+def _split_plan(B: int, H_Q: int, H_KV: int, D: int, max_tiles: int, per_sequence: bool, num_splits: int):
+    """(splits, workspace bytes) of a decode launch: a function of the sizes alone."""
+    lib = _lib.lib()
+    if num_splits <= 0:
+        num_splits = lib.kitty_decode_attn_default_splits(B, H_KV, max_tiles, int(per_sequence))
+    return num_splits, lib.kitty_decode_attn_workspace_bytes(B, H_Q, D, num_splits)
 
 
 def kitty_attention_forward(
@@ -40,22 +50,20 @@ def kitty_attention_forward(
     if H_KV != kv_cache.H_KV or B > kv_cache.MAX_BS:
         raise ValueError("query does not match the cache (H_KV or batch size)")
 
-    lib = _lib.lib()
-    if kv_cache.seq_counts is None:
-        max_tiles = 1 + (kv_cache.get_total_length() - kv_cache.Sink_Count + kv_cache.PAGE_SIZE - 1) // kv_cache.PAGE_SIZE
-    else:
+    per_sequence = kv_cache.seq_counts is not None
+    if per_sequence:
         max_tiles = 2 + kv_cache.MAX_PAGE
-    if not num_splits or num_splits <= 0:
-        num_splits = lib.kitty_decode_attn_default_splits(B, H_KV, max_tiles, int(kv_cache.seq_counts is not None))
-    ws_bytes = lib.kitty_decode_attn_workspace_bytes(B, H_Q, D, num_splits)
+    else:
+        max_tiles = 1 + (kv_cache.get_total_length() - kv_cache.Sink_Count + kv_cache.PAGE_SIZE - 1) // kv_cache.PAGE_SIZE
+    num_splits, ws_bytes = _split_plan(B, H_Q, H_KV, D, max_tiles, per_sequence, num_splits or 0)
     ws = kv_cache.workspace(ws_bytes)
     # [B, T=1, H_Q, D], the layout HF attention modules expect (kitty_attention.py:475-481)
-    attn_output = torch.empty((B, t_query, H_Q, D), dtype=query.dtype, device=query.device)
-    desc = kv_cache.descriptor()
-    rc = lib.kitty_decode_attn(desc, query.data_ptr(), B, H_Q, float(scaling), attn_output.data_ptr(),
-                               ws.data_ptr(), ws.numel(), num_splits, variant,
-                               _lib.current_stream_ptr(query.device))
-    _lib.check(rc, "kitty_attention_forward")
+    attn_output = query.new_empty((B, t_query, H_Q, D))
+    rc = _lib.lib().kitty_decode_attn(kv_cache.descriptor(), query.data_ptr(), B, H_Q, float(scaling),
+                                      attn_output.data_ptr(), ws.data_ptr(), ws.numel(), num_splits, variant,
+                                      _lib.current_stream_ptr(query.device))
+    if rc:
+        _lib.check(rc, "kitty_attention_forward")
     return attn_output, None
 
 

@@ -33,6 +33,17 @@ def prefill_split(len_prefill: int, S: int, P: int) -> dict:
     return dict(sink=sink, qbuf_k=qbuf_k, pages_k=pages_k, local_v=local_v, qbuf_v=qbuf_v, pages_v=pages_v)
 
 
+def _row_source(L: KVCache_Layer, x: torch.Tensor) -> torch.Tensor:
+    """``x [B, H_KV, 1, D]`` as the append kernel reads it: fp16 on the cache's device, D contiguous, rows on
+    16-byte boundaries.  What a slice assignment would have converted or moved is converted here."""
+    if x.dtype != torch.float16 or x.device != L.KeyCache.device:
+        x = x.to(L.KeyCache.device, torch.float16)
+    st = x.stride()
+    if st[3] != 1 or st[0] % 8 or st[1] % 8 or x.data_ptr() % 16:
+        x = x.clone(memory_format=torch.contiguous_format)
+    return x
+
+
 class KittyCache(_HFCache):
     """Kitty KV cache: fp16 sink + packed 2-bit pages (25 % of key channels at 4 bit) + fp16
     residual windows that are flushed into packed pages when full."""
@@ -77,6 +88,9 @@ class KittyCache(_HFCache):
         if kvcache.device_counters:
             self._append_token_device(kvcache, key_states, value_states)
             return False
+        if kvcache.on_hip:
+            self._append_row(kvcache, key_states, value_states)
+            return False
         with torch.no_grad():
             if kvcache.Sink_Count < kvcache.S:
                 idx = kvcache.Sink_Count
@@ -99,6 +113,24 @@ class KittyCache(_HFCache):
                     kvcache.Local_Buffer_V[:B, :, w, :] = value_states[:, :, 0, :]
                     kvcache.Write_Offset_Local_V = (w + 1) % kvcache.PAGE_SIZE
         return False
+
+    @staticmethod
+    def _append_row(L: KVCache_Layer, key_states: torch.Tensor, value_states: torch.Tensor) -> None:
+        """The decode branch of ``update`` on the GPU: one launch writes the rows, then the host counters
+        follow (kitty.py:102-123)."""
+        if L.Sink_Count >= L.S:
+            assert L.Q_Buffer_Count_K < L.PAGE_SIZE
+            assert L.Local_Count_V < L.PAGE_SIZE or L.Q_Buffer_Count_V < L.PAGE_SIZE
+        B, H, _, D = key_states.shape
+        if H != L.H_KV or D != L.D or B > L.MAX_BS or value_states.shape != key_states.shape:
+            raise ValueError(f"key_states / value_states must be [B <= {L.MAX_BS}, {L.H_KV}, 1, {L.D}]")
+        key_states, value_states = _row_source(L, key_states), _row_source(L, value_states)
+        ks, vs = key_states.stride(), value_states.stride()
+        rc = _lib.lib().kitty_append_row(L.descriptor(), key_states.data_ptr(), value_states.data_ptr(), 2 * ks[0],
+                                         2 * ks[1], 2 * vs[0], 2 * vs[1], B, _lib.current_stream_ptr(key_states.device))
+        if rc:
+            _lib.check(rc, "KittyCache.update")
+        L.step_host_counters()
 
     def quantize_prefill(self, layer_idx: int = 0) -> None:
         """Split the stashed prefill into sink / packed pages / fp16 residuals (kitty.py:126-192)."""

@@ -94,6 +94,7 @@ class KVCache_Layer:
         self.active_batch = MAX_BS
         self._workspace: Optional[torch.Tensor] = None
         self._desc: Optional[_lib.KittyKVLayer] = None
+        self.on_hip = self.KeyCache.is_cuda
 
     def get_total_length(self) -> int:
         """Total number of cached tokens (the reference's :85-95, including its K == V check)."""
@@ -179,8 +180,8 @@ class KVCache_Layer:
             d.cache_pages_k, d.cache_pages_v = self.KeyCache.shape[0], self.ValueCache.shape[0]
             d.status = self.status.data_ptr()
             self._desc = d
-        for i, v in enumerate(self.counts()):
-            d.counts[i] = int(v)
+            self._desc_counts = d.counts          # a view of the struct's array
+        self._desc_counts[:] = self.counts()
         d.seq_counts = None if self.seq_counts is None else self.seq_counts.data_ptr()
         return d
 
