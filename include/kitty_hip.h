@@ -239,6 +239,24 @@ int kitty_prefill_attn(const kitty_kv_layer* layer,
                        int B, int H_Q, int T_q, float scaling, void* out, void* stream);
 
 /*
+ * The same with the walk over the tokens cut into num_splits shares, for chunks that alone would leave most
+ * of the device idle: a partial per row and share goes to the workspace, a second launch merges them.
+ * num_splits = 1: kitty_prefill_attn itself (workspace unused, may be NULL).  Otherwise workspace: at least
+ * kitty_prefill_attn_workspace_bytes(B,H_Q,D,T_q,num_splits) bytes, 256-aligned.
+ * kitty_prefill_attn_default_splits: how many shares pay; max_tiles = 1 + the 128-token tiles after the
+ * sink of the longest sequence.  Results do not depend on num_splits beyond the order of fp32 sums and the
+ * running maximum that the fp16 probabilities refer to.
+ */
+size_t kitty_prefill_attn_workspace_bytes(int B, int H_Q, int D, int T_q, int num_splits);
+int kitty_prefill_attn_default_splits(int B, int H_Q, int H_KV, int D, int T_q, int max_tiles);
+int kitty_prefill_attn_split(const kitty_kv_layer* layer,
+                             const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
+                             const void* k_new, const void* v_new,
+                             int64_t new_stride_b, int64_t new_stride_h, int64_t new_stride_t,
+                             int B, int H_Q, int T_q, float scaling, void* out,
+                             void* workspace, size_t workspace_bytes, int num_splits, void* stream);
+
+/*
  * Decode-time bookkeeping with per-sequence counters kept on the device (layer->seq_counts must be
  * set; it is read AND written; layer->status, when set, is written).  The reference keeps one set of host ints for the whole batch and
  * drives slice copies from them (KittyCache.update, kitty.py:97-123; quantize_decode,

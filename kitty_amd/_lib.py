@@ -64,6 +64,11 @@ _SIGNATURES = {
                                          c_void_p]),
     "kitty_prefill_attn": (c_int, [POINTER(KittyKVLayer), c_void_p, c_int64, c_int64, c_int64, c_void_p, c_void_p,
                                    c_int64, c_int64, c_int64, c_int, c_int, c_int, c_float, c_void_p, c_void_p]),
+    "kitty_prefill_attn_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
+    "kitty_prefill_attn_default_splits": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int]),
+    "kitty_prefill_attn_split": (c_int, [POINTER(KittyKVLayer), c_void_p, c_int64, c_int64, c_int64, c_void_p, c_void_p,
+                                         c_int64, c_int64, c_int64, c_int, c_int, c_int, c_float, c_void_p, c_void_p,
+                                         c_size_t, c_int, c_void_p]),
     "kitty_append_token": (c_int, [POINTER(KittyKVLayer), c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_void_p,
                                    c_int64, c_int, c_void_p]),
     "kitty_append_row": (c_int, [POINTER(KittyKVLayer), c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int,

@@ -14,7 +14,8 @@ void launch_decode_mfma(const kitty_kv_layer& L, const void* q, int B, int H_Q, 
 void launch_prefill_attn(const kitty_kv_layer& L, const void* q, int64_t q_stride_b, int64_t q_stride_h,
                          int64_t q_stride_t, const void* k_new, const void* v_new, int64_t new_stride_b,
                          int64_t new_stride_h, int64_t new_stride_t, int B, int H_Q, int Tq, float scaling,
-                         void* out, hipStream_t stream);
+                         void* out, float* ws_ml, float* ws_acc, int num_splits, hipStream_t stream);
+int prefill_splits(int B, int H_Q, int H_KV, int Tq, int tiles, int units);
 // head dimensions other than 128 (any_dim.hip)
 void launch_decode_any(const kitty_kv_layer& L, const void* q, int B, int H_Q, float scaling, float* ws_ml,
                        float* ws_acc, int num_splits, hipStream_t stream);
@@ -227,10 +228,30 @@ extern "C" int kitty_decode_attn(const kitty_kv_layer* layer, const void* q, int
   return kitty_decode_attn_merge(workspace, workspace_bytes, B, H_Q, layer->D, num_splits, out, stream);
 }
 
+extern "C" size_t kitty_prefill_attn_workspace_bytes(int B, int H_Q, int D, int T_q, int num_splits) {
+  if (B <= 0 || H_Q <= 0 || T_q <= 0 || !head_dim_supported(D) || num_splits <= 1) return 0;
+  const size_t rows = (size_t)B * T_q;
+  return ((rows * H_Q * num_splits * 2 * sizeof(float) + 255) & ~(size_t)255) + rows * H_Q * num_splits * D * sizeof(float);
+}
+
+extern "C" int kitty_prefill_attn_default_splits(int B, int H_Q, int H_KV, int D, int T_q, int max_tiles) {
+  if (B <= 0 || H_KV <= 0 || H_Q < H_KV || H_Q / H_KV > 16 || T_q <= 0 || max_tiles <= 0 || D != kD) return 1;
+  return prefill_splits(B, H_Q, H_KV, T_q, max_tiles + c_div_up(T_q, kPage), device_simds() / 4);
+}
+
 extern "C" int kitty_prefill_attn(const kitty_kv_layer* layer, const void* q, int64_t q_stride_b,
                                   int64_t q_stride_h, int64_t q_stride_t, const void* k_new, const void* v_new,
                                   int64_t new_stride_b, int64_t new_stride_h, int64_t new_stride_t, int B, int H_Q,
                                   int T_q, float scaling, void* out, void* stream) {
+  return kitty_prefill_attn_split(layer, q, q_stride_b, q_stride_h, q_stride_t, k_new, v_new, new_stride_b, new_stride_h,
+                                  new_stride_t, B, H_Q, T_q, scaling, out, nullptr, 0, 1, stream);
+}
+
+extern "C" int kitty_prefill_attn_split(const kitty_kv_layer* layer, const void* q, int64_t q_stride_b,
+                                        int64_t q_stride_h, int64_t q_stride_t, const void* k_new, const void* v_new,
+                                        int64_t new_stride_b, int64_t new_stride_h, int64_t new_stride_t, int B, int H_Q,
+                                        int T_q, float scaling, void* out, void* workspace, size_t workspace_bytes,
+                                        int num_splits, void* stream) {
   int max_tiles = 0;
   if (int rc = check_layer(layer, q, B, H_Q, &max_tiles)) return rc;
   KITTY_REQUIRE(k_new && v_new && out, KITTY_E_NULL, "k_new / v_new / out is NULL");
@@ -242,12 +263,23 @@ extern "C" int kitty_prefill_attn(const kitty_kv_layer* layer, const void* q, in
                 KITTY_E_ALIGN, "q, k_new, v_new and out need 16-byte aligned bases and strides");
   KITTY_REQUIRE(q_stride_t >= layer->D * 2 && new_stride_t >= layer->D * 2, KITTY_E_ALIGN,
                 "a token stride is smaller than one row of D fp16 values");
+  KITTY_REQUIRE(num_splits >= 1 && num_splits <= 1024, KITTY_E_RANGE, "num_splits=%d out of range", num_splits);
+  float *ws_ml = nullptr, *ws_acc = nullptr;
+  if (num_splits > 1) {
+    KITTY_REQUIRE(workspace != nullptr, KITTY_E_NULL, "workspace is NULL");
+    KITTY_REQUIRE(((uintptr_t)workspace % 256) == 0, KITTY_E_ALIGN, "workspace needs 256-byte alignment");
+    const size_t need = kitty_prefill_attn_workspace_bytes(B, H_Q, layer->D, T_q, num_splits);
+    KITTY_REQUIRE(workspace_bytes >= need, KITTY_E_WORKSPACE, "workspace of %zu bytes is smaller than the %zu needed for %d splits",
+                  workspace_bytes, need, num_splits);
+    ws_ml = (float*)workspace;
+    ws_acc = (float*)((uint8_t*)workspace + (need - (size_t)B * T_q * H_Q * num_splits * layer->D * sizeof(float)));
+  }
   if (layer->D != kD) {
     launch_prefill_any(*layer, q, q_stride_b, q_stride_h, q_stride_t, k_new, v_new, new_stride_b, new_stride_h,
                        new_stride_t, B, H_Q, T_q, scaling, out, (hipStream_t)stream);
     return check_launch("kitty_prefill_attn");
   }
   launch_prefill_attn(*layer, q, q_stride_b, q_stride_h, q_stride_t, k_new, v_new, new_stride_b, new_stride_h,
-                      new_stride_t, B, H_Q, T_q, scaling, out, (hipStream_t)stream);
+                      new_stride_t, B, H_Q, T_q, scaling, out, ws_ml, ws_acc, num_splits, (hipStream_t)stream);
   return check_launch("kitty_prefill_attn");
 }

@@ -34,6 +34,9 @@
 #define KITTY_PV_PRIO 2
 
 namespace kitty {
+// merge pass over independent rows (rows_merge.hip)
+void launch_rows_merge(int D, const float* ws_ml, const float* ws_acc, void* out, int64_t rows, int num_splits,
+                       bool keep_nan, hipStream_t stream);
 namespace {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
@@ -117,7 +120,7 @@ __device__ __forceinline__ uint32_t dequant_pair(uint32_t c, half2v scale, half2
   return __builtin_bit_cast(uint32_t, r);
 }
 
-template <bool BOOST>
+template <bool BOOST, bool SPLIT>
 struct Prefill {
   const kitty_kv_layer& L;
   const SeqCounts c;
@@ -136,12 +139,15 @@ struct Prefill {
   // current one, and the barrier that ends every iteration of the walk publishes it.  Reading and
   // checking the ids where they are used - a load whose value the next instructions need, in every
   // iteration of every workgroup - cost this kernel 10 %.
+  // Body tiles are counted from id_base(), the first one of this workgroup's share.
   static constexpr int kIdChunk = 64;
-  int32_t (*page_ids)[2][kIdChunk];   // [chunk & 1][K, V][body tile % kIdChunk]
+  int32_t (*page_ids)[2][kIdChunk];   // [chunk & 1][K, V][(body tile - id_base()) % kIdChunk]
+  int first_id = 0;
+  __device__ __forceinline__ int id_base() const { return SPLIT ? first_id : 0; }
 
   __device__ __forceinline__ void stage_page_ids(int chunk) const {
     if (tid < 2 * kIdChunk) {
-      const int side = tid / kIdChunk, i = chunk * kIdChunk + tid % kIdChunk;
+      const int side = tid / kIdChunk, i = id_base() + chunk * kIdChunk + tid % kIdChunk;
       if (i < (side ? c.pv : c.pk)) {
         const int64_t pg = side ? L.page_table_v[(int64_t)b * L.page_table_v_stride_b + i]
                                 : L.page_table_k[(int64_t)b * L.page_table_k_stride_b + i];
@@ -153,7 +159,8 @@ struct Prefill {
   // (every lane reads the same word and keeps it in a vector register: made a scalar again with
   // v_readfirstlane, with the tile addresses then computed on the scalar unit, the kernel is 4 % slower)
   __device__ __forceinline__ int64_t staged_page(int side, int i) const {
-    return page_ids[(i / kIdChunk) & 1][side][i % kIdChunk];
+    const int r = i - id_base();
+    return page_ids[(r / kIdChunk) & 1][side][r % kIdChunk];
   }
 
   __device__ TileSrc tile(int t) const {
@@ -330,6 +337,9 @@ struct WaveAcc {
 // issued between the exponentials of sub-tile s, so that a wave's instruction stream mixes matrix
 // and vector work instead of alternating long runs of each.
 // limit[nt]: tokens of the tile with index < limit are visible to the row of column tile nt.
+// SPLIT: the walk starts anywhere in the sequence, so a row may see nothing of the first sub-tile (and
+// then, causally, nothing at all of this share): its running maximum must stay a number.
+template <bool SPLIT>
 struct TileAttend {
   const uint8_t* kb;   // K tile + this lane's corner of a transposing read
   const uint8_t* vb;   // V tile + the same corner
@@ -390,7 +400,7 @@ struct TileAttend {
 #pragma unroll
       for (int nt = 0; nt < kNT; ++nt) {
         const float col = max_over_lane_groups(mt_[nt]);
-        const float dm = A.first ? col : fmaxf(col, 0.f);
+        const float dm = !A.first ? fmaxf(col, 0.f) : SPLIT && col == -INFINITY ? 0.f : col;
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
@@ -467,22 +477,38 @@ struct TileAttend {
   }
 };
 
-template <bool BOOST>
+// Chunk positions per workgroup: the chunk cut into as few blocks as 256 rows allow, all of the same size
+// (a chunk of 200 positions, four heads per group: 4 x 50 instead of 3 x 64 + 8), so that the rows are
+// dense and a wavefront without rows has none of them to multiply.
+__host__ __device__ inline int block_positions(int G, int Tq) {
+  const int most = kRows / G;
+  return c_div_up(Tq, c_div_up(Tq, most));
+}
+
+// SPLIT: blockIdx.x = block * num_splits + split; a workgroup walks its share of the tiles and leaves a
+// partial per row (running maximum, running sum, un-normalised output) for prefill_merge_kernel.  One
+// workgroup fills a compute unit (147 KB of LDS), and a short chunk has few of them: 200 positions over
+// 12k cached tokens, 32 / 8 heads, are 32 workgroups of 98 tiles on 256 units; in 7 shares they are 224 of 14
+// tiles, and a layer (attention and append) takes 146 us instead of 555 (see prefill_splits).
+template <bool BOOST, bool SPLIT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves / 4, kWaves / 4))) void prefill_attn_kernel(
     kitty_kv_layer L, const uint8_t* __restrict__ q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
     const uint8_t* __restrict__ k_new, const uint8_t* __restrict__ v_new, int64_t new_stride_b,
-    int64_t new_stride_h, int64_t new_stride_t, int H_Q, int Tq, float scaling, __half* __restrict__ out) {
+    int64_t new_stride_h, int64_t new_stride_t, int H_Q, int Tq, float scaling, __half* __restrict__ out,
+    float* __restrict__ ws_ml, float* __restrict__ ws_acc, int num_splits) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  __shared__ int32_t s_page_ids[2][2][Prefill<BOOST>::kIdChunk];
+  __shared__ int32_t s_page_ids[2][2][Prefill<BOOST, SPLIT>::kIdChunk];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, kg = lane >> 4, n = lane & 15;
   const int b = blockIdx.z, h = blockIdx.y;
   const int G = H_Q / L.H_KV;
-  const int PB = kRows / G;                              // chunk positions per workgroup
-  const int blk = (int)gridDim.x - 1 - (int)blockIdx.x;   // longest causal extent first
+  const int PB = block_positions(G, Tq);                 // chunk positions per workgroup
+  const int split = SPLIT ? (int)blockIdx.x % num_splits : 0;
+  const int blk = SPLIT ? ((int)gridDim.x - 1 - (int)blockIdx.x) / num_splits
+                        : (int)gridDim.x - 1 - (int)blockIdx.x;   // longest causal extent first
   const int p0 = blk * PB;
 
   const SeqCounts cnt = load_counts(L, b);
-  Prefill<BOOST> P{L, cnt, b, h, tid,
+  Prefill<BOOST, SPLIT> P{L, cnt, b, h, tid,
                    k_new + (int64_t)b * new_stride_b + (int64_t)h * new_stride_h,
                    v_new + (int64_t)b * new_stride_b + (int64_t)h * new_stride_h,
                    new_stride_t, min(Tq, p0 + PB), 0, 0, 0, 0};
@@ -491,6 +517,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
   P.first_body = cnt.sink > 0 ? 1 : 0;
   P.first_chunk = P.first_body + P.n_body;
   P.n_tiles = P.first_chunk + c_div_up(P.kv_chunk, kPage);
+  int t_begin = 0, t_end = P.n_tiles;
+  if (SPLIT) {
+    const int share = c_div_up(P.n_tiles, num_splits);
+    t_begin = min(split * share, P.n_tiles);
+    t_end = min(t_begin + share, P.n_tiles);
+    P.first_id = max(t_begin - P.first_body, 0);
+  }
 
   // this lane's query rows: column n of row tile nt is row 16 kNT w + 16 nt + n
   half8 qreg[4][kNT];
@@ -529,30 +562,33 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
   // packed bytes of tile t+2 are on their way.  The waves of a SIMD take the two jobs in opposite
   // order (waves 0..3 convert first, waves 4..7 multiply first), so that one does vector work
   // while the other keeps the matrix pipe busy.  One barrier per tile.
-  const int nt_ = P.n_tiles;
   const bool convert_first = w < kWaves / 2;
+  const bool has_rows = !SPLIT || 16 * kNT * w < G * PB;   // (tested in full blocks it costs 2 %)
   Stage ga, gb;                       // tile t+1, tile t+2
   P.stage_page_ids(0);
   __syncthreads();
-  TileSrc cur = P.tile(0), nxt = cur, nn = cur;
-  P.issue(cur, ga);
-  P.finish(cur, ga, lds, lds + 2 * kTile);
-  if (nt_ > 1) {
-    nxt = P.tile(1);
-    P.issue(nxt, ga);
+  TileSrc cur, nxt, nn;
+  if (!SPLIT || t_begin < t_end) {    // (the last splits of a short walk are empty)
+    cur = P.tile(t_begin), nxt = cur, nn = cur;
+    P.issue(cur, ga);
+    P.finish(cur, ga, lds, lds + 2 * kTile);
+    if (t_begin + 1 < t_end) {
+      nxt = P.tile(t_begin + 1);
+      P.issue(nxt, ga);
+    }
   }
   __syncthreads();
 #pragma unroll 1
-  for (int t = 0; t < nt_; ++t) {
-    const int buf = t & 1;
-    const bool more = t + 1 < nt_;
-    if (t + 2 < nt_) {
+  for (int t = t_begin; t < t_end; ++t) {
+    const int buf = (t - t_begin) & 1;
+    const bool more = t + 1 < t_end;
+    if (t + 2 < t_end) {
       nn = P.tile(t + 2);
       P.issue(nn, gb);
     }
     {   // half way through a chunk of page ids: stage the next one (tile() is at body tile t + 2 - first_body)
-      const int i = t + 2 - P.first_body;
-      if (i >= 0 && i % Prefill<BOOST>::kIdChunk == Prefill<BOOST>::kIdChunk / 2) P.stage_page_ids(i / Prefill<BOOST>::kIdChunk + 1);
+      const int i = t + 2 - P.first_body - P.id_base();
+      if (i >= 0 && i % Prefill<BOOST, SPLIT>::kIdChunk == Prefill<BOOST, SPLIT>::kIdChunk / 2) P.stage_page_ids(i / Prefill<BOOST, SPLIT>::kIdChunk + 1);
     }
     uint8_t* kn = lds + (buf ^ 1) * kTile;
     uint8_t* vn = lds + (2 + (buf ^ 1)) * kTile;
@@ -562,13 +598,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
     for (int nt = 0; nt < kNT; ++nt)
       limit[nt] = cur.chunk_t0 >= 0 ? min(cur.ntok, qpos[nt] - cur.chunk_t0 + 1) : cur.ntok;
     const bool masked = cur.chunk_t0 >= 0 || cur.ntok < kPage;
-    {
+    if (has_rows) {
       // the lane's corner inside a 16-lane transposing read: row n / 4 of 4, columns 4 (n % 4) ..;
       // made opaque so that every read's offset stays a small immediate on these two bases
       uint32_t ok_ = buf * kTile + (4 * kg + (n >> 2)) * kPitch + (n & 3) * 8;
       uint32_t ov_ = ok_ + 2 * kTile;
       asm volatile("" : "+v"(ok_), "+v"(ov_));
-      const TileAttend T{lds + ok_, lds + ov_, qreg, A, sc2, masked, limit, kg};
+      const TileAttend<SPLIT> T{lds + ok_, lds + ov_, qreg, A, sc2, masked, limit, kg};
       T.run((cur.ntok + 31) >> 5);
     }
     if (more && !convert_first) P.finish(nxt, ga, kn, vn);
@@ -585,9 +621,21 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
     l += xor_lanes(l, 16);
     l += xor_lanes(l, 32);
     if (qpos[nt] < 0) continue;
-    const float inv = 1.f / l;
     const int r = 16 * kNT * w + 16 * nt + n;
     const int g_ = r / PB;
+    if (SPLIT) {
+      const int64_t row = (((int64_t)b * Tq + qpos[nt]) * H_Q + (h * G + g_)) * num_splits + split;
+      if (kg == 0) *(float2*)(ws_ml + row * 2) = float2{l == 0.f ? -INFINITY : A.m[nt], l};   // 0: this row saw nothing here
+      float* arow = ws_acc + row * kD;
+#pragma unroll
+      for (int ct = 0; ct < 8; ++ct) {
+        const float4v o = A.o[ct][nt];
+        *(float2*)(arow + 16 * ct + 2 * kg) = float2{o[0], o[2]};
+        *(float2*)(arow + 16 * ct + 2 * kg + 8) = float2{o[1], o[3]};
+      }
+      continue;
+    }
+    const float inv = 1.f / l;
     __half* orow = out + (((int64_t)b * Tq + qpos[nt]) * H_Q + (h * G + g_)) * kD;
 #pragma unroll
     for (int ct = 0; ct < 8; ++ct) {
@@ -604,26 +652,53 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
 
 int prefill_lds_bytes() { return kLdsBytes; }
 
+// How many shares the walk over the tiles is cut into.  A workgroup has a compute unit to itself, so a launch
+// of W workgroups takes ceil(W / units) rounds of its longest walk; cutting the walk in s shortens the walk
+// and multiplies the workgroups.  What a share costs besides its tiles is about three tiles' time (filling
+// the pipeline, 128 KB of partials); the merge reads 512 bytes a row and share.  A tile takes 5.4 us with all
+// rows in use.  The smallest total wins; ties go to fewer shares.
+// `tiles`: 128-token tiles the layer holds (sink included) plus those of the chunk.
+int prefill_splits(int B, int H_Q, int H_KV, int Tq, int tiles, int units) {
+  const int G = H_Q / H_KV;
+  if ((int64_t)B * Tq > 65535) return 1;   // the merge's grid; such a launch has enough workgroups
+  const int64_t wgs = (int64_t)c_div_up(Tq, block_positions(G, Tq)) * H_KV * B;
+  const float rows = (float)B * (float)Tq * (float)H_Q;
+  int best = 1;
+  float best_us = 0.f;
+  for (int s = 1; s <= 64 && (s == 1 || 2 * s <= tiles); ++s) {
+    const int64_t rounds = (wgs * s + units - 1) / units;
+    float us = 5.4f * (float)rounds * (float)(c_div_up(tiles, s) + 3);
+    if (s > 1) us += 4.f + rows * (float)s * 3.5e-4f;   // write + read of 1 KB at about 3 TB/s
+    if (s == 1 || us < 0.95f * best_us) best = s, best_us = us;
+  }
+  return best;
+}
+
 void launch_prefill_attn(const kitty_kv_layer& L, const void* q, int64_t q_stride_b, int64_t q_stride_h,
                          int64_t q_stride_t, const void* k_new, const void* v_new, int64_t new_stride_b,
                          int64_t new_stride_h, int64_t new_stride_t, int B, int H_Q, int Tq, float scaling,
-                         void* out, hipStream_t stream) {
+                         void* out, float* ws_ml, float* ws_acc, int num_splits, hipStream_t stream) {
   const int G = H_Q / L.H_KV;
-  const int PB = kRows / G;
-  dim3 grid(c_div_up(Tq, PB), L.H_KV, B), block(kThreads);
-#define KITTY_LAUNCH_PREFILL(BOOST)                                                                              \
+  const int blocks = c_div_up(Tq, block_positions(G, Tq));
+  dim3 grid(blocks * num_splits, L.H_KV, B), block(kThreads);
+#define KITTY_LAUNCH_PREFILL(BOOST, SPLIT)                                                                       \
   do {                                                                                                           \
     /* more LDS than the default per-workgroup limit; per device, so set on every launch */                      \
-    (void)hipFuncSetAttribute((const void*)prefill_attn_kernel<BOOST>,                                           \
+    (void)hipFuncSetAttribute((const void*)prefill_attn_kernel<BOOST, SPLIT>,                                    \
                               hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);                            \
-    hipLaunchKernelGGL((prefill_attn_kernel<BOOST>), grid, block, kLdsBytes, stream, L, (const uint8_t*)q,       \
+    hipLaunchKernelGGL((prefill_attn_kernel<BOOST, SPLIT>), grid, block, kLdsBytes, stream, L, (const uint8_t*)q, \
                        q_stride_b, q_stride_h, q_stride_t, (const uint8_t*)k_new, (const uint8_t*)v_new,         \
-                       new_stride_b, new_stride_h, new_stride_t, H_Q, Tq, scaling, (__half*)out);                \
+                       new_stride_b, new_stride_h, new_stride_t, H_Q, Tq, scaling, (__half*)out, ws_ml, ws_acc,  \
+                       num_splits);                                                                              \
   } while (0)
-  if (L.D_BOOSTED > 0)
-    KITTY_LAUNCH_PREFILL(true);
-  else
-    KITTY_LAUNCH_PREFILL(false);
+  if (num_splits > 1) {
+    if (L.D_BOOSTED > 0) KITTY_LAUNCH_PREFILL(true, true);
+    else KITTY_LAUNCH_PREFILL(false, true);
+    launch_rows_merge(kD, ws_ml, ws_acc, out, (int64_t)B * Tq * H_Q, num_splits, /* keep_nan */ true, stream);
+  } else {
+    if (L.D_BOOSTED > 0) KITTY_LAUNCH_PREFILL(true, false);
+    else KITTY_LAUNCH_PREFILL(false, false);
+  }
 #undef KITTY_LAUNCH_PREFILL
 }
 

@@ -28,6 +28,14 @@ def _split_plan(B: int, H_Q: int, H_KV: int, D: int, max_tiles: int, per_sequenc
     return num_splits, lib.kitty_decode_attn_workspace_bytes(B, H_Q, D, num_splits)
 
 
+@functools.lru_cache(maxsize=4096)
+def _chunk_split_plan(B: int, H_Q: int, H_KV: int, D: int, T_q: int, max_tiles: int):
+    """(splits, workspace bytes) of a chunked-prefill launch: a function of the sizes alone."""
+    lib = _lib.lib()
+    num_splits = lib.kitty_prefill_attn_default_splits(B, H_Q, H_KV, D, T_q, max_tiles)
+    return num_splits, lib.kitty_prefill_attn_workspace_bytes(B, H_Q, D, T_q, num_splits)
+
+
 def kitty_attention_forward(
     module: nn.Module,
     query: torch.Tensor,
@@ -106,12 +114,17 @@ def kitty_prefill_attention(
         value_states = value_states.contiguous()
         key_states = key_states.contiguous()
 
-    lib = _lib.lib()
-    attn_output = torch.empty((B, T_q, H_Q, D), dtype=query.dtype, device=query.device)
-    desc = kv_cache.descriptor()
+    attn_output = query.new_empty((B, T_q, H_Q, D))
+    # tiles of the longest sequence (with counters on the device the host ints shadow it; any number of shares is right)
+    max_tiles = 1 + kv_cache.PageCount_K + (kv_cache.Q_Buffer_Count_K > 0)
+    num_splits, ws_bytes = _chunk_split_plan(B, H_Q, H_KV, D, T_q, max_tiles)
+    # scratch of this call alone (tens of MB at most): torch's allocator hands the same block to the next layer
+    ws = query.new_empty(ws_bytes, dtype=torch.uint8) if num_splits > 1 else None
     qs, ks = [x * 2 for x in query.stride()], [x * 2 for x in key_states.stride()]
-    rc = lib.kitty_prefill_attn(desc, query.data_ptr(), qs[0], qs[1], qs[2], key_states.data_ptr(),
-                                value_states.data_ptr(), ks[0], ks[1], ks[2], B, H_Q, T_q, float(scaling),
-                                attn_output.data_ptr(), _lib.current_stream_ptr(query.device))
+    rc = _lib.lib().kitty_prefill_attn_split(kv_cache.descriptor(), query.data_ptr(), qs[0], qs[1], qs[2],
+                                             key_states.data_ptr(), value_states.data_ptr(), ks[0], ks[1], ks[2], B, H_Q,
+                                             T_q, float(scaling), attn_output.data_ptr(),
+                                             None if ws is None else ws.data_ptr(), ws_bytes, num_splits,
+                                             _lib.current_stream_ptr(query.device))
     _lib.check(rc, "kitty_prefill_attention")
     return attn_output, None
