@@ -161,7 +161,7 @@ int kitty_quant_pack_v(const void* value, int64_t stride_b, int64_t stride_h, in
  * num_splits <= 0 picks kitty_decode_attn_default_splits() (max_tiles = 1 + the 128-token tiles
  * after the sink of the longest sequence; per_sequence_counts = layer->seq_counts is set).
  * variant: 0 = default kernel, 1 = the plain reference-order kernel (fp16 dequantization, no
- * matrix cores).  For D = 64 / 256 both values run the same plain kernel.
+ * matrix cores).  For D = 64 / 256 both values run the same kernel, in the reference's order.
  */
 size_t kitty_decode_attn_workspace_bytes(int B, int H_Q, int D, int num_splits);
 int kitty_decode_attn_default_splits(int B, int H_KV, int max_tiles, int per_sequence_counts);

@@ -2,15 +2,14 @@
 //
 // The reference takes the head dimension from the model's config and promotes a quarter of the key
 // channels (kitty.py:39-44); its kernels take D as a parameter (kitty_quant_pack.py:42-45, 180-181;
-// kitty_attention.py:59-62, 253-254).  The tuned kernels of this library are written for D = 128, the
+// kitty_attention.py:59-62, 253-254).  The other kernels of this library are written for D = 128, the
 // size of every model the reference names.  The kernels here cover the other sizes with the same
-// arithmetic and the same storage format - plain vector-ALU code, one template parameter for D:
+// arithmetic and the same storage format, one template parameter for D:
 //
-//   quant_k_any_kernel / quant_v_any_kernel   quantize-and-pack, boost selection fused or given
-//   attn_any_kernel<D, false, ROWS>           decode attention, split pass (the reference's order of
-//                                             operations: fp16 dequantization with both roundings)
-//   attn_any_kernel<D, true, 16>              chunked-prefill attention, one pass
-//   merge_any_kernel                          the merge pass of split-K
+//   quant_k_any_kernel / quant_v_any_kernel   quantize-and-pack, boost selection fused or given (vector ALUs)
+//   attn_any_kernel<D, false, 1>              decode attention, split pass (the reference's order of
+//                                             operations: fp16 dequantization with both roundings; matrix cores)
+//   attn_any_kernel<D, true, NT>              chunked-prefill attention, in one pass or in shares
 //
 // Wire format for general D (PAGE = 128 tokens): a K page-head is 32 D bytes of low plane (channel d at
 // 32 d), 32 d_boost bytes of high plane (slot s at 32 (D + s)) and D bytes of slot map; a V page-head is
@@ -19,9 +18,13 @@
 #include "quant_arith.h"
 
 namespace kitty {
+// merge pass over independent rows (rows_merge.hip)
+void launch_rows_merge(int D, const float* ws_ml, const float* ws_acc, void* out, int64_t rows, int num_splits,
+                       bool keep_nan, hipStream_t stream);
 namespace {
 
-constexpr int kMaxRows = 16;   // query rows per workgroup at most: the group's heads (decode), heads x positions (prefill)
+// column tiles of 16 query rows per workgroup in chunked prefill: as many as the output's accumulators leave room for
+constexpr int kPrefillTiles64 = 4, kPrefillTiles256 = 2;
 
 // ---------------------------------------------------------------------------------------------
 // quantize and pack
@@ -165,241 +168,440 @@ __global__ __launch_bounds__(128) void quant_v_any_kernel(
 // ---------------------------------------------------------------------------------------------
 // attention
 // ---------------------------------------------------------------------------------------------
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef float float4v __attribute__((ext_vector_type(4)));
+typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
+typedef short short4v __attribute__((ext_vector_type(4)));
+
+constexpr float kLog2e = 1.44269504088896340736f;
+constexpr uint32_t kCodeMask = 0x00030003u;    // the lowest code of both 16-bit pieces of a word
+constexpr uint32_t kCodeMagic = 0x64006400u;   // fp16 1024 in both halves: 1024 + code is exact
+constexpr float kProbScale = 4096.f;           // probabilities as matrix operands: see below
+
+__device__ __forceinline__ float4v mfma16(const uint32_t (&a)[4], const uint32_t (&b)[4], float4v c) {
+  const uint4v av = {a[0], a[1], a[2], a[3]}, bv = {b[0], b[1], b[2], b[3]};
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, av), __builtin_bit_cast(half8, bv), c, 0, 0, 0);
+}
+// Transposing LDS read: lane i of a 16-lane block receives 16-bit piece i of the four 32-byte rows whose
+// 8-byte quarters lanes 4r .. 4r+3 address; r0 = (row 0, row 1), r1 = (row 2, row 3).
+__device__ __forceinline__ void lds_tr(const uint8_t* p, uint32_t& r0, uint32_t& r1) {
+  const short4v v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((short4v __attribute__((address_space(3)))*)p);
+  const uint2 u = __builtin_bit_cast(uint2, v);
+  r0 = u.x;
+  r1 = u.y;
+}
+__device__ __forceinline__ float4v mfma16(const uint32_t (&a)[4], const uint4& b, float4v c) {
+  const uint32_t bb[4] = {b.x, b.y, b.z, b.w};
+  return mfma16(a, bb, c);
+}
+__device__ __forceinline__ uint32_t low_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x05040100u); }
+__device__ __forceinline__ uint32_t high_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
 // fp16(code) * scale + zero with BOTH operations rounded to fp16 (kitty_attention.py:162-165, 317-320 as
-// eager torch and the Triton interpreter evaluate them).
-__device__ inline float dequant_two(uint32_t code, __half scale, __half zero) {
+// eager torch and the Triton interpreter evaluate them), for the two codes of a word that has kCodeMagic set.
+__device__ __forceinline__ uint32_t dequant_word(uint32_t c, uint32_t scale, uint32_t zero) {
 #pragma clang fp contract(off)
-  const _Float16 s = static_cast<__half_raw>(scale).data;
-  const _Float16 z = static_cast<__half_raw>(zero).data;
-  const _Float16 c = (_Float16)(float)code;
-  const _Float16 prod = c * s;
-  const _Float16 r = prod + z;
-  return (float)r;
+  const half2v f = __builtin_bit_cast(half2v, c) - half2v{(_Float16)1024.f, (_Float16)1024.f};
+  const half2v m = f * __builtin_bit_cast(half2v, scale);
+  const half2v r = m + __builtin_bit_cast(half2v, zero);
+  return __builtin_bit_cast(uint32_t, r);
+}
+// maximum over lanes l, l^16, l^32, l^48
+__device__ __forceinline__ float max_over_lane_groups(float v) {
+  const unsigned b = __builtin_bit_cast(unsigned, v);
+  const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+  const unsigned r0 = r[0], r1 = r[1];   // as scalars first: a bit_cast of r[1] itself reads element 0
+  const float m = fmaxf(__builtin_bit_cast(float, r0), __builtin_bit_cast(float, r1));
+  const unsigned c = __builtin_bit_cast(unsigned, m);
+  const auto q = __builtin_amdgcn_permlane32_swap(c, c, false, false);
+  const unsigned q0 = q[0], q1 = q[1];
+  return fmaxf(__builtin_bit_cast(float, q0), __builtin_bit_cast(float, q1));
 }
 
-// Up to 16 query rows of one (batch row, kv head) against a range of 128-token tiles.
+// LDS of one workgroup: the packed bytes of a tile as they lie in memory, or (at the end) one round of the
+// sum over the wavefronts.
+struct AnyLds {
+  int zero_row, k_meta, v_raw, v_meta, bytes;
+  __host__ __device__ AnyLds(int D, int DB) {
+    zero_row = k_head_bytes_d(D, DB);          // 32 zero bytes: the high-plane row of a channel that has none
+    k_meta = zero_row + kRowBytes;
+    v_raw = k_meta + 4 * D;
+    v_meta = v_raw + v_head_bytes_d(D);
+    bytes = v_meta + 4 * kPage;
+    if (bytes < 16384) bytes = 16384;
+  }
+  // with the operands of NT column tiles of query rows
+  int with_q(int D, int NT) const { return bytes + D / 32 * NT * 1024; }
+};
+
+// 16 NT query rows of one (batch row, kv head) against a range of 128-token tiles, on the matrix cores.
 // Decode (PREFILL false): grid (splits, H_KV, B); the rows are the G heads of the group; the partial
 // (running max in log2 units, running sum, un-normalised output) goes to the split-K workspace.
-// Prefill: grid (blocks of 16 / G chunk positions, H_KV, B); row r is head r / PB at chunk position
-// p0 + r % PB; after the layer's own tiles come the chunk's rows, causally; the normalised output
-// goes to out [B, T_q, H_Q, D].
-// Logits: thread = (token, half of the channels).  Output: thread = (channel, 1 / (256 / D) of the tile's
-// tokens).  Logits and probabilities stay fp32.
-template <int D, bool PREFILL, int ROWS>
-__global__ __launch_bounds__(256) void attn_any_kernel(
+// Prefill: grid (blocks of 16 NT / G chunk positions x splits, H_KV, B); row r is head r / PB at chunk position
+// p0 + r % PB; after the layer's own tiles come the chunk's rows, causally; the normalised output goes to
+// out [B, T_q, H_Q, D], or with ws_ml set a partial per row to the workspace.
+//
+// What bounds it is turning codes into fp16 numbers with the reference's two roundings: 8 vector instructions
+// per two key codes, 5 per two value codes, once per code.  So every code is unpacked in the register in which the
+// matrix instruction takes it, by one lane of one wavefront: the packed bytes of a tile go to LDS as they
+// are (loaded into registers while the tile before is worked on), a transposing read hands lane n the 8 codes
+// 8n .. 8n+7 of several plane rows, and `(X >> 2u) & mask` is then one register of the operand of
+//   S^T[token 8n + u][row] = sum_ch  K[token][ch] * Q[row][ch]           (A = K, B = Q in registers)
+//   O^T[ch 8n + u][row]    = sum_tok V[tok][ch]   * P^T[tok][row]        (A = V, B = P)
+// Wavefront w owns tokens 8i + 2w and 8i + 2w + 1 of every tile, with a running maximum, a sum and an output of its
+// own: its accumulator of the first product holds, lane for lane, the B operand of the second (lane group kg:
+// tokens 32kg + 8j + 2w, + 1), and the wavefronts meet only where a tile is staged and once at the end.
+// fp16 rows (sink, windows, the chunk) are loaded from memory in operand order.
+// Probabilities stay fp32 numbers: 4096 p is split into two fp16 numbers (22 bits; a remainder below fp16's
+// normal range is below 2^-26 of the row's largest probability), each a matrix operand of its own.
+// A decode layer (append, this kernel, merge) on MI355X, against the version on the vector ALUs before it:
+//   D = 64,  B = 8, 6100 tokens, 32 / 8 heads:  79 -> 31 us
+//   D = 256, B = 2, 9000 tokens, 16 / 8 heads: 194 -> 36 us
+template <int D, bool PREFILL, int NT>
+__global__ __launch_bounds__(256, PREFILL ? 1 : 2) void attn_any_kernel(
     kitty_kv_layer L, const uint8_t* __restrict__ q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
     const uint8_t* __restrict__ k_new, const uint8_t* __restrict__ v_new, int64_t new_stride_b,
     int64_t new_stride_h, int64_t new_stride_t, int H_Q, int Tq, float scaling, float* __restrict__ ws_ml,
     float* __restrict__ ws_acc, int num_splits, __half* __restrict__ out) {
-  constexpr int kParts = 256 / D;   // token parts of the output phase
-  constexpr int kPartTok = kPage / kParts;
-  static_assert(D == 64 || D == 128 || D == 256, "head dimensions with a whole number of token parts");
+  static_assert(D == 64 || D == 256, "128 has kernels of its own");
+  constexpr int kHalves = D == 256 ? 2 : 1;      // V rows in pieces of 128 channels
+  constexpr int kU = D == 256 ? 8 : 4;           // channels of a lane within a piece
+  constexpr int kOT = kHalves * kU;              // 16-channel tiles of the output
+  constexpr int kRows = 16 * NT;
+  constexpr int kKIter = (kRowBytes * 2 * D + D) / 16 / 256 + 1;
+  constexpr int kVIter = (D + 127) / 128;
   const int h = blockIdx.y, b = blockIdx.z;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, kg = lane >> 4, n = lane & 15;
   const int G = H_Q / L.H_KV;
   const int DB = L.D_BOOSTED;
   const SeqCounts c = load_counts(L, b);
-  const int PB = PREFILL ? max(1, ROWS / G) : 1;
-  const int R = PREFILL ? G * PB : G;
-  const int p0 = PREFILL ? (int)blockIdx.x * PB : 0;
+  const int PB = PREFILL ? max(1, kRows / G) : 1;
+  const int split = PREFILL ? (int)blockIdx.x % num_splits : (int)blockIdx.x;
+  const int p0 = PREFILL ? ((int)blockIdx.x / num_splits) * PB : 0;
   const int kv_chunk = PREFILL ? min(Tq, p0 + PB) : 0;           // chunk tokens this workgroup can see
   const int n_tiles = c.ntiles + (kv_chunk + kPage - 1) / kPage;
-  int tile_begin = 0, tile_end = n_tiles;
-  if (!PREFILL) {
-    const int per = (c.ntiles + num_splits - 1) / num_splits;
-    tile_begin = (int)blockIdx.x * per;
-    tile_end = min(c.ntiles, tile_begin + per);
-  }
+  const int share = (n_tiles + num_splits - 1) / num_splits;
+  const int tile_begin = min(split * share, n_tiles), tile_end = min(n_tiles, tile_begin + share);
   int bad_page = 0;
 
-  __shared__ __attribute__((aligned(16))) float s_q[D][ROWS];        // [channel][row]: a thread reads the rows of a channel at once
-  __shared__ __attribute__((aligned(16))) uint8_t s_codes[kRowBytes * 2 * D + D];   // a K page-head with d_boost up to D
-  __shared__ __half2 s_meta[D > kPage ? D : kPage];
-  __shared__ __attribute__((aligned(16))) float s_p[kPage][ROWS];    // [token][row]
-  __shared__ union {
-    float part[2][ROWS][kPage];        // logits: [half of the channels][row][token]
-    float o[kParts][ROWS][D];          // the output's partial sums at the end
-  } s_u;
-  __shared__ float s_m[ROWS], s_l[ROWS], s_alpha[ROWS];
-  __shared__ int s_pos[ROWS];          // prefill: chunk position of a row, -1 = no such row
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  __shared__ float s_m[4][kRows], s_l[4][kRows];
+  const AnyLds at(D, DB);
+  if (tid < 2) ((uint4*)(lds + at.zero_row))[tid] = uint4{0u, 0u, 0u, 0u};
 
-  if (tid < ROWS) {
-    s_m[tid] = -INFINITY;
-    s_l[tid] = 0.f;
-    int pos = 0;
-    if (PREFILL) pos = (tid < R && p0 + tid % PB < Tq) ? p0 + tid % PB : -1;
-    s_pos[tid] = pos;
-  }
-  for (int i = tid; i < R * D; i += 256) {
-    const int r = i / D, d = i % D;
-    const int g = PREFILL ? r / PB : r, pos = PREFILL ? min(p0 + r % PB, Tq - 1) : 0;
-    const uint8_t* row = q + (int64_t)b * q_stride_b + (int64_t)(h * G + g) * q_stride_h + (int64_t)pos * q_stride_t;
-    s_q[d][r] = __half2float(((const __half*)row)[d]);
-  }
-  float acc_o[ROWS];
+  // the query rows as operands, one copy in LDS for the four wavefronts (16 bytes a lane): k-slots 0..3 of chunk kc
+  // are channels 32 kc + 4 kg .., 4..7 those 16 further
+  uint4* const s_q = (uint4*)(lds + at.bytes);   // [D / 32][NT][64 lanes]
+  int qpos[NT], qhead[NT];   // chunk position (decode: 0), -1 = no such row; head within the group
 #pragma unroll
-  for (int g = 0; g < ROWS; ++g) acc_o[g] = 0.f;
-  __syncthreads();
+  for (int nt = 0; nt < NT; ++nt) {
+    const int r = 16 * nt + n, g = r / PB, pos = p0 + r % PB;
+    const bool ok = g < G && pos < (PREFILL ? Tq : 1);
+    qpos[nt] = ok ? pos : -1;
+    qhead[nt] = g;
+    const uint8_t* row = q + (int64_t)b * q_stride_b + (int64_t)(h * G + (ok ? g : 0)) * q_stride_h +
+                         (int64_t)(ok ? pos : 0) * q_stride_t;
+#pragma unroll
+    for (int kc = w; kc < D / 32; kc += 4) {
+      const uint2 x0 = *(const uint2*)(row + (32 * kc + 4 * kg) * 2);
+      const uint2 x1 = *(const uint2*)(row + (32 * kc + 16 + 4 * kg) * 2);
+      s_q[(kc * NT + nt) * 64 + lane] = ok ? uint4{x0.x, x0.y, x1.x, x1.y} : uint4{0u, 0u, 0u, 0u};
+    }
+  }
 
-  const int t = tid & 127, half = tid >> 7;
-  const int od = tid % D, opart = tid / D;
+  float4v O[kOT][NT];
+  float m_run[NT], l_run[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    m_run[nt] = -INFINITY, l_run[nt] = 0.f;
+#pragma unroll
+    for (int t = 0; t < kOT; ++t) O[t][nt] = float4v{0.f, 0.f, 0.f, 0.f};
+  }
+  const float sc2 = scaling * kLog2e;
   const int64_t sink_base = (int64_t)b * L.sink_stride_b + (int64_t)h * L.sink_stride_h;
   const int64_t win_base = (int64_t)b * L.win_stride_b + (int64_t)h * L.win_stride_h;
-  const uint8_t* kc = PREFILL ? k_new + (int64_t)b * new_stride_b + (int64_t)h * new_stride_h : nullptr;
-  const uint8_t* vc = PREFILL ? v_new + (int64_t)b * new_stride_b + (int64_t)h * new_stride_h : nullptr;
+  const int k_words = k_head_bytes_d(D, DB) / 16;
 
+  // the packed bytes of a tile on their way to LDS
+  uint4v pk[kKIter] = {}, pv[kVIter] = {}, pm = {};
+  auto k_is_packed = [&](int tile) { return tile > 0 && tile < c.ntiles && tile - 1 < c.pk; };
+  auto v_is_packed = [&](int tile) { return tile > 0 && tile < c.ntiles && tile - 1 < c.pv; };
+  auto fetch = [&](int tile) {
+    if (k_is_packed(tile)) {
+      const int64_t pg = checked_page(page_id(L.page_table_k, (int64_t)b * L.page_table_k_stride_b + tile - 1), L.cache_pages_k, bad_page);
+      const uint4v* src = (const uint4v*)(L.key_cache + pg * L.key_cache_stride_page + (int64_t)h * k_head_bytes_d(D, DB));
+#pragma unroll
+      for (int i = 0; i < kKIter; ++i)
+        if (i * 256 + tid < k_words) pk[i] = src[i * 256 + tid];
+      if (tid < D / 4)
+        pm = ((const uint4v*)((const uint8_t*)L.key_meta + pg * L.key_meta_stride_page + (int64_t)h * D * 4))[tid];
+    }
+    if (v_is_packed(tile)) {
+      const int64_t pg = checked_page(page_id(L.page_table_v, (int64_t)b * L.page_table_v_stride_b + tile - 1), L.cache_pages_v, bad_page);
+      const uint4v* src = (const uint4v*)(L.value_cache + pg * L.value_cache_stride_page + (int64_t)h * v_head_bytes_d(D));
+#pragma unroll
+      for (int i = 0; i < kVIter; ++i)
+        if (i * 256 + tid < 2 * D) pv[i] = src[i * 256 + tid];
+      if (tid >= 64 && tid < 96)
+        pm = ((const uint4v*)((const uint8_t*)L.value_meta + pg * L.value_meta_stride_page + (int64_t)h * kPage * 4))[tid - 64];
+    }
+  };
+  auto stage = [&](int tile) {
+    if (k_is_packed(tile)) {
+#pragma unroll
+      for (int i = 0; i < kKIter; ++i)
+        if (i * 256 + tid < k_words) ((uint4v*)lds)[i * 256 + tid] = pk[i];
+      if (tid < D / 4) ((uint4v*)(lds + at.k_meta))[tid] = pm;
+    }
+    if (v_is_packed(tile)) {
+#pragma unroll
+      for (int i = 0; i < kVIter; ++i)
+        if (i * 256 + tid < 2 * D) ((uint4v*)(lds + at.v_raw))[i * 256 + tid] = pv[i];
+      if (tid >= 64 && tid < 96) ((uint4v*)(lds + at.v_meta))[tid - 64] = pm;
+    }
+  };
+
+  if (tile_begin < tile_end) fetch(tile_begin);
+#pragma unroll 1
   for (int tile = tile_begin; tile < tile_end; ++tile) {
     const bool chunk = tile >= c.ntiles;                       // a tile of the new chunk (prefill only)
     const int chunk_t0 = chunk ? (tile - c.ntiles) * kPage : 0;
     const int body = tile - 1;                                  // -1 = sink
     const int ntok = chunk ? min(kPage, kv_chunk - chunk_t0) : tile == 0 ? c.sink : min(kPage, c.nbody - body * kPage);
-    const bool k_packed = !chunk && tile > 0 && body < c.pk;
-    const bool v_packed = !chunk && tile > 0 && body < c.pv;
+    const bool k_packed = k_is_packed(tile), v_packed = v_is_packed(tile);
+    __syncthreads();   // everyone is done with the tile before
+    stage(tile);
+    __syncthreads();
+    if (tile + 1 < tile_end) fetch(tile + 1);
+    if (ntok <= 0) continue;   // an empty sink
 
-    // ---- logits -----------------------------------------------------------------------------
-    float acc[ROWS];
+    // ---- logits of tokens 8i + 2w + e: S[e][nt][j] is token 32 kg + 8 j + 2 w + e, row 16 nt + n -------------------
+    float4v S[2][NT];
 #pragma unroll
-    for (int g = 0; g < ROWS; ++g) acc[g] = 0.f;
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) S[e][nt] = float4v{0.f, 0.f, 0.f, 0.f};
     if (k_packed) {
-      const int64_t pg = checked_page(page_id(L.page_table_k, (int64_t)b * L.page_table_k_stride_b + body), L.cache_pages_k, bad_page);
-      const uint8_t* src = L.key_cache + pg * L.key_cache_stride_page + (int64_t)h * k_head_bytes_d(D, DB);
-      for (int i = tid; i < k_head_bytes_d(D, DB) / 16; i += 256) ((uint4*)s_codes)[i] = ((const uint4*)src)[i];
-      if (tid < D)
-        s_meta[tid] = *(const __half2*)((const uint8_t*)L.key_meta + pg * L.key_meta_stride_page +
-                                        ((int64_t)h * D + tid) * 4);
-      __syncthreads();
-      const int sh = 2 * (t & 3);
-      const uint8_t* idx = s_codes + kRowBytes * (D + DB);
-      for (int d = half * (D / 2); d < (half + 1) * (D / 2); ++d) {
-        uint32_t code = (s_codes[d * kRowBytes + (t >> 2)] >> sh) & 3u;
-        const uint32_t slot = idx[d];
-        if (slot < (uint32_t)DB) code |= ((s_codes[(D + slot) * kRowBytes + (t >> 2)] >> sh) & 3u) << 2;
-        const __half2 m = s_meta[d];
-        const float x = dequant_two(code, __low2half(m), __high2half(m));
+      const int sh = 4 * w;
+      const uint8_t* idx = lds + kRowBytes * (D + DB);
+      const int quarter = (n & 3) * 8;
+#pragma unroll 2
+      for (int kc = 0; kc < D / 32; ++kc) {
+        const int r0 = 32 * kc + 4 * kg, mine = r0 + (n >> 2);
+        uint32_t X[4], H[4], sc[4], zr[4];
+        lds_tr(lds + mine * kRowBytes + quarter, X[0], X[1]);
+        lds_tr(lds + (mine + 16) * kRowBytes + quarter, X[2], X[3]);
+        const int s0 = idx[mine], s1 = idx[mine + 16];
+        lds_tr(lds + (s0 < DB ? (D + s0) * kRowBytes : at.zero_row) + quarter, H[0], H[1]);
+        lds_tr(lds + (s1 < DB ? (D + s1) * kRowBytes : at.zero_row) + quarter, H[2], H[3]);
+        const uint4 m0 = *(const uint4*)(lds + at.k_meta + r0 * 4), m1 = *(const uint4*)(lds + at.k_meta + (r0 + 16) * 4);
+        sc[0] = low_halves(m0.x, m0.y), zr[0] = high_halves(m0.x, m0.y);
+        sc[1] = low_halves(m0.z, m0.w), zr[1] = high_halves(m0.z, m0.w);
+        sc[2] = low_halves(m1.x, m1.y), zr[2] = high_halves(m1.x, m1.y);
+        sc[3] = low_halves(m1.z, m1.w), zr[3] = high_halves(m1.z, m1.w);
+        uint4 qq[NT];
 #pragma unroll
-        for (int g = 0; g < ROWS; ++g)
-          if (g < R) acc[g] += s_q[d][g] * x;
+        for (int nt = 0; nt < NT; ++nt) qq[nt] = s_q[(kc * NT + nt) * 64 + lane];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          uint32_t a[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const uint32_t lo = ((X[i] >> (sh + 2 * e)) & kCodeMask) | kCodeMagic;
+            const uint32_t hi = (H[i] >> (sh + 2 * e)) & kCodeMask;
+            a[i] = dequant_word((hi << 2) | lo, sc[i], zr[i]);
+          }
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) S[e][nt] = mfma16(a, qq[nt], S[e][nt]);
+        }
       }
-    } else if (t < ntok) {
-      const __half* row = chunk      ? (const __half*)(kc + (int64_t)(chunk_t0 + t) * new_stride_t)
-                          : tile == 0 ? (const __half*)((const uint8_t*)L.sink_k + sink_base) + (int64_t)t * D
-                                      : (const __half*)((const uint8_t*)L.qbuf_k + win_base) + (int64_t)t * D;
-      for (int d = half * (D / 2); d < (half + 1) * (D / 2); ++d) {
-        const float x = __half2float(row[d]);
+    } else {
+      const uint8_t* base = chunk ? k_new + (int64_t)b * new_stride_b + (int64_t)h * new_stride_h + (int64_t)chunk_t0 * new_stride_t
+                          : tile == 0 ? (const uint8_t*)L.sink_k + sink_base : (const uint8_t*)L.qbuf_k + win_base;
+      const int64_t stride = chunk ? new_stride_t : (int64_t)(2 * D);
 #pragma unroll
-        for (int g = 0; g < ROWS; ++g)
-          if (g < R) acc[g] += s_q[d][g] * x;
+      for (int e = 0; e < 2; ++e) {
+        // a token past the end repeats the last one: its logits are masked below
+        const uint8_t* row = base + (int64_t)min(8 * n + 2 * w + e, ntok - 1) * stride;
+#pragma unroll 4
+        for (int kc = 0; kc < D / 32; ++kc) {
+          const uint2 x0 = *(const uint2*)(row + (32 * kc + 4 * kg) * 2);
+          const uint2 x1 = *(const uint2*)(row + (32 * kc + 16 + 4 * kg) * 2);
+          const uint32_t a[4] = {x0.x, x0.y, x1.x, x1.y};
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) S[e][nt] = mfma16(a, s_q[(kc * NT + nt) * 64 + lane], S[e][nt]);
+        }
       }
     }
-#pragma unroll
-    for (int g = 0; g < ROWS; ++g)
-      if (g < R) s_u.part[half][g][t] = acc[g];
-    __syncthreads();
 
-    // ---- online softmax: one wave per query row ------------------------------------------------
-    for (int g = wave; g < R; g += 4) {
-      // tokens of the tile this row sees: all of them, or (the chunk's own tiles) those up to its position
-      int lim = ntok;
-      if (PREFILL) lim = s_pos[g] < 0 ? 0 : chunk ? min(ntok, s_pos[g] - chunk_t0 + 1) : ntok;
-      float v0 = -INFINITY, v1 = -INFINITY;
-      if (lane < lim) v0 = (s_u.part[0][g][lane] + s_u.part[1][g][lane]) * scaling;
-      if (lane + 64 < lim) v1 = (s_u.part[0][g][lane + 64] + s_u.part[1][g][lane + 64]) * scaling;
-      float mxv = fmaxf(v0, v1);
+    // ---- online softmax of this wavefront's tokens ----------------------------------------------
+    uint32_t ph[NT][4], pl[NT][4];
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1) mxv = fmaxf(mxv, __shfl_xor(mxv, o));
-      const float m_old = s_m[g];
-      const float m_new = fmaxf(m_old, mxv);
-      const float p0v = (v0 == -INFINITY) ? 0.f : __expf(v0 - m_new);
-      const float p1v = (v1 == -INFINITY) ? 0.f : __expf(v1 - m_new);
-      float sum = p0v + p1v;
+    for (int nt = 0; nt < NT; ++nt) {
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
-      const float alpha = (m_old == -INFINITY) ? 0.f : __expf(m_old - m_new);
-      s_p[lane][g] = p0v;
-      s_p[lane + 64][g] = p1v;
-      if (lane == 0) { s_m[g] = m_new; s_l[g] = s_l[g] * alpha + sum; s_alpha[g] = alpha; }
+      for (int e = 0; e < 2; ++e) S[e][nt] *= sc2;
+      if (chunk || ntok < kPage) {
+        // tokens of the tile this row sees: all of them, or (the chunk's own tiles) those up to its position
+        const int lim = chunk ? min(ntok, qpos[nt] - chunk_t0 + 1) : ntok;
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (32 * kg + 8 * j + 2 * w + e >= lim) S[e][nt][j] = -INFINITY;
+      }
+      float mx = fmaxf(fmaxf(fmaxf(S[0][nt][0], S[0][nt][1]), fmaxf(S[0][nt][2], S[0][nt][3])),
+                       fmaxf(fmaxf(S[1][nt][0], S[1][nt][1]), fmaxf(S[1][nt][2], S[1][nt][3])));
+      mx = max_over_lane_groups(mx);
+      const float m_old = m_run[nt], m_new = fmaxf(m_old, mx);
+      if (__any(m_new > m_old)) {
+        const float alpha = m_old == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_old - m_new);
+        l_run[nt] *= alpha;
+#pragma unroll
+        for (int t = 0; t < kOT; ++t) O[t][nt] *= alpha;
+        m_run[nt] = m_new;
+      }
+      const float ref = m_run[nt] == -INFINITY ? 0.f : m_run[nt];
+      float sum = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float p0v = __builtin_amdgcn_exp2f(S[0][nt][j] - ref), p1v = __builtin_amdgcn_exp2f(S[1][nt][j] - ref);
+        sum += p0v + p1v;
+        const float x0 = p0v * kProbScale, x1 = p1v * kProbScale;
+        const half2v hi = {(_Float16)x0, (_Float16)x1};
+        const half2v lo = {(_Float16)(x0 - (float)hi[0]), (_Float16)(x1 - (float)hi[1])};
+        ph[nt][j] = __builtin_bit_cast(uint32_t, hi);
+        pl[nt][j] = __builtin_bit_cast(uint32_t, lo);
+      }
+      l_run[nt] += sum;
     }
-    // ---- stage V ---------------------------------------------------------------------------
+
+    // ---- O += P V over the same tokens ------------------------------------------------------------
+    const int t0 = 32 * kg + 2 * w;   // register j of an operand: tokens t0 + 8 j, t0 + 8 j + 1
     if (v_packed) {
-      const int64_t pg = checked_page(page_id(L.page_table_v, (int64_t)b * L.page_table_v_stride_b + body), L.cache_pages_v, bad_page);
-      const uint8_t* src = L.value_cache + pg * L.value_cache_stride_page + (int64_t)h * v_head_bytes_d(D);
-      for (int i = tid; i < v_head_bytes_d(D) / 16; i += 256) ((uint4*)s_codes)[i] = ((const uint4*)src)[i];
-      if (tid < kPage)
-        s_meta[tid] = *(const __half2*)((const uint8_t*)L.value_meta + pg * L.value_meta_stride_page +
-                                        ((int64_t)h * kPage + tid) * 4);
-    }
-    __syncthreads();
-
-    // ---- out += P V : thread = (channel, part of the tile's tokens) ---------------------------
-    {
+      uint32_t sc[4], zr[4];
 #pragma unroll
-      for (int g = 0; g < ROWS; ++g)
-        if (g < R) acc_o[g] *= s_alpha[g];
-      const int t0 = opart * kPartTok, t1 = min(ntok, (opart + 1) * kPartTok);
-      for (int tt = t0; tt < t1; ++tt) {
-        float x;
-        if (v_packed) {
-          const uint32_t code = (s_codes[tt * (D / 4) + (od >> 2)] >> (2 * (od & 3))) & 3u;
-          const __half2 m = s_meta[tt];
-          x = dequant_two(code, __low2half(m), __high2half(m));
-        } else if (chunk) {
-          x = __half2float(((const __half*)(vc + (int64_t)(chunk_t0 + tt) * new_stride_t))[od]);
-        } else if (tile == 0) {
-          x = __half2float(((const __half*)((const uint8_t*)L.sink_v + sink_base))[(int64_t)tt * D + od]);
-        } else {
-          x = __half2float(v_tail_row(L, c, b, h, (body - c.pv) * kPage + tt, D)[od]);
+      for (int j = 0; j < 4; ++j) {
+        uint2 mm = *(const uint2*)(lds + at.v_meta + (t0 + 8 * j) * 4);
+        if (ntok < kPage) {           // a token that does not count is 0, whatever its bytes say
+          if (t0 + 8 * j >= ntok) mm.x = 0u;
+          if (t0 + 8 * j + 1 >= ntok) mm.y = 0u;
+        }
+        sc[j] = low_halves(mm.x, mm.y), zr[j] = high_halves(mm.x, mm.y);
+      }
+      const int rr = n >> 2, tok = t0 + (rr & 1) + 8 * (rr >> 1);
+#pragma unroll
+      for (int hf = 0; hf < kHalves; ++hf) {
+        // D = 64: a row has 8 pieces; lanes n and n + 8 both receive piece n % 8 and take its lower and upper four codes
+        const uint8_t* p = lds + at.v_raw + tok * (D / 4) + hf * kRowBytes + (D == 64 ? n & 1 : n & 3) * 8;
+        uint32_t X[4];
+        lds_tr(p, X[0], X[1]);
+        lds_tr(p + 16 * (D / 4), X[2], X[3]);
+        if (D == 64) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) X[j] >>= n & 8;
         }
 #pragma unroll
-        for (int g = 0; g < ROWS; ++g)
-          if (g < R) acc_o[g] += s_p[tt][g] * x;   // (a masked token has probability 0)
+        for (int u = 0; u < kU; ++u) {
+          uint32_t a[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) a[j] = dequant_word(((X[j] >> (2 * u)) & kCodeMask) | kCodeMagic, sc[j], zr[j]);
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) {
+            O[hf * kU + u][nt] = mfma16(a, ph[nt], O[hf * kU + u][nt]);
+            O[hf * kU + u][nt] = mfma16(a, pl[nt], O[hf * kU + u][nt]);
+          }
+        }
+      }
+    } else {
+      const uint8_t* rows[8];   // the rows of tokens t0 + 8 j + e
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int tok = min(t0 + 8 * (i >> 1) + (i & 1), ntok - 1);
+        if (chunk) rows[i] = v_new + (int64_t)b * new_stride_b + (int64_t)h * new_stride_h + (int64_t)(chunk_t0 + tok) * new_stride_t;
+        else if (tile == 0) rows[i] = (const uint8_t*)L.sink_v + sink_base + (int64_t)tok * (2 * D);
+        else rows[i] = (const uint8_t*)v_tail_row(L, c, b, h, (body - c.pv) * kPage + tok, D);
+      }
+#pragma unroll
+      for (int hf = 0; hf < kHalves; ++hf) {
+        const int ch = D == 256 ? 128 * hf + 8 * n : 8 * (n & 7) + 4 * (n >> 3);
+        asm volatile("" ::: "memory");   // one piece's rows in flight at a time: both would cost 32 registers more
+        typedef uint32_t words __attribute__((ext_vector_type(kU / 2)));
+        words x[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          x[i] = *(const words*)(rows[i] + ch * 2);
+          if (t0 + 8 * (i >> 1) + (i & 1) >= ntok) x[i] = words{};   // probability 0 times what a dead row may hold must be 0
+        }
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+          uint32_t a[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            a[j] = u & 1 ? high_halves(x[2 * j][u >> 1], x[2 * j + 1][u >> 1]) : low_halves(x[2 * j][u >> 1], x[2 * j + 1][u >> 1]);
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) {
+            O[hf * kU + u][nt] = mfma16(a, ph[nt], O[hf * kU + u][nt]);
+            O[hf * kU + u][nt] = mfma16(a, pl[nt], O[hf * kU + u][nt]);
+          }
+        }
       }
     }
-    __syncthreads();
   }
 
   if (tid == 0) report_bad_page(L, b, bad_page);
+  // ---- the wavefronts' partials meet: a common maximum, then sums of four output tiles at a time ---------------
 #pragma unroll
-  for (int g = 0; g < ROWS; ++g)
-    if (g < R) s_u.o[opart][g][od] = acc_o[g];
+  for (int nt = 0; nt < NT; ++nt) {
+    float l = l_run[nt];
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    if (kg == 0) s_m[w][16 * nt + n] = m_run[nt], s_l[w][16 * nt + n] = l;
+  }
   __syncthreads();
-  for (int i = tid; i < R * D; i += 256) {
-    const int g = i / D, d = i % D;
-    float o = 0.f;
 #pragma unroll
-    for (int pp = 0; pp < kParts; ++pp) o += s_u.o[pp][g][d];
-    if (PREFILL) {
-      const int pos = s_pos[g];
-      if (pos >= 0) {
-        const float l = s_l[g];
-        out[(((int64_t)b * Tq + pos) * H_Q + (h * G + g / PB)) * D + d] = __float2half_rn(l > 0.f ? o / l : 0.f);
+  for (int nt = 0; nt < NT; ++nt) {
+    const int r = 16 * nt + n;
+    const float mm = fmaxf(fmaxf(s_m[0][r], s_m[1][r]), fmaxf(s_m[2][r], s_m[3][r]));
+    const float own = m_run[nt] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run[nt] - mm) * (1.f / kProbScale);
+#pragma unroll
+    for (int t = 0; t < kOT; ++t) O[t][nt] *= own;
+  }
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    // (this thread's part of the result: 4 channels of row n of column tile nt)
+    const int r = 16 * nt + n;
+    float mm = -INFINITY, l = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) mm = fmaxf(mm, s_m[i][r]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) l += s_m[i][r] == -INFINITY ? 0.f : s_l[i][r] * __builtin_amdgcn_exp2f(s_m[i][r] - mm);
+    const bool partial = !PREFILL || ws_ml != nullptr;
+    int64_t row = 0;   // of the workspace, or of out
+    if (PREFILL) row = ((int64_t)b * Tq + qpos[nt]) * H_Q + h * G + qhead[nt];
+    else row = (int64_t)b * H_Q + h * G + qhead[nt];
+    if (partial) row = row * num_splits + split;
+    if (partial && qpos[nt] >= 0 && w == 0 && kg == 0) *(float2*)(ws_ml + row * 2) = float2{mm, l};
+#pragma unroll
+    for (int t4 = 0; t4 < kOT; t4 += 4) {
+      __syncthreads();
+#pragma unroll
+      for (int t = 0; t < 4; ++t) ((float4v*)lds)[(w * 4 + t) * 64 + lane] = O[t4 + t][nt];
+      __syncthreads();
+      float4v o = float4v{0.f, 0.f, 0.f, 0.f};   // tile t4 + w, summed over the wavefronts
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o += ((const float4v*)lds)[(i * 4 + w) * 64 + lane];
+      if (qpos[nt] >= 0) {
+        const int t = t4 + w;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int x = 4 * kg + j;
+          const int ch = D == 256 ? 128 * (t >> 3) + 8 * x + (t & 7) : 8 * (x & 7) + 4 * (x >> 3) + t;
+          if (partial) ws_acc[row * D + ch] = o[j];
+          else out[row * D + ch] = __float2half_rn(l > 0.f ? o[j] / l : 0.f);
+        }
       }
-    } else {
-      const int64_t row = ((int64_t)b * H_Q + (int64_t)h * G + g) * num_splits + blockIdx.x;
-      ws_acc[row * D + d] = o;
-      if (d == 0) { ws_ml[row * 2] = s_m[g] * 1.44269504088896f; ws_ml[row * 2 + 1] = s_l[g]; }
     }
   }
-}
-
-// out[b, 0, hq, :] = sum_s acc_s * 2^(m_s - m) / sum_s l_s * 2^(m_s - m); one block per query head, one
-// thread per channel.
-template <int D>
-__global__ __launch_bounds__(D) void merge_any_kernel(const float* __restrict__ ws_ml, const float* __restrict__ ws_acc,
-                                                       __half* __restrict__ out, int num_splits) {
-  const int64_t head = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
-  const int64_t row0 = head * num_splits;
-  const int d = threadIdx.x;
-  float m = -INFINITY;
-  for (int s = 0; s < num_splits; ++s) m = fmaxf(m, ws_ml[(row0 + s) * 2]);
-  float l = 0.f, o = 0.f;
-  for (int s = 0; s < num_splits; ++s) {
-    const float ms = ws_ml[(row0 + s) * 2];
-    if (ms == -INFINITY) continue;   // an empty split
-    const float w = exp2f(ms - m);
-    l += ws_ml[(row0 + s) * 2 + 1] * w;
-    o += ws_acc[(row0 + s) * D + d] * w;
-  }
-  out[head * D + d] = __float2half_rn(l > 0.f ? o / l : 0.f);
 }
 
 template <int D>
@@ -453,48 +655,51 @@ void launch_decode_any(const kitty_kv_layer& L, const void* q, int B, int H_Q, f
                        float* ws_acc, int num_splits, hipStream_t stream) {
   const dim3 grid(num_splits, L.H_KV, B), block(256);
   const int64_t qb = (int64_t)H_Q * L.D * 2, qh = (int64_t)L.D * 2;
-  const int G = H_Q / L.H_KV;
-  // the kernel is instantiated for 4, 8 and 16 query rows: a group of 4 heads does not pay for 16
-#define KITTY_ATTN_ANY(DD, RR)                                                                                       \
-  hipLaunchKernelGGL((attn_any_kernel<DD, false, RR>), grid, block, 0, stream, L, (const uint8_t*)q, qb, qh,         \
-                     (int64_t)0, nullptr, nullptr, (int64_t)0, (int64_t)0, (int64_t)0, H_Q, 1, scaling, ws_ml,       \
-                     ws_acc, num_splits, nullptr)
-  if (L.D == 64) {
-    if (G <= 4) KITTY_ATTN_ANY(64, 4);
-    else if (G <= 8) KITTY_ATTN_ANY(64, 8);
-    else KITTY_ATTN_ANY(64, 16);
-  } else {
-    if (G <= 4) KITTY_ATTN_ANY(256, 4);
-    else if (G <= 8) KITTY_ATTN_ANY(256, 8);
-    else KITTY_ATTN_ANY(256, 16);
-  }
-#undef KITTY_ATTN_ANY
+  const int lds = AnyLds(L.D, L.D_BOOSTED).with_q(L.D, 1);
+  if (L.D == 64)
+    hipLaunchKernelGGL((attn_any_kernel<64, false, 1>), grid, block, lds, stream, L, (const uint8_t*)q, qb, qh, (int64_t)0,
+                       nullptr, nullptr, (int64_t)0, (int64_t)0, (int64_t)0, H_Q, 1, scaling, ws_ml, ws_acc, num_splits, nullptr);
+  else
+    hipLaunchKernelGGL((attn_any_kernel<256, false, 1>), grid, block, lds, stream, L, (const uint8_t*)q, qb, qh, (int64_t)0,
+                       nullptr, nullptr, (int64_t)0, (int64_t)0, (int64_t)0, H_Q, 1, scaling, ws_ml, ws_acc, num_splits, nullptr);
 }
 
-void launch_merge_any(int D, const float* ws_ml, const float* ws_acc, void* out, int B, int H_Q, int num_splits,
-                      hipStream_t stream) {
-  const dim3 grid(H_Q, B);
-  if (D == 64)
-    hipLaunchKernelGGL((merge_any_kernel<64>), grid, dim3(64), 0, stream, ws_ml, ws_acc, (__half*)out, num_splits);
-  else
-    hipLaunchKernelGGL((merge_any_kernel<256>), grid, dim3(256), 0, stream, ws_ml, ws_acc, (__half*)out, num_splits);
+namespace {
+// chunk positions per workgroup
+int any_positions(int D, int G) {
+  const int rows = 16 * (D == 64 ? kPrefillTiles64 : kPrefillTiles256);
+  return rows / G > 0 ? rows / G : 1;
+}
+}  // namespace
+
+// Shares of a chunk's walk: enough workgroups for two on every compute unit (what their registers allow at
+// D = 256), of at least two tiles each.
+int prefill_splits_any(int B, int H_Q, int H_KV, int D, int Tq, int tiles, int units) {
+  const int PB = any_positions(D, H_Q / H_KV);
+  const int64_t wgs = (int64_t)((Tq + PB - 1) / PB) * H_KV * B;
+  int64_t s = 2 * units / wgs;
+  if (s > tiles / 2) s = tiles / 2;
+  if (s > 64) s = 64;
+  return s < 1 ? 1 : (int)s;
 }
 
 void launch_prefill_any(const kitty_kv_layer& L, const void* q, int64_t q_stride_b, int64_t q_stride_h,
                         int64_t q_stride_t, const void* k_new, const void* v_new, int64_t new_stride_b,
                         int64_t new_stride_h, int64_t new_stride_t, int B, int H_Q, int Tq, float scaling, void* out,
-                        hipStream_t stream) {
-  const int G = H_Q / L.H_KV;
-  const int PB = kMaxRows / G > 0 ? kMaxRows / G : 1;
-  const dim3 grid((Tq + PB - 1) / PB, L.H_KV, B), block(256);
+                        float* ws_ml, float* ws_acc, int num_splits, hipStream_t stream) {
+  const int PB = any_positions(L.D, H_Q / L.H_KV);
+  const dim3 grid((Tq + PB - 1) / PB * num_splits, L.H_KV, B), block(256);
+  const int lds = AnyLds(L.D, L.D_BOOSTED).with_q(L.D, L.D == 64 ? kPrefillTiles64 : kPrefillTiles256);
   if (L.D == 64)
-    hipLaunchKernelGGL((attn_any_kernel<64, true, kMaxRows>), grid, block, 0, stream, L, (const uint8_t*)q, q_stride_b,
+    hipLaunchKernelGGL((attn_any_kernel<64, true, kPrefillTiles64>), grid, block, lds, stream, L, (const uint8_t*)q, q_stride_b,
                        q_stride_h, q_stride_t, (const uint8_t*)k_new, (const uint8_t*)v_new, new_stride_b,
-                       new_stride_h, new_stride_t, H_Q, Tq, scaling, nullptr, nullptr, 1, (__half*)out);
+                       new_stride_h, new_stride_t, H_Q, Tq, scaling, ws_ml, ws_acc, num_splits, (__half*)out);
   else
-    hipLaunchKernelGGL((attn_any_kernel<256, true, kMaxRows>), grid, block, 0, stream, L, (const uint8_t*)q, q_stride_b,
+    hipLaunchKernelGGL((attn_any_kernel<256, true, kPrefillTiles256>), grid, block, lds, stream, L, (const uint8_t*)q, q_stride_b,
                        q_stride_h, q_stride_t, (const uint8_t*)k_new, (const uint8_t*)v_new, new_stride_b,
-                       new_stride_h, new_stride_t, H_Q, Tq, scaling, nullptr, nullptr, 1, (__half*)out);
+                       new_stride_h, new_stride_t, H_Q, Tq, scaling, ws_ml, ws_acc, num_splits, (__half*)out);
+  if (num_splits > 1)
+    launch_rows_merge(L.D, ws_ml, ws_acc, out, (int64_t)B * Tq * H_Q, num_splits, /* keep_nan */ false, stream);
 }
 
 }  // namespace kitty

@@ -19,12 +19,14 @@ int prefill_splits(int B, int H_Q, int H_KV, int Tq, int tiles, int units);
 // head dimensions other than 128 (any_dim.hip)
 void launch_decode_any(const kitty_kv_layer& L, const void* q, int B, int H_Q, float scaling, float* ws_ml,
                        float* ws_acc, int num_splits, hipStream_t stream);
-void launch_merge_any(int D, const float* ws_ml, const float* ws_acc, void* out, int B, int H_Q, int num_splits,
-                      hipStream_t stream);
 void launch_prefill_any(const kitty_kv_layer& L, const void* q, int64_t q_stride_b, int64_t q_stride_h,
                         int64_t q_stride_t, const void* k_new, const void* v_new, int64_t new_stride_b,
                         int64_t new_stride_h, int64_t new_stride_t, int B, int H_Q, int Tq, float scaling, void* out,
-                        hipStream_t stream);
+                        float* ws_ml, float* ws_acc, int num_splits, hipStream_t stream);
+int prefill_splits_any(int B, int H_Q, int H_KV, int D, int Tq, int tiles, int units);
+// merge pass over independent rows (rows_merge.hip)
+void launch_rows_merge(int D, const float* ws_ml, const float* ws_acc, void* out, int64_t rows, int num_splits,
+                       bool keep_nan, hipStream_t stream);
 }  // namespace kitty
 
 using namespace kitty;
@@ -178,7 +180,7 @@ extern "C" int kitty_decode_attn_split(const kitty_kv_layer* layer, const void* 
   const kitty_kv_layer& L = *layer;
   float* ws_ml = (float*)workspace;
   float* ws_acc = (float*)((uint8_t*)workspace + ws_ml_bytes(B, H_Q, num_splits));
-  if (L.D != kD) {   // one kernel for both variants: the reference's order of operations on the vector ALUs
+  if (L.D != kD) {   // one kernel for both variants: the reference's order of operations
     if (ev0) (void)hipEventRecord(ev0, (hipStream_t)stream);
     launch_decode_any(L, q, B, H_Q, scaling, ws_ml, ws_acc, num_splits, (hipStream_t)stream);
     if (ev1) (void)hipEventRecord(ev1, (hipStream_t)stream);
@@ -210,7 +212,7 @@ extern "C" int kitty_decode_attn_merge(const void* workspace, size_t workspace_b
   if (int rc = check_workspace(workspace, workspace_bytes, B, H_Q, num_splits, D)) return rc;
   const float* ws_ml = (const float*)workspace;
   const float* ws_acc = (const float*)((const uint8_t*)workspace + ws_ml_bytes(B, H_Q, num_splits));
-  if (D != kD) launch_merge_any(D, ws_ml, ws_acc, out, B, H_Q, num_splits, (hipStream_t)stream);
+  if (D != kD) launch_rows_merge(D, ws_ml, ws_acc, out, (int64_t)B * H_Q, num_splits, /* keep_nan */ false, (hipStream_t)stream);
   else launch_decode_merge(ws_ml, ws_acc, out, B, H_Q, num_splits, (hipStream_t)stream);
   return check_launch("kitty_decode_attn_merge");
 }
@@ -235,7 +237,8 @@ extern "C" size_t kitty_prefill_attn_workspace_bytes(int B, int H_Q, int D, int 
 }
 
 extern "C" int kitty_prefill_attn_default_splits(int B, int H_Q, int H_KV, int D, int T_q, int max_tiles) {
-  if (B <= 0 || H_KV <= 0 || H_Q < H_KV || H_Q / H_KV > 16 || T_q <= 0 || max_tiles <= 0 || D != kD) return 1;
+  if (B <= 0 || H_KV <= 0 || H_Q < H_KV || H_Q / H_KV > 16 || T_q <= 0 || max_tiles <= 0 || !head_dim_supported(D)) return 1;
+  if (D != kD) return prefill_splits_any(B, H_Q, H_KV, D, T_q, max_tiles + c_div_up(T_q, kPage), device_simds() / 4);
   return prefill_splits(B, H_Q, H_KV, T_q, max_tiles + c_div_up(T_q, kPage), device_simds() / 4);
 }
 
@@ -276,7 +279,7 @@ extern "C" int kitty_prefill_attn_split(const kitty_kv_layer* layer, const void*
   }
   if (layer->D != kD) {
     launch_prefill_any(*layer, q, q_stride_b, q_stride_h, q_stride_t, k_new, v_new, new_stride_b, new_stride_h,
-                       new_stride_t, B, H_Q, T_q, scaling, out, (hipStream_t)stream);
+                       new_stride_t, B, H_Q, T_q, scaling, out, ws_ml, ws_acc, num_splits, (hipStream_t)stream);
     return check_launch("kitty_prefill_attn");
   }
   launch_prefill_attn(*layer, q, q_stride_b, q_stride_h, q_stride_t, k_new, v_new, new_stride_b, new_stride_h,

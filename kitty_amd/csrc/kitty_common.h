@@ -20,7 +20,7 @@ constexpr int kVBytes = kPage * kRowBytes;               // 4096: a V page-head
 __host__ __device__ inline int k_head_bytes(int d_boost) { return kRowBytes * (kD + d_boost) + kD; }
 // Other head dimensions (the reference derives everything from config.head_dim, kitty.py:39-44, and its
 // kernels take D as a parameter, kitty_quant_pack.py:42-45, kitty_attention.py:59-62): 64 and 256 run
-// on plain kernels of their own (any_dim.hip); the tuned kernels are those for 128.
+// on kernels of their own (any_dim.hip).
 __host__ __device__ inline bool head_dim_supported(int d) { return d == 64 || d == kD || d == 256; }
 __host__ __device__ inline int k_head_bytes_d(int head_dim, int d_boost) {
   return kRowBytes * (head_dim + d_boost) + head_dim;
