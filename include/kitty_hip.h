@@ -304,6 +304,26 @@ int kitty_append_chunk(const kitty_kv_layer* layer, const void* k_new, const voi
                        int64_t stride_b, int64_t stride_h, int64_t stride_t, int B, int T, void* stream);
 
 /*
+ * kitty_append_chunk with the layer's scalar counters (layer->counts; seq_counts must be NULL): one chunk for every
+ * sequence of the batch in two launches.  The caller advances its counters by the closed form of the state
+ * machine.  Rows of a Q-buffer past its fill count are left as the last page that went through it lies there.  A page whose table entry is outside the cache is not written.
+ */
+int kitty_append_chunk_host(const kitty_kv_layer* layer, const void* k_new, const void* v_new, int64_t stride_b,
+                            int64_t stride_h, int64_t stride_t, int B, int T, void* stream);
+
+/*
+ * A prompt into rows first_row .. first_row + B - 1 of a layer that hold nothing: what KittyCache.quantize_prefill
+ * does (kitty.py:126-192) - sink rows, packed pages (through entries 0 .. of those rows of the page tables, channel
+ * selection fused), Q-buffer rows and the local ring in order of age.  k_new / v_new: fp16 [B,H_KV,T,D], D contiguous,
+ * byte strides of their own, 16-byte aligned.  The caller owns the counters (layer->counts and seq_counts are not
+ * read).  A page whose table entry is outside the cache is not written, and recorded in layer->status.
+ * One launch at D = 128; at D = 64 / 256 the quantizers are two more.
+ */
+int kitty_pack_prompt(const kitty_kv_layer* layer, int first_row, const void* k_new, int64_t k_stride_b,
+                      int64_t k_stride_h, int64_t k_stride_t, const void* v_new, int64_t v_stride_b,
+                      int64_t v_stride_h, int64_t v_stride_t, int B, int T, void* stream);
+
+/*
  * One token per sequence with the layer's scalar counters (layer->counts; seq_counts must be NULL): the
  * slice copies of KittyCache.update's decode branch (kitty.py:97-123) as one launch, for every supported
  * head dimension.  k_new / v_new: fp16 [B,H_KV,1,D], D contiguous, byte strides of their own, 16-byte

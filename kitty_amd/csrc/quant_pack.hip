@@ -673,23 +673,25 @@ struct ChunkPlan {
   int rk2, rv2, lv2, off2;
 };
 
-// the counters part; `ok` still lacks the page ids (chunk_pages_ok)
-__device__ inline ChunkPlan chunk_plan(const kitty_kv_layer& L, int b, int T) {
-  const int32_t* cnt = L.seq_counts + b * KITTY_SEQ_COUNT_FIELDS;
+// the counters part; `ok` still lacks the page ids (chunk_pages_ok).  HOST: one set of counters for the batch, in
+// the layer itself, which the host has checked.
+template <bool HOST = false>
+__host__ __device__ inline ChunkPlan chunk_plan(const kitty_kv_layer& L, int b, int T) {
+  const int32_t* cnt = HOST ? L.counts : L.seq_counts + b * KITTY_SEQ_COUNT_FIELDS;
   ChunkPlan p;
-  p.active = !(cnt[KITTY_CNT_FLAGS] & KITTY_SEQ_INACTIVE);
+  p.active = HOST || !(cnt[KITTY_CNT_FLAGS] & KITTY_SEQ_INACTIVE);
   p.sink = cnt[KITTY_CNT_SINK]; p.pk = cnt[KITTY_CNT_PAGES_K]; p.rk = cnt[KITTY_CNT_QBUF_K];
   p.pv = cnt[KITTY_CNT_PAGES_V]; p.rv = cnt[KITTY_CNT_QBUF_V]; p.lv = cnt[KITTY_CNT_LOCAL_V];
   p.off = cnt[KITTY_CNT_LOCAL_OFF] & (kPage - 1);
   const bool sane = p.sink >= 0 && p.sink <= L.S && p.pk >= 0 && p.pv >= 0 && p.rk >= 0 && p.rv >= 0 && p.lv >= 0 &&
                     p.lv <= kPage && p.rk <= kPage && p.rv <= kPage;
-  p.a = sane ? min(L.S - p.sink, T) : 0;
+  p.a = sane ? (L.S - p.sink < T ? L.S - p.sink : T) : 0;
   p.n = T - p.a;
   p.npk = (p.rk + p.n) / kPage;
   p.rk2 = (p.rk + p.n) % kPage;
-  p.lv2 = min(kPage, p.lv + p.n);
+  p.lv2 = p.lv + p.n < kPage ? p.lv + p.n : kPage;
   p.e = p.lv + p.n - p.lv2;
-  p.er = min(p.e, p.lv);
+  p.er = p.e < p.lv ? p.e : p.lv;
   p.npv = (p.rv + p.e) / kPage;
   p.rv2 = (p.rv + p.e) % kPage;
   p.off2 = (p.off + p.e) & (kPage - 1);
@@ -736,26 +738,31 @@ struct VStreamRows {
   }
 };
 
-// grid (2 * max_pages, H_KV, B): blockIdx.x < max_pages: new K page blockIdx.x, else new V page
+// grid (2 * max_pages, H_KV, B): blockIdx.x < max_pages: new K page blockIdx.x, else new V page.  With the
+// counters on the device a sequence takes the whole chunk or nothing; with host counters (HOST) a page whose id
+// is outside the cache is left out alone, as kitty_quant_pack_k / _v leave it out.
+template <bool HOST>
 __global__ __launch_bounds__(256) void chunk_quant_kernel(kitty_kv_layer L, const uint8_t* __restrict__ k_new,
                                                           const uint8_t* __restrict__ v_new, int64_t stride_b,
                                                           int64_t stride_h, int64_t stride_t, int T, int max_pages) {
   const int h = blockIdx.y, b = blockIdx.z;
   const bool vside = (int)blockIdx.x >= max_pages;
   const int p = vside ? blockIdx.x - max_pages : blockIdx.x;
-  const ChunkPlan c = chunk_plan(L, b, T);
+  const ChunkPlan c = chunk_plan<HOST>(L, b, T);
   if (!c.active || p >= (vside ? c.npv : c.npk)) return;        // uniform over the block
-  if (!chunk_pages_ok(L, b, c)) return;
+  if (!HOST && !chunk_pages_ok(L, b, c)) return;
   const int64_t w = (int64_t)b * L.win_stride_b + (int64_t)h * L.win_stride_h;
   const int64_t src = (int64_t)b * stride_b + (int64_t)h * stride_h + (int64_t)c.a * stride_t;
   if (!vside) {
     const int64_t pg = L.page_table_k[(int64_t)b * L.page_table_k_stride_b + c.pk + p];
+    if (HOST && (pg < 0 || pg >= L.cache_pages_k)) return;
     quant_k_page<1>(KStreamRows{(const uint8_t*)L.qbuf_k + w, k_new + src, stride_t, c.rk, p * kPage}, L.D_BOOSTED,
                     nullptr, nullptr,
                     const_cast<uint8_t*>(L.key_cache) + pg * L.key_cache_stride_page + (int64_t)h * k_head_bytes(L.D_BOOSTED),
                     (uint8_t*)L.key_meta + pg * L.key_meta_stride_page + (int64_t)h * kD * 4);
   } else {
     const int64_t pg = L.page_table_v[(int64_t)b * L.page_table_v_stride_b + c.pv + p];
+    if (HOST && (pg < 0 || pg >= L.cache_pages_v)) return;
     quant_v_page(VStreamRows{(const uint8_t*)L.qbuf_v + w, (const uint8_t*)L.local_v + w, v_new + src, stride_t, c.rv,
                              c.er, c.off, p * kPage},
                  const_cast<uint8_t*>(L.value_cache) + pg * L.value_cache_stride_page + (int64_t)h * kVBytes,
@@ -766,14 +773,15 @@ __global__ __launch_bounds__(256) void chunk_quant_kernel(kitty_kv_layer L, cons
 // grid (H_KV, B): the fp16 rows of one (b, h) after the chunk - sink rows, what is left of the two
 // streams (the new Q-buffer contents) and the ring.  Runs after chunk_quant_kernel, which reads the
 // old Q-buffers and ring.  Rows are moved by 16 lanes x 16 bytes.
+template <bool HOST>
 __global__ __launch_bounds__(256) void chunk_rows_kernel(kitty_kv_layer L, const uint8_t* __restrict__ k_new,
                                                          const uint8_t* __restrict__ v_new, int64_t stride_b,
                                                          int64_t stride_h, int64_t stride_t, int T) {
   __shared__ uint4 s_stage[kPage][16];   // ring rows on their way to the V Q-buffer
   const int h = blockIdx.x, b = blockIdx.y;
-  const ChunkPlan c = chunk_plan(L, b, T);
+  const ChunkPlan c = chunk_plan<HOST>(L, b, T);
   if (!c.active) return;
-  if (!chunk_pages_ok(L, b, c)) return;
+  if (!HOST && !chunk_pages_ok(L, b, c)) return;
   const int piece = threadIdx.x & 15, r0 = threadIdx.x >> 4;
   const int64_t w = (int64_t)b * L.win_stride_b + (int64_t)h * L.win_stride_h;
   const uint8_t* ksrc = k_new + (int64_t)b * stride_b + (int64_t)h * stride_h;
@@ -791,22 +799,31 @@ __global__ __launch_bounds__(256) void chunk_rows_kernel(kitty_kv_layer L, const
   ksrc += (int64_t)c.a * stride_t;
   vsrc += (int64_t)c.a * stride_t;
   // K: stream rows 128 npk + i -> Q_Buffer_K[i]; rows that already sit there stay (no page was cut)
-  for (int i = (c.npk ? 0 : c.rk) + r0; i < c.rk2; i += 16)
-    ((uint4*)((uint8_t*)L.qbuf_k + w + (int64_t)i * (kD * 2)))[piece] =
-        row16(ksrc + (int64_t)(c.npk * kPage + i - c.rk) * stride_t);
+  // (HOST: and past the fill count the rows of the page that went through the Q-buffer, as they would lie there)
+  const int k_end = HOST && c.npk > 0 && c.rk > 0 ? kPage : c.rk2;
+  for (int i = (c.npk ? 0 : c.rk) + r0; i < k_end; i += 16) {
+    const int s = i < c.rk2 ? c.npk * kPage + i : i;
+    if (s >= c.rk) ((uint4*)((uint8_t*)L.qbuf_k + w + (int64_t)i * (kD * 2)))[piece] = row16(ksrc + (int64_t)(s - c.rk) * stride_t);
+  }
   // V: the same, but a stream row may lie in the ring, whose slots are about to be overwritten:
   // those rows go through LDS
-  const int v_first = c.npv * kPage;
   const int lo = c.npv ? 0 : c.rv;
-  for (int i = lo + r0; i < c.rv2; i += 16) {
-    const int s = v_first + i;
-    if (s >= c.rv && s < c.rv + c.er)
+  // (HOST: of the new pages that hold buffered or ring rows the last went through the Q-buffer last - unless it is
+  // the ring itself, in one piece)
+  const int waiting = c.rv + c.er;
+  const bool through = HOST && c.npv > 0 && waiting > 0 && !(c.rv == 0 && c.er == kPage && c.off == 0);
+  const int last = min((waiting - 1) / kPage, c.npv - 1), v_end = through ? kPage : c.rv2;
+  auto stream_row = [&](int i) { return i < c.rv2 ? c.npv * kPage + i : last * kPage + i; };
+  for (int i = lo + r0; i < v_end; i += 16) {
+    const int s = stream_row(i);
+    if (s >= c.rv && s < waiting)
       s_stage[i][piece] = row16((const uint8_t*)L.local_v + w + (int64_t)((c.off + s - c.rv) & (kPage - 1)) * (kD * 2));
   }
   __syncthreads();
-  for (int i = lo + r0; i < c.rv2; i += 16) {
-    const int s = v_first + i;
-    const uint4 v = (s < c.rv + c.er) ? s_stage[i][piece] : row16(vsrc + (int64_t)(s - c.rv - c.er) * stride_t);
+  for (int i = lo + r0; i < v_end; i += 16) {
+    const int s = stream_row(i);
+    if (s < c.rv) continue;   // lies there already
+    const uint4 v = s < waiting ? s_stage[i][piece] : row16(vsrc + (int64_t)(s - waiting) * stride_t);
     ((uint4*)((uint8_t*)L.qbuf_v + w + (int64_t)i * (kD * 2)))[piece] = v;
   }
   // ring: the chunk rows that stay take the slots single steps would have given them
@@ -835,6 +852,93 @@ __global__ __launch_bounds__(64) void chunk_advance_kernel(kitty_kv_layer L, int
   cnt[KITTY_CNT_QBUF_V] = c.rv2;
   cnt[KITTY_CNT_LOCAL_V] = c.lv2;
   cnt[KITTY_CNT_LOCAL_OFF] = c.off2;
+}
+
+// ---------------------------------------------------------------------------------------------
+// A prompt into empty rows of a layer, in one launch: what KittyCache.quantize_prefill does (kitty.py:126-192).
+// Nothing it reads is written by it, so the three kinds of work share a grid:
+//   blockIdx.x < npk: K page;  < npk + npv: V page;  else: 64 KB of fp16 rows (sink, Q-buffers, ring in order of age).
+// A short prompt is launch latency (B = 1, 700 tokens: five row copies of 4.5 us and two quantizers of 8 and 5, 55 us
+// a layer with the host's part; 8.5 in one launch); a long one is memory bandwidth, where the K pages' arithmetic
+// and the V pages' streaming now overlap (B = 4, 32k tokens: quantizers of 60 and 53 us and the copies, 131 us;
+// 113 in one launch, 5.5 TB/s).
+// At D != 128 the quantizers stay launches of their own (npk = npv = 0 here).
+// ---------------------------------------------------------------------------------------------
+struct PromptRows {   // [first, first + n) of the prompt -> rows 0 .. n - 1 of a window
+  int n, first;
+};
+struct PromptPlan {
+  int npk, npv;
+  PromptRows sink, qk, qv, ring;
+};
+__host__ __device__ inline PromptPlan prompt_plan(int S, int T) {
+  PromptPlan p;
+  const int sink = S < T ? S : T, n = T - sink, lv = n < kPage ? n : kPage;
+  p.npk = n / kPage;
+  p.npv = (n - lv) / kPage;
+  p.sink = PromptRows{sink, 0};
+  p.qk = PromptRows{n % kPage, sink + p.npk * kPage};
+  p.qv = PromptRows{(n - lv) % kPage, sink + p.npv * kPage};
+  p.ring = PromptRows{lv, T - lv};
+  return p;
+}
+constexpr int kRowPieces = 1024;   // 16-byte pieces of fp16 rows per workgroup
+
+__global__ __launch_bounds__(256) void pack_prompt_kernel(kitty_kv_layer L, int first_row, const uint8_t* __restrict__ k_new,
+                                                          int64_t k_sb, int64_t k_sh, int64_t k_st,
+                                                          const uint8_t* __restrict__ v_new, int64_t v_sb, int64_t v_sh,
+                                                          int64_t v_st, int T, int npk, int npv) {
+  const int h = blockIdx.y, b = first_row + blockIdx.z;
+  const uint8_t* k = k_new + (int64_t)blockIdx.z * k_sb + (int64_t)h * k_sh;
+  const uint8_t* v = v_new + (int64_t)blockIdx.z * v_sb + (int64_t)h * v_sh;
+  int x = blockIdx.x;
+  const int sink = L.S < T ? L.S : T;
+  if (x < npk) {
+    const int64_t pg = L.page_table_k[(int64_t)b * L.page_table_k_stride_b + x];
+    if (pg < 0 || pg >= L.cache_pages_k) {   // never write outside the cache; leave a record instead
+      if (L.status && threadIdx.x == 0) L.status[b * KITTY_STATUS_FIELDS + KITTY_STATUS_BAD_PAGE_WRITE] = 1;
+      return;
+    }
+    quant_k_page<1>(StridedRows{k + (int64_t)(sink + x * kPage) * k_st, k_st}, L.D_BOOSTED, nullptr, nullptr,
+                    const_cast<uint8_t*>(L.key_cache) + pg * L.key_cache_stride_page + (int64_t)h * k_head_bytes(L.D_BOOSTED),
+                    (uint8_t*)L.key_meta + pg * L.key_meta_stride_page + (int64_t)h * kD * 4);
+    return;
+  }
+  x -= npk;
+  if (x < npv) {
+    const int64_t pg = L.page_table_v[(int64_t)b * L.page_table_v_stride_b + x];
+    if (pg < 0 || pg >= L.cache_pages_v) {
+      if (L.status && threadIdx.x == 0) L.status[b * KITTY_STATUS_FIELDS + KITTY_STATUS_BAD_PAGE_WRITE] = 1;
+      return;
+    }
+    quant_v_page(StridedRows{v + (int64_t)(sink + x * kPage) * v_st, v_st},
+                 const_cast<uint8_t*>(L.value_cache) + pg * L.value_cache_stride_page + (int64_t)h * kVBytes,
+                 (uint8_t*)L.value_meta + pg * L.value_meta_stride_page + (int64_t)h * kPage * 4);
+    return;
+  }
+  x -= npv;
+  const PromptPlan p = prompt_plan(L.S, T);
+  const int pieces = L.D >> 3;   // 16-byte pieces of a row: 8, 16 or 32
+  const int64_t row_bytes = (int64_t)L.D * 2;
+  const int64_t so = (int64_t)b * L.sink_stride_b + (int64_t)h * L.sink_stride_h;
+  const int64_t wo = (int64_t)b * L.win_stride_b + (int64_t)h * L.win_stride_h;
+  const struct { PromptRows r; uint8_t* dst; const uint8_t* src; int64_t st; } part[5] = {
+      {p.sink, (uint8_t*)L.sink_k + so, k, k_st}, {p.sink, (uint8_t*)L.sink_v + so, v, v_st},
+      {p.qk, (uint8_t*)L.qbuf_k + wo, k, k_st},   {p.qv, (uint8_t*)L.qbuf_v + wo, v, v_st},
+      {p.ring, (uint8_t*)L.local_v + wo, v, v_st}};
+#pragma unroll
+  for (int j = 0; j < kRowPieces / 256; ++j) {
+    const int i = x * kRowPieces + j * 256 + threadIdx.x;
+    int row = i / pieces;
+    const int off = (i - row * pieces) * 16;
+#pragma unroll
+    for (int s = 0; s < 5; ++s) {
+      if (row >= 0 && row < part[s].r.n)
+        *(uint4*)(part[s].dst + row * row_bytes + off) =
+            *(const uint4*)(part[s].src + (int64_t)(part[s].r.first + row) * part[s].st + off);
+      row -= part[s].r.n;
+    }
+  }
 }
 
 int check_src(const void* p, int64_t sb, int64_t sh, int64_t st, int B, int H, int T, int D, int t_offset,
@@ -952,10 +1056,11 @@ extern "C" int kitty_quant_pack_v(const void* value, int64_t stride_b, int64_t s
 }
 
 namespace {
-int check_append_layer(const kitty_kv_layer* layer, int B) {
+int check_append_layer(const kitty_kv_layer* layer, int B, bool device_counters = true) {
   KITTY_REQUIRE(layer != nullptr, KITTY_E_NULL, "layer is NULL");
   const kitty_kv_layer& L = *layer;
-  KITTY_REQUIRE(L.seq_counts != nullptr, KITTY_E_NULL, "this entry point needs per-sequence counters (seq_counts)");
+  KITTY_REQUIRE(!device_counters || L.seq_counts != nullptr, KITTY_E_NULL,
+                "this entry point needs per-sequence counters (seq_counts)");
   KITTY_REQUIRE(L.D == kD && L.PAGE_SIZE == kPage, KITTY_E_SHAPE,
                 "the device-counter entry points are built for head_dim 128 and page_size 128 (other head dimensions "
                 "keep the counters on the host), got D=%d page_size=%d", L.D, L.PAGE_SIZE);
@@ -1055,10 +1160,84 @@ extern "C" int kitty_append_chunk(const kitty_kv_layer* layer, const void* k_new
                 KITTY_E_ALIGN, "k_new / v_new need 16-byte aligned bases and strides with D contiguous");
   const int max_pages = (T + kPage - 1) / kPage;   // a stream holds at most 127 rows before the chunk
   const hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(chunk_quant_kernel, dim3(2 * max_pages, layer->H_KV, B), dim3(256), 0, st, *layer,
+  hipLaunchKernelGGL(chunk_quant_kernel<false>, dim3(2 * max_pages, layer->H_KV, B), dim3(256), 0, st, *layer,
                      (const uint8_t*)k_new, (const uint8_t*)v_new, stride_b, stride_h, stride_t, T, max_pages);
-  hipLaunchKernelGGL(chunk_rows_kernel, dim3(layer->H_KV, B), dim3(256), 0, st, *layer, (const uint8_t*)k_new,
+  hipLaunchKernelGGL(chunk_rows_kernel<false>, dim3(layer->H_KV, B), dim3(256), 0, st, *layer, (const uint8_t*)k_new,
                      (const uint8_t*)v_new, stride_b, stride_h, stride_t, T);
   hipLaunchKernelGGL(chunk_advance_kernel, dim3(B), dim3(64), 0, st, *layer, T);
   return check_launch("kitty_append_chunk");
+}
+
+extern "C" int kitty_append_chunk_host(const kitty_kv_layer* layer, const void* k_new, const void* v_new,
+                                       int64_t stride_b, int64_t stride_h, int64_t stride_t, int B, int T, void* stream) {
+  if (int rc = check_append_layer(layer, B, /* device_counters */ false)) return rc;
+  KITTY_REQUIRE(layer->seq_counts == nullptr, KITTY_E_RANGE,
+                "the layer's counters live on the device (seq_counts): use kitty_append_chunk");
+  KITTY_REQUIRE(k_new && v_new, KITTY_E_NULL, "k_new / v_new is NULL");
+  KITTY_REQUIRE(T >= 1 && T <= (1 << 24), KITTY_E_RANGE, "T=%d out of range", T);
+  KITTY_REQUIRE(((uintptr_t)k_new % 16) == 0 && ((uintptr_t)v_new % 16) == 0 && stride_b % 16 == 0 &&
+                    stride_h % 16 == 0 && stride_t % 16 == 0 && stride_t >= kD * 2,
+                KITTY_E_ALIGN, "k_new / v_new need 16-byte aligned bases and strides with D contiguous");
+  const ChunkPlan c = chunk_plan<true>(*layer, 0, T);
+  KITTY_REQUIRE(c.ok, KITTY_E_RANGE, "a cache counter is out of range, a Q-buffer is full, or the chunk exceeds MAX_PAGE=%d",
+                layer->MAX_PAGE);
+  const int max_pages = c.npk > c.npv ? c.npk : c.npv;
+  const hipStream_t st = (hipStream_t)stream;
+  if (max_pages > 0)
+    hipLaunchKernelGGL(chunk_quant_kernel<true>, dim3(2 * max_pages, layer->H_KV, B), dim3(256), 0, st, *layer,
+                       (const uint8_t*)k_new, (const uint8_t*)v_new, stride_b, stride_h, stride_t, T, max_pages);
+  hipLaunchKernelGGL(chunk_rows_kernel<true>, dim3(layer->H_KV, B), dim3(256), 0, st, *layer, (const uint8_t*)k_new,
+                     (const uint8_t*)v_new, stride_b, stride_h, stride_t, T);
+  return check_launch("kitty_append_chunk_host");
+}
+
+extern "C" int kitty_pack_prompt(const kitty_kv_layer* layer, int first_row, const void* k_new, int64_t k_stride_b,
+                                 int64_t k_stride_h, int64_t k_stride_t, const void* v_new, int64_t v_stride_b,
+                                 int64_t v_stride_h, int64_t v_stride_t, int B, int T, void* stream) {
+  KITTY_REQUIRE(layer && k_new && v_new, KITTY_E_NULL, "layer / k_new / v_new is NULL");
+  const kitty_kv_layer& L = *layer;
+  KITTY_REQUIRE(head_dim_supported(L.D) && L.PAGE_SIZE == kPage && L.S >= 0 && L.S <= kPage && L.MAX_PAGE >= 0, KITTY_E_SHAPE,
+                "kernels are built for head_dim 64, 128 or 256, page_size 128 and S <= 128, got D=%d page_size=%d S=%d",
+                L.D, L.PAGE_SIZE, L.S);
+  KITTY_REQUIRE(L.D_BOOSTED >= 0 && L.D_BOOSTED <= L.D && L.D_BOOSTED <= 255 && k_head_bytes_d(L.D, L.D_BOOSTED) % 16 == 0,
+                KITTY_E_SHAPE, "unsupported D_BOOSTED=%d", L.D_BOOSTED);
+  KITTY_REQUIRE(L.H_KV >= 1 && L.H_KV <= 65535 && B >= 1 && B <= 65535 && first_row >= 0 && T >= 1 && T <= (1 << 24), KITTY_E_RANGE,
+                "bad H_KV=%d, B=%d, first_row=%d or T=%d", L.H_KV, B, first_row, T);
+  KITTY_REQUIRE(L.sink_k && L.sink_v && L.qbuf_k && L.qbuf_v && L.local_v, KITTY_E_NULL, "a cache tensor pointer is NULL");
+  KITTY_REQUIRE((((uintptr_t)k_new | (uintptr_t)v_new | (uintptr_t)L.sink_k | (uintptr_t)L.sink_v | (uintptr_t)L.qbuf_k |
+                  (uintptr_t)L.qbuf_v | (uintptr_t)L.local_v) % 16) == 0 &&
+                    ((k_stride_b | k_stride_h | k_stride_t | v_stride_b | v_stride_h | v_stride_t | L.sink_stride_b |
+                      L.sink_stride_h | L.win_stride_b | L.win_stride_h) % 16) == 0 && ((uintptr_t)L.status % 4) == 0,
+                KITTY_E_ALIGN, "k_new, v_new and the windows need 16-byte aligned bases and strides");
+  const PromptPlan p = prompt_plan(L.S, T);
+  KITTY_REQUIRE(p.npk <= L.MAX_PAGE, KITTY_E_RANGE, "a prompt of %d tokens exceeds MAX_PAGE=%d", T, L.MAX_PAGE);
+  const int64_t need_k = (int64_t)L.H_KV * k_head_bytes_d(L.D, L.D_BOOSTED), need_v = (int64_t)L.H_KV * v_head_bytes_d(L.D);
+  if (p.npk > 0)
+    if (int rc = check_dst(L.page_table_k, 0, L.key_cache, L.key_cache_stride_page, L.key_meta, L.key_meta_stride_page,
+                           L.cache_pages_k, need_k, (int64_t)L.H_KV * L.D * 4))
+      return rc;
+  if (p.npv > 0)
+    if (int rc = check_dst(L.page_table_v, 0, L.value_cache, L.value_cache_stride_page, L.value_meta,
+                           L.value_meta_stride_page, L.cache_pages_v, need_v, (int64_t)L.H_KV * kPage * 4))
+      return rc;
+  const hipStream_t st = (hipStream_t)stream;
+  const int pieces = (2 * p.sink.n + p.qk.n + p.qv.n + p.ring.n) * (L.D / 8), row_blocks = (pieces + kRowPieces - 1) / kRowPieces;
+  const int npk = L.D == kD ? p.npk : 0, npv = L.D == kD ? p.npv : 0;
+  hipLaunchKernelGGL(pack_prompt_kernel, dim3(npk + npv + row_blocks, L.H_KV, B), dim3(256), 0, st, L, first_row,
+                     (const uint8_t*)k_new, k_stride_b, k_stride_h, k_stride_t, (const uint8_t*)v_new, v_stride_b,
+                     v_stride_h, v_stride_t, T, npk, npv);
+  if (L.D != kD) {
+    int32_t* status = L.status ? L.status + (int64_t)first_row * KITTY_STATUS_FIELDS : nullptr;
+    if (p.npk > 0)
+      launch_quant_k_any(L.D, 1, k_new, k_stride_b, k_stride_h, k_stride_t, B, L.H_KV, p.sink.n, p.npk, L.D_BOOSTED,
+                         nullptr, nullptr, L.page_table_k + (int64_t)first_row * L.page_table_k_stride_b,
+                         L.page_table_k_stride_b, 0, const_cast<uint8_t*>(L.key_cache), L.key_cache_stride_page,
+                         const_cast<void*>(L.key_meta), L.key_meta_stride_page, L.cache_pages_k, status, st);
+    if (p.npv > 0)
+      launch_quant_v_any(L.D, v_new, v_stride_b, v_stride_h, v_stride_t, B, L.H_KV, p.sink.n, p.npv,
+                         L.page_table_v + (int64_t)first_row * L.page_table_v_stride_b, L.page_table_v_stride_b, 0,
+                         const_cast<uint8_t*>(L.value_cache), L.value_cache_stride_page,
+                         const_cast<void*>(L.value_meta), L.value_meta_stride_page, L.cache_pages_v, status, st);
+  }
+  return check_launch("kitty_pack_prompt");
 }

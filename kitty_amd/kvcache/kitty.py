@@ -44,6 +44,15 @@ def _row_source(L: KVCache_Layer, x: torch.Tensor) -> torch.Tensor:
     return x
 
 
+def _kernel_ready(L: KVCache_Layer, x: torch.Tensor) -> bool:
+    """``x [B, H_KV, T, D]`` can be read by the packing kernels as it lies: what tensor copies would convert, move or
+    track stays with them."""
+    st = x.stride()
+    return (x.dtype == torch.float16 and x.device == L.KeyCache.device and st[3] == 1 and st[2] >= L.D
+            and not (st[0] % 8 or st[1] % 8 or st[2] % 8 or x.data_ptr() % 16)
+            and not (x.requires_grad and torch.is_grad_enabled()))
+
+
 class KittyCache(_HFCache):
     """Kitty KV cache: fp16 sink + packed 2-bit pages (25 % of key channels at 4 bit) + fp16
     residual windows that are flushed into packed pages when full."""
@@ -159,6 +168,16 @@ class KittyCache(_HFCache):
         len_local_v, len_qbuf_v, pages_v = n["local_v"], n["qbuf_v"], n["pages_v"]
         if pages_k > kvcache.MAX_PAGE:
             raise ValueError(f"prefill of {len_prefill} tokens exceeds max_length={kvcache.MAX_LEN}")
+        if kvcache.on_hip and self.select == "hip" and 1 <= len_prefill <= 1 << 24 and 1 <= B <= kvcache.MAX_BS - first_row \
+                and K.shape == (B, kvcache.H_KV, len_prefill, kvcache.D) == V.shape \
+                and _kernel_ready(kvcache, K) and _kernel_ready(kvcache, V):
+            ks, vs = K.stride(), V.stride()
+            rc = _lib.lib().kitty_pack_prompt(kvcache.descriptor(), first_row, K.data_ptr(), 2 * ks[0], 2 * ks[1], 2 * ks[2],
+                                              V.data_ptr(), 2 * vs[0], 2 * vs[1], 2 * vs[2], B, len_prefill,
+                                              _lib.current_stream_ptr(K.device))
+            if rc:
+                _lib.check(rc, "KittyCache.quantize_prefill")
+            return n
         kvcache.Sink_Buffer_K[rows, :, :len_sink, :].copy_(K[:, :, :len_sink, :])
         if len_qbuf_k > 0:
             kvcache.Q_Buffer_K[rows, :, :len_qbuf_k, :].copy_(K[:, :, len_prefill - len_qbuf_k:, :])
@@ -379,6 +398,21 @@ class KittyCache(_HFCache):
         new_pv = (L.Q_Buffer_Count_V + evicted) // P
         if L.PageCount_K + new_pk > L.MAX_PAGE or L.PageCount_V + new_pv > L.MAX_PAGE:
             raise ValueError(f"appending {T} tokens exceeds max_length={L.MAX_LEN}")
+        # the whole batch in two launches (a part of it would leave what the rest's Q-buffers hold out of their pages)
+        if L.on_hip and L.D == 128 and self.select == "hip" and 1 <= T <= 1 << 24 and B == L.MAX_BS \
+                and key_states.shape[1] == L.H_KV and key_states.shape[3] == L.D \
+                and L.Q_Buffer_Count_K < P and L.Q_Buffer_Count_V < P and key_states.stride() == value_states.stride() \
+                and _kernel_ready(L, key_states) and _kernel_ready(L, value_states):
+            ks = key_states.stride()
+            rc = _lib.lib().kitty_append_chunk_host(L.descriptor(), key_states.data_ptr(), value_states.data_ptr(), 2 * ks[0],
+                                                    2 * ks[1], 2 * ks[2], B, T, _lib.current_stream_ptr(key_states.device))
+            if rc:
+                _lib.check(rc, "KittyCache.append")
+            L.Sink_Count += a
+            L.PageCount_K, L.Q_Buffer_Count_K = L.PageCount_K + new_pk, (L.Q_Buffer_Count_K + n) % P
+            L.PageCount_V, L.Q_Buffer_Count_V = L.PageCount_V + new_pv, (L.Q_Buffer_Count_V + evicted) % P
+            L.Local_Count_V, L.Write_Offset_Local_V = lv_after, (L.Write_Offset_Local_V + evicted) % P
+            return
         with torch.no_grad():
             if a > 0:
                 L.Sink_Buffer_K[:B, :, L.Sink_Count:L.Sink_Count + a, :].copy_(key_states[:, :, :a, :])
