@@ -165,6 +165,8 @@ int kitty_quant_pack_v(const void* value, int64_t stride_b, int64_t stride_h, in
  */
 size_t kitty_decode_attn_workspace_bytes(int B, int H_Q, int D, int num_splits);
 int kitty_decode_attn_default_splits(int B, int H_KV, int max_tiles, int per_sequence_counts);
+/* the same for a given head dimension (kitty_decode_attn_default_splits is the rule for D = 128) */
+int kitty_decode_attn_default_splits_d(int B, int H_KV, int D, int max_tiles, int per_sequence_counts);
 int kitty_decode_attn(const kitty_kv_layer* layer, const void* q, int B, int H_Q, float scaling,
                       void* out, void* workspace, size_t workspace_bytes, int num_splits,
                       int variant, void* stream);

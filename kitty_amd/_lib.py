@@ -54,6 +54,7 @@ _SIGNATURES = {
                                    c_void_p, c_void_p]),
     "kitty_decode_attn_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),
     "kitty_decode_attn_default_splits": (c_int, [c_int, c_int, c_int, c_int]),
+    "kitty_decode_attn_default_splits_d": (c_int, [c_int, c_int, c_int, c_int, c_int]),
     "kitty_decode_attn_split": (c_int, [POINTER(KittyKVLayer), c_void_p, c_int, c_int, c_float, c_void_p, c_size_t,
                                         c_int, c_int, c_void_p]),
     "kitty_decode_attn_merge": (c_int, [c_void_p, c_size_t, c_int, c_int, c_int, c_int, c_void_p, c_void_p]),

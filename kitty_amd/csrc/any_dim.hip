@@ -14,6 +14,8 @@
 // Wire format for general D (PAGE = 128 tokens): a K page-head is 32 D bytes of low plane (channel d at
 // 32 d), 32 d_boost bytes of high plane (slot s at 32 (D + s)) and D bytes of slot map; a V page-head is
 // 128 rows of D / 4 bytes; metadata as for D = 128 with D resp. 128 (scale, zero) pairs per head.
+#include <type_traits>
+
 #include "decode_common.h"
 #include "quant_arith.h"
 
@@ -175,8 +177,7 @@ typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
 typedef short short4v __attribute__((ext_vector_type(4)));
 
 constexpr float kLog2e = 1.44269504088896340736f;
-constexpr uint32_t kCodeMask = 0x00030003u;    // the lowest code of both 16-bit pieces of a word
-constexpr uint32_t kCodeMagic = 0x64006400u;   // fp16 1024 in both halves: 1024 + code is exact
+constexpr uint32_t kCodeMagic = 0x64006400u;   // fp16 1024 in both halves: 1024 + n is exact for n < 1024
 constexpr float kProbScale = 4096.f;           // probabilities as matrix operands: see below
 
 __device__ __forceinline__ float4v mfma16(const uint32_t (&a)[4], const uint32_t (&b)[4], float4v c) {
@@ -198,13 +199,23 @@ __device__ __forceinline__ float4v mfma16(const uint32_t (&a)[4], const uint4& b
 __device__ __forceinline__ uint32_t low_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x05040100u); }
 __device__ __forceinline__ uint32_t high_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
 // fp16(code) * scale + zero with BOTH operations rounded to fp16 (kitty_attention.py:162-165, 317-320 as
-// eager torch and the Triton interpreter evaluate them), for the two codes of a word that has kCodeMagic set.
+// eager torch and the Triton interpreter evaluate them), for two codes.  `c` holds 1024 + code * 2^SHIFT in each
+// half (a code may stay at the bit where it lies): (1024 + code * 2^SHIFT) * 2^-SHIFT - 1024 * 2^-SHIFT is exact.
+template <int SHIFT>
 __device__ __forceinline__ uint32_t dequant_word(uint32_t c, uint32_t scale, uint32_t zero) {
 #pragma clang fp contract(off)
-  const half2v f = __builtin_bit_cast(half2v, c) - half2v{(_Float16)1024.f, (_Float16)1024.f};
+  constexpr _Float16 k = (_Float16)(1.0f / (1 << SHIFT)), o = (_Float16)(1024.0f / (1 << SHIFT));
+  const half2v x = __builtin_bit_cast(half2v, c);
+  const half2v f = SHIFT == 0 ? x - half2v{o, o} : __builtin_elementwise_fma(x, half2v{k, k}, half2v{-o, -o});
   const half2v m = f * __builtin_bit_cast(half2v, scale);
   const half2v r = m + __builtin_bit_cast(half2v, zero);
   return __builtin_bit_cast(uint32_t, r);
+}
+// the value codes of d-tile u of a word: codes 0 .. 4 where they lie, the others after one shift for the three
+template <int U>
+__device__ __forceinline__ uint32_t dequant_v(uint32_t x, uint32_t x10, uint32_t scale, uint32_t zero) {
+  constexpr int k = 2 * (U < 5 ? U : U - 5);
+  return dequant_word<k>(((U < 5 ? x : x10) & (0x00030003u << k)) | kCodeMagic, scale, zero);
 }
 // maximum over lanes l, l^16, l^32, l^48
 __device__ __forceinline__ float max_over_lane_groups(float v) {
@@ -241,8 +252,8 @@ struct AnyLds {
 // p0 + r % PB; after the layer's own tiles come the chunk's rows, causally; the normalised output goes to
 // out [B, T_q, H_Q, D], or with ws_ml set a partial per row to the workspace.
 //
-// What bounds it is turning codes into fp16 numbers with the reference's two roundings: 8 vector instructions
-// per two key codes, 5 per two value codes, once per code.  So every code is unpacked in the register in which the
+// What bounds it is turning codes into fp16 numbers with the reference's two roundings: 6 vector instructions
+// per two key codes, 4 per two value codes, once per code.  So every code is unpacked in the register in which the
 // matrix instruction takes it, by one lane of one wavefront: the packed bytes of a tile go to LDS as they
 // are (loaded into registers while the tile before is worked on), a transposing read hands lane n the 8 codes
 // 8n .. 8n+7 of several plane rows, and `(X >> 2u) & mask` is then one register of the operand of
@@ -255,10 +266,10 @@ struct AnyLds {
 // Probabilities stay fp32 numbers: 4096 p is split into two fp16 numbers (22 bits; a remainder below fp16's
 // normal range is below 2^-26 of the row's largest probability), each a matrix operand of its own.
 // A decode layer (append, this kernel, merge) on MI355X, against the version on the vector ALUs before it:
-//   D = 64,  B = 8, 6100 tokens, 32 / 8 heads:  79 -> 31 us
+//   D = 64,  B = 8, 6100 tokens, 32 / 8 heads:  79 -> 26 us
 //   D = 256, B = 2, 9000 tokens, 16 / 8 heads: 194 -> 36 us
 template <int D, bool PREFILL, int NT>
-__global__ __launch_bounds__(256, PREFILL ? 1 : 2) void attn_any_kernel(
+__global__ __launch_bounds__(256, PREFILL ? 1 : D == 64 ? 3 : 2) void attn_any_kernel(
     kitty_kv_layer L, const uint8_t* __restrict__ q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
     const uint8_t* __restrict__ k_new, const uint8_t* __restrict__ v_new, int64_t new_stride_b,
     int64_t new_stride_h, int64_t new_stride_t, int H_Q, int Tq, float scaling, float* __restrict__ ws_ml,
@@ -326,9 +337,14 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : 2) void attn_any_kernel(
   uint4v pk[kKIter] = {}, pv[kVIter] = {}, pm = {};
   auto k_is_packed = [&](int tile) { return tile > 0 && tile < c.ntiles && tile - 1 < c.pk; };
   auto v_is_packed = [&](int tile) { return tile > 0 && tile < c.ntiles && tile - 1 < c.pv; };
+  int64_t id_k = 0, id_v = 0;   // of the tile fetched next, asked for one tile ahead: the load behind them waits for nothing
+  auto ask = [&](int tile) {
+    if (tile < tile_end && k_is_packed(tile)) id_k = page_id(L.page_table_k, (int64_t)b * L.page_table_k_stride_b + tile - 1);
+    if (tile < tile_end && v_is_packed(tile)) id_v = page_id(L.page_table_v, (int64_t)b * L.page_table_v_stride_b + tile - 1);
+  };
   auto fetch = [&](int tile) {
     if (k_is_packed(tile)) {
-      const int64_t pg = checked_page(page_id(L.page_table_k, (int64_t)b * L.page_table_k_stride_b + tile - 1), L.cache_pages_k, bad_page);
+      const int64_t pg = checked_page(id_k, L.cache_pages_k, bad_page);
       const uint4v* src = (const uint4v*)(L.key_cache + pg * L.key_cache_stride_page + (int64_t)h * k_head_bytes_d(D, DB));
 #pragma unroll
       for (int i = 0; i < kKIter; ++i)
@@ -337,7 +353,7 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : 2) void attn_any_kernel(
         pm = ((const uint4v*)((const uint8_t*)L.key_meta + pg * L.key_meta_stride_page + (int64_t)h * D * 4))[tid];
     }
     if (v_is_packed(tile)) {
-      const int64_t pg = checked_page(page_id(L.page_table_v, (int64_t)b * L.page_table_v_stride_b + tile - 1), L.cache_pages_v, bad_page);
+      const int64_t pg = checked_page(id_v, L.cache_pages_v, bad_page);
       const uint4v* src = (const uint4v*)(L.value_cache + pg * L.value_cache_stride_page + (int64_t)h * v_head_bytes_d(D));
 #pragma unroll
       for (int i = 0; i < kVIter; ++i)
@@ -345,6 +361,7 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : 2) void attn_any_kernel(
       if (tid >= 64 && tid < 96)
         pm = ((const uint4v*)((const uint8_t*)L.value_meta + pg * L.value_meta_stride_page + (int64_t)h * kPage * 4))[tid - 64];
     }
+    ask(tile + 1);
   };
   auto stage = [&](int tile) {
     if (k_is_packed(tile)) {
@@ -361,7 +378,7 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : 2) void attn_any_kernel(
     }
   };
 
-  if (tile_begin < tile_end) fetch(tile_begin);
+  if (tile_begin < tile_end) ask(tile_begin), fetch(tile_begin);
 #pragma unroll 1
   for (int tile = tile_begin; tile < tile_end; ++tile) {
     const bool chunk = tile >= c.ntiles;                       // a tile of the new chunk (prefill only)
@@ -382,7 +399,6 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : 2) void attn_any_kernel(
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) S[e][nt] = float4v{0.f, 0.f, 0.f, 0.f};
     if (k_packed) {
-      const int sh = 4 * w;
       const uint8_t* idx = lds + kRowBytes * (D + DB);
       const int quarter = (n & 3) * 8;
 #pragma unroll 2
@@ -402,27 +418,30 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : 2) void attn_any_kernel(
         uint4 qq[NT];
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) qq[nt] = s_q[(kc * NT + nt) * 64 + lane];
+        uint32_t a0[4], a1[4];
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          uint32_t a[4];
+        for (int i = 0; i < 4; ++i) {
+          const uint32_t lo = X[i] >> (4 * w), hi = (H[i] >> (4 * w)) << 2;   // code e: bits 2e, 2e + 1 of lo, two further up in hi
+          const uint32_t c0 = (lo & 0x00030003u) | (hi & ~0x00030003u), c1 = (lo & 0x000c000cu) | (hi & ~0x000c000cu);
+          a0[i] = dequant_word<0>((c0 & 0x000f000fu) | kCodeMagic, sc[i], zr[i]);
+          a1[i] = dequant_word<2>((c1 & 0x003c003cu) | kCodeMagic, sc[i], zr[i]);
+        }
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const uint32_t lo = ((X[i] >> (sh + 2 * e)) & kCodeMask) | kCodeMagic;
-            const uint32_t hi = (H[i] >> (sh + 2 * e)) & kCodeMask;
-            a[i] = dequant_word((hi << 2) | lo, sc[i], zr[i]);
-          }
-#pragma unroll
-          for (int nt = 0; nt < NT; ++nt) S[e][nt] = mfma16(a, qq[nt], S[e][nt]);
+        for (int nt = 0; nt < NT; ++nt) {
+          S[0][nt] = mfma16(a0, qq[nt], S[0][nt]);
+          S[1][nt] = mfma16(a1, qq[nt], S[1][nt]);
         }
       }
     } else {
       const uint8_t* base = chunk ? k_new + (int64_t)b * new_stride_b + (int64_t)h * new_stride_h + (int64_t)chunk_t0 * new_stride_t
                           : tile == 0 ? (const uint8_t*)L.sink_k + sink_base : (const uint8_t*)L.qbuf_k + win_base;
       const int64_t stride = chunk ? new_stride_t : (int64_t)(2 * D);
+      int first = 8 * n + 2 * w;
+      asm volatile("" : "+v"(first));   // these addresses are formed here, not kept in registers over the packed tiles
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
         // a token past the end repeats the last one: its logits are masked below
-        const uint8_t* row = base + (int64_t)min(8 * n + 2 * w + e, ntok - 1) * stride;
+        const uint8_t* row = base + (int64_t)min(first + e, ntok - 1) * stride;
 #pragma unroll 4
         for (int kc = 0; kc < D / 32; ++kc) {
           const uint2 x0 = *(const uint2*)(row + (32 * kc + 4 * kg) * 2);
@@ -500,26 +519,42 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : 2) void attn_any_kernel(
 #pragma unroll
           for (int j = 0; j < 4; ++j) X[j] >>= n & 8;
         }
+        uint32_t X10[4];
 #pragma unroll
-        for (int u = 0; u < kU; ++u) {
+        for (int j = 0; j < 4; ++j) X10[j] = X[j] >> 10;
+        auto tile = [&](auto u_) {
+          constexpr int u = decltype(u_)::value;
           uint32_t a[4];
 #pragma unroll
-          for (int j = 0; j < 4; ++j) a[j] = dequant_word(((X[j] >> (2 * u)) & kCodeMask) | kCodeMagic, sc[j], zr[j]);
+          for (int j = 0; j < 4; ++j) a[j] = dequant_v<u>(X[j], X10[j], sc[j], zr[j]);
 #pragma unroll
           for (int nt = 0; nt < NT; ++nt) {
             O[hf * kU + u][nt] = mfma16(a, ph[nt], O[hf * kU + u][nt]);
             O[hf * kU + u][nt] = mfma16(a, pl[nt], O[hf * kU + u][nt]);
           }
+        };
+        tile(std::integral_constant<int, 0>{}), tile(std::integral_constant<int, 1>{});
+        tile(std::integral_constant<int, 2>{}), tile(std::integral_constant<int, 3>{});
+        if constexpr (kU == 8) {
+          tile(std::integral_constant<int, 4>{}), tile(std::integral_constant<int, 5>{});
+          tile(std::integral_constant<int, 6>{}), tile(std::integral_constant<int, 7>{});
         }
       }
     } else {
+      int first = t0;
+      asm volatile("" : "+v"(first));   // as above
+      // rows u < lows of one tensor, then the ring's (a tail tile only)
+      const int u0 = chunk || tile == 0 ? 0 : (body - c.pv) * kPage, lows = chunk || tile == 0 ? kPage : c.rv;
+      const uint8_t* low = chunk ? v_new + (int64_t)b * new_stride_b + (int64_t)h * new_stride_h + (int64_t)chunk_t0 * new_stride_t
+                         : tile == 0 ? (const uint8_t*)L.sink_v + sink_base : (const uint8_t*)L.qbuf_v + win_base;
+      const int64_t stride = chunk ? new_stride_t : (int64_t)(2 * D);
+      const uint8_t* ring = (const uint8_t*)L.local_v + win_base;
       const uint8_t* rows[8];   // the rows of tokens t0 + 8 j + e
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const int tok = min(t0 + 8 * (i >> 1) + (i & 1), ntok - 1);
-        if (chunk) rows[i] = v_new + (int64_t)b * new_stride_b + (int64_t)h * new_stride_h + (int64_t)(chunk_t0 + tok) * new_stride_t;
-        else if (tile == 0) rows[i] = (const uint8_t*)L.sink_v + sink_base + (int64_t)tok * (2 * D);
-        else rows[i] = (const uint8_t*)v_tail_row(L, c, b, h, (body - c.pv) * kPage + tok, D);
+        const int u = u0 + min(first + 8 * (i >> 1) + (i & 1), ntok - 1);
+        const int64_t in_low = (int64_t)u * stride, in_ring = (int64_t)((c.off + u - lows) & (kPage - 1)) * (2 * D);
+        rows[i] = (u < lows ? low : ring) + (u < lows ? in_low : in_ring);
       }
 #pragma unroll
       for (int hf = 0; hf < kHalves; ++hf) {
@@ -530,7 +565,7 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : 2) void attn_any_kernel(
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           x[i] = *(const words*)(rows[i] + ch * 2);
-          if (t0 + 8 * (i >> 1) + (i & 1) >= ntok) x[i] = words{};   // probability 0 times what a dead row may hold must be 0
+          if (first + 8 * (i >> 1) + (i & 1) >= ntok) x[i] = words{};   // probability 0 times what a dead row may hold must be 0
         }
 #pragma unroll
         for (int u = 0; u < kU; ++u) {
@@ -671,6 +706,21 @@ int any_positions(int D, int G) {
   return rows / G > 0 ? rows / G : 1;
 }
 }  // namespace
+
+// Splits of a decode walk.  Three workgroups fit a compute unit at D = 64 (registers), two at D = 256.  Long walks are
+// cut for three per unit (D = 256, B = 4, 30000 tokens: 99 us with 24 splits, 114 with 64, 126 with 8; D = 64, B = 8, 6100
+// tokens: 23.7 us with 10 splits of five tiles, 27.0 with 17 of three), shares of under three tiles for two, so that there
+// is no second round of them (D = 256, B = 2, 9000 tokens: 30 us with 24 splits of three tiles, 32 with 36 of two).
+// Where all of it fits at once a split is a tile: each costs 1.5 to 3.5 us of latency (D = 256, B = 1, 2000 tokens: 13.5 us
+// with 17 splits, 16.9 with 9).
+int decode_splits_any(int B, int H_KV, int tiles, int units) {
+  const int64_t walks = (int64_t)B * H_KV;
+  int64_t s = 3 * units / walks;
+  if (s > 0 && tiles / s < 3) s = 2 * units / walks;
+  if (s > tiles) s = tiles;
+  if (s > 512) s = 512;
+  return s < 1 ? 1 : (int)s;
+}
 
 // Shares of a chunk's walk: enough workgroups for two on every compute unit (what their registers allow at
 // D = 256), of at least two tiles each.

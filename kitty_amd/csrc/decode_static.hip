@@ -62,7 +62,7 @@ extern "C" int kitty_decode_attn_static(const kitty_kv_layer* layer, const void*
   const size_t per_split = ws_total_bytes(B, H_Q, 1, layer->D) + 768;   // an upper bound of the growth per split
   if (num_splits <= 0) {
     // the default of kitty_decode_attn, cut back to what the array holds
-    num_splits = kitty_decode_attn_default_splits(B, layer->H_KV, max_tiles, layer->seq_counts != nullptr);
+    num_splits = kitty_decode_attn_default_splits_d(B, layer->H_KV, layer->D, max_tiles, layer->seq_counts != nullptr);
     const size_t fit = KITTY_STATIC_WORKSPACE_BYTES / per_split;
     if ((size_t)num_splits > fit) num_splits = (int)fit;
     KITTY_REQUIRE(num_splits >= 1, KITTY_E_WORKSPACE,

@@ -24,7 +24,7 @@ def _split_plan(B: int, H_Q: int, H_KV: int, D: int, max_tiles: int, per_sequenc
     """(splits, workspace bytes) of a decode launch: a function of the sizes alone."""
     lib = _lib.lib()
     if num_splits <= 0:
-        num_splits = lib.kitty_decode_attn_default_splits(B, H_KV, max_tiles, int(per_sequence))
+        num_splits = lib.kitty_decode_attn_default_splits_d(B, H_KV, D, max_tiles, int(per_sequence))
     return num_splits, lib.kitty_decode_attn_workspace_bytes(B, H_Q, D, num_splits)
 
 
