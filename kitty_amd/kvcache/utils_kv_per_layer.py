@@ -185,6 +185,13 @@ class KVCache_Layer:
         d.seq_counts = None if self.seq_counts is None else self.seq_counts.data_ptr()
         return d
 
+    def empty_descriptor(self) -> "_lib.KittyKVLayer":
+        """This layer as if it held nothing: what a prompt attends to before it is packed."""
+        d = _lib.KittyKVLayer.from_buffer_copy(self.descriptor())
+        d.counts[:] = [0] * _lib.SEQ_COUNT_FIELDS
+        d.seq_counts = None
+        return d
+
     def workspace(self, nbytes: int) -> torch.Tensor:
         """Split-K scratch, grown on demand and kept with the layer (the reference allocates its
         score tensor on every call, kitty_attention.py:425-430)."""
