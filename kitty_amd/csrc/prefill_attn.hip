@@ -44,8 +44,10 @@ typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float float4v __attribute__((ext_vector_type(4)));
 typedef short short4v __attribute__((ext_vector_type(4)));
+typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
 
 constexpr int kPitch = 288;                   // bytes per LDS row: 128 fp16 + 32 bytes of padding
+constexpr int kRowPitch = 272;                // of a K tile in the dense kernel
 constexpr int kTile = kPage * kPitch;         // 36864 bytes, one K or V tile
 constexpr int kLdsBytes = 4 * kTile;          // K and V, two buffers each
 constexpr int kRows = 256;                    // query rows per workgroup
@@ -90,6 +92,12 @@ __device__ __forceinline__ half4 lds_tr(const uint8_t* p) {
 // matrix-core A operand: k-slots 0..3 from the 4 LDS rows at p, k-slots 4..7 from 16 rows further
 __device__ __forceinline__ half8 load_a(const uint8_t* p) {
   const half4 a0 = lds_tr(p), a1 = lds_tr(p + 16 * kPitch);
+  return __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+// the dense kernel's: channels 4 kg .. of a 32-channel chunk and those 16 further, from one fp16 row
+__device__ __forceinline__ half8 load_row_a(const uint8_t* p) {
+  const half4 a0 = *(const half4*)p, a1 = *(const half4*)(p + 32);
   return __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
@@ -339,9 +347,10 @@ struct WaveAcc {
 // limit[nt]: tokens of the tile with index < limit are visible to the row of column tile nt.
 // SPLIT: the walk starts anywhere in the sequence, so a row may see nothing of the first sub-tile (and
 // then, causally, nothing at all of this share): its running maximum must stay a number.
-template <bool SPLIT>
+// DENSE: tokens and channels lie in their natural order, and K as [token][channel] (see dense_attn_kernel).
+template <bool SPLIT, bool DENSE>
 struct TileAttend {
-  const uint8_t* kb;   // K tile + this lane's corner of a transposing read
+  const uint8_t* kb;   // K tile + this lane's corner of a transposing read; DENSE: + its row and channels
   const uint8_t* vb;   // V tile + the same corner
   const half8 (&q)[4][kNT];
   WaveAcc& A;
@@ -355,12 +364,12 @@ struct TileAttend {
     for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
       for (int nt = 0; nt < kNT; ++nt) S[mt][nt] = float4v{0.f, 0.f, 0.f, 0.f};
-    const uint8_t* kbase = kb + sub * 64;
+    const uint8_t* kbase = kb + sub * (DENSE ? 32 * kRowPitch : 64);
 #pragma unroll
     for (int c = 0; c < 4; ++c)
 #pragma unroll
       for (int mt = 0; mt < 2; ++mt) {
-        const half8 a = load_a(kbase + (32 * c) * kPitch + mt * 32);
+        const half8 a = DENSE ? load_row_a(kbase + mt * 16 * kRowPitch + c * 64) : load_a(kbase + (32 * c) * kPitch + mt * 32);
 #pragma unroll
         for (int nt = 0; nt < kNT; ++nt) S[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, q[c][nt], S[mt][nt], 0, 0, 0);
       }
@@ -379,7 +388,7 @@ struct TileAttend {
         for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const int tok = 32 * sub + 16 * mt + 2 * kg + (i >> 1) + 8 * (i & 1);
+            const int tok = 32 * sub + 16 * mt + (DENSE ? 4 * kg + i : 2 * kg + (i >> 1) + 8 * (i & 1));
             if (tok >= limit[nt]) S[mt][nt][i] = -INFINITY;
           }
       asm volatile("" ::: "memory");   // keep this a branch, not selects on every tile
@@ -604,7 +613,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
       uint32_t ok_ = buf * kTile + (4 * kg + (n >> 2)) * kPitch + (n & 3) * 8;
       uint32_t ov_ = ok_ + 2 * kTile;
       asm volatile("" : "+v"(ok_), "+v"(ov_));
-      const TileAttend<SPLIT> T{lds + ok_, lds + ov_, qreg, A, sc2, masked, limit, kg};
+      const TileAttend<SPLIT, false> T{lds + ok_, lds + ov_, qreg, A, sc2, masked, limit, kg};
       T.run((cur.ntok + 31) >> 5);
     }
     if (more && !convert_first) P.finish(nxt, ga, kn, vn);
@@ -648,6 +657,159 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
   report_bad_page(L, b, P.bad_page);   // by whichever thread met one
 }
 
+// A chunk over a layer that holds nothing: dense causal attention.  The frame is that of the kernel above - 256
+// rows a workgroup, two tile buffers, waves of a SIMD that stage and multiply in opposite order - but every tile is
+// fp16 rows, so nothing has to be permuted to meet codes: a row is copied as it lies, loaded into registers while the
+// tile before it is worked on.  K stays [token][channel] with 272 bytes from row to row (16 rows x two lane groups of
+// 8-byte operand reads on 64 different banks); V [token][channel] is read transposed.  On the kernel above such a tile
+// costs twice a packed one: its rows are fetched when they are needed, K goes in by 16-bit transposing stores, every
+// tile is masked.  Workgroups of one kv head share an XCD, whose L2 then serves its keys and values, longest first.
+// Bound by the vector and LDS work around the matrix instructions (exponentials, operand reads).
+// B = 2, 3001 tokens, 32 / 8 heads: 448 us on the kernel above, 238 here (620 TFLOP/s).
+template <bool SPLIT>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves / 4, kWaves / 4))) void dense_attn_kernel(
+    const uint8_t* __restrict__ q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
+    const uint8_t* __restrict__ k_new, const uint8_t* __restrict__ v_new, int64_t new_stride_b, int64_t new_stride_h,
+    int64_t new_stride_t, int H_Q, int H_KV, int Tq, float scaling, __half* __restrict__ out, float* __restrict__ ws_ml,
+    float* __restrict__ ws_acc, int num_splits, int heads) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, kg = lane >> 4, n = lane & 15;
+  // blockIdx.x -> (kv head of a batch row, block x split): consecutive workgroups go to the XCDs in turn
+  const int id = blockIdx.x;
+  int head, item;
+  if (heads % 8 == 0) {
+    const int per_xcd = heads / 8, j = id / 8;
+    head = (j % per_xcd) * 8 + id % 8, item = j / per_xcd;
+  } else {
+    head = id % heads, item = id / heads;
+  }
+  const int b = head / H_KV, h = head % H_KV;
+  const int G = H_Q / H_KV;
+  const int PB = block_positions(G, Tq);
+  const int split = SPLIT ? item % num_splits : 0;
+  const int blk = c_div_up(Tq, PB) - 1 - (SPLIT ? item / num_splits : item);   // longest causal extent first
+  const int p0 = blk * PB, kv = min(Tq, p0 + PB);
+  const int n_tiles = c_div_up(kv, kPage);
+  int t_begin = 0, t_end = n_tiles;
+  if (SPLIT) {
+    const int share = c_div_up(n_tiles, num_splits);
+    t_begin = min(split * share, n_tiles);
+    t_end = min(t_begin + share, n_tiles);
+  }
+  const uint8_t* kc = k_new + (int64_t)b * new_stride_b + (int64_t)h * new_stride_h;
+  const uint8_t* vc = v_new + (int64_t)b * new_stride_b + (int64_t)h * new_stride_h;
+
+  half8 qreg[4][kNT];
+  int qpos[kNT];
+#pragma unroll
+  for (int nt = 0; nt < kNT; ++nt) {
+    const int r = 16 * kNT * w + 16 * nt + n;
+    const int g = r / PB, pos = p0 + r % PB;
+    const bool ok = g < G && pos < Tq;
+    qpos[nt] = ok ? pos : -1;
+    const uint8_t* row = q + (int64_t)b * q_stride_b + (int64_t)(h * G + (ok ? g : 0)) * q_stride_h +
+                         (int64_t)(ok ? pos : 0) * q_stride_t;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      uint2 x0 = *(const uint2*)(row + (32 * c + 4 * kg) * 2);
+      uint2 x1 = *(const uint2*)(row + (32 * c + 16 + 4 * kg) * 2);
+      if (!ok) x0 = x1 = uint2{0u, 0u};
+      const uint4 x = uint4{x0.x, x0.y, x1.x, x1.y};
+      qreg[c][nt] = __builtin_bit_cast(half8, x);
+    }
+  }
+  WaveAcc A;
+#pragma unroll
+  for (int ct = 0; ct < 8; ++ct)
+#pragma unroll
+    for (int nt = 0; nt < kNT; ++nt) A.o[ct][nt] = float4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int nt = 0; nt < kNT; ++nt) A.m[nt] = 0.f, A.l[nt] = 0.f;
+  A.first = true;
+  const float sc2 = scaling * kLog2e;
+
+  // a thread stages 16-byte pieces part, part + 4, .. of one token
+  const int e = tid / kParts, part = tid % kParts;
+  uint4v kk[2 * kW], vv[2 * kW];
+  auto issue = [&](int t) {
+    const int tok = t * kPage + e;
+    const int64_t off = (int64_t)min(tok, kv - 1) * new_stride_t + part * 16;
+#pragma unroll
+    for (int i = 0; i < 2 * kW; ++i) {
+      kk[i] = *(const uint4v*)(kc + off + i * (16 * kParts));
+      vv[i] = *(const uint4v*)(vc + off + i * (16 * kParts));
+    }
+    if (tok >= kv) {   // dead rows of V must be finite
+#pragma unroll
+      for (int i = 0; i < 2 * kW; ++i) vv[i] = uint4v{0u, 0u, 0u, 0u};
+    }
+  };
+  auto finish = [&](int buf) {
+    uint8_t* kt = lds + buf * kTile + e * kRowPitch + part * 16;
+    uint8_t* vt = lds + (2 + buf) * kTile + e * kPitch + part * 16;
+#pragma unroll
+    for (int i = 0; i < 2 * kW; ++i) {
+      *(uint4v*)(kt + i * (16 * kParts)) = kk[i];
+      *(uint4v*)(vt + i * (16 * kParts)) = vv[i];
+    }
+  };
+  const bool stage_first = w < kWaves / 2;
+  if (!SPLIT || t_begin < t_end) {
+    issue(t_begin);
+    finish(0);
+    if (t_begin + 1 < t_end) issue(t_begin + 1);
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int t = t_begin; t < t_end; ++t) {
+    const int buf = (t - t_begin) & 1;
+    auto stage_next = [&] {
+      if (t + 1 < t_end) finish(buf ^ 1);
+      if (t + 2 < t_end) issue(t + 2);
+    };
+    if (stage_first) stage_next();
+    const int t0 = t * kPage, ntok = min(kPage, kv - t0);
+    int limit[kNT];
+#pragma unroll
+    for (int nt = 0; nt < kNT; ++nt) limit[nt] = min(ntok, qpos[nt] - t0 + 1);
+    // a full tile in front of the workgroup's first position is seen whole by every row
+    const bool masked = t0 + kPage - 1 > p0;
+    {
+      uint32_t ok_ = buf * kTile + n * kRowPitch + kg * 8;
+      uint32_t ov_ = (2 + buf) * kTile + (4 * kg + (n >> 2)) * kPitch + (n & 3) * 8;
+      asm volatile("" : "+v"(ok_), "+v"(ov_));
+      const TileAttend<SPLIT, true> T{lds + ok_, lds + ov_, qreg, A, sc2, masked, limit, kg};
+      T.run((ntok + 31) >> 5);
+    }
+    if (!stage_first) stage_next();
+    __syncthreads();
+  }
+
+#pragma unroll
+  for (int nt = 0; nt < kNT; ++nt) {
+    float l = A.l[nt];
+    l += xor_lanes(l, 16);
+    l += xor_lanes(l, 32);
+    if (qpos[nt] < 0) continue;
+    const int r = 16 * kNT * w + 16 * nt + n;
+    const int64_t row = ((int64_t)b * Tq + qpos[nt]) * H_Q + (h * G + r / PB);
+    if (SPLIT) {
+      const int64_t prow = row * num_splits + split;
+      if (kg == 0) *(float2*)(ws_ml + prow * 2) = float2{l == 0.f ? -INFINITY : A.m[nt], l};   // 0: this row saw nothing here
+#pragma unroll
+      for (int ct = 0; ct < 8; ++ct) *(float4v*)(ws_acc + prow * kD + 16 * ct + 4 * kg) = A.o[ct][nt];
+      continue;
+    }
+    const float inv = 1.f / l;
+#pragma unroll
+    for (int ct = 0; ct < 8; ++ct) {
+      const float4v o = A.o[ct][nt] * inv;
+      __half2 x[2] = {__floats2half2_rn(o[0], o[1]), __floats2half2_rn(o[2], o[3])};
+      *(uint2*)(out + row * kD + 16 * ct + 4 * kg) = *(const uint2*)x;
+    }
+  }
+}
+
 }  // namespace
 
 int prefill_lds_bytes() { return kLdsBytes; }
@@ -681,6 +843,27 @@ void launch_prefill_attn(const kitty_kv_layer& L, const void* q, int64_t q_strid
   const int G = H_Q / L.H_KV;
   const int blocks = c_div_up(Tq, block_positions(G, Tq));
   dim3 grid(blocks * num_splits, L.H_KV, B), block(kThreads);
+  const int* c = L.counts;
+  const int64_t dense_wgs = (int64_t)blocks * num_splits * L.H_KV * B;
+  if (!L.seq_counts && c[KITTY_CNT_SINK] == 0 && c[KITTY_CNT_PAGES_K] + c[KITTY_CNT_QBUF_K] == 0 && dense_wgs <= INT32_MAX) {
+    // (check_layer: as many values as keys)
+#define KITTY_LAUNCH_DENSE(SPLIT)                                                                                \
+  do {                                                                                                           \
+    (void)hipFuncSetAttribute((const void*)dense_attn_kernel<SPLIT>, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes); \
+    hipLaunchKernelGGL((dense_attn_kernel<SPLIT>), dim3((unsigned)dense_wgs), block, kLdsBytes, stream, (const uint8_t*)q, \
+                       q_stride_b, q_stride_h, q_stride_t, (const uint8_t*)k_new, (const uint8_t*)v_new, new_stride_b, \
+                       new_stride_h, new_stride_t, H_Q, L.H_KV, Tq, scaling, (__half*)out, ws_ml, ws_acc, num_splits,  \
+                       L.H_KV * B);                                                                              \
+  } while (0)
+    if (num_splits > 1) {
+      KITTY_LAUNCH_DENSE(true);
+      launch_rows_merge(kD, ws_ml, ws_acc, out, (int64_t)B * Tq * H_Q, num_splits, /* keep_nan */ true, stream);
+    } else {
+      KITTY_LAUNCH_DENSE(false);
+    }
+#undef KITTY_LAUNCH_DENSE
+    return;
+  }
 #define KITTY_LAUNCH_PREFILL(BOOST, SPLIT)                                                                       \
   do {                                                                                                           \
     /* more LDS than the default per-workgroup limit; per device, so set on every launch */                      \

@@ -20,7 +20,7 @@ def _setup(B, T, H_Q, H, layout):
 
 
 @pytest.mark.parametrize("T", [1, 31, 129, 257, 700])
-@pytest.mark.parametrize("H_Q,H,layout", [(2, 2, "token-major"), (8, 2, "contiguous"), (24, 2, "token-major")])
+@pytest.mark.parametrize("H_Q,H,layout", [(2, 2, "token-major"), (8, 2, "contiguous"), (24, 2, "token-major"), (8, 8, "token-major"), (8, 4, "contiguous")])
 def test_prompt_attention(T, H_Q, H, layout):
     if not torch.cuda.is_available():
         pytest.skip("needs a GPU")
