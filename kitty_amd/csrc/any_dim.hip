@@ -266,7 +266,7 @@ struct AnyLds {
 // Probabilities stay fp32 numbers: 4096 p is split into two fp16 numbers (22 bits; a remainder below fp16's
 // normal range is below 2^-26 of the row's largest probability), each a matrix operand of its own.
 // A decode layer (append, this kernel, merge) on MI355X, against the version on the vector ALUs before it:
-//   D = 64,  B = 8, 6100 tokens, 32 / 8 heads:  79 -> 26 us
+//   D = 64,  B = 8, 6100 tokens, 32 / 8 heads:  79 -> 25 us
 //   D = 256, B = 2, 9000 tokens, 16 / 8 heads: 194 -> 36 us
 template <int D, bool PREFILL, int NT>
 __global__ __launch_bounds__(256, PREFILL ? 1 : D == 64 ? 3 : 2) void attn_any_kernel(
@@ -291,8 +291,14 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : D == 64 ? 3 : 2) void attn_any_k
   const int p0 = PREFILL ? ((int)blockIdx.x / num_splits) * PB : 0;
   const int kv_chunk = PREFILL ? min(Tq, p0 + PB) : 0;           // chunk tokens this workgroup can see
   const int n_tiles = c.ntiles + (kv_chunk + kPage - 1) / kPage;
-  const int share = (n_tiles + num_splits - 1) / num_splits;
-  const int tile_begin = min(split * share, n_tiles), tile_end = min(n_tiles, tile_begin + share);
+  int tile_begin, tile_end;
+  if (D == 64) {   // shares that differ by at most one tile (B = 8, 6100 tokens: 24.1 -> 22.8 us)
+    const int least = n_tiles / num_splits, longer = n_tiles - least * num_splits;
+    tile_begin = split * least + min(split, longer), tile_end = tile_begin + least + (split < longer ? 1 : 0);
+  } else {         // equal ones, the last may be empty: at D = 256 the compiler's code for the above costs 5 %
+    const int share = (n_tiles + num_splits - 1) / num_splits;
+    tile_begin = min(split * share, n_tiles), tile_end = min(n_tiles, tile_begin + share);
+  }
   int bad_page = 0;
 
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -709,7 +715,7 @@ int any_positions(int D, int G) {
 
 // Splits of a decode walk.  Three workgroups fit a compute unit at D = 64 (registers), two at D = 256.  Long walks are
 // cut for three per unit (D = 256, B = 4, 30000 tokens: 99 us with 24 splits, 114 with 64, 126 with 8; D = 64, B = 8, 6100
-// tokens: 23.7 us with 10 splits of five tiles, 27.0 with 17 of three), shares of under three tiles for two, so that there
+// tokens: 22.8 us with 12 splits of four or five tiles, 25.5 with 17), shares of under three tiles for two, so that there
 // is no second round of them (D = 256, B = 2, 9000 tokens: 30 us with 24 splits of three tiles, 32 with 36 of two).
 // Where all of it fits at once a split is a tile: each costs 1.5 to 3.5 us of latency (D = 256, B = 1, 2000 tokens: 13.5 us
 // with 17 splits, 16.9 with 9).
