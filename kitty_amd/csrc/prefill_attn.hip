@@ -606,7 +606,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
 #pragma unroll
     for (int nt = 0; nt < kNT; ++nt)
       limit[nt] = cur.chunk_t0 >= 0 ? min(cur.ntok, qpos[nt] - cur.chunk_t0 + 1) : cur.ntok;
-    const bool masked = cur.chunk_t0 >= 0 || cur.ntok < kPage;
+    // (a tile of the chunk that ends in front of the workgroup's first position is seen whole by every row)
+    const bool masked = cur.ntok < kPage || (cur.chunk_t0 >= 0 && cur.chunk_t0 + kPage - 1 > p0);
     if (has_rows) {
       // the lane's corner inside a 16-lane transposing read: row n / 4 of 4, columns 4 (n % 4) ..;
       // made opaque so that every read's offset stays a small immediate on these two bases
@@ -831,7 +832,7 @@ int prefill_splits(int B, int H_Q, int H_KV, int Tq, int tiles, int units) {
     const int64_t rounds = (wgs * s + units - 1) / units;
     float us = 5.4f * (float)rounds * (float)(c_div_up(tiles, s) + 3);
     if (s > 1) us += 4.f + rows * (float)s * 3.5e-4f;   // write + read of 1 KB at about 3 TB/s
-    if (s == 1 || us < 0.95f * best_us) best = s, best_us = us;
+    if (s == 1 || us < 0.98f * best_us) best = s, best_us = us;
   }
   return best;
 }

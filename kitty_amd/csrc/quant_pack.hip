@@ -770,15 +770,19 @@ __global__ __launch_bounds__(256) void chunk_quant_kernel(kitty_kv_layer L, cons
   }
 }
 
-// grid (H_KV, B): the fp16 rows of one (b, h) after the chunk - sink rows, what is left of the two
+// grid (H_KV, B, 2): the fp16 rows of one (b, h) after the chunk - sink rows, what is left of the two
 // streams (the new Q-buffer contents) and the ring.  Runs after chunk_quant_kernel, which reads the
 // old Q-buffers and ring.  Rows are moved by 16 lanes x 16 bytes.
+// 64 rows at a time and the keys' rows beside the values' (blockIdx.z): the loops below wait for memory once per
+// turn (with 16 rows at a time and both in one workgroup: 12.3 us for 200 tokens, 8 kv heads, half of what that append took).
+constexpr int kRowThreads = 1024, kRowStep = kRowThreads / 16;
 template <bool HOST>
-__global__ __launch_bounds__(256) void chunk_rows_kernel(kitty_kv_layer L, const uint8_t* __restrict__ k_new,
+__global__ __launch_bounds__(kRowThreads) void chunk_rows_kernel(kitty_kv_layer L, const uint8_t* __restrict__ k_new,
                                                          const uint8_t* __restrict__ v_new, int64_t stride_b,
                                                          int64_t stride_h, int64_t stride_t, int T) {
   __shared__ uint4 s_stage[kPage][16];   // ring rows on their way to the V Q-buffer
   const int h = blockIdx.x, b = blockIdx.y;
+  const bool values = blockIdx.z != 0;
   const ChunkPlan c = chunk_plan<HOST>(L, b, T);
   if (!c.active) return;
   if (!HOST && !chunk_pages_ok(L, b, c)) return;
@@ -790,20 +794,22 @@ __global__ __launch_bounds__(256) void chunk_rows_kernel(kitty_kv_layer L, const
   // sink
   {
     const int64_t so = (int64_t)b * L.sink_stride_b + (int64_t)h * L.sink_stride_h;
-    for (int i = r0; i < c.a; i += 16) {
-      ((uint4*)((uint8_t*)L.sink_k + so + (int64_t)(c.sink + i) * (kD * 2)))[piece] = row16(ksrc + (int64_t)i * stride_t);
-      ((uint4*)((uint8_t*)L.sink_v + so + (int64_t)(c.sink + i) * (kD * 2)))[piece] = row16(vsrc + (int64_t)i * stride_t);
-    }
+    uint8_t* sink = (uint8_t*)(values ? L.sink_v : L.sink_k) + so;
+    for (int i = r0; i < c.a; i += kRowStep)
+      ((uint4*)(sink + (int64_t)(c.sink + i) * (kD * 2)))[piece] = row16((values ? vsrc : ksrc) + (int64_t)i * stride_t);
   }
   if (c.n == 0) return;
   ksrc += (int64_t)c.a * stride_t;
   vsrc += (int64_t)c.a * stride_t;
   // K: stream rows 128 npk + i -> Q_Buffer_K[i]; rows that already sit there stay (no page was cut)
   // (HOST: and past the fill count the rows of the page that went through the Q-buffer, as they would lie there)
-  const int k_end = HOST && c.npk > 0 && c.rk > 0 ? kPage : c.rk2;
-  for (int i = (c.npk ? 0 : c.rk) + r0; i < k_end; i += 16) {
-    const int s = i < c.rk2 ? c.npk * kPage + i : i;
-    if (s >= c.rk) ((uint4*)((uint8_t*)L.qbuf_k + w + (int64_t)i * (kD * 2)))[piece] = row16(ksrc + (int64_t)(s - c.rk) * stride_t);
+  if (!values) {
+    const int k_end = HOST && c.npk > 0 && c.rk > 0 ? kPage : c.rk2;
+    for (int i = (c.npk ? 0 : c.rk) + r0; i < k_end; i += kRowStep) {
+      const int s = i < c.rk2 ? c.npk * kPage + i : i;
+      if (s >= c.rk) ((uint4*)((uint8_t*)L.qbuf_k + w + (int64_t)i * (kD * 2)))[piece] = row16(ksrc + (int64_t)(s - c.rk) * stride_t);
+    }
+    return;
   }
   // V: the same, but a stream row may lie in the ring, whose slots are about to be overwritten:
   // those rows go through LDS
@@ -814,13 +820,13 @@ __global__ __launch_bounds__(256) void chunk_rows_kernel(kitty_kv_layer L, const
   const bool through = HOST && c.npv > 0 && waiting > 0 && !(c.rv == 0 && c.er == kPage && c.off == 0);
   const int last = min((waiting - 1) / kPage, c.npv - 1), v_end = through ? kPage : c.rv2;
   auto stream_row = [&](int i) { return i < c.rv2 ? c.npv * kPage + i : last * kPage + i; };
-  for (int i = lo + r0; i < v_end; i += 16) {
+  for (int i = lo + r0; i < v_end; i += kRowStep) {
     const int s = stream_row(i);
     if (s >= c.rv && s < waiting)
       s_stage[i][piece] = row16((const uint8_t*)L.local_v + w + (int64_t)((c.off + s - c.rv) & (kPage - 1)) * (kD * 2));
   }
   __syncthreads();
-  for (int i = lo + r0; i < v_end; i += 16) {
+  for (int i = lo + r0; i < v_end; i += kRowStep) {
     const int s = stream_row(i);
     if (s < c.rv) continue;   // lies there already
     const uint4 v = s < waiting ? s_stage[i][piece] : row16(vsrc + (int64_t)(s - waiting) * stride_t);
@@ -828,7 +834,7 @@ __global__ __launch_bounds__(256) void chunk_rows_kernel(kitty_kv_layer L, const
   }
   // ring: the chunk rows that stay take the slots single steps would have given them
   const int base = c.lv < kPage ? c.lv : c.off;
-  for (int j = c.e - c.er + r0; j < c.n; j += 16)
+  for (int j = c.e - c.er + r0; j < c.n; j += kRowStep)
     ((uint4*)((uint8_t*)L.local_v + w + (int64_t)((base + j) & (kPage - 1)) * (kD * 2)))[piece] =
         row16(vsrc + (int64_t)j * stride_t);
 }
@@ -1162,7 +1168,7 @@ extern "C" int kitty_append_chunk(const kitty_kv_layer* layer, const void* k_new
   const hipStream_t st = (hipStream_t)stream;
   hipLaunchKernelGGL(chunk_quant_kernel<false>, dim3(2 * max_pages, layer->H_KV, B), dim3(256), 0, st, *layer,
                      (const uint8_t*)k_new, (const uint8_t*)v_new, stride_b, stride_h, stride_t, T, max_pages);
-  hipLaunchKernelGGL(chunk_rows_kernel<false>, dim3(layer->H_KV, B), dim3(256), 0, st, *layer, (const uint8_t*)k_new,
+  hipLaunchKernelGGL(chunk_rows_kernel<false>, dim3(layer->H_KV, B, 2), dim3(kRowThreads), 0, st, *layer, (const uint8_t*)k_new,
                      (const uint8_t*)v_new, stride_b, stride_h, stride_t, T);
   hipLaunchKernelGGL(chunk_advance_kernel, dim3(B), dim3(64), 0, st, *layer, T);
   return check_launch("kitty_append_chunk");
@@ -1186,7 +1192,7 @@ extern "C" int kitty_append_chunk_host(const kitty_kv_layer* layer, const void* 
   if (max_pages > 0)
     hipLaunchKernelGGL(chunk_quant_kernel<true>, dim3(2 * max_pages, layer->H_KV, B), dim3(256), 0, st, *layer,
                        (const uint8_t*)k_new, (const uint8_t*)v_new, stride_b, stride_h, stride_t, T, max_pages);
-  hipLaunchKernelGGL(chunk_rows_kernel<true>, dim3(layer->H_KV, B), dim3(256), 0, st, *layer, (const uint8_t*)k_new,
+  hipLaunchKernelGGL(chunk_rows_kernel<true>, dim3(layer->H_KV, B, 2), dim3(kRowThreads), 0, st, *layer, (const uint8_t*)k_new,
                      (const uint8_t*)v_new, stride_b, stride_h, stride_t, T);
   return check_launch("kitty_append_chunk_host");
 }
