@@ -245,6 +245,7 @@ extern "C" size_t kitty_prefill_attn_workspace_bytes(int B, int H_Q, int D, int 
 
 extern "C" int kitty_prefill_attn_default_splits(int B, int H_Q, int H_KV, int D, int T_q, int max_tiles) {
   if (B <= 0 || H_KV <= 0 || H_Q < H_KV || H_Q / H_KV > 16 || T_q <= 0 || max_tiles <= 0 || !head_dim_supported(D)) return 1;
+  if ((int64_t)T_q * 64 > (1 << 22) || (int64_t)B * T_q * H_Q > (1 << 26)) return 1;   // (fills the device alone)
   if (D != kD) return prefill_splits_any(B, H_Q, H_KV, D, T_q, max_tiles + c_div_up(T_q, kPage), device_simds() / 4);
   return prefill_splits(B, H_Q, H_KV, T_q, max_tiles + c_div_up(T_q, kPage), device_simds() / 4);
 }
@@ -276,6 +277,8 @@ extern "C" int kitty_prefill_attn_split(const kitty_kv_layer* layer, const void*
   KITTY_REQUIRE(num_splits >= 1 && num_splits <= 1024, KITTY_E_RANGE, "num_splits=%d out of range", num_splits);
   float *ws_ml = nullptr, *ws_acc = nullptr;
   if (num_splits > 1) {
+    KITTY_REQUIRE((int64_t)T_q * num_splits <= (1 << 22) && (int64_t)B * T_q * H_Q <= (1 << 26), KITTY_E_RANGE,
+                  "T_q=%d, num_splits=%d: a chunk of this size is not cut into shares", T_q, num_splits);   // grid limits
     KITTY_REQUIRE(workspace != nullptr, KITTY_E_NULL, "workspace is NULL");
     KITTY_REQUIRE(((uintptr_t)workspace % 256) == 0, KITTY_E_ALIGN, "workspace needs 256-byte alignment");
     const size_t need = kitty_prefill_attn_workspace_bytes(B, H_Q, layer->D, T_q, num_splits);

@@ -846,7 +846,7 @@ void launch_prefill_attn(const kitty_kv_layer& L, const void* q, int64_t q_strid
   dim3 grid(blocks * num_splits, L.H_KV, B), block(kThreads);
   const int* c = L.counts;
   const int64_t dense_wgs = (int64_t)blocks * num_splits * L.H_KV * B;
-  if (!L.seq_counts && c[KITTY_CNT_SINK] == 0 && c[KITTY_CNT_PAGES_K] + c[KITTY_CNT_QBUF_K] == 0 && dense_wgs <= INT32_MAX) {
+  if (!L.seq_counts && c[KITTY_CNT_SINK] == 0 && c[KITTY_CNT_PAGES_K] + c[KITTY_CNT_QBUF_K] == 0 && dense_wgs <= (1 << 22)) {   // (grid limit)
     // (check_layer: as many values as keys)
 #define KITTY_LAUNCH_DENSE(SPLIT)                                                                                \
   do {                                                                                                           \

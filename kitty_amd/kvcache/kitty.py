@@ -97,7 +97,8 @@ class KittyCache(_HFCache):
         if kvcache.device_counters:
             self._append_token_device(kvcache, key_states, value_states)
             return False
-        if kvcache.on_hip:
+        if kvcache.on_hip and 1 <= B <= kvcache.MAX_BS \
+                and key_states.shape == (B, kvcache.H_KV, 1, kvcache.D) == value_states.shape:
             self._append_row(kvcache, key_states, value_states)
             return False
         with torch.no_grad():
@@ -130,9 +131,7 @@ class KittyCache(_HFCache):
         if L.Sink_Count >= L.S:
             assert L.Q_Buffer_Count_K < L.PAGE_SIZE
             assert L.Local_Count_V < L.PAGE_SIZE or L.Q_Buffer_Count_V < L.PAGE_SIZE
-        B, H, _, D = key_states.shape
-        if H != L.H_KV or D != L.D or B > L.MAX_BS or value_states.shape != key_states.shape:
-            raise ValueError(f"key_states / value_states must be [B <= {L.MAX_BS}, {L.H_KV}, 1, {L.D}]")
+        B = key_states.shape[0]
         key_states, value_states = _row_source(L, key_states), _row_source(L, value_states)
         ks, vs = key_states.stride(), value_states.stride()
         rc = _lib.lib().kitty_append_row(L.descriptor(), key_states.data_ptr(), value_states.data_ptr(), 2 * ks[0],

@@ -94,7 +94,10 @@ class KVCache_Layer:
         self.active_batch = MAX_BS
         self._workspace: Optional[torch.Tensor] = None
         self._desc: Optional[_lib.KittyKVLayer] = None
-        self.on_hip = self.KeyCache.is_cuda
+        # the shapes the append and packing kernels are built for; other layers (whose attention they refuse) keep
+        # tensor copies for their fp16 rows
+        self.on_hip = (self.KeyCache.is_cuda and D in (64, 128, 256) and PAGE_SIZE == 128 and 0 <= S <= 128
+                       and 0 <= D_BOOSTED <= min(D, 255))
 
     def get_total_length(self) -> int:
         """Total number of cached tokens (the reference's :85-95, including its K == V check)."""
