@@ -355,6 +355,14 @@ int kitty_fake_quant(void* data, int64_t stride_b, int64_t stride_h, int64_t str
                      const uint8_t* promote_mask, int64_t mask_stride_b, int64_t mask_stride_h,
                      int64_t mask_stride_tile, int promote_bit, void* stream);
 
+/*
+ * kitty_fake_quant with groups along the channels (axis 1) from one tensor into another: tokens [t_offset, t_offset +
+ * n_tokens) of src [B,H,T,D] arrive in data quantized, the others as they are.  The tensors must not overlap.
+ */
+int kitty_fake_quant_from(const void* src, int64_t src_stride_b, int64_t src_stride_h, int64_t src_stride_t, void* data,
+                          int64_t stride_b, int64_t stride_h, int64_t stride_t, int B, int H, int T, int D, int t_offset,
+                          int n_tokens, int group_size, int bit, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

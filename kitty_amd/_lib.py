@@ -81,6 +81,8 @@ _SIGNATURES = {
                                         c_int, c_void_p]),
     "kitty_pack_prompt": (c_int, [POINTER(KittyKVLayer), c_int, c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int64,
                                   c_int64, c_int64, c_int, c_int, c_void_p]),
+    "kitty_fake_quant_from": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int, c_int,
+                                      c_int, c_int, c_int, c_int, c_int, c_int, c_void_p]),
     "kitty_fake_quant": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_int, c_int, c_int, c_int, c_int, c_int,
                                  c_int, c_int, c_int, c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p]),
 }

@@ -198,6 +198,20 @@ class KittyKVCache(_HFCache):
         if hi > lo:
             fake_quant_tokens_(self.value_cache[layer], lo, hi - lo, 1, self.cfg.group_size, self.cfg.vbits)
 
+    def _values_from(self, x: torch.Tensor, buf: torch.Tensor, lo: int, hi: int) -> bool:
+        """A prompt's values into an empty buffer, ``[lo, hi)`` quantized, in one launch.  False, and nothing done, for
+        what a tensor copy would have converted, moved or tracked, and without quantization."""
+        c, (B, nh, L, D), st = self.cfg, x.shape, x.stride()
+        if c.vbits >= 16 or x.dtype != torch.float16 or x.device != buf.device or st[3] != 1 or st[0] % 8 or st[1] % 8 \
+                or st[2] % 8 or x.data_ptr() % 16 or L > 1 << 24 or (x.requires_grad and torch.is_grad_enabled()):
+            return False
+        bs = buf.stride()
+        rc = _lib.lib().kitty_fake_quant_from(x.data_ptr(), st[0] * 2, st[1] * 2, st[2] * 2, buf.data_ptr(), bs[0] * 2,
+                                              bs[1] * 2, bs[2] * 2, B, nh, L, D, lo, hi - lo, c.group_size, c.vbits,
+                                              _lib.current_stream_ptr(buf.device))
+        _lib.check(rc, "KittyKVCache.update")
+        return True
+
     def _run(self, layer: int, jobs: list) -> None:
         for kind, lo, hi in jobs:
             (self._quant_k if kind == "k" else self._quant_v)(layer, lo, hi)
@@ -223,17 +237,22 @@ class KittyKVCache(_HFCache):
             if self.max_length is not None and L > self.max_length:
                 raise ValueError(f"prompt of {L} tokens exceeds max_length={self.max_length}")
             cap = self.max_length if self.max_length is not None else max(2 * L, L + 1024)
-            for store, x in ((self.key_cache, key_states), (self.value_cache, value_states)):
-                buf = torch.empty((B, nh, cap, D), dtype=torch.float16, device=key_states.device)
-                buf[:, :, :L].copy_(x)
-                store.append(buf)
-            self._len.append(L)
-            self._pending.append([])
+            v_from = v_to = c.sink_length                       # the values to quantize
             if L > c.sink_length + c.buffer_length:
                 n = L - c.sink_length
                 nq = n - n % c.buffer_length
                 jobs.append(("k", c.sink_length, c.sink_length + nq))
-                jobs.append(("v", c.sink_length, c.sink_length + (nq if c.VCache_BitDecoding else n - c.buffer_length)))
+                v_to = c.sink_length + (nq if c.VCache_BitDecoding else n - c.buffer_length)
+            for store, x in ((self.key_cache, key_states), (self.value_cache, value_states)):
+                buf = torch.empty((B, nh, cap, D), dtype=torch.float16, device=key_states.device)
+                if store is self.value_cache and v_to > v_from and self._values_from(x, buf, v_from, v_to):
+                    v_to = v_from                               # quantized on their way in
+                else:
+                    buf[:, :, :L].copy_(x)
+                store.append(buf)
+            self._len.append(L)
+            self._pending.append([])
+            jobs.append(("v", v_from, v_to))
             self._run(layer_idx, jobs)
             if c.PostQuant:
                 return key_states, value_states        # the prompt's attention sees the prompt as it came
