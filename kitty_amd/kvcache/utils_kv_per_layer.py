@@ -94,6 +94,7 @@ class KVCache_Layer:
         self.active_batch = MAX_BS
         self._workspace: Optional[torch.Tensor] = None
         self._desc: Optional[_lib.KittyKVLayer] = None
+        self._desc_counts = None
         # the shapes the append and packing kernels are built for; other layers (whose attention they refuse) keep
         # tensor copies for their fp16 rows
         self.on_hip = (self.KeyCache.is_cuda and D in (64, 128, 256) and PAGE_SIZE == 128 and 0 <= S <= 128
@@ -155,6 +156,12 @@ class KVCache_Layer:
             assert self.Q_Buffer_Count_V < self.PAGE_SIZE
             self.Q_Buffer_Count_V += 1
             self.Write_Offset_Local_V = (self.Write_Offset_Local_V + 1) % self.PAGE_SIZE
+
+    # ---- copies -------------------------------------------------------------------------------
+    def __getstate__(self) -> dict:
+        """What ``copy.deepcopy`` and ``pickle`` take along: everything but the view of this layer's own
+        memory that ``descriptor`` makes again, and the scratch."""
+        return dict(self.__dict__, _desc=None, _desc_counts=None, _workspace=None)
 
     # ---- C-ABI view -------------------------------------------------------------------------
     def counts(self):
