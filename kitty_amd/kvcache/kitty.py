@@ -33,11 +33,11 @@ def prefill_split(len_prefill: int, S: int, P: int) -> dict:
     return dict(sink=sink, qbuf_k=qbuf_k, pages_k=pages_k, local_v=local_v, qbuf_v=qbuf_v, pages_v=pages_v)
 
 
-def _row_source(L: KVCache_Layer, x: torch.Tensor) -> torch.Tensor:
+def _row_source(device: torch.device, x: torch.Tensor) -> torch.Tensor:
     """``x [B, H_KV, 1, D]`` as the append kernel reads it: fp16 on the cache's device, D contiguous, rows on
     16-byte boundaries.  What a slice assignment would have converted or moved is converted here."""
-    if x.dtype != torch.float16 or x.device != L.KeyCache.device:
-        x = x.to(L.KeyCache.device, torch.float16)
+    if x.dtype != torch.float16 or x.device != device:
+        x = x.to(device, torch.float16)
     st = x.stride()
     if st[3] != 1 or st[0] % 8 or st[1] % 8 or x.data_ptr() % 16:
         x = x.clone(memory_format=torch.contiguous_format)
@@ -131,8 +131,8 @@ class KittyCache(_HFCache):
         if L.Sink_Count >= L.S:
             assert L.Q_Buffer_Count_K < L.PAGE_SIZE
             assert L.Local_Count_V < L.PAGE_SIZE or L.Q_Buffer_Count_V < L.PAGE_SIZE
-        B = key_states.shape[0]
-        key_states, value_states = _row_source(L, key_states), _row_source(L, value_states)
+        B, device = key_states.shape[0], L.KeyCache.device
+        key_states, value_states = _row_source(device, key_states), _row_source(device, value_states)
         ks, vs = key_states.stride(), value_states.stride()
         rc = _lib.lib().kitty_append_row(L.descriptor(), key_states.data_ptr(), value_states.data_ptr(), 2 * ks[0],
                                          2 * ks[1], 2 * vs[0], 2 * vs[1], B, _lib.current_stream_ptr(key_states.device))

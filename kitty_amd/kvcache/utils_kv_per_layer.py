@@ -20,6 +20,7 @@ against the reference keeps working.  Differences, all additive:
   no page assigned); see ``paging.PagedKittyCache``.
 """
 import math
+import operator
 from typing import Optional
 
 import torch
@@ -27,8 +28,24 @@ import torch
 from .. import _lib
 
 
+def _layer_tensor(name: str) -> property:
+    """A tensor attribute whose address the layer's C descriptor holds: assigning another tensor drops the descriptor."""
+    slot = "_" + name
+
+    def assign(layer, tensor):
+        layer.__dict__[slot] = tensor
+        layer.__dict__["_desc"] = None
+
+    return property(operator.attrgetter(slot), assign)
+
+
 class KVCache_Layer:
     """KV cache of a single layer; pages are statically allocated."""
+
+    _TENSORS = ("KeyCache", "KeyCache_metadata", "ValueCache", "ValueCache_metadata", "PageTable_K", "PageTable_V",
+                "Sink_Buffer_K", "Sink_Buffer_V", "Q_Buffer_K", "Q_Buffer_V", "Local_Buffer_V", "status")
+    (KeyCache, KeyCache_metadata, ValueCache, ValueCache_metadata, PageTable_K, PageTable_V, Sink_Buffer_K, Sink_Buffer_V,
+     Q_Buffer_K, Q_Buffer_V, Local_Buffer_V, status) = map(_layer_tensor, _TENSORS)
 
     def __init__(self, MAX_BS: int, MAX_LEN: int, H_KV: int, D: int, D_BOOSTED: int, LOW_BIT: int, HIGH_BIT: int,
                  PAGE_SIZE: int, S: int, device="cuda", *, n_pages: Optional[int] = None,
@@ -94,11 +111,15 @@ class KVCache_Layer:
         self.active_batch = MAX_BS
         self._workspace: Optional[torch.Tensor] = None
         self._desc: Optional[_lib.KittyKVLayer] = None
-        self._desc_counts = None
-        # the shapes the append and packing kernels are built for; other layers (whose attention they refuse) keep
-        # tensor copies for their fp16 rows
-        self.on_hip = (self.KeyCache.is_cuda and D in (64, 128, 256) and PAGE_SIZE == 128 and 0 <= S <= 128
-                       and 0 <= D_BOOSTED <= min(D, 255))
+        self._desc_counts = self._desc_at = None
+        self._kernel_shape = (D in (64, 128, 256) and PAGE_SIZE == 128 and 0 <= S <= 128
+                              and 0 <= D_BOOSTED <= min(D, 255))
+
+    @property
+    def on_hip(self) -> bool:
+        """The shapes the append and packing kernels are built for, on a GPU; other layers (whose attention they
+        refuse) keep tensor copies for their fp16 rows."""
+        return self._kernel_shape and self._KeyCache.is_cuda
 
     def get_total_length(self) -> int:
         """Total number of cached tokens (the reference's :85-95, including its K == V check)."""
@@ -161,7 +182,7 @@ class KVCache_Layer:
     def __getstate__(self) -> dict:
         """What ``copy.deepcopy`` and ``pickle`` take along: everything but the view of this layer's own
         memory that ``descriptor`` makes again, and the scratch."""
-        return dict(self.__dict__, _desc=None, _desc_counts=None, _workspace=None)
+        return dict(self.__dict__, _desc=None, _desc_counts=None, _desc_at=None, _workspace=None)
 
     # ---- C-ABI view -------------------------------------------------------------------------
     def counts(self):
@@ -169,27 +190,28 @@ class KVCache_Layer:
                 self.Q_Buffer_Count_V, self.Local_Count_V, self.Write_Offset_Local_V, 0]
 
     def descriptor(self) -> "_lib.KittyKVLayer":
-        """struct kitty_kv_layer for this layer; pointers are cached, counters refreshed."""
-        d = self._desc
-        if d is None:
+        """struct kitty_kv_layer for this layer as it is now.  The struct is kept; a tensor that is replaced drops it
+        (``_layer_tensor``), and so does storage that moved under the tensors (offloading moves all of them: two
+        addresses are compared, all twelve would cost a decode step 1 us of the host's time per layer).  Counters always."""
+        d, at = self._desc, (self._KeyCache.data_ptr(), self._Q_Buffer_K.data_ptr())
+        if d is None or at != self._desc_at:
+            tensors = [getattr(self, n) for n in self._TENSORS]
+            where = tensors[0].device
+            for n, t in zip(self._TENSORS, tensors):
+                if t.device != where:
+                    raise ValueError(f"the layer's tensors are on different devices: KeyCache on {where}, {n} on {t.device}")
             d = _lib.KittyKVLayer()
             d.H_KV, d.D, d.D_BOOSTED, d.PAGE_SIZE, d.S, d.MAX_PAGE = (
                 self.H_KV, self.D, self.D_BOOSTED, self.PAGE_SIZE, self.S, self.MAX_PAGE)
-            d.key_cache, d.key_cache_stride_page = self.KeyCache.data_ptr(), self.KeyCache.stride(0)
-            d.key_meta, d.key_meta_stride_page = self.KeyCache_metadata.data_ptr(), self.KeyCache_metadata.stride(0) * 2
-            d.value_cache, d.value_cache_stride_page = self.ValueCache.data_ptr(), self.ValueCache.stride(0)
-            d.value_meta = self.ValueCache_metadata.data_ptr()
-            d.value_meta_stride_page = self.ValueCache_metadata.stride(0) * 2
-            d.page_table_k, d.page_table_k_stride_b = self.PageTable_K.data_ptr(), self.PageTable_K.stride(0)
-            d.page_table_v, d.page_table_v_stride_b = self.PageTable_V.data_ptr(), self.PageTable_V.stride(0)
-            d.sink_k, d.sink_v = self.Sink_Buffer_K.data_ptr(), self.Sink_Buffer_V.data_ptr()
+            (d.key_cache, d.key_meta, d.value_cache, d.value_meta, d.page_table_k, d.page_table_v, d.sink_k, d.sink_v,
+             d.qbuf_k, d.qbuf_v, d.local_v, d.status) = [t.data_ptr() for t in tensors]
+            d.key_cache_stride_page, d.key_meta_stride_page = self.KeyCache.stride(0), self.KeyCache_metadata.stride(0) * 2
+            d.value_cache_stride_page, d.value_meta_stride_page = self.ValueCache.stride(0), self.ValueCache_metadata.stride(0) * 2
+            d.page_table_k_stride_b, d.page_table_v_stride_b = self.PageTable_K.stride(0), self.PageTable_V.stride(0)
             d.sink_stride_b, d.sink_stride_h = self.Sink_Buffer_K.stride(0) * 2, self.Sink_Buffer_K.stride(1) * 2
-            d.qbuf_k, d.qbuf_v = self.Q_Buffer_K.data_ptr(), self.Q_Buffer_V.data_ptr()
-            d.local_v = self.Local_Buffer_V.data_ptr()
             d.win_stride_b, d.win_stride_h = self.Q_Buffer_K.stride(0) * 2, self.Q_Buffer_K.stride(1) * 2
             d.cache_pages_k, d.cache_pages_v = self.KeyCache.shape[0], self.ValueCache.shape[0]
-            d.status = self.status.data_ptr()
-            self._desc = d
+            self._desc, self._desc_at = d, at
             self._desc_counts = d.counts          # a view of the struct's array
         self._desc_counts[:] = self.counts()
         d.seq_counts = None if self.seq_counts is None else self.seq_counts.data_ptr()
