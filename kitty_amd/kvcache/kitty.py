@@ -97,7 +97,8 @@ class KittyCache(_HFCache):
         if kvcache.device_counters:
             self._append_token_device(kvcache, key_states, value_states)
             return False
-        if kvcache.on_hip and 1 <= B <= kvcache.MAX_BS \
+        # (per-sequence counters set by hand: the host ints still say where the rows go, the kernel would not look at them)
+        if kvcache.on_hip and kvcache.seq_counts is None and 1 <= B <= kvcache.MAX_BS \
                 and key_states.shape == (B, kvcache.H_KV, 1, kvcache.D) == value_states.shape:
             self._append_row(kvcache, key_states, value_states)
             return False
@@ -398,7 +399,7 @@ class KittyCache(_HFCache):
         if L.PageCount_K + new_pk > L.MAX_PAGE or L.PageCount_V + new_pv > L.MAX_PAGE:
             raise ValueError(f"appending {T} tokens exceeds max_length={L.MAX_LEN}")
         # the whole batch in two launches (a part of it would leave what the rest's Q-buffers hold out of their pages)
-        if L.on_hip and L.D == 128 and self.select == "hip" and 1 <= T <= 1 << 24 and B == L.MAX_BS \
+        if L.on_hip and L.seq_counts is None and L.D == 128 and self.select == "hip" and 1 <= T <= 1 << 24 and B == L.MAX_BS \
                 and key_states.shape[1] == L.H_KV and key_states.shape[3] == L.D \
                 and L.Q_Buffer_Count_K < P and L.Q_Buffer_Count_V < P and key_states.stride() == value_states.stride() \
                 and _kernel_ready(L, key_states) and _kernel_ready(L, value_states):

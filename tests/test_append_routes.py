@@ -35,3 +35,49 @@ def test_other_head_dims_and_broadcast_rows_still_append():
         assert a.counts() == b.counts()
         for n in ("Sink_Buffer_K", "Sink_Buffer_V", "Q_Buffer_K", "Q_Buffer_V", "Local_Buffer_V"):
             assert torch.equal(getattr(a, n).cpu(), getattr(b, n)), (D, n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_layers_with_counters_set_by_hand_still_append(D):
+    """``seq_counts`` assigned without ``enable_device_counters``: attention reads them, ``update`` and ``append`` go by
+    the host ints, as on any layer."""
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    by_hand, plain = _cache(D, "cuda"), _cache(D, "cuda")
+    gen = torch.Generator(device="cuda").manual_seed(D)
+    rnd = lambda T: torch.randn(2, 2, T, D, generator=gen, device="cuda", dtype=torch.float16)
+    a, b = by_hand.kv_cache[0], plain.kv_cache[0]
+    rows = [rnd(100), rnd(100)]
+    for c in (by_hand, plain):
+        c.update(*rows, 0)
+        c.quantize_prefill(0)
+    a.seq_counts = torch.tensor([a.counts()] * 2, dtype=torch.int32, device="cuda")
+    for T in (1, 1, 70, 1):
+        rows = [rnd(T), rnd(T)]
+        for c in (by_hand, plain):
+            if T == 1:
+                assert c.update(*rows, 0) is False
+                c.quantize_decode(0)
+            else:
+                c.append(*rows, 0)
+    assert a.counts() == b.counts()
+    for n in ("Sink_Buffer_K", "Sink_Buffer_V", "Q_Buffer_K", "Q_Buffer_V", "Local_Buffer_V", "KeyCache", "KeyCache_metadata",
+              "ValueCache", "ValueCache_metadata"):
+        assert torch.equal(getattr(a, n), getattr(b, n)), n
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_counters_set_by_hand_take_the_copies(D, monkeypatch):
+    from kitty_amd.kvcache import kitty as module
+    c = _cache(D, "cpu")
+    L = c.kv_cache[0]
+    L.Sink_Count, L.Q_Buffer_Count_K, L.Local_Count_V = 32, 5, 5
+    L.seq_counts = torch.tensor([L.counts()] * 2, dtype=torch.int32)
+    monkeypatch.setattr(type(L), "on_hip", True)                       # as on a GPU, but a launch is an error
+    monkeypatch.setattr(module._lib, "lib", lambda: pytest.fail("a kernel was launched"))
+    x = torch.ones(2, 2, 1, D).half()
+    assert c.update(x, x, 0) is False and L.Q_Buffer_Count_K == 6 and bool((L.Q_Buffer_K[:, :, 5] == 1).all())
+    x = torch.full((2, 2, 3, D), 2.0).half()
+    c.append(x, x, 0)
+    assert L.Q_Buffer_Count_K == 9 and bool((L.Q_Buffer_K[:, :, 6:9] == 2).all()) and bool((L.Local_Buffer_V[:, :, 6:9] == 2).all())
