@@ -112,7 +112,8 @@ class KVCache_Layer:
         self._workspace: Optional[torch.Tensor] = None
         self._desc: Optional[_lib.KittyKVLayer] = None
         self._desc_counts = self._desc_at = None
-        self._kernel_shape = (D in (64, 128, 256) and PAGE_SIZE == 128 and 0 <= S <= 128
+        # (an empty sink or page tensor has no address to hand over)
+        self._kernel_shape = (D in (64, 128, 256) and PAGE_SIZE == 128 and 1 <= S <= 128 and self.MAX_PAGE >= 1
                               and 0 <= D_BOOSTED <= min(D, 255))
 
     @property

@@ -81,3 +81,44 @@ def test_counters_set_by_hand_take_the_copies(D, monkeypatch):
     x = torch.full((2, 2, 3, D), 2.0).half()
     c.append(x, x, 0)
     assert L.Q_Buffer_Count_K == 9 and bool((L.Q_Buffer_K[:, :, 6:9] == 2).all()) and bool((L.Local_Buffer_V[:, :, 6:9] == 2).all())
+
+
+def _odd_layer(device, S, max_len):
+    from kitty_amd.kvcache.utils_kv_per_layer import KVCache_Layer
+    c = _cache(128, device)
+    c.kv_cache[0] = KVCache_Layer(2, max_len, 2, 128, 32, 2, 4, 128, S, device=device)
+    return c
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,max_len,steps", [(0, 512, (300,)), (0, 512, (300, 40)), (32, 0, (50, 1, 30))])
+def test_layers_without_a_sink_or_without_pages_still_take_tokens(S, max_len, steps):
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    c = _odd_layer("cuda", S, max_len)
+    L = c.kv_cache[0]
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    K = torch.randn(2, 2, sum(steps), 128, generator=gen, device="cuda", dtype=torch.float16)
+    V = torch.randn(2, 2, sum(steps), 128, generator=gen, device="cuda", dtype=torch.float16)
+    c.update(K[:, :, :steps[0]], V[:, :, :steps[0]], 0)
+    c.quantize_prefill(0)
+    t = steps[0]
+    for n in steps[1:]:
+        if n == 1:
+            assert c.update(K[:, :, t:t + 1], V[:, :, t:t + 1], 0) is False
+        else:
+            c.append(K[:, :, t:t + n], V[:, :, t:t + n], 0)
+        t += n
+    assert L.get_total_length() == t and L.PageCount_K == (t - S) // 128
+    rk = L.Q_Buffer_Count_K
+    assert torch.equal(L.Q_Buffer_K[:, :, :rk], K[:, :, t - rk:t]) and torch.equal(L.Sink_Buffer_K, K[:, :, :S])
+
+
+@pytest.mark.parametrize("S,max_len", [(0, 512), (32, 0)])
+def test_layers_without_a_sink_or_without_pages_are_not_for_the_kernels(S, max_len, monkeypatch):
+    L = _odd_layer("cpu", S, max_len).kv_cache[0]
+    monkeypatch.setattr(type(L), "_KeyCache", types.SimpleNamespace(is_cuda=True), raising=False)
+    del L.__dict__["_KeyCache"]
+    assert L.on_hip is False
+    L._kernel_shape = True
+    assert L.on_hip is True
