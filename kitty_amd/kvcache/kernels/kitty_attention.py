@@ -139,7 +139,8 @@ def _launch_chunk(desc, query, key_states, value_states, scaling, out, ws, ws_by
 def prompt_attention_ready(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, kv_cache: KVCache_Layer) -> bool:
     """The chunk kernel can run a prompt's dense causal attention on these tensors as they lie.  What stays with
     torch's attention: other types, devices and head dimensions (at 64 and 256 the kernel keeps 22-bit probabilities
-    and is slower than a dense kernel), rows off the 16-byte grid, and whatever is being differentiated or traced."""
+    and is slower than a dense kernel), rows off the 16-byte grid, autocast (which gives the result its type), and whatever
+    is being differentiated or traced."""
     if not kv_cache.on_hip or kv_cache.D != 128 or kv_cache.MAX_PAGE < 1:
         return False
     B, H_Q, T, D = query.shape
@@ -147,7 +148,7 @@ def prompt_attention_ready(query: torch.Tensor, key: torch.Tensor, value: torch.
     if key.shape != (B, H, T, 128) or value.shape != key.shape or D != 128 or H_Q % H or not 1 <= H_Q // H <= MAX_KV_GROUP \
             or not 1 <= T <= 1 << 24 or not 1 <= B <= 65535 or key.stride() != value.stride():
         return False
-    if torch.compiler.is_compiling() or torch.autograd.forward_ad._current_level >= 0:
+    if torch.compiler.is_compiling() or torch.autograd.forward_ad._current_level >= 0 or torch.is_autocast_enabled("cuda"):
         return False
     grad = torch.is_grad_enabled()
     for x in (query, key, value):

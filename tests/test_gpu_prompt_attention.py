@@ -57,3 +57,16 @@ def test_what_stays_with_torch():
     out, _ = hf.kitty_attention(types.SimpleNamespace(layer_idx=0), qg, kk, vv, None, scaling=128 ** -0.5)
     out.float().sum().backward()
     assert torch.isfinite(qg.grad).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_autocast_gives_the_result_its_type(dtype):
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    hf, cache, q, k, v = _setup(1, 40, 4, 2, "token-major")
+    with torch.autocast("cuda", dtype=dtype):
+        kk, vv = cache.update(k, v, 0)
+        out, _ = hf.kitty_attention(types.SimpleNamespace(layer_idx=0), q, kk, vv, None, scaling=128 ** -0.5)
+        ref = torch.nn.functional.scaled_dot_product_attention(q, k.repeat_interleave(2, 1), v.repeat_interleave(2, 1), is_causal=True,
+                                                               scale=128 ** -0.5).transpose(1, 2)
+    assert out.dtype == ref.dtype == dtype and torch.equal(out, ref) and cache.get_seq_length(0) == 40
