@@ -7,6 +7,9 @@ import ctypes
 import os
 from ctypes import POINTER, c_char_p, c_float, c_int, c_int32, c_int64, c_size_t, c_uint8, c_void_p
 
+import torch
+from torch.autograd import forward_ad
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libkitty_hip.so")
 ABI_VERSION = 2
@@ -126,9 +129,25 @@ def require_hip(t, name: str) -> None:
             f"{name} lives on {t.device}; the Kitty kernels are HIP kernels for MI355X and there is no CPU path")
 
 
+def launchable(device) -> bool:
+    """A raw launch may stand in for tensor operations on ``device``: nothing records the operations (a jit trace,
+    forward-mode AD; a kernel would be invisible to both) and raw launches go to that device, i.e. it is the current one.
+    Callers look at gradients themselves."""
+    # (no public question for "is a dual level active": without the name, tensor operations are always kept)
+    return (getattr(forward_ad, "_current_level", 0) < 0 and not _is_tracing()
+            and device.index in (None, _current_device()))
+
+
 def current_stream_ptr(device) -> int:
     """Torch's current stream on ``device`` as a raw ``hipStream_t`` (the Stream object that
     ``torch.cuda.current_stream`` builds around it costs the host 1.5 us a call)."""
-    import torch
+    if _raw_stream is None:
+        return torch.cuda.current_stream(device).cuda_stream
     index = device.index
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+    return _raw_stream(_current_device() if index is None else index)
+
+
+# the private names behind torch.cuda.current_stream, current_device and jit.is_tracing, where this build of torch has them
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+_is_tracing = getattr(torch._C, "_is_tracing", torch.jit.is_tracing)

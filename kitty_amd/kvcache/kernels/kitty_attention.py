@@ -148,7 +148,7 @@ def prompt_attention_ready(query: torch.Tensor, key: torch.Tensor, value: torch.
     if key.shape != (B, H, T, 128) or value.shape != key.shape or D != 128 or H_Q % H or not 1 <= H_Q // H <= MAX_KV_GROUP \
             or not 1 <= T <= 1 << 24 or not 1 <= B <= 65535 or key.stride() != value.stride():
         return False
-    if torch.compiler.is_compiling() or torch.autograd.forward_ad._current_level >= 0 or torch.is_autocast_enabled("cuda"):
+    if torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda") or not _lib.launchable(kv_cache.KeyCache.device):
         return False
     grad = torch.is_grad_enabled()
     for x in (query, key, value):

@@ -99,7 +99,8 @@ class KittyCache(_HFCache):
             return False
         # (per-sequence counters set by hand: the host ints still say where the rows go, the kernel would not look at them)
         if kvcache.on_hip and kvcache.seq_counts is None and 1 <= B <= kvcache.MAX_BS \
-                and key_states.shape == (B, kvcache.H_KV, 1, kvcache.D) == value_states.shape:
+                and key_states.shape == (B, kvcache.H_KV, 1, kvcache.D) == value_states.shape \
+                and _lib.launchable(kvcache.KeyCache.device):
             self._append_row(kvcache, key_states, value_states)
             return False
         with torch.no_grad():
@@ -170,7 +171,7 @@ class KittyCache(_HFCache):
             raise ValueError(f"prefill of {len_prefill} tokens exceeds max_length={kvcache.MAX_LEN}")
         if kvcache.on_hip and self.select == "hip" and 1 <= len_prefill <= 1 << 24 and 1 <= B <= kvcache.MAX_BS - first_row \
                 and K.shape == (B, kvcache.H_KV, len_prefill, kvcache.D) == V.shape \
-                and _kernel_ready(kvcache, K) and _kernel_ready(kvcache, V):
+                and _kernel_ready(kvcache, K) and _kernel_ready(kvcache, V) and _lib.launchable(K.device):
             ks, vs = K.stride(), V.stride()
             rc = _lib.lib().kitty_pack_prompt(kvcache.descriptor(), first_row, K.data_ptr(), 2 * ks[0], 2 * ks[1], 2 * ks[2],
                                               V.data_ptr(), 2 * vs[0], 2 * vs[1], 2 * vs[2], B, len_prefill,
@@ -402,7 +403,7 @@ class KittyCache(_HFCache):
         if L.on_hip and L.seq_counts is None and L.D == 128 and self.select == "hip" and 1 <= T <= 1 << 24 and B == L.MAX_BS \
                 and key_states.shape[1] == L.H_KV and key_states.shape[3] == L.D \
                 and L.Q_Buffer_Count_K < P and L.Q_Buffer_Count_V < P and key_states.stride() == value_states.stride() \
-                and _kernel_ready(L, key_states) and _kernel_ready(L, value_states):
+                and _kernel_ready(L, key_states) and _kernel_ready(L, value_states) and _lib.launchable(key_states.device):
             ks = key_states.stride()
             rc = _lib.lib().kitty_append_chunk_host(L.descriptor(), key_states.data_ptr(), value_states.data_ptr(), 2 * ks[0],
                                                     2 * ks[1], 2 * ks[2], B, T, _lib.current_stream_ptr(key_states.device))

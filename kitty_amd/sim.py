@@ -203,7 +203,8 @@ class KittyKVCache(_HFCache):
         what a tensor copy would have converted, moved or tracked, and without quantization."""
         c, (B, nh, L, D), st = self.cfg, x.shape, x.stride()
         if c.vbits >= 16 or x.dtype != torch.float16 or x.device != buf.device or st[3] != 1 or st[0] % 8 or st[1] % 8 \
-                or st[2] % 8 or x.data_ptr() % 16 or L > 1 << 24 or (x.requires_grad and torch.is_grad_enabled()):
+                or st[2] % 8 or x.data_ptr() % 16 or L > 1 << 24 or (x.requires_grad and torch.is_grad_enabled()) \
+                or not _lib.launchable(x.device):
             return False
         bs = buf.stride()
         rc = _lib.lib().kitty_fake_quant_from(x.data_ptr(), st[0] * 2, st[1] * 2, st[2] * 2, buf.data_ptr(), bs[0] * 2,
