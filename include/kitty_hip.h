@@ -158,14 +158,15 @@ int kitty_quant_pack_v(const void* value, int64_t stride_b, int64_t stride_h, in
  * split-K pass (QK^T, online softmax, PV per split of the sequence) and a merge pass.
  * q: fp16 [B,H_Q,1,D] contiguous.  out: fp16 [B,1,H_Q,D] contiguous.
  * workspace: at least kitty_decode_attn_workspace_bytes(B,H_Q,D,num_splits) bytes, 256-aligned.
- * num_splits <= 0 picks kitty_decode_attn_default_splits() (max_tiles = 1 + the 128-token tiles
- * after the sink of the longest sequence; per_sequence_counts = layer->seq_counts is set).
+ * num_splits <= 0 picks kitty_decode_attn_default_splits_d() (max_tiles = 1 + the 128-token tiles
+ * after the sink of the longest sequence; per_sequence_counts = layer->seq_counts is set), or for D = 64 / 256
+ * kitty_decode_attn_default_splits() where the workspace holds only that many.
  * variant: 0 = default kernel, 1 = the plain reference-order kernel (fp16 dequantization, no
  * matrix cores).  For D = 64 / 256 both values run the same kernel, in the reference's order.
  */
 size_t kitty_decode_attn_workspace_bytes(int B, int H_Q, int D, int num_splits);
 int kitty_decode_attn_default_splits(int B, int H_KV, int max_tiles, int per_sequence_counts);
-/* the same for a given head dimension (kitty_decode_attn_default_splits is the rule for D = 128) */
+/* the rule for a given head dimension; for D = 128 the same as kitty_decode_attn_default_splits */
 int kitty_decode_attn_default_splits_d(int B, int H_KV, int D, int max_tiles, int per_sequence_counts);
 int kitty_decode_attn(const kitty_kv_layer* layer, const void* q, int B, int H_Q, float scaling,
                       void* out, void* workspace, size_t workspace_bytes, int num_splits,

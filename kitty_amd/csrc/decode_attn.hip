@@ -229,8 +229,15 @@ extern "C" int kitty_decode_attn(const kitty_kv_layer* layer, const void* q, int
                                  void* stream) {
   int max_tiles = 0;
   if (int rc = check_layer(layer, q, B, H_Q, &max_tiles)) return rc;
-  if (num_splits <= 0)
-    num_splits = kitty_decode_attn_default_splits_d(B, layer->H_KV, layer->D, max_tiles, layer->seq_counts != nullptr);
+  if (num_splits <= 0) {
+    const int per_sequence = layer->seq_counts != nullptr;
+    num_splits = kitty_decode_attn_default_splits_d(B, layer->H_KV, layer->D, max_tiles, per_sequence);
+    // kitty_decode_attn_default_splits was the rule for every head dimension: a workspace sized by it is enough
+    if (layer->D != kD && workspace_bytes < ws_total_bytes(B, H_Q, num_splits, layer->D)) {
+      const int fewer = kitty_decode_attn_default_splits(B, layer->H_KV, max_tiles, per_sequence);
+      if (fewer < num_splits) num_splits = fewer;
+    }
+  }
   if (int rc = kitty_decode_attn_split(layer, q, B, H_Q, scaling, workspace, workspace_bytes, num_splits, variant,
                                        stream))
     return rc;
