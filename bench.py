@@ -529,6 +529,11 @@ def lib_check():
     assert torch.cuda.is_available(), "bench.py needs a GPU"
 
 
+def product_splits(lib, B, H_KV, D, max_tiles, per_sequence):
+    """The splits that ``kitty_attention_forward`` takes for these sizes."""
+    return lib.kitty_decode_attn_default_splits_d(B, H_KV, D, max_tiles, int(per_sequence))
+
+
 class DecodeBench:
     """One decode workload resident in HBM: the packed caches (made by the quantizer under test, enough
     independent copies to rotate over more than 3x the Infinity Cache), q, the workspace, and the
@@ -545,7 +550,7 @@ class DecodeBench:
         self.B, self.H_Q, self.H_KV, self.T = B, H_Q, H_KV, T
         D = self.D = getattr(args, "head_dim", 128)
         if D != 128:
-            self.desc = self.desc.replace("D=128", f"D={D}") + " - the plain kernels for other head dimensions"
+            self.desc = self.desc.replace("D=128", f"D={D}") + " - the kernels for other head dimensions"
             if workload == "c2":
                 raise ValueError("per-sequence counters on the device (c2) are built for head_dim 128")
         cfg = types.SimpleNamespace(num_hidden_layers=1, head_dim=D, num_key_value_heads=H_KV,
@@ -608,8 +613,7 @@ class DecodeBench:
                              dtype=torch.float32).half()
         self.out = torch.empty((B, 1, H_Q, D), dtype=torch.float16, device=dev)
         max_tiles = (2 + L0.MAX_PAGE) if seq_counts is not None else 1 + (T - L0.Sink_Count + 127) // 128
-        self.splits = args.splits or self.lib.kitty_decode_attn_default_splits(B, H_KV, max_tiles,
-                                                                               int(seq_counts is not None))
+        self.splits = args.splits or product_splits(self.lib, B, H_KV, D, max_tiles, seq_counts is not None)
         self.ws_bytes = self.lib.kitty_decode_attn_workspace_bytes(B, H_Q, D, self.splits)
         self.ws = torch.empty(self.ws_bytes, dtype=torch.uint8, device=dev)
         if seq_counts is not None:
@@ -866,7 +870,7 @@ def main():
     ap.add_argument("--splits", type=int, default=0)
     ap.add_argument("--variant", type=int, default=0)
     ap.add_argument("--head-dim", type=int, default=128, choices=[64, 128, 256],
-                    help="c0 / c1 / c4 with another head dimension (the untuned kernels for 64 and 256)")
+                    help="c0 / c1 / c4 with another head dimension (the kernels for 64 and 256)")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--no-other-workloads", action="store_true",
                     help="default workload only: leave out the `workloads` key (configs[0], [2], [3], [4], the plain "
@@ -893,7 +897,7 @@ def main():
     lib_check()
     headline = DecodeBench(args.workload, args.variant, args)
     result = headline.headline(args)
-    if args.head_dim != 128:     # a side measurement of the plain kernels: neither the host baseline nor the other configs
+    if args.head_dim != 128:     # a side measurement of the kernels for 64 and 256: neither the host baseline nor the other configs
         args.no_cpu_baseline = args.no_other_workloads = True
         result["roofline"]["traffic"] = None
     if not args.no_cpu_baseline:

@@ -7,6 +7,8 @@ import sys
 import types
 from pathlib import Path
 
+import pytest
+
 ROOT = Path(__file__).resolve().parent.parent
 sys.path.insert(0, str(ROOT))
 import bench  # noqa: E402
@@ -37,3 +39,12 @@ def test_algorithmic_bytes_follow_the_head_dimension():
         v_page = 32 * D + 4 * 128
         assert packed == 2 * 2 * (3 * k_page + 2 * v_page)
         assert total == packed + 2 * 2 * (2 * D) * (2 * 32 + 96 + 96 + 128) + 2 * (2 * 8 * D * 2)
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_the_measured_launch_is_the_products(D):
+    from kitty_amd import _lib
+    from kitty_amd.kvcache.kernels.kitty_attention import _split_plan
+    for B, H_KV, tiles, per_sequence in ((1, 8, 33, False), (16, 8, 257, False), (4, 2, 100, True)):
+        assert bench.product_splits(_lib.lib(), B, H_KV, D, tiles, per_sequence) == \
+            _split_plan(B, 4 * H_KV, H_KV, D, tiles, per_sequence, 0)[0]
