@@ -246,8 +246,8 @@ int kitty_prefill_attn(const kitty_kv_layer* layer,
  * of the device idle: a partial per row and share goes to the workspace, a second launch merges them.
  * num_splits = 1: kitty_prefill_attn itself (workspace unused, may be NULL).  Otherwise workspace: at least
  * kitty_prefill_attn_workspace_bytes(B,H_Q,D,T_q,num_splits) bytes, 256-aligned.
- * kitty_prefill_attn_default_splits: how many shares pay; max_tiles = 1 + the 128-token tiles after the
- * sink of the longest sequence.  Results do not depend on num_splits beyond the order of fp32 sums and the
+ * kitty_prefill_attn_default_splits: how many shares pay, their workspace 128 MB at most; max_tiles = 1 + the 128-token
+ * tiles after the sink of the longest sequence.  Results do not depend on num_splits beyond the order of fp32 sums and the
  * running maximum that the fp16 probabilities refer to.
  */
 size_t kitty_prefill_attn_workspace_bytes(int B, int H_Q, int D, int T_q, int num_splits);

@@ -729,13 +729,13 @@ int decode_splits_any(int B, int H_KV, int tiles, int units) {
 }
 
 // Shares of a chunk's walk: enough workgroups for two on every compute unit (what their registers allow at
-// D = 256), of at least two tiles each.
-int prefill_splits_any(int B, int H_Q, int H_KV, int D, int Tq, int tiles, int units) {
+// D = 256), of at least two tiles each.  `most`: shares the scratch allows.
+int prefill_splits_any(int B, int H_Q, int H_KV, int D, int Tq, int tiles, int units, int most) {
   const int PB = any_positions(D, H_Q / H_KV);
   const int64_t wgs = (int64_t)((Tq + PB - 1) / PB) * H_KV * B;
   int64_t s = 2 * units / wgs;
   if (s > tiles / 2) s = tiles / 2;
-  if (s > 64) s = 64;
+  if (s > most) s = most;
   return s < 1 ? 1 : (int)s;
 }
 

@@ -15,7 +15,7 @@ void launch_prefill_attn(const kitty_kv_layer& L, const void* q, int64_t q_strid
                          int64_t q_stride_t, const void* k_new, const void* v_new, int64_t new_stride_b,
                          int64_t new_stride_h, int64_t new_stride_t, int B, int H_Q, int Tq, float scaling,
                          void* out, float* ws_ml, float* ws_acc, int num_splits, hipStream_t stream);
-int prefill_splits(int B, int H_Q, int H_KV, int Tq, int tiles, int units);
+int prefill_splits(int B, int H_Q, int H_KV, int Tq, int tiles, int units, int most);
 // head dimensions other than 128 (any_dim.hip)
 void launch_decode_any(const kitty_kv_layer& L, const void* q, int B, int H_Q, float scaling, float* ws_ml,
                        float* ws_acc, int num_splits, hipStream_t stream);
@@ -24,7 +24,7 @@ void launch_prefill_any(const kitty_kv_layer& L, const void* q, int64_t q_stride
                         int64_t new_stride_h, int64_t new_stride_t, int B, int H_Q, int Tq, float scaling, void* out,
                         float* ws_ml, float* ws_acc, int num_splits, hipStream_t stream);
 int decode_splits_any(int B, int H_KV, int tiles, int units);
-int prefill_splits_any(int B, int H_Q, int H_KV, int D, int Tq, int tiles, int units);
+int prefill_splits_any(int B, int H_Q, int H_KV, int D, int Tq, int tiles, int units, int most);
 // merge pass over independent rows (rows_merge.hip)
 void launch_rows_merge(int D, const float* ws_ml, const float* ws_acc, void* out, int64_t rows, int num_splits,
                        bool keep_nan, hipStream_t stream);
@@ -253,8 +253,12 @@ extern "C" size_t kitty_prefill_attn_workspace_bytes(int B, int H_Q, int D, int 
 extern "C" int kitty_prefill_attn_default_splits(int B, int H_Q, int H_KV, int D, int T_q, int max_tiles) {
   if (B <= 0 || H_KV <= 0 || H_Q < H_KV || H_Q / H_KV > 16 || T_q <= 0 || max_tiles <= 0 || !head_dim_supported(D)) return 1;
   if ((int64_t)T_q * 64 > (1 << 22) || (int64_t)B * T_q * H_Q > (1 << 26)) return 1;   // (fills the device alone)
-  if (D != kD) return prefill_splits_any(B, H_Q, H_KV, D, T_q, max_tiles + c_div_up(T_q, kPage), device_simds() / 4);
-  return prefill_splits(B, H_Q, H_KV, T_q, max_tiles + c_div_up(T_q, kPage), device_simds() / 4);
+  // scratch of at most 128 MB, what a model's MLP holds for a chunk of some 4000 tokens: one chunk in 150 of sizes a
+  // server sees would take more (up to 310 MB), and loses 7 % on average by the rule's own estimate (at 64 MB: one in 40, 17 %)
+  const size_t share = (size_t)B * T_q * H_Q * (D + 2) * sizeof(float), budget = ((size_t)128 << 20) - 256;
+  const int most = share >= budget ? 1 : (int)(budget / share < 64 ? budget / share : 64);
+  if (D != kD) return prefill_splits_any(B, H_Q, H_KV, D, T_q, max_tiles + c_div_up(T_q, kPage), device_simds() / 4, most);
+  return prefill_splits(B, H_Q, H_KV, T_q, max_tiles + c_div_up(T_q, kPage), device_simds() / 4, most);
 }
 
 extern "C" int kitty_prefill_attn(const kitty_kv_layer* layer, const void* q, int64_t q_stride_b,

@@ -820,15 +820,15 @@ int prefill_lds_bytes() { return kLdsBytes; }
 // and multiplies the workgroups.  What a share costs besides its tiles is about three tiles' time (filling
 // the pipeline, 128 KB of partials); the merge reads 512 bytes a row and share.  A tile takes 5.4 us with all
 // rows in use.  The smallest total wins; ties go to fewer shares.
-// `tiles`: 128-token tiles the layer holds (sink included) plus those of the chunk.
-int prefill_splits(int B, int H_Q, int H_KV, int Tq, int tiles, int units) {
+// `tiles`: 128-token tiles the layer holds (sink included) plus those of the chunk; `most`: shares the scratch allows.
+int prefill_splits(int B, int H_Q, int H_KV, int Tq, int tiles, int units, int most) {
   const int G = H_Q / H_KV;
   if ((int64_t)B * Tq > 65535) return 1;   // the merge's grid; such a launch has enough workgroups
   const int64_t wgs = (int64_t)c_div_up(Tq, block_positions(G, Tq)) * H_KV * B;
   const float rows = (float)B * (float)Tq * (float)H_Q;
   int best = 1;
   float best_us = 0.f;
-  for (int s = 1; s <= 64 && (s == 1 || 2 * s <= tiles); ++s) {
+  for (int s = 1; s <= most && (s == 1 || 2 * s <= tiles); ++s) {
     const int64_t rounds = (wgs * s + units - 1) / units;
     float us = 5.4f * (float)rounds * (float)(c_div_up(tiles, s) + 3);
     if (s > 1) us += 4.f + rows * (float)s * 3.5e-4f;   // write + read of 1 KB at about 3 TB/s

@@ -118,7 +118,7 @@ def kitty_prefill_attention(
     # tiles of the longest sequence (with counters on the device the host ints shadow it; any number of shares is right)
     max_tiles = 1 + kv_cache.PageCount_K + (kv_cache.Q_Buffer_Count_K > 0)
     num_splits, ws_bytes = _chunk_split_plan(B, H_Q, H_KV, D, T_q, max_tiles)
-    # scratch of this call alone (tens of MB at most): torch's allocator hands the same block to the next layer
+    # scratch of this call alone (128 MB at most, by the rule): torch's allocator hands the same block to the next layer
     ws = query.new_empty(ws_bytes, dtype=torch.uint8) if num_splits > 1 else None
     _launch_chunk(kv_cache.descriptor(), query, key_states, value_states, scaling, attn_output, ws, ws_bytes, num_splits,
                   "kitty_prefill_attention")
