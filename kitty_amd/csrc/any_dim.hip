@@ -615,13 +615,18 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : D == 64 ? 3 : 2) void attn_any_k
 #pragma unroll
     for (int i = 0; i < 4; ++i) mm = fmaxf(mm, s_m[i][r]);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) l += s_m[i][r] == -INFINITY ? 0.f : s_l[i][r] * __builtin_amdgcn_exp2f(s_m[i][r] - mm);
+    for (int i = 0; i < 4; ++i)   // (a wavefront whose logits are all NaN has -inf for a maximum and NaN for a sum, which must stay)
+      l += s_l[i][r] * (s_m[i][r] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s_m[i][r] - mm));
     const bool partial = !PREFILL || ws_ml != nullptr;
     int64_t row = 0;   // of the workspace, or of out
     if (PREFILL) row = ((int64_t)b * Tq + qpos[nt]) * H_Q + h * G + qhead[nt];
     else row = (int64_t)b * H_Q + h * G + qhead[nt];
     if (partial) row = row * num_splits + split;
-    if (partial && qpos[nt] >= 0 && w == 0 && kg == 0) *(float2*)(ws_ml + row * 2) = float2{mm, l};
+    if (partial && qpos[nt] >= 0 && w == 0 && kg == 0) {
+      // a share of nothing but NaN counts in a chunk, whose walk may be one share or many (the merge passes over -inf)
+      if (PREFILL && l != l) mm = 0.f;
+      *(float2*)(ws_ml + row * 2) = float2{mm, l};
+    }
 #pragma unroll
     for (int t4 = 0; t4 < kOT; t4 += 4) {
       __syncthreads();

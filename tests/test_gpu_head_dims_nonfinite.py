@@ -1,0 +1,94 @@
+"""NaN and infinities at head dimensions 64 and 256: a row one of whose logits is NaN or +inf comes out as 0, a logit of
+-inf is a token that is not there - whichever wavefront, tile or share meets the token, and whatever else that one met."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import kitty_oracle as O
+from tests.helpers import make_kv
+
+pytestmark = pytest.mark.gpu
+
+
+def _state(D, T, seed):
+    import kitty_amd
+    from tests import gpu_util as u
+    k, v = make_kv(2, 2, T, D=D, seed=seed)
+    cache = kitty_amd.KittyCache(u.cfg(2, 4, D=D), 2, 2048)
+    ol = O.OracleLayer(2, 2048, 2, D=D, D_BOOSTED=D // 4)
+    cache.update(u.to_dev(k), u.to_dev(v), 0)
+    cache.quantize_prefill(0)
+    ol.update(k, v)
+    ol.quantize_prefill()
+    return u, cache.kv_cache[0], ol
+
+
+def _query(D, T_q, seed):
+    q = np.random.default_rng(seed).standard_normal((2, 4, T_q, D)).astype(np.float16)
+    q[:, ::2, :, 0], q[:, 1::2, :, 0] = 1, -1         # even heads see +inf where a key's first channel is +inf, odd ones -inf
+    return q
+
+
+def _plant(L, ol, token, value):
+    """Channel 0 of a key of (batch row 1, kv head 0) that lies in the sink or the Q-buffer."""
+    sink = token < 32
+    t = token if sink else (token - 32) % 128
+    (L.Sink_Buffer_K if sink else L.Q_Buffer_K)[1, 0, t, 0] = value
+    (ol.Sink_Buffer_K if sink else ol.Q_Buffer_K)[1, 0, t, 0] = value
+
+
+def _expect(ref, value):
+    """The oracle's result with the rows of (1, kv head 0) that meet a NaN or +inf logit set to 0."""
+    ref = ref.copy()
+    if np.isnan(value):
+        ref[1, :, :2] = 0
+    else:
+        ref[1, :, 0] = 0                               # head 0 (+inf); head 1 sees -inf
+    return ref
+
+
+def _close(out, ref, what):
+    got = out.float().cpu().numpy().astype(np.float64)
+    assert np.isfinite(got).all() and (np.abs(got - ref) <= 2.0 ** -11 * np.abs(ref) + 2e-5).all(), what
+
+
+# (tokens, the planted one): alone in its wavefront's share of the tile, with others, in the sink, in a tail tile
+PLACES = [(3, 2), (9, 2), (32, 31), (35, 34), (32 + 128 + 3, 32 + 128 + 2), (32 + 256 + 70, 32 + 256 + 69), (32 + 256 + 70, 5)]
+
+
+@pytest.mark.parametrize("D", [64, 256])
+@pytest.mark.parametrize("T,token", PLACES)
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_decode(D, T, token, value):
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    from kitty_amd.kvcache.kernels import kitty_attention_forward
+    u, L, ol = _state(D, T, T)
+    q = _query(D, 1, T)
+    with np.errstate(all="ignore"):
+        _plant(L, ol, token, value)
+        ref = _expect(O.decode_attention(ol, q, D ** -0.5, reference_rounding=False, dequant="two"), value)
+    out, _ = kitty_attention_forward(u.module(2, 4), u.to_dev(q), L, D ** -0.5, num_splits=1)
+    _close(out, ref, (D, T, token))
+
+
+@pytest.mark.parametrize("D", [64, 256])
+@pytest.mark.parametrize("T,token", PLACES)
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+@pytest.mark.parametrize("T_q", [1, 17])
+def test_chunk(D, T, token, value, T_q, monkeypatch):
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    from kitty_amd import _lib
+    from kitty_amd.kvcache.kernels import kitty_attention as A
+    u, L, ol = _state(D, T, T)
+    k, v = make_kv(2, 2, T_q, D=D, seed=T_q)
+    q = _query(D, T_q, T)
+    with np.errstate(all="ignore"):
+        _plant(L, ol, token, value)
+        ref = _expect(O.chunk_attention(ol, q, k, v, D ** -0.5, dequant="two"), value)
+    for s in (1, 3, 20):
+        monkeypatch.setattr(A, "_chunk_split_plan",
+                            lambda *a, s=s: (s, _lib.lib().kitty_prefill_attn_workspace_bytes(2, 4, D, T_q, s)))
+        out, _ = A.kitty_prefill_attention(u.module(2, 4), u.to_dev(q), u.to_dev(k), u.to_dev(v), L, D ** -0.5)
+        _close(out, ref, (D, T, token, s))
