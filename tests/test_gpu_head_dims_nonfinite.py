@@ -1,5 +1,6 @@
-"""NaN and infinities at head dimensions 64 and 256: a row one of whose logits is NaN or +inf comes out as 0, a logit of
--inf is a token that is not there - whichever wavefront, tile or share meets the token, and whatever else that one met."""
+"""NaN and infinities in attention.  Head dimensions 64 and 256: a row one of whose logits is NaN or +inf comes out as 0, a logit of
+-inf is a token that is not there - whichever wavefront, tile or share meets the token, and whatever else that one met.  Head dimension 128, chunks and prompts: such a row is NaN, in
+one walk and in shares, and a prompt's rows in front of the token do not see it."""
 import numpy as np
 import pytest
 import torch
@@ -92,3 +93,57 @@ def test_chunk(D, T, token, value, T_q, monkeypatch):
                             lambda *a, s=s: (s, _lib.lib().kitty_prefill_attn_workspace_bytes(2, 4, D, T_q, s)))
         out, _ = A.kitty_prefill_attention(u.module(2, 4), u.to_dev(q), u.to_dev(k), u.to_dev(v), L, D ** -0.5)
         _close(out, ref, (D, T, token, s))
+
+
+@pytest.mark.parametrize("T,token", [(3, 2), (32, 31), (32 + 128 + 3, 32 + 128 + 2), (32 + 256 + 70, 5)])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_chunk_128(T, token, value, monkeypatch):
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    from kitty_amd import _lib
+    from kitty_amd.kvcache.kernels import kitty_attention as A
+    u, L, ol = _state(128, T, T)
+    k, v = make_kv(2, 2, 17, seed=17)
+    q = _query(128, 17, T)
+    with np.errstate(all="ignore"):
+        _plant(L, ol, token, value)
+        ref = _expect(O.chunk_attention(ol, q, k, v, 128 ** -0.5, dequant="two"), value)
+    nan = np.zeros(ref.shape, bool)
+    nan[1, :, :2 if np.isnan(value) else 1] = True
+    for s in (1, 3, 20):
+        monkeypatch.setattr(A, "_chunk_split_plan",
+                            lambda *a, s=s: (s, _lib.lib().kitty_prefill_attn_workspace_bytes(2, 4, 128, 17, s)))
+        out, _ = A.kitty_prefill_attention(u.module(2, 4), u.to_dev(q), u.to_dev(k), u.to_dev(v), L, 128 ** -0.5)
+        got = out.float().cpu().numpy()
+        assert (np.isnan(got) == nan).all(), s
+        # fp16 probabilities (2^-11 each, relative) weigh rows of at most max|v|; half a unit of the fp16 result
+        bound = 2.0 ** -11 * float(np.abs(v).max() + 4) + 2.0 ** -11 * np.abs(ref)
+        assert (np.abs(got - ref)[~nan] <= bound[~nan]).all(), s
+
+
+@pytest.mark.parametrize("T,token", [(5, 0), (40, 33), (300, 140), (700, 699)])
+@pytest.mark.parametrize("shares", [1, 2, 5])
+def test_prompt(T, token, shares, monkeypatch):
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    import kitty_amd
+    from kitty_amd import _lib
+    from kitty_amd.kvcache.kernels import kitty_attention as A
+    from tests import gpu_util as u
+    k, v = make_kv(1, 2, T, seed=T)
+    k[0, 0, token, 3] = np.nan
+    q = np.random.default_rng(T).standard_normal((1, 4, T, 128)).astype(np.float16)
+    L = kitty_amd.KittyCache(u.cfg(2, 4), 1, 1024).kv_cache[0]
+    qd, kd, vd = u.to_dev(q), u.to_dev(k), u.to_dev(v)
+    monkeypatch.setattr(A, "_chunk_split_plan", lambda *a: (shares, _lib.lib().kitty_prefill_attn_workspace_bytes(1, 4, 128, T, shares)))
+    assert A.prompt_attention_ready(qd, kd, vd, L)
+    got = A.kitty_prompt_attention(qd, kd, vd, L, 128 ** -0.5)[0].float().cpu().numpy()      # [T, 4, 128]
+    assert np.isnan(got[token:, :2]).all()
+    clean = got.copy()
+    clean[token:, :2] = 0
+    assert np.isfinite(clean).all()
+    k[0, 0, token, 3] = 0
+    ref = np.concatenate([O.prefill_attention(q[0, 2 * h:2 * h + 2], k[0, h:h + 1], v[0, h:h + 1], 128 ** -0.5, 0) for h in (0, 1)])
+    ref = ref.transpose(1, 0, 2)
+    ref[token:, :2] = 0
+    assert (np.abs(clean - ref) <= 2.0 ** -11 * np.abs(v).max() + 2.0 ** -11 * np.abs(ref)).all()
