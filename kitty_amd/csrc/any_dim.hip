@@ -178,7 +178,8 @@ typedef short short4v __attribute__((ext_vector_type(4)));
 
 constexpr float kLog2e = 1.44269504088896340736f;
 constexpr uint32_t kCodeMagic = 0x64006400u;   // fp16 1024 in both halves: 1024 + n is exact for n < 1024
-constexpr float kProbScale = 4096.f;           // probabilities as matrix operands: see below
+constexpr float kProbScale = 32768.f;          // probabilities as matrix operands: see below
+constexpr int kProbParts = 3;
 
 __device__ __forceinline__ float4v mfma16(const uint32_t (&a)[4], const uint32_t (&b)[4], float4v c) {
   const uint4v av = {a[0], a[1], a[2], a[3]}, bv = {b[0], b[1], b[2], b[3]};
@@ -263,11 +264,12 @@ struct AnyLds {
 // own: its accumulator of the first product holds, lane for lane, the B operand of the second (lane group kg:
 // tokens 32kg + 8j + 2w, + 1), and the wavefronts meet only where a tile is staged and once at the end.
 // fp16 rows (sink, windows, the chunk) are loaded from memory in operand order.
-// Probabilities stay fp32 numbers: 4096 p is split into two fp16 numbers (22 bits; a remainder below fp16's
-// normal range is below 2^-26 of the row's largest probability), each a matrix operand of its own.
+// Probabilities stay fp32 numbers: 32768 p is split into three fp16 numbers, each a matrix operand of its own.
+// Together they are the fp32 number itself from 2^-16 of the row's largest probability on; below that they miss it by
+// at most 2^-40 of the largest.
 // A decode layer (append, this kernel, merge) on MI355X, against the version on the vector ALUs before it:
 //   D = 64,  B = 8, 6100 tokens, 32 / 8 heads:  79 -> 25 us
-//   D = 256, B = 2, 9000 tokens, 16 / 8 heads: 194 -> 36 us
+//   D = 256, B = 2, 9000 tokens, 16 / 8 heads: 194 -> 38 us
 template <int D, bool PREFILL, int NT>
 __global__ __launch_bounds__(256, PREFILL ? 1 : D == 64 ? 3 : 2) void attn_any_kernel(
     kitty_kv_layer L, const uint8_t* __restrict__ q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
@@ -460,7 +462,7 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : D == 64 ? 3 : 2) void attn_any_k
     }
 
     // ---- online softmax of this wavefront's tokens ----------------------------------------------
-    uint32_t ph[NT][4], pl[NT][4];
+    uint32_t pr[kProbParts][NT][4];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
 #pragma unroll
@@ -491,11 +493,13 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : D == 64 ? 3 : 2) void attn_any_k
       for (int j = 0; j < 4; ++j) {
         const float p0v = __builtin_amdgcn_exp2f(S[0][nt][j] - ref), p1v = __builtin_amdgcn_exp2f(S[1][nt][j] - ref);
         sum += p0v + p1v;
-        const float x0 = p0v * kProbScale, x1 = p1v * kProbScale;
-        const half2v hi = {(_Float16)x0, (_Float16)x1};
-        const half2v lo = {(_Float16)(x0 - (float)hi[0]), (_Float16)(x1 - (float)hi[1])};
-        ph[nt][j] = __builtin_bit_cast(uint32_t, hi);
-        pl[nt][j] = __builtin_bit_cast(uint32_t, lo);
+        float x0 = p0v * kProbScale, x1 = p1v * kProbScale;
+#pragma unroll
+        for (int i = 0; i < kProbParts; ++i) {
+          const half2v part = {(_Float16)x0, (_Float16)x1};
+          pr[i][nt][j] = __builtin_bit_cast(uint32_t, part);
+          x0 -= (float)part[0], x1 -= (float)part[1];   // exact
+        }
       }
       l_run[nt] += sum;
     }
@@ -534,10 +538,9 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : D == 64 ? 3 : 2) void attn_any_k
 #pragma unroll
           for (int j = 0; j < 4; ++j) a[j] = dequant_v<u>(X[j], X10[j], sc[j], zr[j]);
 #pragma unroll
-          for (int nt = 0; nt < NT; ++nt) {
-            O[hf * kU + u][nt] = mfma16(a, ph[nt], O[hf * kU + u][nt]);
-            O[hf * kU + u][nt] = mfma16(a, pl[nt], O[hf * kU + u][nt]);
-          }
+          for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int i = 0; i < kProbParts; ++i) O[hf * kU + u][nt] = mfma16(a, pr[i][nt], O[hf * kU + u][nt]);
         };
         tile(std::integral_constant<int, 0>{}), tile(std::integral_constant<int, 1>{});
         tile(std::integral_constant<int, 2>{}), tile(std::integral_constant<int, 3>{});
@@ -580,10 +583,9 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : D == 64 ? 3 : 2) void attn_any_k
           for (int j = 0; j < 4; ++j)
             a[j] = u & 1 ? high_halves(x[2 * j][u >> 1], x[2 * j + 1][u >> 1]) : low_halves(x[2 * j][u >> 1], x[2 * j + 1][u >> 1]);
 #pragma unroll
-          for (int nt = 0; nt < NT; ++nt) {
-            O[hf * kU + u][nt] = mfma16(a, ph[nt], O[hf * kU + u][nt]);
-            O[hf * kU + u][nt] = mfma16(a, pl[nt], O[hf * kU + u][nt]);
-          }
+          for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int i = 0; i < kProbParts; ++i) O[hf * kU + u][nt] = mfma16(a, pr[i][nt], O[hf * kU + u][nt]);
         }
       }
     }

@@ -138,7 +138,7 @@ def _launch_chunk(desc, query, key_states, value_states, scaling, out, ws, ws_by
 
 def prompt_attention_ready(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, kv_cache: KVCache_Layer) -> bool:
     """The chunk kernel can run a prompt's dense causal attention on these tensors as they lie.  What stays with
-    torch's attention: other types, devices and head dimensions (at 64 and 256 the kernel keeps 22-bit probabilities
+    torch's attention: other types, devices and head dimensions (at 64 and 256 the kernel keeps fp32 probabilities
     and is slower than a dense kernel), rows off the 16-byte grid, autocast (which gives the result its type), and whatever
     is being differentiated or traced."""
     if not kv_cache.on_hip or kv_cache.D != 128 or kv_cache.MAX_PAGE < 1:

@@ -1,7 +1,7 @@
 """Attention at head dimensions 64 and 256 where the matrix-core kernel's lane maps can go wrong: tiles with one
 token, with a token more or less than a page, windows whose ring has turned, every group size around the 16-row column
 tile, walks cut into more shares than there are tiles.  The kernel dequantizes with the reference's two roundings and
-keeps probabilities to 22 bits, so beyond the output's own fp16 rounding only fp32 sums remain."""
+keeps probabilities as fp32 numbers, so beyond the output's own fp16 rounding only fp32 sums remain."""
 import numpy as np
 import pytest
 import torch
