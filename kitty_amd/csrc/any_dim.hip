@@ -218,6 +218,14 @@ __device__ __forceinline__ uint32_t dequant_v(uint32_t x, uint32_t x10, uint32_t
   constexpr int k = 2 * (U < 5 ? U : U - 5);
   return dequant_word<k>(((U < 5 ? x : x10) & (0x00030003u << k)) | kCodeMagic, scale, zero);
 }
+// infinities as the largest finite number: operands of the second and third part of a probability, which may be 0 or negative
+// (the first part, times the infinity itself, has already made the sum infinite).  Costs the fp16 rows two instructions a
+// word and packed tiles a look at their scales: 3 % at D = 64 and D = 256 (the steps named at the kernel: 101 -> 104, 150 -> 156 us)
+__device__ __forceinline__ uint32_t finite_word(uint32_t x) {
+  const half2v top = {(_Float16)65504.f, (_Float16)65504.f};
+  const half2v v = __builtin_elementwise_min(__builtin_elementwise_max(__builtin_bit_cast(half2v, x), -top), top);
+  return __builtin_bit_cast(uint32_t, v);
+}
 // maximum over lanes l, l^16, l^32, l^48
 __device__ __forceinline__ float max_over_lane_groups(float v) {
   const unsigned b = __builtin_bit_cast(unsigned, v);
@@ -268,8 +276,8 @@ struct AnyLds {
 // Together they are the fp32 number itself from 2^-16 of the row's largest probability on; below that they miss it by
 // at most 2^-40 of the largest.
 // A decode layer (append, this kernel, merge) on MI355X, against the version on the vector ALUs before it:
-//   D = 64,  B = 8, 6100 tokens, 32 / 8 heads:  79 -> 25 us
-//   D = 256, B = 2, 9000 tokens, 16 / 8 heads: 194 -> 38 us
+//   D = 64,  B = 8, 6100 tokens, 32 / 8 heads:  79 -> 26 us
+//   D = 256, B = 2, 9000 tokens, 16 / 8 heads: 194 -> 39 us
 template <int D, bool PREFILL, int NT>
 __global__ __launch_bounds__(256, PREFILL ? 1 : D == 64 ? 3 : 2) void attn_any_kernel(
     kitty_kv_layer L, const uint8_t* __restrict__ q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
@@ -506,6 +514,18 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : D == 64 ? 3 : 2) void attn_any_k
 
     // ---- O += P V over the same tokens ------------------------------------------------------------
     const int t0 = 32 * kg + 2 * w;   // register j of an operand: tokens t0 + 8 j, t0 + 8 j + 1
+    auto weigh = [&](uint32_t (&a)[4], int t, bool infinities) {
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) O[t][nt] = mfma16(a, pr[0][nt], O[t][nt]);
+      if (infinities) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) a[j] = finite_word(a[j]);
+      }
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int i = 1; i < kProbParts; ++i) O[t][nt] = mfma16(a, pr[i][nt], O[t][nt]);
+    };
     if (v_packed) {
       uint32_t sc[4], zr[4];
 #pragma unroll
@@ -517,6 +537,11 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : D == 64 ? 3 : 2) void attn_any_k
         }
         sc[j] = low_halves(mm.x, mm.y), zr[j] = high_halves(mm.x, mm.y);
       }
+      // 3 scale + zero stays finite where both are below 2^13; elsewhere a value may be infinite
+      uint32_t big = 0u;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) big |= ((sc[j] & 0x7fff7fffu) + 0x10001000u) | ((zr[j] & 0x7fff7fffu) + 0x10001000u);
+      const bool wild = __any((big & 0x80008000u) != 0u);
       const int rr = n >> 2, tok = t0 + (rr & 1) + 8 * (rr >> 1);
 #pragma unroll
       for (int hf = 0; hf < kHalves; ++hf) {
@@ -537,10 +562,7 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : D == 64 ? 3 : 2) void attn_any_k
           uint32_t a[4];
 #pragma unroll
           for (int j = 0; j < 4; ++j) a[j] = dequant_v<u>(X[j], X10[j], sc[j], zr[j]);
-#pragma unroll
-          for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-            for (int i = 0; i < kProbParts; ++i) O[hf * kU + u][nt] = mfma16(a, pr[i][nt], O[hf * kU + u][nt]);
+          weigh(a, hf * kU + u, wild);
         };
         tile(std::integral_constant<int, 0>{}), tile(std::integral_constant<int, 1>{});
         tile(std::integral_constant<int, 2>{}), tile(std::integral_constant<int, 3>{});
@@ -582,10 +604,7 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : D == 64 ? 3 : 2) void attn_any_k
 #pragma unroll
           for (int j = 0; j < 4; ++j)
             a[j] = u & 1 ? high_halves(x[2 * j][u >> 1], x[2 * j + 1][u >> 1]) : low_halves(x[2 * j][u >> 1], x[2 * j + 1][u >> 1]);
-#pragma unroll
-          for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-            for (int i = 0; i < kProbParts; ++i) O[hf * kU + u][nt] = mfma16(a, pr[i][nt], O[hf * kU + u][nt]);
+          weigh(a, hf * kU + u, true);
         }
       }
     }

@@ -147,3 +147,38 @@ def test_prompt(T, token, shares, monkeypatch):
     ref = ref.transpose(1, 0, 2)
     ref[token:, :2] = 0
     assert (np.abs(clean - ref) <= 2.0 ** -11 * np.abs(v).max() + 2.0 ** -11 * np.abs(ref)).all()
+
+
+@pytest.mark.parametrize("D", [64, 256])
+@pytest.mark.parametrize("T,token", [(3, 1), (40, 31), (32 + 128 + 100, 32 + 128 + 60), (32 + 384, 32 + 20)])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_infinite_values(D, T, token, splits):
+    """A value that is infinite makes its channel infinite and no other: +-inf in fp16 rows; in packed pages a range so
+    wide that the reference's fp16 arithmetic overflows (code * scale beyond 65504)."""
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    import kitty_amd
+    from kitty_amd.kvcache.kernels import kitty_attention_forward
+    from tests import gpu_util as u
+    k, v = make_kv(1, 2, T, D=D, seed=T)
+    packed = token >= 32 and token < T - 128
+    if packed:
+        v[0, 0, token, ::2], v[0, 0, token, 1::2] = -60000, 60000
+    else:
+        v[0, 0, token, 3], v[0, 0, token, D - 2] = np.inf, -np.inf
+    cache = kitty_amd.KittyCache(u.cfg(2, 4, D=D), 1, 2048)
+    ol = O.OracleLayer(1, 2048, 2, D=D, D_BOOSTED=D // 4)
+    with np.errstate(all="ignore"):
+        cache.update(u.to_dev(k), u.to_dev(v), 0)
+        cache.quantize_prefill(0)
+        ol.update(k, v)
+        ol.quantize_prefill()
+        q = np.random.default_rng(T).standard_normal((1, 4, 1, D)).astype(np.float16)
+        ref = O.decode_attention(ol, q, D ** -0.5, reference_rounding=False, dequant="two")
+    assert (ol.PageCount_V * 128 > token - 32 >= 0) == packed and np.isinf(ref).any() and not np.isnan(ref).any()
+    out, _ = kitty_attention_forward(u.module(2, 4), u.to_dev(q), cache.kv_cache[0], D ** -0.5, num_splits=splits)
+    got = out.float().cpu().numpy().astype(np.float64)
+    inf = np.isinf(ref)
+    assert (got[inf] == ref[inf]).all()
+    big = 60000 if packed else 8                            # fp32 sums over terms of that size
+    assert (np.abs(got - ref)[~inf] <= 2.0 ** -11 * np.abs(ref[~inf]) + 2.5e-6 * big).all()
