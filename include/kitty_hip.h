@@ -309,7 +309,8 @@ int kitty_append_chunk(const kitty_kv_layer* layer, const void* k_new, const voi
 /*
  * kitty_append_chunk with the layer's scalar counters (layer->counts; seq_counts must be NULL): one chunk for every
  * sequence of the batch in two launches.  The caller advances its counters by the closed form of the state
- * machine.  Rows of a Q-buffer past its fill count are left as the last page that went through it lies there.  A page whose table entry is outside the cache is not written.
+ * machine.  Rows of a Q-buffer past its fill count are left as the last page that went through it lies there.
+ * A page whose table entry is outside the cache is not written, and recorded in layer->status.
  */
 int kitty_append_chunk_host(const kitty_kv_layer* layer, const void* k_new, const void* v_new, int64_t stride_b,
                             int64_t stride_h, int64_t stride_t, int B, int T, void* stream);

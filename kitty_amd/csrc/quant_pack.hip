@@ -740,7 +740,7 @@ struct VStreamRows {
 
 // grid (2 * max_pages, H_KV, B): blockIdx.x < max_pages: new K page blockIdx.x, else new V page.  With the
 // counters on the device a sequence takes the whole chunk or nothing; with host counters (HOST) a page whose id
-// is outside the cache is left out alone, as kitty_quant_pack_k / _v leave it out.
+// is outside the cache is left out alone and recorded, as kitty_quant_pack_k / _v do it.
 template <bool HOST>
 __global__ __launch_bounds__(256) void chunk_quant_kernel(kitty_kv_layer L, const uint8_t* __restrict__ k_new,
                                                           const uint8_t* __restrict__ v_new, int64_t stride_b,
@@ -755,14 +755,20 @@ __global__ __launch_bounds__(256) void chunk_quant_kernel(kitty_kv_layer L, cons
   const int64_t src = (int64_t)b * stride_b + (int64_t)h * stride_h + (int64_t)c.a * stride_t;
   if (!vside) {
     const int64_t pg = L.page_table_k[(int64_t)b * L.page_table_k_stride_b + c.pk + p];
-    if (HOST && (pg < 0 || pg >= L.cache_pages_k)) return;
+    if (HOST && (pg < 0 || pg >= L.cache_pages_k)) {
+      if (L.status && threadIdx.x == 0) L.status[b * KITTY_STATUS_FIELDS + KITTY_STATUS_BAD_PAGE_WRITE] = 1;
+      return;
+    }
     quant_k_page<1>(KStreamRows{(const uint8_t*)L.qbuf_k + w, k_new + src, stride_t, c.rk, p * kPage}, L.D_BOOSTED,
                     nullptr, nullptr,
                     const_cast<uint8_t*>(L.key_cache) + pg * L.key_cache_stride_page + (int64_t)h * k_head_bytes(L.D_BOOSTED),
                     (uint8_t*)L.key_meta + pg * L.key_meta_stride_page + (int64_t)h * kD * 4);
   } else {
     const int64_t pg = L.page_table_v[(int64_t)b * L.page_table_v_stride_b + c.pv + p];
-    if (HOST && (pg < 0 || pg >= L.cache_pages_v)) return;
+    if (HOST && (pg < 0 || pg >= L.cache_pages_v)) {
+      if (L.status && threadIdx.x == 0) L.status[b * KITTY_STATUS_FIELDS + KITTY_STATUS_BAD_PAGE_WRITE] = 1;
+      return;
+    }
     quant_v_page(VStreamRows{(const uint8_t*)L.qbuf_v + w, (const uint8_t*)L.local_v + w, v_new + src, stride_t, c.rv,
                              c.er, c.off, p * kPage},
                  const_cast<uint8_t*>(L.value_cache) + pg * L.value_cache_stride_page + (int64_t)h * kVBytes,

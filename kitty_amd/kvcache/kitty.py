@@ -491,7 +491,7 @@ class KittyCache(_HFCache):
             if L.Q_Buffer_Count_K == 0 and hi - lo >= P:
                 pages = (hi - lo) // P
                 quantize_pack_k(src, lo, pages, L.PageTable_K, L.PageCount_K, L.KeyCache, L.KeyCache_metadata, P,
-                                L.D_BOOSTED, select=self.select)
+                                L.D_BOOSTED, select=self.select, status=L.status)
                 L.PageCount_K += pages
                 lo += pages * P
                 continue
@@ -501,7 +501,7 @@ class KittyCache(_HFCache):
             lo += m
             if L.Q_Buffer_Count_K == P:
                 quantize_pack_k(L.Q_Buffer_K, 0, 1, L.PageTable_K, L.PageCount_K, L.KeyCache, L.KeyCache_metadata,
-                                P, L.D_BOOSTED, select=self.select)
+                                P, L.D_BOOSTED, select=self.select, status=L.status)
                 L.PageCount_K += 1
                 L.Q_Buffer_Count_K = 0
 
@@ -511,7 +511,8 @@ class KittyCache(_HFCache):
         while lo < hi:
             if L.Q_Buffer_Count_V == 0 and hi - lo >= P:
                 pages = (hi - lo) // P
-                quantize_pack_v(src, lo, pages, L.PageTable_V, L.PageCount_V, L.ValueCache, L.ValueCache_metadata, P)
+                quantize_pack_v(src, lo, pages, L.PageTable_V, L.PageCount_V, L.ValueCache, L.ValueCache_metadata, P,
+                                status=L.status)
                 L.PageCount_V += pages
                 lo += pages * P
                 continue
@@ -521,7 +522,7 @@ class KittyCache(_HFCache):
             lo += m
             if L.Q_Buffer_Count_V == P:
                 quantize_pack_v(L.Q_Buffer_V, 0, 1, L.PageTable_V, L.PageCount_V, L.ValueCache,
-                                L.ValueCache_metadata, P)
+                                L.ValueCache_metadata, P, status=L.status)
                 L.PageCount_V += 1
                 L.Q_Buffer_Count_V = 0
 

@@ -77,3 +77,27 @@ def test_chunk(T0, chunks):
     with pytest.raises(ValueError, match="max_length"):
         fast.append(k, k, 0)
     assert fast.kv_cache[0].counts() == before
+
+
+@pytest.mark.parametrize("side,entry", [("K", 0), ("K", 2), ("V", 0), ("V", 1)])
+@pytest.mark.parametrize("T0,T", [(100, 600), (40, 500), (32 + 128, 500)])
+def test_chunk_records_a_page_id_outside_the_cache(side, entry, T0, T):
+    """Both routes: the page is not written, everything else is, and ``check_status`` says whose page it was."""
+    D, H, B = 128, 2, 2
+    g = torch.Generator().manual_seed(T0 + T)
+    fast, slow, whole = (_cache(D, H, B, 2048) for _ in range(3))
+    rows = [tuple(torch.randn(B, n, H, D, generator=g).half().cuda().transpose(1, 2) for _ in range(2)) for n in (T0, T)]
+    for c in (fast, slow):
+        getattr(c.kv_cache[0], "PageTable_" + side)[1, entry] = 10 ** 6
+    for c, f in ((fast, lambda x: x), (slow, _odd), (whole, lambda x: x)):
+        for k, v in rows:
+            c.append(f(k), f(v), 0)
+    _same(fast, slow, (side, entry))
+    for c in (fast, slow):
+        assert c.check_status(raise_on_error=False)["bad_page_write"].tolist() == [[0, 1]]
+        with pytest.raises(RuntimeError, match="bad_page_write"):
+            c.check_status()
+    whole.check_status()
+    L, W = fast.kv_cache[0], whole.kv_cache[0]
+    name = "KeyCache" if side == "K" else "ValueCache"
+    assert not getattr(L, name)[L.MAX_PAGE + entry].any() and getattr(W, name)[L.MAX_PAGE + entry].any()
