@@ -305,7 +305,7 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : D == 64 ? 3 : 2) void attn_any_k
   if (D == 64) {   // shares that differ by at most one tile (B = 8, 6100 tokens: 24.1 -> 22.8 us)
     const int least = n_tiles / num_splits, longer = n_tiles - least * num_splits;
     tile_begin = split * least + min(split, longer), tile_end = tile_begin + least + (split < longer ? 1 : 0);
-  } else {         // equal ones, the last may be empty: at D = 256 the compiler's code for the above costs 5 %
+  } else {         // equal ones (the last shorter): at D = 256 the compiler's code for the above costs 5 %
     const int share = (n_tiles + num_splits - 1) / num_splits;
     tile_begin = min(split * share, n_tiles), tile_end = min(n_tiles, tile_begin + share);
   }
@@ -737,6 +737,13 @@ int any_positions(int D, int G) {
   const int rows = 16 * (D == 64 ? kPrefillTiles64 : kPrefillTiles256);
   return rows / G > 0 ? rows / G : 1;
 }
+// Shares of ceil(tiles / s) tiles, as the kernel cuts them at D = 256, may leave the last of them empty: 65 tiles in 64 shares are
+// 33 of two.  Those workgroups would load the queries and write partials for the merge to read.
+int without_empty_shares(int D, int tiles, int s) {
+  if (D == 64) return s;   // shares that differ by at most one tile
+  const int share = (tiles + s - 1) / s;
+  return (tiles + share - 1) / share;
+}
 }  // namespace
 
 // Splits of a decode walk.  Three workgroups fit a compute unit at D = 64 (registers), two at D = 256.  Long walks are
@@ -745,13 +752,13 @@ int any_positions(int D, int G) {
 // is no second round of them (D = 256, B = 2, 9000 tokens: 30 us with 24 splits of three tiles, 32 with 36 of two).
 // Where all of it fits at once a split is a tile: each costs 1.5 to 3.5 us of latency (D = 256, B = 1, 2000 tokens: 13.5 us
 // with 17 splits, 16.9 with 9).
-int decode_splits_any(int B, int H_KV, int tiles, int units) {
+int decode_splits_any(int B, int H_KV, int D, int tiles, int units) {
   const int64_t walks = (int64_t)B * H_KV;
   int64_t s = 3 * units / walks;
   if (s > 0 && tiles / s < 3) s = 2 * units / walks;
   if (s > tiles) s = tiles;
   if (s > 512) s = 512;
-  return s < 1 ? 1 : (int)s;
+  return without_empty_shares(D, tiles, s < 1 ? 1 : (int)s);
 }
 
 // Shares of a chunk's walk: enough workgroups for two on every compute unit (what their registers allow at
@@ -762,7 +769,7 @@ int prefill_splits_any(int B, int H_Q, int H_KV, int D, int Tq, int tiles, int u
   int64_t s = 2 * units / wgs;
   if (s > tiles / 2) s = tiles / 2;
   if (s > most) s = most;
-  return s < 1 ? 1 : (int)s;
+  return without_empty_shares(D, tiles, s < 1 ? 1 : (int)s);
 }
 
 void launch_prefill_any(const kitty_kv_layer& L, const void* q, int64_t q_stride_b, int64_t q_stride_h,

@@ -23,7 +23,7 @@ void launch_prefill_any(const kitty_kv_layer& L, const void* q, int64_t q_stride
                         int64_t q_stride_t, const void* k_new, const void* v_new, int64_t new_stride_b,
                         int64_t new_stride_h, int64_t new_stride_t, int B, int H_Q, int Tq, float scaling, void* out,
                         float* ws_ml, float* ws_acc, int num_splits, hipStream_t stream);
-int decode_splits_any(int B, int H_KV, int tiles, int units);
+int decode_splits_any(int B, int H_KV, int D, int tiles, int units);
 int prefill_splits_any(int B, int H_Q, int H_KV, int D, int Tq, int tiles, int units, int most);
 // merge pass over independent rows (rows_merge.hip)
 void launch_rows_merge(int D, const float* ws_ml, const float* ws_acc, void* out, int64_t rows, int num_splits,
@@ -87,7 +87,7 @@ extern "C" int kitty_decode_attn_default_splits(int B, int H_KV, int max_tiles, 
 extern "C" int kitty_decode_attn_default_splits_d(int B, int H_KV, int D, int max_tiles, int per_sequence_counts) {
   if (D == kD || !head_dim_supported(D) || B <= 0 || H_KV <= 0 || max_tiles <= 0)
     return kitty_decode_attn_default_splits(B, H_KV, max_tiles, per_sequence_counts);
-  return decode_splits_any(B, H_KV, max_tiles, device_simds() / 4);
+  return decode_splits_any(B, H_KV, D, max_tiles, device_simds() / 4);
 }
 
 namespace {
