@@ -13,8 +13,8 @@
  * Each function names the reference interface it replaces (paths relative to the reference
  * checkout, src/kitty/kvcache/...).
  *
- * Head dimensions: D = 128 runs on the tuned kernels; D = 64 and D = 256 are served by plain kernels
- * with the same arithmetic and storage format (the reference's kernels take D as a parameter,
+ * Head dimensions: D = 128 runs on kernels written for it; D = 64 and D = 256 have their own (attention on the matrix
+ * cores, quantizers of one thread per channel or token) with the same arithmetic and storage format (the reference's kernels take D as a parameter,
  * kernels/kitty_quant_pack.py:42-45, kernels/kitty_attention.py:59-62); any other D is KITTY_E_SHAPE.
  * PAGE_SIZE is 128.
  */

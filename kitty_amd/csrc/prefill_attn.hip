@@ -495,10 +495,10 @@ __host__ __device__ inline int block_positions(int G, int Tq) {
 }
 
 // SPLIT: blockIdx.x = block * num_splits + split; a workgroup walks its share of the tiles and leaves a
-// partial per row (running maximum, running sum, un-normalised output) for prefill_merge_kernel.  One
+// partial per row (running maximum, running sum, un-normalised output) for rows_merge_kernel.  One
 // workgroup fills a compute unit (147 KB of LDS), and a short chunk has few of them: 200 positions over
-// 12k cached tokens, 32 / 8 heads, are 32 workgroups of 98 tiles on 256 units; in 7 shares they are 224 of 14
-// tiles, and a layer (attention and append) takes 146 us instead of 555 (see prefill_splits).
+// 12k cached tokens, 32 / 8 heads, are 32 workgroups of 98 tiles on 256 units; in 8 shares they are 256 of 13
+// tiles, and a layer (attention and append) takes 118 us instead of 555 (see prefill_splits).
 template <bool BOOST, bool SPLIT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves / 4, kWaves / 4))) void prefill_attn_kernel(
     kitty_kv_layer L, const uint8_t* __restrict__ q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
@@ -665,8 +665,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
 // 8-byte operand reads on 64 different banks); V [token][channel] is read transposed.  On the kernel above such a tile
 // costs twice a packed one: its rows are fetched when they are needed, K goes in by 16-bit transposing stores, every
 // tile is masked.  Workgroups of one kv head share an XCD, whose L2 then serves its keys and values, longest first.
-// Bound by the vector and LDS work around the matrix instructions (exponentials, operand reads).
-// B = 2, 3001 tokens, 32 / 8 heads: 448 us on the kernel above, 238 here (620 TFLOP/s).
+// Bound, as the kernel above, by matrix, LDS and vector phases that overlap little.
+// B = 2, 3001 tokens, 32 / 8 heads: 448 us on the kernel above, 233 here (633 TFLOP/s; trace, launches back to back once the
+// clock is up - the first ones of a process take 265).
 template <bool SPLIT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves / 4, kWaves / 4))) void dense_attn_kernel(
     const uint8_t* __restrict__ q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
@@ -823,7 +824,7 @@ int prefill_lds_bytes() { return kLdsBytes; }
 // `tiles`: 128-token tiles the layer holds (sink included) plus those of the chunk; `most`: shares the scratch allows.
 int prefill_splits(int B, int H_Q, int H_KV, int Tq, int tiles, int units, int most) {
   const int G = H_Q / H_KV;
-  if ((int64_t)B * Tq > 65535) return 1;   // the merge's grid; such a launch has enough workgroups
+  if ((int64_t)B * Tq > 65535) return 1;   // more than a workgroup per compute unit for every query head: the device is full
   const int64_t wgs = (int64_t)c_div_up(Tq, block_positions(G, Tq)) * H_KV * B;
   const float rows = (float)B * (float)Tq * (float)H_Q;
   int best = 1;

@@ -2,7 +2,7 @@
 channels, src/kitty/kvcache/kitty.py:39-44; its kernels take D as a parameter): quantizer, cache plugin,
 decode attention and chunked-prefill attention against the oracle, whose quantizer is pinned at these sizes
 by the reference's own output (tests/golden/quant_k_v_d64.npz, quant_k_v_d256.npz).  These sizes run on
-plain kernels of their own; packed bytes bit-exact, attention within 2e-3 of float64 attention over the
+kernels of their own; packed bytes bit-exact, attention within 2e-3 of float64 attention over the
 reference's twice-rounded fp16 dequantization."""
 import numpy as np
 import pytest
