@@ -6,28 +6,36 @@
 // k^ = fp16(code) * scale + zero evaluated in fp16 (kitty_attention.py:162-165, 317-320).
 //
 // The work is a dense contraction (G * T_q query rows per KV head), so it runs on the matrix
-// cores, flash-attention style.  One workgroup of 4 wavefronts owns 256 query rows of one
+// cores, flash-attention style.  One workgroup of 8 wavefronts, two per SIMD, owns 256 query rows of one
 // (batch row, KV head): PB = 256 / G consecutive chunk positions times the G query heads of the
-// group; wavefront w owns rows 64w .. 64w+63.  The workgroup walks the sequence in 128-token
-// tiles.  Each tile is brought into LDS once, as fp16, by all 256 threads: packed pages are
+// group; wavefront w owns rows 32w .. 32w+31.  The workgroup walks the sequence in 128-token
+// tiles.  Each tile is brought into LDS once, as fp16, by all 512 threads: packed pages are
 // dequantized on the way (exactly the reference's two fp16 roundings), fp16 rows are copied.
 // Two tile buffers alternate: while tile t is multiplied, tile t+1 is converted into the other
 // buffer and the packed bytes of tile t+2 are in flight; one barrier per tile.
 //
-// Matrix-core formulation (v_mfma_f32_16x16x32_f16; lane = 16 kg + n holds A[n][8 k-slots],
-// B[8 k-slots][n], C[4kg .. 4kg+3][n]):
+// Matrix-core formulation (v_mfma_f32_32x32x16_f16; lane = 32 kg + n holds A[n][8 k-slots],
+// B[8 k-slots][n], C[8 (i / 4) + 4 kg + i % 4][n], i = 0 .. 15):
 //   S^T[pos][row]  = sum_ch  K[pos][ch]  * Q[row][ch]      A = keys,   B = queries (registers)
 //   O^T[cp][row]   = sum_pos V[pos][cp]  * P^T[pos][row]   A = values, B = probabilities
 // The accumulator of the first product is, lane for lane, the B operand of the second: k-slot j
-// of lane group kg stands for position 16 (j / 4) + 4 kg + j % 4 of a 32-position sub-tile.
+// of lane group kg stands for position 8 (j / 4) + 4 kg + j % 4 of 16.  A lane holds 16 logits of ONE row, so
+// the running maximum and sum are one register each and a reduction over a row is one exchange between two lanes.
 //
 // LDS layouts, chosen so that dequantization writes 128-bit rows and the matrix-core operands
 // come out of `ds_read_b64_tr_b16` (a 16-lane block reads 4 rows x 16 columns and lane i
 // receives column i of the 4 rows):
-//   K tile: [channel][position]       V tile: [position][channel slot]      row pitch 288 bytes
+//   K tile: [channel][position]       V tile: [position][channel slot]      row pitch 272 bytes
 // "position" and "channel slot" are the order in which codes fall out of a plane word when it is
 // masked with 0x00030003 << 2u: slot 2u + e of a 16-block is element u + 8e.  Keys and values use
 // the same token permutation, the output undoes the channel permutation.
+//
+// What bounds it: power and the vector unit, in turn.  B = 4, 32 / 8 heads, 2048 positions over 30720 cached tokens:
+// 5.13 -> 4.7 ms (830 -> 910 TFLOP/s; the matrix instructions alone, on the same frame, take 3.1).  Per wave and tile, against
+// v_mfma_f32_16x16x32 (two rows per lane, twice the matrix instructions) with 288-byte rows: 100 vector instructions,
+// 60 scalar ones and a dependent load (the boost slot) less, and a quarter of the bank conflicts.
+#include <type_traits>
+
 #include "decode_common.h"
 
 // wave priority while a wave issues the PV MFMAs (the other wave of the SIMD fills the gaps)
@@ -43,40 +51,24 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float float4v __attribute__((ext_vector_type(4)));
+typedef float float16v __attribute__((ext_vector_type(16)));
 typedef short short4v __attribute__((ext_vector_type(4)));
 typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
 
-constexpr int kPitch = 288;                   // bytes per LDS row: 128 fp16 + 32 bytes of padding
-constexpr int kRowPitch = 272;                // of a K tile in the dense kernel
-constexpr int kTile = kPage * kPitch;         // 36864 bytes, one K or V tile
+constexpr int kPitch = 272;                   // bytes per LDS row: 128 fp16 + 16 bytes of padding
+constexpr int kTile = kPage * kPitch;         // 34816 bytes, one K or V tile
 constexpr int kLdsBytes = 4 * kTile;          // K and V, two buffers each
 constexpr int kRows = 256;                    // query rows per workgroup
 constexpr int kWaves = 8;                     // two per SIMD: one does vector work while the other feeds the matrix pipe
 constexpr int kThreads = 64 * kWaves;
-constexpr int kNT = kRows / (16 * kWaves);    // 16-row column tiles per wave
-constexpr int kParts = kThreads / 128;        // threads that share one row of a tile while staging it
-constexpr int kW = 8 / kParts;                // 16-code words of a packed row per thread
-constexpr int kPartBytes = 256 / kParts;      // bytes of an fp16 row per thread
+constexpr int kWaveRows = kRows / kWaves;     // 32: one column tile of the matrix instruction per wave
+constexpr int kParts = 4;                     // threads that share one packed row of a tile while staging it
+constexpr int kSubs = 2;                      // sub-tiles of 32 positions that share one look at the maxima
 constexpr float kLog2e = 1.4426950408889634f;
-
-enum SrcKind : int { SRC_PACKED = 0, SRC_ROWS = 1, SRC_VTAIL = 2 };
-
-// where the keys and the values of one 128-token tile come from
-struct TileSrc {
-  int k_kind, v_kind;
-  const uint8_t* k_ptr;   // packed: the page-head;  rows: first row
-  const uint8_t* k_meta;
-  const uint8_t* v_ptr;
-  const uint8_t* v_meta;
-  int64_t k_stride, v_stride;   // rows: bytes between tokens
-  int v_u0;                     // v-tail: index of the tile's first token in [Q_Buffer_V | ring]
-  int ntok;                     // valid tokens
-  int chunk_t0;                 // >= 0: tile of the new chunk starting at this chunk position
-};
 
 // what issue() leaves in flight for a packed tile (fp16 rows are few and are copied by finish())
 struct Stage {
-  uint32_t klo[kW], khi[kW], v[kW];
+  uint2 klo, khi, v;
   uint32_t kmeta, vmeta;
 };
 
@@ -89,33 +81,29 @@ __device__ __forceinline__ half4 lds_tr(const uint8_t* p) {
   return __builtin_bit_cast(half4, r);
 }
 
-// matrix-core A operand: k-slots 0..3 from the 4 LDS rows at p, k-slots 4..7 from 16 rows further
+// matrix-core A operand: k-slots 0..3 from the 4 LDS rows at p, k-slots 4..7 from 8 rows further
 __device__ __forceinline__ half8 load_a(const uint8_t* p) {
-  const half4 a0 = lds_tr(p), a1 = lds_tr(p + 16 * kPitch);
+  const half4 a0 = lds_tr(p), a1 = lds_tr(p + 8 * kPitch);
   return __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
-// the dense kernel's: channels 4 kg .. of a 32-channel chunk and those 16 further, from one fp16 row
-__device__ __forceinline__ half8 load_row_a(const uint8_t* p) {
-  const half4 a0 = *(const half4*)p, a1 = *(const half4*)(p + 32);
-  return __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
-}
-
-// Maximum over the four lane groups (lanes l, l^16, l^32, l^48) with the row-swap instructions of
-// gfx950: two vector instructions per step, where a shuffle would be a round trip through LDS.
-// v_permlane16_swap exchanges rows 1 and 3 of its first operand with rows 0 and 2 of its second.
-__device__ __forceinline__ float max_over_lane_groups(float v) {
+// Maximum over lanes l and l^32 with the half-swap instruction of gfx950: two vector instructions, where a
+// shuffle would be a round trip through LDS.
+__device__ __forceinline__ float max_over_lane_halves(float v) {
   const unsigned b = __builtin_bit_cast(unsigned, v);
-  const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
-  const unsigned r0 = r[0], r1 = r[1];   // as scalars first: a bit_cast of r[1] itself reads element 0
-  const float m = vmax(__builtin_bit_cast(float, r0), __builtin_bit_cast(float, r1));
-  const unsigned c = __builtin_bit_cast(unsigned, m);
-  const auto q = __builtin_amdgcn_permlane32_swap(c, c, false, false);
-  const unsigned q0 = q[0], q1 = q[1];
+  const auto q = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  const unsigned q0 = q[0], q1 = q[1];   // as scalars first: a bit_cast of q[1] itself reads element 0
   return vmax(__builtin_bit_cast(float, q0), __builtin_bit_cast(float, q1));
 }
 
 __device__ __forceinline__ float xor_lanes(float v, int mask) { return __shfl_xor(v, mask); }
+
+// where the 16 tokens 16 g .. of a channel's row lie in a K tile: the two groups of a 32-token sub-tile 128 bytes apart
+__device__ __forceinline__ int token_group_bytes(int g) { return 32 * (g >> 1) + 128 * (g & 1); }
+// A 16-lane block of a transposing read takes every second row of eight, so that the rows of 272 bytes that two blocks
+// read (16 positions of either 128-byte half) and the four rows of four 64-byte pieces that 16 lanes write
+// meet each of the 64 banks once: row 8 a + 2 j + k is k-slot 4 k + j of its eight.
+__device__ __forceinline__ int row_slot(int r) { return (r & ~7) | ((r & 1) << 2) | ((r >> 1) & 3); }
 
 // fp16(code) * scale + zero with both roundings, for two codes at a time; `c` holds the codes as
 // integers in its two halves.
@@ -128,6 +116,20 @@ __device__ __forceinline__ uint32_t dequant_pair(uint32_t c, half2v scale, half2
   return __builtin_bit_cast(uint32_t, r);
 }
 
+// The same for 4-bit codes at bit SHIFT of each half of x, taken where they lie: 1024 + code * 2^SHIFT is a number of
+// fp16, and scaling it down and subtracting is exact.  `magic` is 1024 in both halves, in a register: with the mask as
+// the instruction's only constant, masking and merging are one instruction.
+template <int SHIFT>
+__device__ __forceinline__ uint32_t dequant_code(uint32_t x, uint32_t magic, half2v scale, half2v zero) {
+#pragma clang fp contract(off)
+  constexpr _Float16 k = (_Float16)(1.0f / (1 << SHIFT)), o = (_Float16)(1024.0f / (1 << SHIFT));
+  const half2v c = __builtin_bit_cast(half2v, (x & (0x000f000fu << SHIFT)) | magic);
+  const half2v f = SHIFT == 0 ? c - half2v{o, o} : __builtin_elementwise_fma(c, half2v{k, k}, half2v{-o, -o});
+  const half2v m = f * scale;
+  const half2v r = m + zero;
+  return __builtin_bit_cast(uint32_t, r);
+}
+
 template <bool BOOST, bool SPLIT>
 struct Prefill {
   const kitty_kv_layer& L;
@@ -137,159 +139,154 @@ struct Prefill {
   const uint8_t* v_new;
   int64_t new_stride_t;
   int kv_chunk;      // chunk tokens this workgroup can see
-  int n_body;        // body tiles
   int n_tiles;       // sink + body + chunk tiles actually walked
   int first_body, first_chunk;
   mutable int bad_page = 0;   // a page id outside the cache was met (checked_page)
-  // Page ids reach tile() through LDS, checked: kIdChunk body tiles at a time, the K and V ids are
-  // read by one thread each, range-checked (checked_page) and left as 32-bit numbers in one of two
-  // chunk buffers; the chunk after the current one is staged when the walk is half way through the
-  // current one, and the barrier that ends every iteration of the walk publishes it.  Reading and
-  // checking the ids where they are used - a load whose value the next instructions need, in every
-  // iteration of every workgroup - cost this kernel 10 %.
+  // Addresses reach issue() through LDS, checked: kChunk body tiles at a time, the K and V page ids are read by
+  // one thread each, range-checked (checked_page) and turned into the addresses of this head's bytes and metadata,
+  // in one half of a ring; the chunk after the current one is staged when the walk is half way through the
+  // current one, and the barrier that ends every iteration of the walk publishes it.  (Reading and checking the ids where
+  // they are used - a load whose value the next instructions need, in every iteration of every workgroup - cost this
+  // kernel 10 %; multiplying ids by strides there, on every thread, some 70 of 640 vector instructions a tile.)
   // Body tiles are counted from id_base(), the first one of this workgroup's share.
-  static constexpr int kIdChunk = 64;
-  int32_t (*page_ids)[2][kIdChunk];   // [chunk & 1][K, V][(body tile - id_base()) % kIdChunk]
+  static constexpr int kChunk = 64;
+  typedef const uint8_t* PageTable[4][2 * kChunk];   // [K, K metadata, V, V metadata][(body tile - id_base()) % (2 kChunk)]
+  const uint8_t* (*pages)[2 * kChunk];
   int first_id = 0;
   __device__ __forceinline__ int id_base() const { return SPLIT ? first_id : 0; }
 
-  __device__ __forceinline__ void stage_page_ids(int chunk) const {
-    if (tid < 2 * kIdChunk) {
-      const int side = tid / kIdChunk, i = id_base() + chunk * kIdChunk + tid % kIdChunk;
+  __device__ __forceinline__ void stage_pages(int chunk) const {
+    if (tid < 2 * kChunk) {
+      const int side = tid / kChunk, i = id_base() + chunk * kChunk + tid % kChunk;
       if (i < (side ? c.pv : c.pk)) {
         const int64_t pg = side ? L.page_table_v[(int64_t)b * L.page_table_v_stride_b + i]
                                 : L.page_table_k[(int64_t)b * L.page_table_k_stride_b + i];
-        page_ids[chunk & 1][side][tid % kIdChunk] =
-            (int32_t)checked_page(pg, side ? L.cache_pages_v : L.cache_pages_k, bad_page);
+        const int64_t ok = checked_page(pg, side ? L.cache_pages_v : L.cache_pages_k, bad_page);
+        const uint8_t* at = side ? L.value_cache + ok * L.value_cache_stride_page + (int64_t)h * kVBytes
+                                 : L.key_cache + ok * L.key_cache_stride_page + (int64_t)h * k_head_bytes(L.D_BOOSTED);
+        const uint8_t* meta = side ? (const uint8_t*)L.value_meta + ok * L.value_meta_stride_page + (int64_t)h * kPage * 4
+                                   : (const uint8_t*)L.key_meta + ok * L.key_meta_stride_page + (int64_t)h * kD * 4;
+        const int r = (chunk & 1) * kChunk + tid % kChunk;
+        pages[2 * side][r] = at;
+        pages[2 * side + 1][r] = meta;
       }
     }
   }
-  // (every lane reads the same word and keeps it in a vector register: made a scalar again with
-  // v_readfirstlane, with the tile addresses then computed on the scalar unit, the kernel is 4 % slower)
-  __device__ __forceinline__ int64_t staged_page(int side, int i) const {
-    const int r = i - id_base();
-    return page_ids[(r / kIdChunk) & 1][side][r % kIdChunk];
+  __device__ __forceinline__ const uint8_t* page(int which, int i) const {
+    return pages[which][(i - id_base()) & (2 * kChunk - 1)];
   }
 
-  __device__ TileSrc tile(int t) const {
-    TileSrc s;
-    s.chunk_t0 = -1;
-    s.k_meta = s.v_meta = nullptr;
-    s.v_u0 = 0;
-    const int64_t win = (int64_t)b * L.win_stride_b + (int64_t)h * L.win_stride_h;
-    if (t < first_body) {   // the sink rows
-      const int64_t off = (int64_t)b * L.sink_stride_b + (int64_t)h * L.sink_stride_h;
-      s.k_kind = s.v_kind = SRC_ROWS;
-      s.k_ptr = (const uint8_t*)L.sink_k + off;
-      s.v_ptr = (const uint8_t*)L.sink_v + off;
-      s.k_stride = s.v_stride = kD * 2;
-      s.ntok = c.sink;
-    } else if (t < first_chunk) {
-      const int i = t - first_body;
-      s.ntok = min(kPage, c.nbody - i * kPage);
-      if (i < c.pk) {
-        const int64_t pg = staged_page(0, i);
-        s.k_kind = SRC_PACKED;
-        s.k_ptr = L.key_cache + pg * L.key_cache_stride_page + (int64_t)h * k_head_bytes(L.D_BOOSTED);
-        s.k_meta = (const uint8_t*)L.key_meta + pg * L.key_meta_stride_page + (int64_t)h * kD * 4;
-      } else {
-        s.k_kind = SRC_ROWS;
-        s.k_ptr = (const uint8_t*)L.qbuf_k + win;
-        s.k_stride = kD * 2;
-      }
-      if (i < c.pv) {
-        const int64_t pg = staged_page(1, i);
-        s.v_kind = SRC_PACKED;
-        s.v_ptr = L.value_cache + pg * L.value_cache_stride_page + (int64_t)h * kVBytes;
-        s.v_meta = (const uint8_t*)L.value_meta + pg * L.value_meta_stride_page + (int64_t)h * kPage * 4;
-      } else {
-        s.v_kind = SRC_VTAIL;
-        s.v_ptr = nullptr;
-        s.v_u0 = (i - c.pv) * kPage;
-      }
-      s.v_stride = 0;
-    } else {
-      const int t0 = (t - first_chunk) * kPage;
-      s.k_kind = s.v_kind = SRC_ROWS;
-      s.k_ptr = k_new + (int64_t)t0 * new_stride_t;
-      s.v_ptr = v_new + (int64_t)t0 * new_stride_t;
-      s.k_stride = s.v_stride = new_stride_t;
-      s.ntok = min(kPage, kv_chunk - t0);
-      s.chunk_t0 = t0;
-    }
-    return s;
+  __device__ __forceinline__ int body(int t) const { return t - first_body; }   // -1: the sink
+  __device__ __forceinline__ bool k_packed(int t) const { return t >= first_body && t - first_body < c.pk && t < first_chunk; }
+  __device__ __forceinline__ bool v_packed(int t) const { return t >= first_body && t - first_body < c.pv && t < first_chunk; }
+  __device__ __forceinline__ int tokens(int t) const {
+    return t < first_body ? c.sink : t < first_chunk ? min(kPage, c.nbody - body(t) * kPage) : min(kPage, kv_chunk - chunk_pos(t));
+  }
+  __device__ __forceinline__ int chunk_pos(int t) const { return (t - first_chunk) * kPage; }   // < 0: not a tile of the chunk
+
+  // what a thread takes of packed rows: a K channel's tokens 32 part .., dealt so that 16 lanes write to 64 different banks; the
+  // channels 32 part .. of the value row that belongs in LDS row tid / 4
+  __device__ __forceinline__ int part() const { return tid % kParts; }
+  __device__ __forceinline__ int key_channel() const {
+    return (tid >> 6) * 16 + ((tid >> 4) & 3) * 2 + ((tid >> 2) & 1) + ((tid >> 3) & 1) * 8;
+  }
+  __device__ __forceinline__ int value_row() const { return tid / kParts; }
+  __device__ __forceinline__ int value_token() const {   // slot 2u + e of a 16-block is token u + 8e
+    const int m = row_slot(value_row());
+    return (m & ~15) | ((m >> 1) & 7) | ((m & 1) << 3);
+  }
+
+  // The boost slot of this thread's channel in tile t.  The high plane's words lie where it says: asked for a tile before
+  // issue(), or every wave would wait for one load in order to start the next.
+  // (FULL, here and below: tile t is known to be a page on both sides)
+  template <bool FULL>
+  __device__ __forceinline__ int ask_slot(int t) const {
+    return BOOST && (FULL || k_packed(t)) ? page(0, body(t))[kLoBytes + L.D_BOOSTED * kRowBytes + key_channel()] : 255;
   }
 
   // ---- stage 1: global loads of a packed tile into registers ----------------------------------
-  __device__ __forceinline__ void issue(const TileSrc& s, Stage& g) const {
-    const int e = tid / kParts, part = tid % kParts;   // element (channel or token) and its part of the row
-    if (s.k_kind == SRC_PACKED) {
-      const uint32_t* lo = (const uint32_t*)(s.k_ptr + e * kRowBytes + part * (4 * kW));
-#pragma unroll
-      for (int w = 0; w < kW; ++w) g.klo[w] = lo[w];
-      g.kmeta = *(const uint32_t*)(s.k_meta + e * 4);
-#pragma unroll
-      for (int w = 0; w < kW; ++w) g.khi[w] = 0u;
-      if (BOOST) {
-        const int slot = s.k_ptr[kLoBytes + L.D_BOOSTED * kRowBytes + e];
-        if (slot < L.D_BOOSTED) {
-          const uint32_t* hi = (const uint32_t*)(s.k_ptr + kLoBytes + slot * kRowBytes + part * (4 * kW));
-#pragma unroll
-          for (int w = 0; w < kW; ++w) g.khi[w] = hi[w];
-        }
-      }
+  template <bool FULL>
+  __device__ __forceinline__ void issue(int t, int slot, Stage& g) const {
+    if (FULL || k_packed(t)) {
+      const uint8_t* at = page(0, body(t));
+      g.klo = *(const uint2*)(at + key_channel() * kRowBytes + part() * 8);
+      g.kmeta = *(const uint32_t*)(page(1, body(t)) + key_channel() * 4);
+      g.khi = uint2{0u, 0u};
+      if (BOOST && slot < L.D_BOOSTED) g.khi = *(const uint2*)(at + kLoBytes + slot * kRowBytes + part() * 8);
     }
-    if (s.v_kind == SRC_PACKED) {
-      const uint32_t* vv = (const uint32_t*)(s.v_ptr + e * kRowBytes + part * (4 * kW));
-#pragma unroll
-      for (int w = 0; w < kW; ++w) g.v[w] = vv[w];
-      g.vmeta = *(const uint32_t*)(s.v_meta + e * 4);
+    if (FULL || v_packed(t)) {
+      g.v = *(const uint2*)(page(2, body(t)) + value_token() * kRowBytes + part() * 8);
+      g.vmeta = *(const uint32_t*)(page(3, body(t)) + value_token() * 4);
     }
   }
 
   // ---- stage 2: registers -> fp16 tile in LDS -----------------------------------------------
-  __device__ __forceinline__ void finish(const TileSrc& s, const Stage& g, uint8_t* kt, uint8_t* vt) const {
-    const int e = tid / kParts, part = tid % kParts;
-    if (s.k_kind == SRC_PACKED) {
-      // thread = one channel, 16 kW tokens: plane words of 16 tokens each
+  template <bool FULL>
+  __device__ __forceinline__ void finish(int t, const Stage& g, uint8_t* kt, uint8_t* vt) const {
+    const int64_t win = (int64_t)b * L.win_stride_b + (int64_t)h * L.win_stride_h;
+    const int64_t sink = (int64_t)b * L.sink_stride_b + (int64_t)h * L.sink_stride_h;
+    const bool in_sink = t < first_body, in_chunk = t >= first_chunk;
+    if (FULL || k_packed(t)) {
+      // thread = one channel, 32 tokens: plane words of 16 tokens each
       const half2v m2 = __builtin_bit_cast(half2v, g.kmeta);
       const half2v scale = {m2[0], m2[0]}, zero = {m2[1], m2[1]};
       const uint32_t k01 = dequant_pair(0x00010000u, scale, zero), k23 = dequant_pair(0x00030002u, scale, zero);
-      uint8_t* row = kt + e * kPitch + part * kPartBytes;
+      uint8_t* row = kt + key_channel() * kPitch + part() * 32;
+      uint32_t magic = 0x64006400u;
+      asm volatile("" : "+v"(magic));
 #pragma unroll
-      for (int w = 0; w < kW; ++w) {
+      for (int w = 0; w < 2; ++w) {
+        const uint32_t lo = w ? g.klo.y : g.klo.x, hi = w ? g.khi.y : g.khi.x;
         uint32_t o[8];
+        if (BOOST) {
+          // even, odd: the four bits of tokens 2j and 2j + 1 of each half of the word in nibble j
+          const uint32_t even = (lo & 0x33333333u) | ((hi << 2) & 0xccccccccu);
+          const uint32_t odd = ((lo >> 2) & 0x33333333u) | (hi & 0xccccccccu);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          uint32_t code = (g.klo[w] >> (2 * u)) & 0x00030003u;
-          if (BOOST) {
-            code |= ((g.khi[w] >> (2 * u)) & 0x00030003u) << 2;
-            o[u] = dequant_pair(code, scale, zero);
-          } else {   // four values per channel: the table of the V side below
+          for (int j = 0; j < 4; j += 2) {
+            const uint32_t x = even >> (4 * j), y = odd >> (4 * j);
+            o[2 * j] = dequant_code<0>(x, magic, scale, zero);
+            o[2 * j + 1] = dequant_code<0>(y, magic, scale, zero);
+            o[2 * j + 2] = dequant_code<4>(x, magic, scale, zero);
+            o[2 * j + 3] = dequant_code<4>(y, magic, scale, zero);
+          }
+        } else {   // four values per channel: the table of the V side below
+#pragma unroll
+          for (int u = 0; u < 8; ++u) {
+            const uint32_t code = (lo >> (2 * u)) & 0x00030003u;
             o[u] = __builtin_amdgcn_perm(k23, k01, code * 0x0202u + 0x01000100u);
           }
         }
-        *(uint4*)(row + w * 32) = uint4{o[0], o[1], o[2], o[3]};
-        *(uint4*)(row + w * 32 + 16) = uint4{o[4], o[5], o[6], o[7]};
+        uint8_t* dst = row + 128 * w;   // token_group_bytes(2 part + w)
+        *(uint4*)dst = uint4{o[0], o[1], o[2], o[3]};
+        *(uint4*)(dst + 16) = uint4{o[4], o[5], o[6], o[7]};
       }
-    } else if (e < s.ntok) {
-      // thread = one token, 16 kW channels: transpose into [channel][slot] with 16-bit stores
-      uint8_t* col = kt + (part * 16 * kW) * kPitch + slot_of(e) * 2;
-      const uint4* src = (const uint4*)(s.k_ptr + (int64_t)e * s.k_stride + part * kPartBytes);
+    } else {
+      // fp16 rows, transposed: a lane = tokens u and u + 8 of a 16-block (neighbours in LDS), a wave = 16 channels
+      int id = tid;
+      asm volatile("" : "+v"(id));   // formed here, not kept in registers over the packed tiles
+      const int64_t stride = in_chunk ? new_stride_t : kD * 2;
+      const uint8_t* rows = in_chunk ? k_new + (int64_t)chunk_pos(t) * new_stride_t
+                            : in_sink ? (const uint8_t*)L.sink_k + sink : (const uint8_t*)L.qbuf_k + win;
+      const int blk = (id & 63) >> 3, tok = blk * 16 + (id & 7), last = tokens(t) - 1, ch = (id >> 6) * 16;
+      // (a row past the last one repeats it: its logits are masked)
+      const uint4* s0 = (const uint4*)(rows + (int64_t)min(tok, last) * stride + ch * 2);
+      const uint4* s1 = (const uint4*)(rows + (int64_t)min(tok + 8, last) * stride + ch * 2);
+      uint8_t* col = kt + ch * kPitch + token_group_bytes(blk) + (id & 7) * 4;
 #pragma unroll
-      for (int i = 0; i < 2 * kW; ++i) {
-        const uint4 x = src[i];
-        const uint32_t w4[4] = {x.x, x.y, x.z, x.w};
+      for (int i = 0; i < 2; ++i) {
+        const uint4 x = s0[i], y = s1[i];
+        const uint32_t x4[4] = {x.x, x.y, x.z, x.w}, y4[4] = {y.x, y.y, y.z, y.w};
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          *(uint16_t*)(col + (8 * i + 2 * j) * kPitch) = (uint16_t)(w4[j] & 0xffffu);
-          *(uint16_t*)(col + (8 * i + 2 * j + 1) * kPitch) = (uint16_t)(w4[j] >> 16);
+          *(uint32_t*)(col + (8 * i + 2 * j) * kPitch) = __builtin_amdgcn_perm(y4[j], x4[j], 0x05040100u);
+          *(uint32_t*)(col + (8 * i + 2 * j + 1) * kPitch) = __builtin_amdgcn_perm(y4[j], x4[j], 0x07060302u);
         }
       }
     }
-    uint8_t* vrow = vt + slot_of(e) * kPitch + part * kPartBytes;
-    if (s.v_kind == SRC_PACKED) {
-      // thread = one token, 16 kW channels: words of 16 channels each
+    uint8_t* vrow = vt + value_row() * kPitch + part() * 64;
+    if (FULL || v_packed(t)) {
+      // thread = one token, 32 channels: words of 16 channels each
       // All of a token's codes share one (scale, zero) and take four values: the four dequantized
       // numbers are computed once (same instructions as dequant_pair, so the same two roundings)
       // and every pair of codes picks its two with a byte permute, selector bytes (2c, 2c+1).
@@ -297,11 +294,12 @@ struct Prefill {
       const half2v scale = {m2[0], m2[0]}, zero = {m2[1], m2[1]};
       const uint32_t t01 = dequant_pair(0x00010000u, scale, zero), t23 = dequant_pair(0x00030002u, scale, zero);
 #pragma unroll
-      for (int w = 0; w < kW; ++w) {
+      for (int w = 0; w < 2; ++w) {
+        const uint32_t word = w ? g.v.y : g.v.x;
         uint32_t o[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-          const uint32_t codes = (g.v[w] >> (2 * u)) & 0x00030003u;
+          const uint32_t codes = (word >> (2 * u)) & 0x00030003u;
           o[u] = __builtin_amdgcn_perm(t23, t01, codes * 0x0202u + 0x01000100u);
         }
         *(uint4*)(vrow + w * 32) = uint4{o[0], o[1], o[2], o[3]};
@@ -309,15 +307,18 @@ struct Prefill {
       }
     } else {
       // 16 channels at a time: slot 2u + e' takes channel u + 8e'; dead rows must be finite
-      const bool ok = e < s.ntok;
-      const uint4* src = nullptr;
+      int e = value_token();
+      asm volatile("" : "+v"(e));
+      const bool ok = e < tokens(t);
+      const uint8_t* row = nullptr;
       if (ok)
-        src = s.v_kind == SRC_VTAIL
-                  ? (const uint4*)((const uint8_t*)v_tail_row(L, c, b, h, s.v_u0 + e) + part * kPartBytes)
-                  : (const uint4*)(s.v_ptr + (int64_t)e * s.v_stride + part * kPartBytes);
+        row = in_chunk ? v_new + (int64_t)(chunk_pos(t) + e) * new_stride_t
+              : in_sink ? (const uint8_t*)L.sink_v + sink + (int64_t)e * (kD * 2)
+                        : (const uint8_t*)v_tail_row(L, c, b, h, (body(t) - c.pv) * kPage + e);
+      const uint4* src = (const uint4*)(row + part() * 64);
       const uint4 zero4 = uint4{0u, 0u, 0u, 0u};
 #pragma unroll
-      for (int w = 0; w < kW; ++w) {
+      for (int w = 0; w < 2; ++w) {
         const uint4 a = ok ? src[2 * w] : zero4, bb = ok ? src[2 * w + 1] : zero4;   // channels 0..7, 8..15
         const uint32_t a4[4] = {a.x, a.y, a.z, a.w}, b4[4] = {bb.x, bb.y, bb.z, bb.w};
         uint32_t o[8];
@@ -333,18 +334,21 @@ struct Prefill {
   }
 };
 
-// One wavefront's state: 16 kNT query rows (kNT column tiles of 16) against the tiles in LDS.
+// One wavefront's state: 32 query rows, one per lane pair (l, l + 32), against the tiles in LDS.
 struct WaveAcc {
-  float4v o[8][kNT];    // O^T: [channel-slot tile][row tile]
-  float m[kNT], l[kNT];   // running max (log2 units) per row tile column, per-lane partial sums
+  float16v o[4];   // O^T: channel slots 16 ct .. 16 ct + 15 and 64 + 16 ct .. of the lane's row
+  float m, l;      // running max (log2 units), per-lane partial sum
   bool first;
 };
 
-// One 128-token tile in (kt, vt) against this wavefront's rows, in sub-tiles of 32 positions (the
-// logits of a sub-tile fit 16 registers).  Software-pipelined: the QK^T MFMAs of sub-tile s+1 are
-// issued between the exponentials of sub-tile s, so that a wave's instruction stream mixes matrix
-// and vector work instead of alternating long runs of each.
-// limit[nt]: tokens of the tile with index < limit are visible to the row of column tile nt.
+// One 128-token tile in (kt, vt) against this wavefront's rows, in groups of SUBS sub-tiles of 32 positions: logits,
+// running maxima, probabilities, output.  A wave's matrix and vector phases follow one another; the other wave of the SIMD
+// fills the pipe that this one leaves idle (issuing the next sub-tile's logits between a sub-tile's exponentials, as an
+// earlier version did, costs 16 registers and gains nothing).  Two sub-tiles per group: when the maximum of any of
+// the wave's 32 rows moves, all 64 output registers are scaled, and among the first few thousand tokens that is nearly every
+// time (B = 2, 3001 tokens: 214 us with 32 positions per look, 204 with 64, 211 with 128, which spills; 189 if it
+// never happened).
+// limit: tokens of the tile with index < limit are visible to the lane's row.
 // SPLIT: the walk starts anywhere in the sequence, so a row may see nothing of the first sub-tile (and
 // then, causally, nothing at all of this share): its running maximum must stay a number.
 // DENSE: tokens and channels lie in their natural order, and K as [token][channel] (see dense_attn_kernel).
@@ -352,137 +356,106 @@ template <bool SPLIT, bool DENSE>
 struct TileAttend {
   const uint8_t* kb;   // K tile + this lane's corner of a transposing read; DENSE: + its row and channels
   const uint8_t* vb;   // V tile + the same corner
-  const half8 (&q)[4][kNT];
+  const half8 (&q)[8];
   WaveAcc& A;
-  const float sc2;
-  const bool masked;
-  const int (&limit)[kNT];
+  const float sc2;     // not negative (the queries carry the sign)
   const int kg;
 
-  __device__ __forceinline__ void qk_issue(int sub, float4v (&S)[2][kNT]) const {
+  __device__ __forceinline__ void qk(int sub, float16v& S) const {
+    const uint8_t* kbase = kb + sub * (DENSE ? 32 * kPitch : 32);
+    S = float16v{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-      for (int nt = 0; nt < kNT; ++nt) S[mt][nt] = float4v{0.f, 0.f, 0.f, 0.f};
-    const uint8_t* kbase = kb + sub * (DENSE ? 32 * kRowPitch : 64);
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-      for (int mt = 0; mt < 2; ++mt) {
-        const half8 a = DENSE ? load_row_a(kbase + mt * 16 * kRowPitch + c * 64) : load_a(kbase + (32 * c) * kPitch + mt * 32);
-#pragma unroll
-        for (int nt = 0; nt < kNT; ++nt) S[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, q[c][nt], S[mt][nt], 0, 0, 0);
-      }
-  }
-
-  // scale, mask, column maxima, and the (rare, wave-uniform) move of the running maxima
-  __device__ __forceinline__ void softmax_head(int sub, float4v (&S)[2][kNT]) const {
-#pragma unroll
-    for (int nt = 0; nt < kNT; ++nt)
-#pragma unroll
-      for (int mt = 0; mt < 2; ++mt) S[mt][nt] = S[mt][nt] * sc2 - A.m[nt];
-    if (masked) {   // one wave-uniform branch: partial tiles and the chunk's own tiles only
-#pragma unroll
-      for (int nt = 0; nt < kNT; ++nt)
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int tok = 32 * sub + 16 * mt + (DENSE ? 4 * kg + i : 2 * kg + (i >> 1) + 8 * (i & 1));
-            if (tok >= limit[nt]) S[mt][nt][i] = -INFINITY;
-          }
-      asm volatile("" ::: "memory");   // keep this a branch, not selects on every tile
-    }
-    // this lane's maxima; a logit above the running maximum of its row (the logits are relative to
-    // it) shows in the lane that holds it, so the maxima over the four lane groups are only formed
-    // when some row's maximum really moves
-    float mt_[kNT];
-#pragma unroll
-    for (int nt = 0; nt < kNT; ++nt) {
-      float mx = vmax3(vmax3(S[0][nt][0], S[0][nt][1], S[0][nt][2]), S[0][nt][3], S[1][nt][0]);
-      mt_[nt] = vmax3(vmax3(mx, S[1][nt][1], S[1][nt][2]), S[1][nt][3], mx);
-    }
-    bool move = A.first;
-#pragma unroll
-    for (int nt = 0; nt < kNT; ++nt) move = move || mt_[nt] > 0.f;
-    if (__any(move)) {
-#pragma unroll
-      for (int nt = 0; nt < kNT; ++nt) {
-        const float col = max_over_lane_groups(mt_[nt]);
-        const float dm = !A.first ? fmaxf(col, 0.f) : SPLIT && col == -INFINITY ? 0.f : col;
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) S[mt][nt][i] -= dm;
-        if (!A.first) {
-          const float alpha = __builtin_amdgcn_exp2f(-dm);
-          A.l[nt] *= alpha;
-#pragma unroll
-          for (int ct = 0; ct < 8; ++ct) A.o[ct][nt] *= alpha;
-        }
-        A.m[nt] += dm;
-      }
-      A.first = false;
+    for (int c = 0; c < 8; ++c) {
+      const half8 a = DENSE ? *(const half8*)(kbase + 32 * c) : load_a(kbase + 16 * c * kPitch);
+      S = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, q[c], S, 0, 0, 0);
     }
   }
 
-  // exponentials, row sums, fp16 probabilities
-  __device__ __forceinline__ void softmax_tail(float4v (&S)[2][kNT], half8 (&p)[kNT]) const {
-#pragma unroll
-    for (int nt = 0; nt < kNT; ++nt) {
-      float sum = 0.f;
-#pragma unroll
-      for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float e = __builtin_amdgcn_exp2f(S[mt][nt][i]);
-          S[mt][nt][i] = e;
-          sum += e;
-        }
-      A.l[nt] += sum;
-      const float4v x0 = S[0][nt], x1 = S[1][nt];
-      p[nt] = half8{(_Float16)x0[0], (_Float16)x0[1], (_Float16)x0[2], (_Float16)x0[3],
-                    (_Float16)x1[0], (_Float16)x1[1], (_Float16)x1[2], (_Float16)x1[3]};
-    }
-  }
-
-  __device__ __forceinline__ void pv(int sub, const half8 (&p)[kNT]) const {
+  __device__ __forceinline__ void pv(int sub, const half8 (&p)[2]) const {
     const uint8_t* vbase = vb + (32 * sub) * kPitch;
 #pragma unroll
-    for (int ct = 0; ct < 8; ++ct) {
-      const half8 a = load_a(vbase + ct * 32);
+    for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-      for (int nt = 0; nt < kNT; ++nt) A.o[ct][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, p[nt], A.o[ct][nt], 0, 0, 0);
-    }
+      for (int ct = 0; ct < 4; ++ct)
+        A.o[ct] = __builtin_amdgcn_mfma_f32_32x32x16_f16(load_a(vbase + 16 * kk * kPitch + ct * 32), p[kk], A.o[ct], 0, 0, 0);
   }
 
-  __device__ __forceinline__ void run(int nsub) const {
-    float4v Sc[2][kNT], Sn[2][kNT];
-    half8 p[kNT];
-    qk_issue(0, Sc);
-#pragma unroll 1
-    for (int sub = 0; sub + 1 < nsub; ++sub) {
-      softmax_head(sub, Sc);
-      // one basic block: 16 operand reads + 16 kNT MFMAs of the next sub-tile between the vector work
-      softmax_tail(Sc, p);
-      qk_issue(sub + 1, Sn);
+  static __device__ __forceinline__ float lane_max(const float16v& S) {
+    const float x0 = vmax3(S[0], S[1], S[2]), x1 = vmax3(S[3], S[4], S[5]), x2 = vmax3(S[6], S[7], S[8]),
+                x3 = vmax3(S[9], S[10], S[11]), x4 = vmax3(S[12], S[13], S[14]);
+    return vmax3(vmax3(x0, x1, x2), vmax(x3, x4), S[15]);
+  }
+
+  // MASKED: a partial tile or one of the chunk's own
+  template <int SUBS, bool MASKED>
+  __device__ __forceinline__ void group(int sub, int limit) const {
+    float16v S[SUBS];
+    half8 p[SUBS][2];
 #pragma unroll
-      for (int k = 0; k < 16; ++k) {
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);     // one LDS read
-        __builtin_amdgcn_sched_group_barrier(0x008, kNT, 0);   // its MFMAs
-        __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);     // a few vector instructions
+    for (int s = 0; s < SUBS; ++s) {
+      qk(sub + s, S[s]);
+      if (MASKED) {   // scaled here (-inf times a scaling of 0 would be NaN)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int tok = 32 * (sub + s) + (DENSE ? 8 * (i >> 2) + 2 * (i & 3) + kg
+                                                  : 16 * (i >> 3) + 4 * ((i >> 2) & 1) + 2 * kg + ((i >> 1) & 1) + 8 * (i & 1));
+          S[s][i] = tok < limit ? S[s][i] * sc2 : -INFINITY;
+        }
       }
-      __builtin_amdgcn_s_setprio(KITTY_PV_PRIO);
-      pv(sub, p);
-      __builtin_amdgcn_s_setprio(0);
-#pragma unroll
-      for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < kNT; ++nt) Sc[mt][nt] = Sn[mt][nt];
     }
-    softmax_head(nsub - 1, Sc);
-    softmax_tail(Sc, p);
-    pv(nsub - 1, p);
+    // vmax3 is assembly, which the compiler's insertion of wait states between a matrix instruction and the first reader of its
+    // result does not see into: 20 of them here, for the last product (16 passes: 19); the ones before it are done by then
+    if (!MASKED) {
+      if (SUBS == 1) asm volatile("s_nop 15\n\ts_nop 3" : "+v"(S[0]));
+      else asm volatile("s_nop 15\n\ts_nop 3" : "+v"(S[0]), "+v"(S[SUBS - 1]));
+    }
+    // this lane's maximum; a logit above the running maximum of its row shows in the lane that holds it, so the maximum
+    // over the two lane groups is only formed when some row's maximum really moves
+    float mx = lane_max(S[0]);
+#pragma unroll
+    for (int s = 1; s < SUBS; ++s) mx = vmax(mx, lane_max(S[s]));
+    if (!MASKED) mx *= sc2;
+    if (__any(A.first || mx > A.m)) {
+      const float col = max_over_lane_halves(mx);
+      if (A.first) {
+        A.m = SPLIT && col == -INFINITY ? 0.f : col;
+        A.first = false;
+      } else {
+        const float m = vmax(A.m, col), alpha = __builtin_amdgcn_exp2f(A.m - m);
+        A.l *= alpha;
+#pragma unroll
+        for (int ct = 0; ct < 4; ++ct) A.o[ct] *= alpha;
+        A.m = m;
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < SUBS; ++s) {
+      float sum = 0.f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        S[s][i] = __builtin_amdgcn_exp2f(MASKED ? S[s][i] - A.m : __builtin_fmaf(S[s][i], sc2, -A.m));
+        sum += S[s][i];
+      }
+      A.l += sum;
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) p[s][kk][j] = (_Float16)S[s][8 * kk + j];
+    }
+    __builtin_amdgcn_s_setprio(KITTY_PV_PRIO);
+#pragma unroll
+    for (int s = 0; s < SUBS; ++s) pv(sub + s, p[s]);
+    __builtin_amdgcn_s_setprio(0);
+  }
+
+  __device__ __forceinline__ void run_masked(int ntok, int limit) const {
+#pragma unroll 1
+    for (int sub = 0; 32 * sub < ntok; ++sub) group<1, true>(sub, limit);
+  }
+  // a whole tile that every row sees
+  __device__ __forceinline__ void run_full() const {
+#pragma unroll
+    for (int sub = 0; sub < 4; sub += kSubs) group<kSubs, false>(sub, kPage);
   }
 };
 
@@ -498,7 +471,7 @@ __host__ __device__ inline int block_positions(int G, int Tq) {
 // partial per row (running maximum, running sum, un-normalised output) for rows_merge_kernel.  One
 // workgroup fills a compute unit (147 KB of LDS), and a short chunk has few of them: 200 positions over
 // 12k cached tokens, 32 / 8 heads, are 32 workgroups of 98 tiles on 256 units; in 8 shares they are 256 of 13
-// tiles, and a layer (attention and append) takes 118 us instead of 555 (see prefill_splits).
+// tiles, and a layer (attention and append) takes 96 us instead of 520 (see prefill_splits).
 template <bool BOOST, bool SPLIT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves / 4, kWaves / 4))) void prefill_attn_kernel(
     kitty_kv_layer L, const uint8_t* __restrict__ q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
@@ -506,8 +479,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
     int64_t new_stride_h, int64_t new_stride_t, int H_Q, int Tq, float scaling, __half* __restrict__ out,
     float* __restrict__ ws_ml, float* __restrict__ ws_acc, int num_splits) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  __shared__ int32_t s_page_ids[2][2][Prefill<BOOST, SPLIT>::kIdChunk];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, kg = lane >> 4, n = lane & 15;
+  __shared__ typename Prefill<BOOST, SPLIT>::PageTable s_pages;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, kg = lane >> 5, n = lane & 31;
   const int b = blockIdx.z, h = blockIdx.y;
   const int G = H_Q / L.H_KV;
   const int PB = block_positions(G, Tq);                 // chunk positions per workgroup
@@ -516,15 +489,16 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
                         : (int)gridDim.x - 1 - (int)blockIdx.x;   // longest causal extent first
   const int p0 = blk * PB;
 
-  const SeqCounts cnt = load_counts(L, b);
+  SeqCounts cnt = load_counts(L, b);
+  for (int* x : {&cnt.sink, &cnt.pk, &cnt.rk, &cnt.pv, &cnt.rv, &cnt.lv, &cnt.off, &cnt.nbody})   // the same in every lane
+    *x = __builtin_amdgcn_readfirstlane(*x);
   Prefill<BOOST, SPLIT> P{L, cnt, b, h, tid,
                    k_new + (int64_t)b * new_stride_b + (int64_t)h * new_stride_h,
                    v_new + (int64_t)b * new_stride_b + (int64_t)h * new_stride_h,
-                   new_stride_t, min(Tq, p0 + PB), 0, 0, 0, 0};
-  P.page_ids = s_page_ids;
-  P.n_body = c_div_up(cnt.nbody, kPage);
+                   new_stride_t, min(Tq, p0 + PB), 0, 0, 0};
+  P.pages = s_pages;
   P.first_body = cnt.sink > 0 ? 1 : 0;
-  P.first_chunk = P.first_body + P.n_body;
+  P.first_chunk = P.first_body + c_div_up(cnt.nbody, kPage);
   P.n_tiles = P.first_chunk + c_div_up(P.kv_chunk, kPage);
   int t_begin = 0, t_end = P.n_tiles;
   if (SPLIT) {
@@ -534,37 +508,36 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
     P.first_id = max(t_begin - P.first_body, 0);
   }
 
-  // this lane's query rows: column n of row tile nt is row 16 kNT w + 16 nt + n
-  half8 qreg[4][kNT];
-  int qpos[kNT];
-#pragma unroll
-  for (int nt = 0; nt < kNT; ++nt) {
-    const int r = 16 * kNT * w + 16 * nt + n;
-    const int g = r / PB, pos = p0 + r % PB;
-    const bool ok = g < G && pos < Tq;
-    qpos[nt] = ok ? pos : -1;
+  // this lane's query row: column n of the wave's tile is row 32 w + n
+  half8 qreg[8];
+  const uint32_t flip = scaling < 0.f ? 0x80008000u : 0u;   // the logits are scaled by a number that is not negative
+  const int r = kWaveRows * w + n, g = r / PB, pos = p0 + r % PB;
+  const bool ok = g < G && pos < Tq;
+  const int qpos = ok ? pos : -1;
+  {
     const uint8_t* row = q + (int64_t)b * q_stride_b + (int64_t)(h * G + (ok ? g : 0)) * q_stride_h +
                          (int64_t)(ok ? pos : 0) * q_stride_t;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      // k-slots 0..3 = channels 32c + 4kg .., k-slots 4..7 = channels 32c + 16 + 4kg ..
-      uint2 x0 = *(const uint2*)(row + (32 * c + 4 * kg) * 2);
-      uint2 x1 = *(const uint2*)(row + (32 * c + 16 + 4 * kg) * 2);
-      if (!ok) x0 = x1 = uint2{0u, 0u};
-      const uint4 x = uint4{x0.x, x0.y, x1.x, x1.y};
-      qreg[c][nt] = __builtin_bit_cast(half8, x);
+    for (int c = 0; c < 8; ++c) {
+      // k-slots = channels 16c + kg, + 2, + 4, .. (row_slot)
+      const uint4 x0 = *(const uint4*)(row + 32 * c), x1 = *(const uint4*)(row + 32 * c + 16);
+      const uint32_t sel = kg ? 0x07060302u : 0x05040100u;
+      uint4 x = uint4{__builtin_amdgcn_perm(x0.y, x0.x, sel), __builtin_amdgcn_perm(x0.w, x0.z, sel),
+                      __builtin_amdgcn_perm(x1.y, x1.x, sel), __builtin_amdgcn_perm(x1.w, x1.z, sel)};
+      if (!ok) x = uint4{0u, 0u, 0u, 0u};
+      x.x ^= flip, x.y ^= flip, x.z ^= flip, x.w ^= flip;
+      qreg[c] = __builtin_bit_cast(half8, x);
     }
   }
 
   WaveAcc A;
 #pragma unroll
-  for (int ct = 0; ct < 8; ++ct)
+  for (int ct = 0; ct < 4; ++ct)
 #pragma unroll
-    for (int nt = 0; nt < kNT; ++nt) A.o[ct][nt] = float4v{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int nt = 0; nt < kNT; ++nt) A.m[nt] = 0.f, A.l[nt] = 0.f;
+    for (int i = 0; i < 16; ++i) A.o[ct][i] = 0.f;
+  A.m = A.l = 0.f;
   A.first = true;
-  const float sc2 = scaling * kLog2e;
+  const float sc2 = fabsf(scaling) * kLog2e;
 
   // Software pipeline over tiles: tile t is multiplied from LDS buffer t & 1 while tile t+1 is
   // turned into fp16 in the other buffer from registers loaded one iteration earlier, and the
@@ -572,87 +545,88 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
   // order (waves 0..3 convert first, waves 4..7 multiply first), so that one does vector work
   // while the other keeps the matrix pipe busy.  One barrier per tile.
   const bool convert_first = w < kWaves / 2;
-  const bool has_rows = !SPLIT || 16 * kNT * w < G * PB;   // (tested in full blocks it costs 2 %)
+  const bool has_rows = !SPLIT || kWaveRows * w < G * PB;   // (tested in full blocks it costs 2 %)
   Stage ga, gb;                       // tile t+1, tile t+2
-  P.stage_page_ids(0);
+  int slot = 255;                     // of tile t+2
+  P.stage_pages(0);
   __syncthreads();
-  TileSrc cur, nxt, nn;
   if (!SPLIT || t_begin < t_end) {    // (the last splits of a short walk are empty)
-    cur = P.tile(t_begin), nxt = cur, nn = cur;
-    P.issue(cur, ga);
-    P.finish(cur, ga, lds, lds + 2 * kTile);
-    if (t_begin + 1 < t_end) {
-      nxt = P.tile(t_begin + 1);
-      P.issue(nxt, ga);
-    }
+    const int s0 = P.template ask_slot<false>(t_begin), s1 = t_begin + 1 < t_end ? P.template ask_slot<false>(t_begin + 1) : 255;
+    P.template issue<false>(t_begin, s0, ga);
+    if (t_begin + 1 < t_end) P.template issue<false>(t_begin + 1, s1, gb);
+    if (t_begin + 2 < t_end) slot = P.template ask_slot<false>(t_begin + 2);
+    P.template finish<false>(t_begin, ga, lds, lds + 2 * kTile);
+    ga = gb;
   }
   __syncthreads();
-#pragma unroll 1
-  for (int t = t_begin; t < t_end; ++t) {
+  // FULL: tiles t .. t + 3 are whole pages on both sides - nearly all of a long walk, and a tile then costs 60 scalar
+  // instructions (a wave issues one in 8 clocks) and the test for masks in each sub-tile less (loops of their own: in one loop
+  // with a branch the output's registers are copied where the paths meet)
+  auto step = [&](auto full, int t) {
+    constexpr bool FULL = decltype(full)::value;
     const int buf = (t - t_begin) & 1;
-    const bool more = t + 1 < t_end;
-    if (t + 2 < t_end) {
-      nn = P.tile(t + 2);
-      P.issue(nn, gb);
-    }
-    {   // half way through a chunk of page ids: stage the next one (tile() is at body tile t + 2 - first_body)
-      const int i = t + 2 - P.first_body - P.id_base();
-      if (i >= 0 && i % Prefill<BOOST, SPLIT>::kIdChunk == Prefill<BOOST, SPLIT>::kIdChunk / 2) P.stage_page_ids(i / Prefill<BOOST, SPLIT>::kIdChunk + 1);
+    const bool more = FULL || t + 1 < t_end;
+    if (FULL || t + 2 < t_end) P.template issue<FULL>(t + 2, slot, gb);
+    if (FULL || t + 3 < t_end) slot = P.template ask_slot<FULL>(t + 3);
+    {   // half way through a chunk of addresses: stage the next one (ask_slot() is at tile t + 3)
+      constexpr int kChunk = Prefill<BOOST, SPLIT>::kChunk;
+      const int i = P.body(t + 3) - P.id_base();
+      if (i >= 0 && i % kChunk == kChunk / 2) P.stage_pages(i / kChunk + 1);
     }
     uint8_t* kn = lds + (buf ^ 1) * kTile;
     uint8_t* vn = lds + (2 + (buf ^ 1)) * kTile;
-    if (more && convert_first) P.finish(nxt, ga, kn, vn);
-    int limit[kNT];
-#pragma unroll
-    for (int nt = 0; nt < kNT; ++nt)
-      limit[nt] = cur.chunk_t0 >= 0 ? min(cur.ntok, qpos[nt] - cur.chunk_t0 + 1) : cur.ntok;
-    // (a tile of the chunk that ends in front of the workgroup's first position is seen whole by every row)
-    const bool masked = cur.ntok < kPage || (cur.chunk_t0 >= 0 && cur.chunk_t0 + kPage - 1 > p0);
+    if (more && convert_first) P.template finish<FULL>(t + 1, ga, kn, vn);
     if (has_rows) {
-      // the lane's corner inside a 16-lane transposing read: row n / 4 of 4, columns 4 (n % 4) ..;
-      // made opaque so that every read's offset stays a small immediate on these two bases
-      uint32_t ok_ = buf * kTile + (4 * kg + (n >> 2)) * kPitch + (n & 3) * 8;
+      // the lane's corner inside a 16-lane transposing read: row 2 j + kg of eight, j = n % 16 / 4 (row_slot), columns
+      // 4 (n % 4) .., the upper 16 lanes of a half 128 bytes further; made opaque so that every read's offset stays a small immediate on these two bases
+      uint32_t ok_ = buf * kTile + (kg + ((n >> 2) & 3) * 2) * kPitch + (n & 3) * 8 + (n >> 4) * 128;
       uint32_t ov_ = ok_ + 2 * kTile;
       asm volatile("" : "+v"(ok_), "+v"(ov_));
-      const TileAttend<SPLIT, false> T{lds + ok_, lds + ov_, qreg, A, sc2, masked, limit, kg};
-      T.run((cur.ntok + 31) >> 5);
+      const TileAttend<SPLIT, false> T{lds + ok_, lds + ov_, qreg, A, sc2, kg};
+      const int ntok = FULL ? kPage : P.tokens(t), chunk_t0 = P.chunk_pos(t);
+      // (a tile of the chunk that ends in front of the workgroup's first position is seen whole by every row)
+      if (FULL || (ntok == kPage && chunk_t0 + kPage - 1 <= p0)) T.run_full();
+      else T.run_masked(ntok, chunk_t0 >= 0 ? min(ntok, qpos - chunk_t0 + 1) : ntok);
     }
-    if (more && !convert_first) P.finish(nxt, ga, kn, vn);
-    cur = nxt;
-    nxt = nn;
+    if (more && !convert_first) P.template finish<FULL>(t + 1, ga, kn, vn);
     ga = gb;
     __syncthreads();
-  }
+  };
+  int t = t_begin;
+  const int full_end = min(P.first_body + min(cnt.pk, cnt.pv), t_end) - 3;
+#pragma unroll 1
+  for (; t < min(P.first_body, t_end); ++t) step(std::false_type{}, t);
+#pragma unroll 1
+  for (; t < full_end; ++t) step(std::true_type{}, t);
+#pragma unroll 1
+  for (; t < t_end; ++t) step(std::false_type{}, t);
 
-  // normalise and store: O^T[ct][nt][i] is channel slot 16 ct + 4 kg + i of row 16 kNT w + 16 nt + n
-#pragma unroll
-  for (int nt = 0; nt < kNT; ++nt) {
-    float l = A.l[nt];
-    l += xor_lanes(l, 16);
-    l += xor_lanes(l, 32);
-    if (qpos[nt] < 0) continue;
-    const int r = 16 * kNT * w + 16 * nt + n;
-    const int g_ = r / PB;
+  // normalise and store: O^T[ct][i] is channel slot 64 (i / 8) + 16 ct + 8 (i / 4 % 2) + 4 kg + i % 4 of the lane's row;
+  // slots 4x + {0, 2} of a 16-block are channels 2x, 2x + 1, slots 4x + {1, 3} are channels 2x + 8, 2x + 9
+  const float l = A.l + xor_lanes(A.l, 32);
+  if (ok) {
+    const int64_t row = ((int64_t)b * Tq + qpos) * H_Q + (h * G + g);
     if (SPLIT) {
-      const int64_t row = (((int64_t)b * Tq + qpos[nt]) * H_Q + (h * G + g_)) * num_splits + split;
-      if (kg == 0) *(float2*)(ws_ml + row * 2) = float2{l == 0.f ? -INFINITY : A.m[nt], l};   // 0: this row saw nothing here
-      float* arow = ws_acc + row * kD;
+      const int64_t prow = row * num_splits + split;
+      if (kg == 0) *(float2*)(ws_ml + prow * 2) = float2{l == 0.f ? -INFINITY : A.m, l};   // 0: this row saw nothing here
 #pragma unroll
-      for (int ct = 0; ct < 8; ++ct) {
-        const float4v o = A.o[ct][nt];
-        *(float2*)(arow + 16 * ct + 2 * kg) = float2{o[0], o[2]};
-        *(float2*)(arow + 16 * ct + 2 * kg + 8) = float2{o[1], o[3]};
-      }
-      continue;
-    }
-    const float inv = 1.f / l;
-    __half* orow = out + (((int64_t)b * Tq + qpos[nt]) * H_Q + (h * G + g_)) * kD;
+      for (int ct = 0; ct < 4; ++ct)
 #pragma unroll
-    for (int ct = 0; ct < 8; ++ct) {
-      const float4v o = A.o[ct][nt] * inv;
-      // slots 4kg + {0, 2} are channels 2kg, 2kg + 1; slots 4kg + {1, 3} are channels 2kg + 8, 2kg + 9
-      *(__half2*)(orow + 16 * ct + 2 * kg) = __floats2half2_rn(o[0], o[2]);
-      *(__half2*)(orow + 16 * ct + 2 * kg + 8) = __floats2half2_rn(o[1], o[3]);
+        for (int i = 0; i < 4; ++i) {
+          float* o = ws_acc + prow * kD + 64 * (i >> 1) + 16 * ct + 4 * (i & 1) + 2 * kg;
+          *(float2*)o = float2{A.o[ct][4 * i], A.o[ct][4 * i + 2]};
+          *(float2*)(o + 8) = float2{A.o[ct][4 * i + 1], A.o[ct][4 * i + 3]};
+        }
+    } else {
+      const float inv = 1.f / l;
+#pragma unroll
+      for (int ct = 0; ct < 4; ++ct)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          __half* o = out + row * kD + 64 * (i >> 1) + 16 * ct + 4 * (i & 1) + 2 * kg;
+          *(__half2*)o = __floats2half2_rn(A.o[ct][4 * i] * inv, A.o[ct][4 * i + 2] * inv);
+          *(__half2*)(o + 8) = __floats2half2_rn(A.o[ct][4 * i + 1] * inv, A.o[ct][4 * i + 3] * inv);
+        }
     }
   }
   report_bad_page(L, b, P.bad_page);   // by whichever thread met one
@@ -660,14 +634,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
 
 // A chunk over a layer that holds nothing: dense causal attention.  The frame is that of the kernel above - 256
 // rows a workgroup, two tile buffers, waves of a SIMD that stage and multiply in opposite order - but every tile is
-// fp16 rows, so nothing has to be permuted to meet codes: a row is copied as it lies, loaded into registers while the
-// tile before it is worked on.  K stays [token][channel] with 272 bytes from row to row (16 rows x two lane groups of
-// 8-byte operand reads on 64 different banks); V [token][channel] is read transposed.  On the kernel above such a tile
-// costs twice a packed one: its rows are fetched when they are needed, K goes in by 16-bit transposing stores, every
-// tile is masked.  Workgroups of one kv head share an XCD, whose L2 then serves its keys and values, longest first.
-// Bound, as the kernel above, by matrix, LDS and vector phases that overlap little.
-// B = 2, 3001 tokens, 32 / 8 heads: 448 us on the kernel above, 233 here (633 TFLOP/s; trace, launches back to back once the
-// clock is up - the first ones of a process take 265).
+// fp16 rows, so nothing has to be permuted to meet codes: a row is copied as it lies (16 lanes a row), loaded into registers
+// while the tile before it is worked on.  K stays [token][channel] and is read 16 bytes a lane, its rows in the order of
+// row_slot; V [token][channel] is read transposed.  On the kernel above such a tile costs twice a packed one: its rows are
+// fetched when they are needed, K is transposed on its way in, every tile is masked.  Workgroups of one kv head share an XCD,
+// whose L2 then serves its keys and values, longest first.  Bound, as the kernel above, by power and the vector unit.
+// B = 2, 3001 tokens, 32 / 8 heads, with the packing of the prompt: 240 -> 204 us.
 template <bool SPLIT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves / 4, kWaves / 4))) void dense_attn_kernel(
     const uint8_t* __restrict__ q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
@@ -675,7 +647,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
     int64_t new_stride_t, int H_Q, int H_KV, int Tq, float scaling, __half* __restrict__ out, float* __restrict__ ws_ml,
     float* __restrict__ ws_acc, int num_splits, int heads) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, kg = lane >> 4, n = lane & 15;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, kg = lane >> 5, n = lane & 31;
   // blockIdx.x -> (kv head of a batch row, block x split): consecutive workgroups go to the XCDs in turn
   const int id = blockIdx.x;
   int head, item;
@@ -701,58 +673,53 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
   const uint8_t* kc = k_new + (int64_t)b * new_stride_b + (int64_t)h * new_stride_h;
   const uint8_t* vc = v_new + (int64_t)b * new_stride_b + (int64_t)h * new_stride_h;
 
-  half8 qreg[4][kNT];
-  int qpos[kNT];
-#pragma unroll
-  for (int nt = 0; nt < kNT; ++nt) {
-    const int r = 16 * kNT * w + 16 * nt + n;
-    const int g = r / PB, pos = p0 + r % PB;
-    const bool ok = g < G && pos < Tq;
-    qpos[nt] = ok ? pos : -1;
+  // this lane's query row: column n of the wave's tile is row 32 w + n
+  half8 qreg[8];
+  const uint32_t flip = scaling < 0.f ? 0x80008000u : 0u;   // the logits are scaled by a number that is not negative
+  const int r = kWaveRows * w + n, g = r / PB, pos = p0 + r % PB;
+  const bool ok = g < G && pos < Tq;
+  const int qpos = ok ? pos : -1;
+  {
     const uint8_t* row = q + (int64_t)b * q_stride_b + (int64_t)(h * G + (ok ? g : 0)) * q_stride_h +
                          (int64_t)(ok ? pos : 0) * q_stride_t;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      uint2 x0 = *(const uint2*)(row + (32 * c + 4 * kg) * 2);
-      uint2 x1 = *(const uint2*)(row + (32 * c + 16 + 4 * kg) * 2);
-      if (!ok) x0 = x1 = uint2{0u, 0u};
-      const uint4 x = uint4{x0.x, x0.y, x1.x, x1.y};
-      qreg[c][nt] = __builtin_bit_cast(half8, x);
+    for (int c = 0; c < 8; ++c) {
+      uint4 x = *(const uint4*)(row + (16 * c + 8 * kg) * 2);   // k-slots = channels 16c + 8kg ..
+      if (!ok) x = uint4{0u, 0u, 0u, 0u};
+      x.x ^= flip, x.y ^= flip, x.z ^= flip, x.w ^= flip;
+      qreg[c] = __builtin_bit_cast(half8, x);
     }
   }
+
   WaveAcc A;
 #pragma unroll
-  for (int ct = 0; ct < 8; ++ct)
+  for (int ct = 0; ct < 4; ++ct)
 #pragma unroll
-    for (int nt = 0; nt < kNT; ++nt) A.o[ct][nt] = float4v{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int nt = 0; nt < kNT; ++nt) A.m[nt] = 0.f, A.l[nt] = 0.f;
+    for (int i = 0; i < 16; ++i) A.o[ct][i] = 0.f;
+  A.m = A.l = 0.f;
   A.first = true;
-  const float sc2 = scaling * kLog2e;
+  const float sc2 = fabsf(scaling) * kLog2e;
 
-  // a thread stages 16-byte pieces part, part + 4, .. of one token
-  const int e = tid / kParts, part = tid % kParts;
-  uint4v kk[2 * kW], vv[2 * kW];
+  // a thread stages 16-byte piece tid % 16 of tokens tid / 16, + 32, ..: 16 lanes write one row, 64 different banks
+  const int e = tid >> 4, part = (tid & 15) * 16;
+  uint4v kk[4], vv[4];
   auto issue = [&](int t) {
-    const int tok = t * kPage + e;
-    const int64_t off = (int64_t)min(tok, kv - 1) * new_stride_t + part * 16;
 #pragma unroll
-    for (int i = 0; i < 2 * kW; ++i) {
-      kk[i] = *(const uint4v*)(kc + off + i * (16 * kParts));
-      vv[i] = *(const uint4v*)(vc + off + i * (16 * kParts));
-    }
-    if (tok >= kv) {   // dead rows of V must be finite
-#pragma unroll
-      for (int i = 0; i < 2 * kW; ++i) vv[i] = uint4v{0u, 0u, 0u, 0u};
+    for (int i = 0; i < 4; ++i) {
+      const int tok = t * kPage + e + 32 * i;
+      const int64_t off = (int64_t)min(tok, kv - 1) * new_stride_t + part;
+      kk[i] = *(const uint4v*)(kc + off);
+      vv[i] = *(const uint4v*)(vc + off);
+      if (tok >= kv) vv[i] = uint4v{0u, 0u, 0u, 0u};   // dead rows of V must be finite
     }
   };
   auto finish = [&](int buf) {
-    uint8_t* kt = lds + buf * kTile + e * kRowPitch + part * 16;
-    uint8_t* vt = lds + (2 + buf) * kTile + e * kPitch + part * 16;
+    uint8_t* kt = lds + buf * kTile + e * kPitch + part;
+    uint8_t* vt = lds + (2 + buf) * kTile + e * kPitch + part;
 #pragma unroll
-    for (int i = 0; i < 2 * kW; ++i) {
-      *(uint4v*)(kt + i * (16 * kParts)) = kk[i];
-      *(uint4v*)(vt + i * (16 * kParts)) = vv[i];
+    for (int i = 0; i < 4; ++i) {
+      *(uint4v*)(kt + 32 * i * kPitch) = kk[i];
+      *(uint4v*)(vt + 32 * i * kPitch) = vv[i];
     }
   };
   const bool stage_first = w < kWaves / 2;
@@ -762,54 +729,54 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
     if (t_begin + 1 < t_end) issue(t_begin + 1);
   }
   __syncthreads();
-#pragma unroll 1
-  for (int t = t_begin; t < t_end; ++t) {
+  // FULL: a tile in front of the workgroup's first position, which every row sees whole
+  auto step = [&](auto full, int t) {
+    constexpr bool FULL = decltype(full)::value;
     const int buf = (t - t_begin) & 1;
     auto stage_next = [&] {
       if (t + 1 < t_end) finish(buf ^ 1);
       if (t + 2 < t_end) issue(t + 2);
     };
     if (stage_first) stage_next();
-    const int t0 = t * kPage, ntok = min(kPage, kv - t0);
-    int limit[kNT];
-#pragma unroll
-    for (int nt = 0; nt < kNT; ++nt) limit[nt] = min(ntok, qpos[nt] - t0 + 1);
-    // a full tile in front of the workgroup's first position is seen whole by every row
-    const bool masked = t0 + kPage - 1 > p0;
     {
-      uint32_t ok_ = buf * kTile + n * kRowPitch + kg * 8;
-      uint32_t ov_ = (2 + buf) * kTile + (4 * kg + (n >> 2)) * kPitch + (n & 3) * 8;
+      // K: the lane's logits are those of k-slots 4 kg .. of V's rows (row_slot)
+      uint32_t ok_ = buf * kTile + ((n & ~7) + 2 * (n & 3) + ((n >> 2) & 1)) * kPitch + kg * 16;
+      uint32_t ov_ = (2 + buf) * kTile + (kg + ((n >> 2) & 3) * 2) * kPitch + (n & 3) * 8 + (n >> 4) * 128;
       asm volatile("" : "+v"(ok_), "+v"(ov_));
-      const TileAttend<SPLIT, true> T{lds + ok_, lds + ov_, qreg, A, sc2, masked, limit, kg};
-      T.run((ntok + 31) >> 5);
+      const int t0 = t * kPage, ntok = min(kPage, kv - t0);
+      const TileAttend<SPLIT, true> T{lds + ok_, lds + ov_, qreg, A, sc2, kg};
+      if (FULL) T.run_full();
+      else T.run_masked(ntok, min(ntok, qpos - t0 + 1));
     }
     if (!stage_first) stage_next();
     __syncthreads();
-  }
+  };
+  int t = t_begin;
+  const int full_end = min(p0 / kPage, t_end);
+#pragma unroll 1
+  for (; t < full_end; ++t) step(std::true_type{}, t);
+#pragma unroll 1
+  for (; t < t_end; ++t) step(std::false_type{}, t);
 
+  const float l = A.l + xor_lanes(A.l, 32);
+  if (!ok) return;
+  const int64_t row = ((int64_t)b * Tq + qpos) * H_Q + (h * G + g);
+  const int64_t prow = row * num_splits + split;
+  if (SPLIT && kg == 0) *(float2*)(ws_ml + prow * 2) = float2{l == 0.f ? -INFINITY : A.m, l};   // 0: this row saw nothing here
+  const float inv = 1.f / l;
 #pragma unroll
-  for (int nt = 0; nt < kNT; ++nt) {
-    float l = A.l[nt];
-    l += xor_lanes(l, 16);
-    l += xor_lanes(l, 32);
-    if (qpos[nt] < 0) continue;
-    const int r = 16 * kNT * w + 16 * nt + n;
-    const int64_t row = ((int64_t)b * Tq + qpos[nt]) * H_Q + (h * G + r / PB);
-    if (SPLIT) {
-      const int64_t prow = row * num_splits + split;
-      if (kg == 0) *(float2*)(ws_ml + prow * 2) = float2{l == 0.f ? -INFINITY : A.m[nt], l};   // 0: this row saw nothing here
+  for (int ct = 0; ct < 4; ++ct)
 #pragma unroll
-      for (int ct = 0; ct < 8; ++ct) *(float4v*)(ws_acc + prow * kD + 16 * ct + 4 * kg) = A.o[ct][nt];
-      continue;
+    for (int i = 0; i < 4; ++i) {   // channels 64 (i / 2) + 16 ct + 8 (i % 2) + 4 kg ..
+      const int ch = 64 * (i >> 1) + 16 * ct + 8 * (i & 1) + 4 * kg;
+      const float4v o = {A.o[ct][4 * i], A.o[ct][4 * i + 1], A.o[ct][4 * i + 2], A.o[ct][4 * i + 3]};
+      if (SPLIT) {
+        *(float4v*)(ws_acc + prow * kD + ch) = o;
+      } else {
+        __half2 x[2] = {__floats2half2_rn(o[0] * inv, o[1] * inv), __floats2half2_rn(o[2] * inv, o[3] * inv)};
+        *(uint2*)(out + row * kD + ch) = *(const uint2*)x;
+      }
     }
-    const float inv = 1.f / l;
-#pragma unroll
-    for (int ct = 0; ct < 8; ++ct) {
-      const float4v o = A.o[ct][nt] * inv;
-      __half2 x[2] = {__floats2half2_rn(o[0], o[1]), __floats2half2_rn(o[2], o[3])};
-      *(uint2*)(out + row * kD + 16 * ct + 4 * kg) = *(const uint2*)x;
-    }
-  }
 }
 
 }  // namespace
