@@ -160,7 +160,7 @@ int kitty_quant_pack_v(const void* value, int64_t stride_b, int64_t stride_h, in
  * workspace: at least kitty_decode_attn_workspace_bytes(B,H_Q,D,num_splits) bytes, 256-aligned.
  * num_splits <= 0 picks kitty_decode_attn_default_splits_d() (max_tiles = 1 + the 128-token tiles
  * after the sink of the longest sequence; per_sequence_counts = layer->seq_counts is set), or for D = 64 / 256
- * kitty_decode_attn_default_splits() where the workspace holds only that many.
+ * kitty_decode_attn_default_splits() where the workspace holds only that many or is exactly of the size for it.
  * variant: 0 = default kernel, 1 = the plain reference-order kernel (fp16 dequantization, no
  * matrix cores).  For D = 64 / 256 both values run the same kernel, in the reference's order.
  */

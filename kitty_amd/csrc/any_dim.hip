@@ -7,16 +7,17 @@
 // arithmetic and the same storage format, one template parameter for D:
 //
 //   quant_k_any_kernel / quant_v_any_kernel   quantize-and-pack, boost selection fused or given (vector ALUs)
-//   attn_any_kernel<D, false, 1>              decode attention, split pass (the reference's order of
+//   attn_any_kernel<256, false, 1>            decode attention over few tokens, split pass (the reference's order of
 //                                             operations: fp16 dequantization with both roundings; matrix cores)
 //   attn_any_kernel<D, true, NT>              chunked-prefill attention, in one pass or in shares
+// Decode attention otherwise: any_decode.hip.
 //
 // Wire format for general D (PAGE = 128 tokens): a K page-head is 32 D bytes of low plane (channel d at
 // 32 d), 32 d_boost bytes of high plane (slot s at 32 (D + s)) and D bytes of slot map; a V page-head is
 // 128 rows of D / 4 bytes; metadata as for D = 128 with D resp. 128 (scale, zero) pairs per head.
 #include <type_traits>
 
-#include "decode_common.h"
+#include "any_dim.h"
 #include "quant_arith.h"
 
 namespace kitty {
@@ -170,74 +171,6 @@ __global__ __launch_bounds__(128) void quant_v_any_kernel(
 // ---------------------------------------------------------------------------------------------
 // attention
 // ---------------------------------------------------------------------------------------------
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-typedef float float4v __attribute__((ext_vector_type(4)));
-typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
-typedef short short4v __attribute__((ext_vector_type(4)));
-
-constexpr float kLog2e = 1.44269504088896340736f;
-constexpr uint32_t kCodeMagic = 0x64006400u;   // fp16 1024 in both halves: 1024 + n is exact for n < 1024
-constexpr float kProbScale = 32768.f;          // probabilities as matrix operands: see below
-constexpr int kProbParts = 3;
-
-__device__ __forceinline__ float4v mfma16(const uint32_t (&a)[4], const uint32_t (&b)[4], float4v c) {
-  const uint4v av = {a[0], a[1], a[2], a[3]}, bv = {b[0], b[1], b[2], b[3]};
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, av), __builtin_bit_cast(half8, bv), c, 0, 0, 0);
-}
-// Transposing LDS read: lane i of a 16-lane block receives 16-bit piece i of the four 32-byte rows whose
-// 8-byte quarters lanes 4r .. 4r+3 address; r0 = (row 0, row 1), r1 = (row 2, row 3).
-__device__ __forceinline__ void lds_tr(const uint8_t* p, uint32_t& r0, uint32_t& r1) {
-  const short4v v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((short4v __attribute__((address_space(3)))*)p);
-  const uint2 u = __builtin_bit_cast(uint2, v);
-  r0 = u.x;
-  r1 = u.y;
-}
-__device__ __forceinline__ float4v mfma16(const uint32_t (&a)[4], const uint4& b, float4v c) {
-  const uint32_t bb[4] = {b.x, b.y, b.z, b.w};
-  return mfma16(a, bb, c);
-}
-__device__ __forceinline__ uint32_t low_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x05040100u); }
-__device__ __forceinline__ uint32_t high_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
-// fp16(code) * scale + zero with BOTH operations rounded to fp16 (kitty_attention.py:162-165, 317-320 as
-// eager torch and the Triton interpreter evaluate them), for two codes.  `c` holds 1024 + code * 2^SHIFT in each
-// half (a code may stay at the bit where it lies): (1024 + code * 2^SHIFT) * 2^-SHIFT - 1024 * 2^-SHIFT is exact.
-template <int SHIFT>
-__device__ __forceinline__ uint32_t dequant_word(uint32_t c, uint32_t scale, uint32_t zero) {
-#pragma clang fp contract(off)
-  constexpr _Float16 k = (_Float16)(1.0f / (1 << SHIFT)), o = (_Float16)(1024.0f / (1 << SHIFT));
-  const half2v x = __builtin_bit_cast(half2v, c);
-  const half2v f = SHIFT == 0 ? x - half2v{o, o} : __builtin_elementwise_fma(x, half2v{k, k}, half2v{-o, -o});
-  const half2v m = f * __builtin_bit_cast(half2v, scale);
-  const half2v r = m + __builtin_bit_cast(half2v, zero);
-  return __builtin_bit_cast(uint32_t, r);
-}
-// the value codes of d-tile u of a word: codes 0 .. 4 where they lie, the others after one shift for the three
-template <int U>
-__device__ __forceinline__ uint32_t dequant_v(uint32_t x, uint32_t x10, uint32_t scale, uint32_t zero) {
-  constexpr int k = 2 * (U < 5 ? U : U - 5);
-  return dequant_word<k>(((U < 5 ? x : x10) & (0x00030003u << k)) | kCodeMagic, scale, zero);
-}
-// infinities as the largest finite number: operands of the second and third part of a probability, which may be 0 or negative
-// (the first part, times the infinity itself, has already made the sum infinite).  Costs the fp16 rows two instructions a
-// word and packed tiles a look at their scales: 3 % at D = 64 and D = 256 (the steps named at the kernel: 101 -> 104, 150 -> 156 us)
-__device__ __forceinline__ uint32_t finite_word(uint32_t x) {
-  const half2v top = {(_Float16)65504.f, (_Float16)65504.f};
-  const half2v v = __builtin_elementwise_min(__builtin_elementwise_max(__builtin_bit_cast(half2v, x), -top), top);
-  return __builtin_bit_cast(uint32_t, v);
-}
-// maximum over lanes l, l^16, l^32, l^48
-__device__ __forceinline__ float max_over_lane_groups(float v) {
-  const unsigned b = __builtin_bit_cast(unsigned, v);
-  const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
-  const unsigned r0 = r[0], r1 = r[1];   // as scalars first: a bit_cast of r[1] itself reads element 0
-  const float m = fmaxf(__builtin_bit_cast(float, r0), __builtin_bit_cast(float, r1));
-  const unsigned c = __builtin_bit_cast(unsigned, m);
-  const auto q = __builtin_amdgcn_permlane32_swap(c, c, false, false);
-  const unsigned q0 = q[0], q1 = q[1];
-  return fmaxf(__builtin_bit_cast(float, q0), __builtin_bit_cast(float, q1));
-}
-
 // LDS of one workgroup: the packed bytes of a tile as they lie in memory, or (at the end) one round of the
 // sum over the wavefronts.
 struct AnyLds {
@@ -275,11 +208,9 @@ struct AnyLds {
 // Probabilities stay fp32 numbers: 32768 p is split into three fp16 numbers, each a matrix operand of its own.
 // Together they are the fp32 number itself from 2^-16 of the row's largest probability on; below that they miss it by
 // at most 2^-40 of the largest.
-// A decode layer (append, this kernel, merge) on MI355X, against the version on the vector ALUs before it:
-//   D = 64,  B = 8, 6100 tokens, 32 / 8 heads:  79 -> 26 us (this kernel 21.4)
-//   D = 256, B = 2, 9000 tokens, 16 / 8 heads: 194 -> 39 us (27.7)
+// For decode, sharing a tile among four wavefronts pays where there are fewer tiles than compute units (any_decode.hip).
 template <int D, bool PREFILL, int NT>
-__global__ __launch_bounds__(256, PREFILL ? 1 : D == 64 ? 3 : 2) void attn_any_kernel(
+__global__ __launch_bounds__(256, PREFILL ? 1 : 2) void attn_any_kernel(
     kitty_kv_layer L, const uint8_t* __restrict__ q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
     const uint8_t* __restrict__ k_new, const uint8_t* __restrict__ v_new, int64_t new_stride_b,
     int64_t new_stride_h, int64_t new_stride_t, int H_Q, int Tq, float scaling, float* __restrict__ ws_ml,
@@ -561,7 +492,7 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : D == 64 ? 3 : 2) void attn_any_k
           constexpr int u = decltype(u_)::value;
           uint32_t a[4];
 #pragma unroll
-          for (int j = 0; j < 4; ++j) a[j] = dequant_v<u>(X[j], X10[j], sc[j], zr[j]);
+          for (int j = 0; j < 4; ++j) a[j] = dequant_v<u>(X[j], X10[j], kCodeMagic, sc[j], zr[j]);
           weigh(a, hf * kU + u, wild);
         };
         tile(std::integral_constant<int, 0>{}), tile(std::integral_constant<int, 1>{});
@@ -718,17 +649,13 @@ void launch_quant_v_any(int D, const void* value, int64_t sb, int64_t sh, int64_
                        cache_pages, status);
 }
 
-void launch_decode_any(const kitty_kv_layer& L, const void* q, int B, int H_Q, float scaling, float* ws_ml,
-                       float* ws_acc, int num_splits, hipStream_t stream) {
+// decode at D = 256
+void launch_decode_by_tile(const kitty_kv_layer& L, const void* q, int B, int H_Q, float scaling, float* ws_ml, float* ws_acc,
+                           int num_splits, hipStream_t stream) {
   const dim3 grid(num_splits, L.H_KV, B), block(256);
-  const int64_t qb = (int64_t)H_Q * L.D * 2, qh = (int64_t)L.D * 2;
-  const int lds = AnyLds(L.D, L.D_BOOSTED).with_q(L.D, 1);
-  if (L.D == 64)
-    hipLaunchKernelGGL((attn_any_kernel<64, false, 1>), grid, block, lds, stream, L, (const uint8_t*)q, qb, qh, (int64_t)0,
-                       nullptr, nullptr, (int64_t)0, (int64_t)0, (int64_t)0, H_Q, 1, scaling, ws_ml, ws_acc, num_splits, nullptr);
-  else
-    hipLaunchKernelGGL((attn_any_kernel<256, false, 1>), grid, block, lds, stream, L, (const uint8_t*)q, qb, qh, (int64_t)0,
-                       nullptr, nullptr, (int64_t)0, (int64_t)0, (int64_t)0, H_Q, 1, scaling, ws_ml, ws_acc, num_splits, nullptr);
+  hipLaunchKernelGGL((attn_any_kernel<256, false, 1>), grid, block, AnyLds(256, L.D_BOOSTED).with_q(256, 1), stream, L, (const uint8_t*)q,
+                     (int64_t)H_Q * 512, (int64_t)512, (int64_t)0, nullptr, nullptr, (int64_t)0, (int64_t)0, (int64_t)0, H_Q, 1, scaling,
+                     ws_ml, ws_acc, num_splits, nullptr);
 }
 
 namespace {
@@ -745,21 +672,6 @@ int without_empty_shares(int D, int tiles, int s) {
   return (tiles + share - 1) / share;
 }
 }  // namespace
-
-// Splits of a decode walk.  Three workgroups fit a compute unit at D = 64 (registers), two at D = 256.  Long walks are
-// cut for three per unit (D = 256, B = 4, 30000 tokens: 99 us with 24 splits, 114 with 64, 126 with 8; D = 64, B = 8, 6100
-// tokens: 22.8 us with 12 splits of four or five tiles, 25.5 with 17), shares of under three tiles for two, so that there
-// is no second round of them (D = 256, B = 2, 9000 tokens: 30 us with 24 splits of three tiles, 32 with 36 of two).
-// Where all of it fits at once a split is a tile: each costs 1.5 to 3.5 us of latency (D = 256, B = 1, 2000 tokens: 13.5 us
-// with 17 splits, 16.9 with 9).
-int decode_splits_any(int B, int H_KV, int D, int tiles, int units) {
-  const int64_t walks = (int64_t)B * H_KV;
-  int64_t s = 3 * units / walks;
-  if (s > 0 && tiles / s < 3) s = 2 * units / walks;
-  if (s > tiles) s = tiles;
-  if (s > 512) s = 512;
-  return without_empty_shares(D, tiles, s < 1 ? 1 : (int)s);
-}
 
 // Shares of a chunk's walk: enough workgroups for two on every compute unit (what their registers allow at
 // D = 256), of at least two tiles each.  `most`: shares the scratch allows.

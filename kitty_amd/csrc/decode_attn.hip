@@ -16,9 +16,9 @@ void launch_prefill_attn(const kitty_kv_layer& L, const void* q, int64_t q_strid
                          int64_t new_stride_h, int64_t new_stride_t, int B, int H_Q, int Tq, float scaling,
                          void* out, float* ws_ml, float* ws_acc, int num_splits, hipStream_t stream);
 int prefill_splits(int B, int H_Q, int H_KV, int Tq, int tiles, int units, int most);
-// head dimensions other than 128 (any_dim.hip)
+// head dimensions other than 128 (any_decode.hip, any_dim.hip)
 void launch_decode_any(const kitty_kv_layer& L, const void* q, int B, int H_Q, float scaling, float* ws_ml,
-                       float* ws_acc, int num_splits, hipStream_t stream);
+                       float* ws_acc, int num_splits, int max_tiles, int units, hipStream_t stream);
 void launch_prefill_any(const kitty_kv_layer& L, const void* q, int64_t q_stride_b, int64_t q_stride_h,
                         int64_t q_stride_t, const void* k_new, const void* v_new, int64_t new_stride_b,
                         int64_t new_stride_h, int64_t new_stride_t, int B, int H_Q, int Tq, float scaling, void* out,
@@ -189,7 +189,7 @@ extern "C" int kitty_decode_attn_split(const kitty_kv_layer* layer, const void* 
   float* ws_acc = (float*)((uint8_t*)workspace + ws_ml_bytes(B, H_Q, num_splits));
   if (L.D != kD) {   // one kernel for both variants: the reference's order of operations
     if (ev0) (void)hipEventRecord(ev0, (hipStream_t)stream);
-    launch_decode_any(L, q, B, H_Q, scaling, ws_ml, ws_acc, num_splits, (hipStream_t)stream);
+    launch_decode_any(L, q, B, H_Q, scaling, ws_ml, ws_acc, num_splits, max_tiles, device_simds() / 4, (hipStream_t)stream);
     if (ev1) (void)hipEventRecord(ev1, (hipStream_t)stream);
   } else if (variant == 0 && decode_mfma_supported(L, H_Q)) {
     uint32_t* ws_plan = (uint32_t*)((uint8_t*)ws_acc + ws_acc_bytes(B, H_Q, num_splits));
@@ -232,10 +232,13 @@ extern "C" int kitty_decode_attn(const kitty_kv_layer* layer, const void* q, int
   if (num_splits <= 0) {
     const int per_sequence = layer->seq_counts != nullptr;
     num_splits = kitty_decode_attn_default_splits_d(B, layer->H_KV, layer->D, max_tiles, per_sequence);
-    // kitty_decode_attn_default_splits was the rule for every head dimension: a workspace sized by it is enough
-    if (layer->D != kD && workspace_bytes < ws_total_bytes(B, H_Q, num_splits, layer->D)) {
-      const int fewer = kitty_decode_attn_default_splits(B, layer->H_KV, max_tiles, per_sequence);
-      if (fewer < num_splits) num_splits = fewer;
+    // kitty_decode_attn_default_splits was the rule for every head dimension: a workspace of its size gets its count, and one that
+    // is too small for the head dimension's own rule does if that is less
+    if (layer->D != kD) {
+      const int other = kitty_decode_attn_default_splits(B, layer->H_KV, max_tiles, per_sequence);
+      if (workspace_bytes == ws_total_bytes(B, H_Q, other, layer->D) ||
+          (workspace_bytes < ws_total_bytes(B, H_Q, num_splits, layer->D) && other < num_splits))
+        num_splits = other;
     }
   }
   if (int rc = kitty_decode_attn_split(layer, q, B, H_Q, scaling, workspace, workspace_bytes, num_splits, variant,
