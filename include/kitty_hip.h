@@ -365,6 +365,26 @@ int kitty_fake_quant_from(const void* src, int64_t src_stride_b, int64_t src_str
                           int64_t stride_b, int64_t stride_h, int64_t stride_t, int B, int H, int T, int D, int t_offset,
                           int n_tokens, int group_size, int bit, void* stream);
 
+/*
+ * kitty_fake_quant with groups along the tokens (axis 0) and the k_promote channels with the largest scores promoted: scores fp16
+ * [B,H,tiles,128] contiguous, one row per 128-token block from t_offset; higher score first, NaN before all, then the lower
+ * channel.  src NULL: in place.  Otherwise tokens [t_offset, t_offset + n_tokens) of src [B,H,T,D] arrive in data quantized, the
+ * others as they are; the tensors must not overlap.
+ */
+int kitty_fake_quant_topk(const void* src, int64_t src_stride_b, int64_t src_stride_h, int64_t src_stride_t, void* data,
+                          int64_t stride_b, int64_t stride_h, int64_t stride_t, int B, int H, int T, int D, int t_offset,
+                          int n_tokens, int group_size, int bit, const void* scores, int k_promote, int promote_bit,
+                          void* stream);
+
+/*
+ * One decode step of the simulator's layer: the rows k_new / v_new [B,H,1,D] to token pos of K / V [B,H,T,D] (same strides),
+ * and, with quant_pos >= 0, token quant_pos of V quantized in place as by kitty_fake_quant with axis 1.
+ */
+int kitty_sim_append(const void* k_new, const void* v_new, int64_t k_new_stride_b, int64_t k_new_stride_h,
+                     int64_t v_new_stride_b, int64_t v_new_stride_h, void* K, void* V, int64_t stride_b, int64_t stride_h,
+                     int64_t stride_t, int B, int H, int T, int D, int pos, int quant_pos, int group_size, int bit,
+                     void* stream);
+
 #ifdef __cplusplus
 }
 #endif

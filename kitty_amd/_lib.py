@@ -86,6 +86,10 @@ _SIGNATURES = {
                                   c_int64, c_int64, c_int, c_int, c_void_p]),
     "kitty_fake_quant_from": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int, c_int,
                                       c_int, c_int, c_int, c_int, c_int, c_int, c_void_p]),
+    "kitty_fake_quant_topk": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int, c_int,
+                                      c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int, c_void_p]),
+    "kitty_sim_append": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_int64, c_int64,
+                                 c_int64, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p]),
     "kitty_fake_quant": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_int, c_int, c_int, c_int, c_int, c_int,
                                  c_int, c_int, c_int, c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p]),
 }

@@ -65,6 +65,17 @@ def build_promote_mask(key_states: torch.Tensor, promote_ratio: float, channel_s
     return mask
 
 
+_own_promote_mask = build_promote_mask
+
+
+def _rows_readable(x: torch.Tensor, device: torch.device) -> bool:
+    """``x`` fp16 [B, nh, T, 128] can be read by the kernels as it lies: what a tensor copy would convert, move or track stays
+    with tensor operations."""
+    st = x.stride()
+    return (x.dtype == torch.float16 and x.device == device and st[3] == 1 and not (st[0] % 8 or st[1] % 8 or st[2] % 8 or x.data_ptr() % 16)
+            and not (x.requires_grad and torch.is_grad_enabled()) and _lib.launchable(device))
+
+
 def fake_quant_tokens_(x: torch.Tensor, t_offset: int, n_tokens: int, axis: int, group_size: int, bit: int,
                        promote_mask: Optional[torch.Tensor] = None, promote_bit: int = 4) -> torch.Tensor:
     """In place on tokens ``[t_offset, t_offset + n_tokens)`` of ``x`` fp16 [B, H, T, 128].
@@ -185,6 +196,8 @@ class KittyKVCache(_HFCache):
     # -- the three quantization steps of the reference, on [lo, hi) of a layer's buffers ----------
     def _quant_k(self, layer: int, lo: int, hi: int) -> None:
         c, K = self.cfg, self.key_cache[layer]
+        if self._quant_k_ranked(K, lo, hi, None):
+            return
         # one mask per 128-token block, from the block as it is before quantization (:204-206, :236-237)
         blocks = K[:, :, lo:hi, :].unflatten(2, (-1, c.buffer_length)).transpose(-1, -2)    # [B, nh, blocks, D, 128]
         if c.channel_selection == 0:          # a fresh permutation per head and block, as the reference draws them
@@ -194,6 +207,35 @@ class KittyKVCache(_HFCache):
             mask = build_promote_mask(blocks, c.promote_ratio, c.channel_selection)
         fake_quant_tokens_(K, lo, hi - lo, 0, c.group_size, c.kbits, mask, c.promote_bit)
 
+    def _quant_k_ranked(self, K: torch.Tensor, lo: int, hi: int, src: Optional[torch.Tensor]) -> bool:
+        """The same with the top-k and its mask inside the quantizer's launch and, with ``src`` [B, nh, L, D], the keys' copy into
+        the empty buffer.  False, and nothing done, where there is no top-k or nothing to quantize, where ``build_promote_mask``
+        has been replaced (it is then called), and for what tensor operations have to handle."""
+        c, (B, nh, _, D) = self.cfg, K.shape
+        k_chan = max(0, min(int(D * c.promote_ratio + 1e-6), D))
+        if c.channel_selection == 0 or not 0 < k_chan < D or c.kbits >= 16 or build_promote_mask is not _own_promote_mask \
+                or not _rows_readable(K, K.device):
+            return False
+        # (a variance is taken from the buffer's layout: the order of torch's sums)
+        if src is not None and not (c.channel_selection == 1 and src.shape[2] <= 1 << 24 and _rows_readable(src, K.device)):
+            return False
+        blocks = (K if src is None else src)[:, :, lo:hi, :].unflatten(2, (-1, c.buffer_length))    # [B, nh, blocks, 128, D]
+        if c.channel_selection == 1:
+            # laid out as the buffer's own blocks would be, whatever the source's order: the order of the mean's sums
+            size = torch.empty(blocks.shape, dtype=blocks.dtype, device=blocks.device)
+            score = torch.abs(blocks.detach(), out=size).transpose(-1, -2).mean(dim=-1)
+        else:
+            blocks = blocks.transpose(-1, -2)
+            score = (blocks - blocks.mean(dim=-1, keepdim=True)).pow(2).mean(dim=-1)
+        score = score.contiguous()
+        ks, ss = K.stride(), (0, 0, 0) if src is None else src.stride()
+        rc = _lib.lib().kitty_fake_quant_topk(None if src is None else src.data_ptr(), ss[0] * 2, ss[1] * 2, ss[2] * 2, K.data_ptr(),
+                                              ks[0] * 2, ks[1] * 2, ks[2] * 2, B, nh, K.shape[2] if src is None else src.shape[2],
+                                              D, lo, hi - lo, c.group_size, c.kbits, score.data_ptr(), k_chan, c.promote_bit,
+                                              _lib.current_stream_ptr(K.device))
+        _lib.check(rc, "KittyKVCache.update")
+        return True
+
     def _quant_v(self, layer: int, lo: int, hi: int) -> None:
         if hi > lo:
             fake_quant_tokens_(self.value_cache[layer], lo, hi - lo, 1, self.cfg.group_size, self.cfg.vbits)
@@ -202,9 +244,7 @@ class KittyKVCache(_HFCache):
         """A prompt's values into an empty buffer, ``[lo, hi)`` quantized, in one launch.  False, and nothing done, for
         what a tensor copy would have converted, moved or tracked, and without quantization."""
         c, (B, nh, L, D), st = self.cfg, x.shape, x.stride()
-        if c.vbits >= 16 or x.dtype != torch.float16 or x.device != buf.device or st[3] != 1 or st[0] % 8 or st[1] % 8 \
-                or st[2] % 8 or x.data_ptr() % 16 or L > 1 << 24 or (x.requires_grad and torch.is_grad_enabled()) \
-                or not _lib.launchable(x.device):
+        if c.vbits >= 16 or L > 1 << 24 or not _rows_readable(x, buf.device):
             return False
         bs = buf.stride()
         rc = _lib.lib().kitty_fake_quant_from(x.data_ptr(), st[0] * 2, st[1] * 2, st[2] * 2, buf.data_ptr(), bs[0] * 2,
@@ -246,11 +286,13 @@ class KittyKVCache(_HFCache):
                 v_to = c.sink_length + (nq if c.VCache_BitDecoding else n - c.buffer_length)
             for store, x in ((self.key_cache, key_states), (self.value_cache, value_states)):
                 buf = torch.empty((B, nh, cap, D), dtype=torch.float16, device=key_states.device)
-                if store is self.value_cache and v_to > v_from and self._values_from(x, buf, v_from, v_to):
+                store.append(buf)
+                if store is self.key_cache and jobs and self._quant_k_ranked(buf, jobs[0][1], jobs[0][2], x):
+                    jobs.pop()                                  # quantized on their way in
+                elif store is self.value_cache and v_to > v_from and self._values_from(x, buf, v_from, v_to):
                     v_to = v_from                               # quantized on their way in
                 else:
                     buf[:, :, :L].copy_(x)
-                store.append(buf)
             self._len.append(L)
             self._pending.append([])
             jobs.append(("v", v_from, v_to))
@@ -259,22 +301,32 @@ class KittyKVCache(_HFCache):
                 return key_states, value_states        # the prompt's attention sees the prompt as it came
             return self.key_cache[layer_idx][:, :, :L], self.value_cache[layer_idx][:, :, :L]
         # decode
-        self.flush_pending(layer_idx)
         L = self._len[layer_idx]
         T_new = key_states.shape[-2]
-        assert T_new == 1, "decode appends one token per step"
-        if self.max_length is not None and L + 1 > self.max_length:
-            raise ValueError(f"cache is full (max_length={self.max_length})")
-        if L + 1 > self.key_cache[layer_idx].shape[2]:                         # no max_length given: double
-            for store in (self.key_cache, self.value_cache):
-                old = store[layer_idx]
-                buf = torch.empty((old.shape[0], old.shape[1], 2 * old.shape[2], old.shape[3]), dtype=old.dtype,
-                                  device=old.device)
-                buf[:, :, :L].copy_(old[:, :, :L])
-                store[layer_idx] = buf
-        K, V = self.key_cache[layer_idx], self.value_cache[layer_idx]
-        K[:, :, L:L + 1].copy_(key_states)
-        V[:, :, L:L + 1].copy_(value_states)
+        pending, self._pending[layer_idx] = self._pending[layer_idx], []
+        # one token's values that the last step left are quantized by the launch that appends this step's rows
+        single = pending.pop() if pending and pending[-1][0] == "v" and pending[-1][2] == pending[-1][1] + 1 else None
+        self._run(layer_idx, pending)
+        try:
+            assert T_new == 1, "decode appends one token per step"
+            if self.max_length is not None and L + 1 > self.max_length:
+                raise ValueError(f"cache is full (max_length={self.max_length})")
+            if L + 1 > self.key_cache[layer_idx].shape[2]:                     # no max_length given: double
+                for store in (self.key_cache, self.value_cache):
+                    old = store[layer_idx]
+                    buf = torch.empty((old.shape[0], old.shape[1], 2 * old.shape[2], old.shape[3]), dtype=old.dtype,
+                                      device=old.device)
+                    buf[:, :, :L].copy_(old[:, :, :L])
+                    store[layer_idx] = buf
+            K, V = self.key_cache[layer_idx], self.value_cache[layer_idx]
+            if self._append_step(K, V, key_states, value_states, L, single):
+                single = None
+            else:
+                K[:, :, L:L + 1].copy_(key_states)
+                V[:, :, L:L + 1].copy_(value_states)
+        finally:
+            if single is not None:
+                self._run(layer_idx, [single])
         L += 1
         self._len[layer_idx] = L
         n = L - c.sink_length - c.buffer_length
@@ -289,3 +341,18 @@ class KittyKVCache(_HFCache):
         else:
             self._run(layer_idx, jobs)
         return K[:, :, :L], V[:, :, :L]
+
+    def _append_step(self, K: torch.Tensor, V: torch.Tensor, k: torch.Tensor, v: torch.Tensor, pos: int, job) -> bool:
+        """A decode step's rows, and ``job``'s one token of values (or None), in one launch.  False, and nothing done, for
+        what tensor operations have to handle."""
+        c, (B, nh, T, D) = self.cfg, K.shape
+        if k.shape != (B, nh, 1, D) or v.shape != k.shape or K.stride() != V.stride() or not _rows_readable(k, K.device) \
+                or not _rows_readable(v, K.device) or not _rows_readable(K, K.device) or not _rows_readable(V, K.device):
+            return False
+        quant = job[1] if job is not None and c.vbits < 16 else -1
+        ks, vs, st = k.stride(), v.stride(), K.stride()
+        rc = _lib.lib().kitty_sim_append(k.data_ptr(), v.data_ptr(), ks[0] * 2, ks[1] * 2, vs[0] * 2, vs[1] * 2, K.data_ptr(),
+                                         V.data_ptr(), st[0] * 2, st[1] * 2, st[2] * 2, B, nh, T, D, pos, quant, c.group_size,
+                                         c.vbits if quant >= 0 else 1, _lib.current_stream_ptr(K.device))
+        _lib.check(rc, "KittyKVCache.update")
+        return True
