@@ -6,7 +6,6 @@
 // size of every model the reference names.  The kernels here cover the other sizes with the same
 // arithmetic and the same storage format, one template parameter for D:
 //
-//   quant_k_any_kernel / quant_v_any_kernel   quantize-and-pack, boost selection fused or given (vector ALUs)
 //   attn_any_kernel<256, false, 1>            decode attention over few tokens, split pass (the reference's order of
 //                                             operations: fp16 dequantization with both roundings; matrix cores)
 //   attn_any_kernel<D, true, NT>              chunked-prefill attention, in one pass or in shares
@@ -18,7 +17,6 @@
 #include <type_traits>
 
 #include "any_dim.h"
-#include "quant_arith.h"
 
 namespace kitty {
 // merge pass over independent rows (rows_merge.hip)
@@ -28,145 +26,6 @@ namespace {
 
 // column tiles of 16 query rows per workgroup in chunked prefill: as many as the output's accumulators leave room for
 constexpr int kPrefillTiles64 = 4, kPrefillTiles256 = 2;
-
-// ---------------------------------------------------------------------------------------------
-// quantize and pack
-// ---------------------------------------------------------------------------------------------
-// One K page of one head: thread d owns channel d and walks the page's 128 tokens twice (the second
-// pass finds the rows in the cache).  MODE 0: slot map given.  1: selection fused.  2: selection only.
-template <int D, int MODE>
-__global__ __launch_bounds__(256) void quant_k_any_kernel(
-    const uint8_t* __restrict__ key, int64_t stride_b, int64_t stride_h, int64_t stride_t, int t_offset, int d_boost,
-    const uint8_t* __restrict__ slot_map_in, uint8_t* __restrict__ slot_map_out, int pages,
-    const int64_t* __restrict__ page_table, int64_t pt_stride_b, int page_offset, uint8_t* __restrict__ cache,
-    int64_t cache_stride_page, uint8_t* __restrict__ meta, int64_t meta_stride_page, int64_t cache_pages,
-    int32_t* __restrict__ status) {
-  static_assert(D <= 256, "one thread per channel");
-  const int p = blockIdx.x, h = blockIdx.y, b = blockIdx.z, H = gridDim.y;
-  const uint8_t* src = key + (int64_t)b * stride_b + (int64_t)h * stride_h + (int64_t)(t_offset + p * kPage) * stride_t;
-  const int64_t slot_off = (((int64_t)b * H + h) * pages + p) * D;
-  uint8_t* dst = nullptr;
-  uint8_t* mdst = nullptr;
-  if (MODE != 2) {
-    const int64_t pg = page_table[(int64_t)b * pt_stride_b + page_offset + p];
-    if (pg < 0 || pg >= cache_pages) {   // never write outside the cache; leave a record instead
-      if (status && threadIdx.x == 0) status[b * KITTY_STATUS_FIELDS + KITTY_STATUS_BAD_PAGE_WRITE] = 1;
-      return;
-    }
-    dst = cache + pg * cache_stride_page + (int64_t)h * k_head_bytes_d(D, d_boost);
-    mdst = meta + pg * meta_stride_page + (int64_t)h * D * 4;
-  }
-  __shared__ uint32_t s_key[D];   // score << 8 | (D - 1 - channel): larger sorts first
-  const int d = threadIdx.x;
-  const bool on = d < D;
-  float mn = INFINITY, mx = -INFINITY;
-  unsigned long long sum = 0;     // exact: every |x| * 2^24 is an integer below 2^40
-  bool saturated = false;
-  if (on) {
-    for (int t = 0; t < kPage; ++t) {
-      const float x = h2f(*(const uint16_t*)(src + (int64_t)t * stride_t + 2 * d));
-      mn = fminf(mn, x);
-      mx = fmaxf(mx, x);
-      if (MODE != 0) {
-        const float v = fabsf(x) * 0x1p24f;
-        if (v < 0x1p41f) sum += (unsigned long long)v;
-        else saturated = true;      // inf or NaN among the inputs
-      }
-    }
-  }
-  uint32_t slot;
-  if (MODE != 0) {
-    // score = mean |x| rounded once to fp16; rank = number of channels that sort before this one
-    // (higher score first, then lower channel index)
-    if (on) s_key[d] = ((uint32_t)(saturated ? 0x7C00 : mean_abs_fp16_bits(sum)) << 8) | (uint32_t)(D - 1 - d);
-    __syncthreads();
-    int rank = 0;
-    if (on) {
-      const uint32_t mine = s_key[d];
-      for (int e = 0; e < D; ++e) rank += s_key[e] > mine;
-    }
-    slot = (uint32_t)(rank < d_boost ? rank : d_boost);
-    if (on && slot_map_out) slot_map_out[slot_off + d] = (uint8_t)slot;
-    if (MODE == 2) return;
-  } else {
-    slot = on ? slot_map_in[slot_off + d] : 0u;
-  }
-  if (!on) return;
-  const float qmax = slot < (uint32_t)d_boost ? 15.0f : 3.0f;
-  float scale = (mx - mn) / qmax;
-  scale = scale < 1e-6f ? 1e-6f : scale;
-  const Divisor k = make_divisor(scale);
-  *(__half2*)(mdst + d * 4) = __halves2half2(__float2half_rn(scale), __float2half_rn(mn));
-  uint32_t lo[8], hi[8];
-#pragma unroll
-  for (int w = 0; w < 8; ++w) {
-    lo[w] = hi[w] = 0u;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const float x = h2f(*(const uint16_t*)(src + (int64_t)(16 * w + i) * stride_t + 2 * d));
-      const uint32_t c = (uint32_t)code_of(x - mn, k, qmax + 0.5f);
-      lo[w] |= (c & 3u) << (2 * i);
-      hi[w] |= (c >> 2) << (2 * i);
-    }
-  }
-  uint4* lo_row = (uint4*)(dst + d * kRowBytes);
-  lo_row[0] = uint4{lo[0], lo[1], lo[2], lo[3]};
-  lo_row[1] = uint4{lo[4], lo[5], lo[6], lo[7]};
-  if (slot < (uint32_t)d_boost) {
-    uint4* hi_row = (uint4*)(dst + (D + slot) * kRowBytes);
-    hi_row[0] = uint4{hi[0], hi[1], hi[2], hi[3]};
-    hi_row[1] = uint4{hi[4], hi[5], hi[6], hi[7]};
-  }
-  dst[kRowBytes * (D + d_boost) + d] = (uint8_t)slot;
-}
-
-// One V page of one head: thread t owns token t and walks its D channels twice.
-template <int D>
-__global__ __launch_bounds__(128) void quant_v_any_kernel(
-    const uint8_t* __restrict__ value, int64_t stride_b, int64_t stride_h, int64_t stride_t, int t_offset,
-    const int64_t* __restrict__ page_table, int64_t pt_stride_b, int page_offset, uint8_t* __restrict__ cache,
-    int64_t cache_stride_page, uint8_t* __restrict__ meta, int64_t meta_stride_page, int64_t cache_pages,
-    int32_t* __restrict__ status) {
-  const int p = blockIdx.x, h = blockIdx.y, b = blockIdx.z, t = threadIdx.x;
-  const int64_t pg = page_table[(int64_t)b * pt_stride_b + page_offset + p];
-  if (pg < 0 || pg >= cache_pages) {
-    if (status && t == 0) status[b * KITTY_STATUS_FIELDS + KITTY_STATUS_BAD_PAGE_WRITE] = 1;
-    return;
-  }
-  const uint8_t* row = value + (int64_t)b * stride_b + (int64_t)h * stride_h + (int64_t)(t_offset + p * kPage + t) * stride_t;
-  uint8_t* dst = cache + pg * cache_stride_page + (int64_t)h * v_head_bytes_d(D) + t * (D / 4);
-  uint8_t* mdst = meta + pg * meta_stride_page + ((int64_t)h * kPage + t) * 4;
-  float mn = INFINITY, mx = -INFINITY;
-  for (int c = 0; c < D / 8; ++c) {
-    const uint4 w = ((const uint4*)row)[c];
-    const uint32_t w4[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float a = h2f((uint16_t)(w4[i] & 0xffffu)), bb = h2f((uint16_t)(w4[i] >> 16));
-      mn = fminf(mn, fminf(a, bb));
-      mx = fmaxf(mx, fmaxf(a, bb));
-    }
-  }
-  float scale = (mx - mn) / 3.0f;
-  scale = scale < 1e-6f ? 1e-6f : scale;
-  const Divisor k = make_divisor(scale);
-  for (int c = 0; c < D / 16; ++c) {   // 16 channels per word of codes: channel e in bits 2 (e % 16)
-    uint32_t packed = 0u;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const uint4 w = ((const uint4*)row)[2 * c + j];
-      const uint32_t w4[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t c0 = (uint32_t)code_of(h2f((uint16_t)(w4[i] & 0xffffu)) - mn, k, 3.5f);
-        const uint32_t c1 = (uint32_t)code_of(h2f((uint16_t)(w4[i] >> 16)) - mn, k, 3.5f);
-        packed |= (c0 | (c1 << 2)) << (4 * (4 * j + i));
-      }
-    }
-    ((uint32_t*)dst)[c] = packed;
-  }
-  *(__half2*)mdst = __halves2half2(__float2half_rn(scale), __float2half_rn(mn));
-}
 
 // ---------------------------------------------------------------------------------------------
 // attention
@@ -602,52 +461,7 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : 2) void attn_any_kernel(
   }
 }
 
-template <int D>
-void quant_k_any(int mode, const void* key, int64_t sb, int64_t sh, int64_t st, int B, int H, int t_offset, int pages,
-                 int d_boost, const uint8_t* slot_in, uint8_t* slot_out, const int64_t* page_table, int64_t pt_stride,
-                 int page_offset, uint8_t* cache, int64_t cache_stride, void* meta, int64_t meta_stride,
-                 int64_t cache_pages, int32_t* status, hipStream_t stream) {
-  const dim3 grid(pages, H, B), block(256);
-#define KITTY_QK_ANY(MODE)                                                                                        \
-  hipLaunchKernelGGL((quant_k_any_kernel<D, MODE>), grid, block, 0, stream, (const uint8_t*)key, sb, sh, st,        \
-                     t_offset, d_boost, slot_in, slot_out, pages, page_table, pt_stride, page_offset, cache,        \
-                     cache_stride, (uint8_t*)meta, meta_stride, cache_pages, status)
-  if (mode == 0) KITTY_QK_ANY(0);
-  else if (mode == 1) KITTY_QK_ANY(1);
-  else KITTY_QK_ANY(2);
-#undef KITTY_QK_ANY
-}
-
 }  // namespace
-
-// mode 0: slot map given; 1: selection fused into the quantizer; 2: selection only (slot_out).
-void launch_quant_k_any(int D, int mode, const void* key, int64_t sb, int64_t sh, int64_t st, int B, int H,
-                        int t_offset, int pages, int d_boost, const uint8_t* slot_in, uint8_t* slot_out,
-                        const int64_t* page_table, int64_t pt_stride, int page_offset, uint8_t* cache,
-                        int64_t cache_stride, void* meta, int64_t meta_stride, int64_t cache_pages, int32_t* status,
-                        hipStream_t stream) {
-  if (D == 64)
-    quant_k_any<64>(mode, key, sb, sh, st, B, H, t_offset, pages, d_boost, slot_in, slot_out, page_table, pt_stride,
-                    page_offset, cache, cache_stride, meta, meta_stride, cache_pages, status, stream);
-  else
-    quant_k_any<256>(mode, key, sb, sh, st, B, H, t_offset, pages, d_boost, slot_in, slot_out, page_table, pt_stride,
-                     page_offset, cache, cache_stride, meta, meta_stride, cache_pages, status, stream);
-}
-
-void launch_quant_v_any(int D, const void* value, int64_t sb, int64_t sh, int64_t st, int B, int H, int t_offset,
-                        int pages, const int64_t* page_table, int64_t pt_stride, int page_offset, uint8_t* cache,
-                        int64_t cache_stride, void* meta, int64_t meta_stride, int64_t cache_pages, int32_t* status,
-                        hipStream_t stream) {
-  const dim3 grid(pages, H, B), block(128);
-  if (D == 64)
-    hipLaunchKernelGGL((quant_v_any_kernel<64>), grid, block, 0, stream, (const uint8_t*)value, sb, sh, st, t_offset,
-                       page_table, pt_stride, page_offset, cache, cache_stride, (uint8_t*)meta, meta_stride,
-                       cache_pages, status);
-  else
-    hipLaunchKernelGGL((quant_v_any_kernel<256>), grid, block, 0, stream, (const uint8_t*)value, sb, sh, st, t_offset,
-                       page_table, pt_stride, page_offset, cache, cache_stride, (uint8_t*)meta, meta_stride,
-                       cache_pages, status);
-}
 
 // decode at D = 256
 void launch_decode_by_tile(const kitty_kv_layer& L, const void* q, int B, int H_Q, float scaling, float* ws_ml, float* ws_acc,

@@ -9,21 +9,10 @@
 // 106-112, 201-204, 227-230): min/max, range, scale = range / qmax (IEEE fp32 divide, floored at
 // 1e-6), (x - min) / scale in fp32, floor(. + 0.5), clamp to [0, qmax]; the stored scale is the
 // fp32 scale rounded to fp16, the stored zero point is the minimum itself.
+#include <type_traits>
+
 #include "half_ops.h"
 #include "quant_arith.h"
-
-namespace kitty {
-// head dimensions other than 128 (any_dim.hip)
-void launch_quant_k_any(int D, int mode, const void* key, int64_t sb, int64_t sh, int64_t st, int B, int H,
-                        int t_offset, int pages, int d_boost, const uint8_t* slot_in, uint8_t* slot_out,
-                        const int64_t* page_table, int64_t pt_stride, int page_offset, uint8_t* cache,
-                        int64_t cache_stride, void* meta, int64_t meta_stride, int64_t cache_pages, int32_t* status,
-                        hipStream_t stream);
-void launch_quant_v_any(int D, const void* value, int64_t sb, int64_t sh, int64_t st, int B, int H, int t_offset,
-                        int pages, const int64_t* page_table, int64_t pt_stride, int page_offset, uint8_t* cache,
-                        int64_t cache_stride, void* meta, int64_t meta_stride, int64_t cache_pages, int32_t* status,
-                        hipStream_t stream);
-}  // namespace kitty
 
 using namespace kitty;
 
@@ -60,8 +49,9 @@ __device__ __forceinline__ float2 fast_offsets(float mn, Divisor k) {
   const bool ok = fabsf(mn * k.r) <= 32.0f && k.d < 3.0e38f;
   return ok ? float2{__builtin_fmaf(-mn, k.r, -kEps), __builtin_fmaf(-mn, k.r, kEps)} : float2{nan, nan};
 }
+// (exact: the lane's own reason to redo them)
 __device__ __forceinline__ void codes_of(const uint32_t (&w)[8], int hi, float mn, float2 cab, Divisor k, float qlim,
-                                         uint32_t& c0123, uint32_t& c4567) {
+                                         bool exact, uint32_t& c0123, uint32_t& c4567) {
   uint32_t a[2] = {0, 0}, b[2] = {0, 0};
 #pragma unroll
   for (int r = 0; r < 8; ++r) {
@@ -69,7 +59,7 @@ __device__ __forceinline__ void codes_of(const uint32_t (&w)[8], int hi, float m
     a[r >> 2] = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fmaf(x, k.r, cab.x), r & 3, a[r >> 2]);
     b[r >> 2] = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fmaf(x, k.r, cab.y), r & 3, b[r >> 2]);
   }
-  if (__any(!(cab.x == cab.x) || a[0] != b[0] || a[1] != b[1])) {
+  if (__any(exact || !(cab.x == cab.x) || a[0] != b[0] || a[1] != b[1])) {
     a[0] = a[1] = 0;
 #pragma unroll
     for (int r = 0; r < 8; ++r)
@@ -88,10 +78,36 @@ __device__ __forceinline__ uint32_t gather_fields(uint32_t c0123, uint32_t c4567
   return ((hi << 8) + lo) >> SHIFT;
 }
 
+// For head dimensions 64 and 256: a NaN takes no part in a group's minimum and maximum and gets the group's largest code.
+// any_nan: one of the lane's halves is a NaN (magnitude above 0x7C00).  range_without_nan: the packed minimum and maximum
+// again, with +inf and -inf in its place.
+template <int N, int M>
+__device__ __forceinline__ bool any_nan(const uint32_t (&w)[N][M]) {
+  uint32_t acc = 0;
+#pragma unroll
+  for (int q = 0; q < N; ++q)
+#pragma unroll
+    for (int r = 0; r < M; ++r) acc |= (w[q][r] & 0x7FFF7FFFu) + 0x03FF03FFu;
+  return (acc & 0x80008000u) != 0;
+}
+__device__ __forceinline__ void range_without_nan(const uint32_t (&w)[8], uint32_t& mn, uint32_t& mx) {
+  mn = 0x7C007C00u, mx = 0xFC00FC00u;
+#pragma unroll
+  for (int r = 0; r < 8; ++r) {
+    const uint32_t bad = (((w[r] & 0x7FFF7FFFu) + 0x03FF03FFu) >> 15 & 0x00010001u) * 0xFFFFu;   // all ones in a half that is a NaN
+    mn = pk_min_f16(mn, (w[r] & ~bad) | (0x7C007C00u & bad));
+    mx = pk_max_f16(mx, (w[r] & ~bad) | (0xFC00FC00u & bad));
+  }
+}
+
 // One K page of one head.  MODE 0: slot map given.  MODE 1: selection fused, then quantize.
-// MODE 2: selection only.  row_of(t): the 256-byte row of token t (0..127) of this head; slot_in /
-// slot_out: 128 bytes (or NULL); dst: the page-head in the cache, meta_dst: its 128 (scale, zero)
-// pairs.  Called by all 256 threads of a workgroup.
+// MODE 2: selection only.  row_of(t): the 2 D-byte row of token t (0..127) of this head; slot_in /
+// slot_out: D bytes (or NULL); dst: the page-head in the cache, meta_dst: its D (scale, zero)
+// pairs.  Called by all 2 D threads of a workgroup: D / 8 lanes beside each other on a row, 16 groups of 8 tokens, at
+// every head dimension.  (At 64 and 256 a thread used to walk one channel, two bytes a load, twice, and the value's one
+// token: the prompts of 4 x 32k tokens x 8 heads at D = 64 and of 2 x 32k at 256 took 350 and 526 us in three launches,
+// 1.0 TB/s; 64 and 135 so, in one, 4.8.  More than 64 registers a thread there, 8 wavefronts a SIMD traded for no spills:
+// 120 and 159 us with them.)
 struct StridedRows {   // the rows of a page that lies in one tensor
   const uint8_t* base;
   int64_t stride_t;
@@ -101,42 +117,43 @@ struct StridedRows {   // the rows of a page that lies in one tensor
     return base + (int64_t)t0 * stride_t + (int64_t)r * stride_t;
   }
 };
-template <int MODE, class ROWS>
+template <int D, int MODE, class ROWS>
 __device__ __forceinline__ void quant_k_page(const ROWS row_of, int d_boost,
                                              const uint8_t* __restrict__ slot_in, uint8_t* __restrict__ slot_out,
                                              uint8_t* __restrict__ dst, uint8_t* __restrict__ meta_dst) {
   const int tid = threadIdx.x;
-  const int tg = tid >> 4;   // tokens tg*8 .. tg*8+7
-  const int c8 = tid & 15;   // channels c8*8 .. c8*8+7
+  constexpr int kC8 = D / 8;      // lanes side by side on a row
+  const int tg = tid / kC8;       // tokens tg*8 .. tg*8+7
+  const int c8 = tid & (kC8 - 1); // channels c8*8 .. c8*8+7
 
   // LDS layouts are chosen so that the 64 lanes of an access fall on 64 different banks.  Per-channel
-  // tables are indexed by pos(channel) = (channel % 8) * 16 + channel / 8: the 16 lanes that share a
+  // tables are indexed by pos(channel) = (channel % 8) * D / 8 + channel / 8: the D / 8 lanes that share a
   // token group work on channels 8 apart and so read / write consecutive entries.  Rows of partials
   // are 80 words (minima / maxima: one per token group, a word of two fp16 channels) or 144 floats
   // (sums: one per pair of token groups) apart, which moves each of the four token groups of a wave to
   // its own quarter of the banks.  All of it stays under 20 KB, so that eight workgroups share a CU:
   // the kernel needs that many to keep the vector units busy across its five barriers.
-  constexpr int kPitchW = kD / 2 + 16, kPitch = kD + 16;
+  constexpr int kPitchW = D / 2 + 16, kPitch = D + 16;
   __shared__ __attribute__((aligned(16))) uint32_t s_pmin[16][kPitchW];   // later: the low plane on its way out
   __shared__ __attribute__((aligned(16))) uint32_t s_pmax[16][kPitchW];   // later: the high plane on its way out
   __shared__ float s_psum[MODE == 0 ? 1 : 8][kPitch];
   // [pos]: min, scale, refined reciprocal of the scale, qmax + 0.5; before the ranking its first half
   // holds s_exact, [pos]: the exact sum of |x| * 2^24 where fp32 leaves a doubt
-  __shared__ float4 s_q[kD];
+  __shared__ float4 s_q[D];
   unsigned long long* const s_exact = (unsigned long long*)s_q;
-  __shared__ uint8_t s_doubt[MODE == 0 ? 1 : kD];              // [pos]
+  __shared__ uint8_t s_doubt[MODE == 0 ? 1 : D];              // [pos]
   __shared__ int s_any_doubt;
-  __shared__ float2 s_cab[kD];   // [pos]: the fast path's two offsets (fast_offsets)
-  // score << 8 | (127 - channel): larger sorts first; after the ranking s_meta, the (scale, zero) pairs by
+  __shared__ float2 s_cab[D];   // [pos]: the fast path's two offsets (fast_offsets)
+  // score << 8 | (D - 1 - channel): larger sorts first; after the ranking s_meta, the (scale, zero) pairs by
   // channel, as they are stored
-  __shared__ __attribute__((aligned(16))) uint32_t s_key[kD];
+  __shared__ __attribute__((aligned(16))) uint32_t s_key[D];
   uint32_t* const s_meta = s_key;
-  __shared__ __attribute__((aligned(16))) uint8_t s_idx[kD];    // slot by channel, as it is stored
-  __shared__ uint8_t s_idx_p[kD];                               // [pos]
+  __shared__ __attribute__((aligned(16))) uint8_t s_idx[D];    // slot by channel, as it is stored
+  __shared__ uint8_t s_idx_p[D];                               // [pos]
   // A given slot map need not use every slot; the high-plane rows of unused slots keep their old bytes
   // (the fused selection fills slots 0 .. d_boost - 1, all of them).
   __shared__ __attribute__((aligned(4))) uint8_t s_slot_used[MODE == 0 ? 256 : 4];
-  static_assert(sizeof(s_pmin) >= kD * 32 && sizeof(s_pmax) >= kD * 32, "the planes reuse the minima and maxima");
+  static_assert(sizeof(s_pmin) >= D * 32 && sizeof(s_pmax) >= D * 32, "the planes reuse the minima and maxima");
   uint8_t* const s_lo = (uint8_t*)&s_pmin[0][0];
   uint8_t* const s_hi = (uint8_t*)&s_pmax[0][0];   // 32 bytes per slot
 
@@ -155,6 +172,8 @@ __device__ __forceinline__ void quant_k_page(const ROWS row_of, int d_boost,
     }
   }
 
+  const bool nan = D != kD && any_nan(w);   // (at D = 128 a NaN counts as it falls; the other head dimensions leave it out of the range)
+
   // per channel the partial min / max (packed fp16, exact) and the partial sum of |x| in fp32 (good
   // enough to rank nearly every channel, see below)
   if (MODE != 0 && tid == 0) s_any_doubt = 0;
@@ -167,33 +186,40 @@ __device__ __forceinline__ void quant_k_page(const ROWS row_of, int d_boost,
       mn = pk_min_f16(mn, w[q][r]);
       mx = pk_max_f16(mx, w[q][r]);
     }
-    s_pmin[tg][q * 16 + c8] = mn;
-    s_pmax[tg][q * 16 + c8] = mx;
+    if (D != kD && nan) range_without_nan(w[q], mn, mx);
+    s_pmin[tg][q * kC8 + c8] = mn;
+    s_pmax[tg][q * kC8 + c8] = mx;
     if (MODE != 0) {
 #pragma unroll
       for (int hi = 0; hi < 2; ++hi) {
         // added as a tree: every term goes through three additions here and a fourth with the
-        // neighbouring token group's sum (lane l ^ 16), whose even member keeps the result
+        // neighbouring token group's sum (lane l ^ D / 8), whose even member keeps the result
         const float own = ((abs_sum_f16(w[q][0], w[q][1], hi) + abs_sum_f16(w[q][2], w[q][3], hi)) +
                            (abs_sum_f16(w[q][4], w[q][5], hi) + abs_sum_f16(w[q][6], w[q][7], hi)));
         const unsigned bits = __builtin_bit_cast(unsigned, own);
-        const auto both = __builtin_amdgcn_permlane16_swap(bits, bits, false, false);
-        const unsigned b0 = both[0], b1 = both[1];   // as scalars first: a bit_cast of both[1] itself reads element 0
+        unsigned b0 = bits, b1;
+        if constexpr (D == 64) {
+          b1 = (unsigned)__builtin_amdgcn_mov_dpp((int)bits, 0x128 /* row_ror:8 */, 0xf, 0xf, true);
+        } else {
+          const auto both = D == 128 ? __builtin_amdgcn_permlane16_swap(bits, bits, false, false)
+                                     : __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
+          b0 = both[0], b1 = both[1];   // as scalars first: a bit_cast of both[1] itself reads element 0
+        }
         if ((tg & 1) == 0)
-          s_psum[tg >> 1][(2 * q + hi) * 16 + c8] = __builtin_bit_cast(float, b0) + __builtin_bit_cast(float, b1);
+          s_psum[tg >> 1][(2 * q + hi) * kC8 + c8] = __builtin_bit_cast(float, b0) + __builtin_bit_cast(float, b1);
       }
     }
   }
   __syncthreads();
 
   // Second stage on lane pairs: lanes 2c and 2c+1 each fold 8 of channel c's 16 partials, then
-  // exchange; with selection they also split the 128 comparisons of the ranking.
+  // exchange; with selection they also split the D comparisons of the ranking.
   // (the pair's channel follows the table order, so that its reads are consecutive too)
   const int pos = tid >> 1, hf = tid & 1;
-  const int ch = (pos & 15) * 8 + (pos >> 4);
+  const int ch = (pos & (kC8 - 1)) * 8 + pos / kC8;
   float ch_min, ch_max;
   {
-    const int word = (pos >> 5) * 16 + (pos & 15);   // the word that holds this channel, in half (pos >> 4) & 1
+    const int word = pos / (2 * kC8) * kC8 + (pos & (kC8 - 1));   // the word that holds this channel, in half (pos / kC8) & 1
     uint32_t mn = s_pmin[hf][word], mx = s_pmax[hf][word];
 #pragma unroll
     for (int i = 2; i < 16; i += 2) {
@@ -202,7 +228,7 @@ __device__ __forceinline__ void quant_k_page(const ROWS row_of, int d_boost,
     }
     mn = pk_min_f16(mn, (uint32_t)__shfl_xor((int)mn, 1));
     mx = pk_max_f16(mx, (uint32_t)__shfl_xor((int)mx, 1));
-    const int sh = (pos & 16);   // 16 for the upper half
+    const int sh = (pos / kC8 & 1) * 16;   // 16 for the upper half
     ch_min = widen_f16(mn >> sh, 0);
     ch_max = widen_f16(mx >> sh, 0);
   }
@@ -236,14 +262,14 @@ __device__ __forceinline__ void quant_k_page(const ROWS row_of, int d_boost,
         s_exact[pos] = 0;
         s_any_doubt = 1;
       } else {
-        s_key[ch] = (score << 8) | (uint32_t)(kD - 1 - ch);
+        s_key[ch] = (score << 8) | (uint32_t)(D - 1 - ch);
       }
     }
     __syncthreads();
     if (s_any_doubt) {   // the same for every thread of the workgroup
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        if (s_doubt[j * 16 + c8]) {
+        if (s_doubt[j * kC8 + c8]) {
           // |x| * 2^24 is an integer below 2^40: its bits from 2^20 up and the rest, added apart
           uint32_t up = 0, low = 0;
 #pragma unroll
@@ -253,29 +279,33 @@ __device__ __forceinline__ void quant_k_page(const ROWS row_of, int d_boost,
             up += (uint32_t)u;
             low += (uint32_t)__builtin_fmaf(u, -0x1p20f, v);
           }
-          atomicAdd(&s_exact[j * 16 + c8], ((unsigned long long)up << 20) + low);
+          atomicAdd(&s_exact[j * kC8 + c8], ((unsigned long long)up << 20) + low);
         }
       }
       __syncthreads();
       if (hf == 0 && s_doubt[pos])
-        s_key[ch] = ((uint32_t)mean_abs_fp16_bits(s_exact[pos]) << 8) | (uint32_t)(kD - 1 - ch);
+        s_key[ch] = ((uint32_t)mean_abs_fp16_bits(s_exact[pos]) << 8) | (uint32_t)(D - 1 - ch);
       __syncthreads();
     }
     // rank = number of channels that sort before this one: higher score, or equal score and lower
-    // channel index.  Each wave ranks 32 channels: a lane holds two of the 128 keys, a channel's key is
+    // channel index.  Each wave ranks 32 channels: a lane holds D / 64 of the D keys, a channel's key is
     // read into every lane, and the lanes whose keys are larger are counted - one compare per 64 pairs
     // of keys, the counting on the scalar unit.
     {
-      const int lane = tid & 63, first = (tid >> 6) * (kD / 4);
-      const uint32_t k0 = s_key[lane], k1 = s_key[lane + 64];
+      const int lane = tid & 63, first = (tid >> 6) * 32;
+      uint32_t own[D / 64];
 #pragma unroll
-      for (int i = 0; i < kD / 16; ++i) {
+      for (int c = 0; c < D / 64; ++c) own[c] = s_key[lane + 64 * c];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
         const uint4 t = *(const uint4*)&s_key[first + 4 * i];
         const uint32_t key[4] = {t.x, t.y, t.z, t.w};
         uint32_t slots = 0;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int rank = __popcll(__ballot(k0 > key[e])) + __popcll(__ballot(k1 > key[e]));
+          int rank = 0;
+#pragma unroll
+          for (int c = 0; c < D / 64; ++c) rank += __popcll(__ballot(own[c] > key[e]));
           slots |= (uint32_t)(rank < d_boost ? rank : d_boost) << (8 * e);
         }
         ((uint32_t*)s_idx)[(first >> 2) + i] = slots;   // the same word from every lane
@@ -314,31 +344,31 @@ __device__ __forceinline__ void quant_k_page(const ROWS row_of, int d_boost,
 
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
-    const int d = c8 * 8 + j, dp = j * 16 + c8;
+    const int d = c8 * 8 + j, dp = j * kC8 + c8;
     const float4 qp = s_q[dp];
     const Divisor k = {qp.y, qp.z};
     uint32_t c0123, c4567;   // the 8 codes (0..15), a byte each
-    codes_of(w[j >> 1], j & 1, qp.x, s_cab[dp], k, qp.w, c0123, c4567);
+    codes_of(w[j >> 1], j & 1, qp.x, s_cab[dp], k, qp.w, nan, c0123, c4567);
     // plane row d, tokens 8 tg ..: byte d * 32 + 2 tg, with the row's 16-byte pieces and its three
     // row-in-octet bits flipped by c8 so that the 16 rows written at once (8 apart) spread over the banks
-    *(uint16_t*)(s_lo + ((d * 32 + tg * 2) ^ (c8 << 4))) = (uint16_t)gather_fields<0>(c0123, c4567);
+    *(uint16_t*)(s_lo + ((d * 32 + tg * 2) ^ ((c8 & 15) << 4))) = (uint16_t)gather_fields<0>(c0123, c4567);
     const uint8_t slot = s_idx_p[dp];
     if (slot < d_boost) *(uint16_t*)(s_hi + slot * kRowBytes + tg * 2) = (uint16_t)gather_fields<2>(c0123, c4567);
   }
   __syncthreads();
   // everything leaves in contiguous pieces: the low plane by all threads (16 bytes each), the high plane by the
-  // first lanes (16 bytes each), the slot map by the second wave and the (scale, zero) pairs by the last two
+  // first lanes (16 bytes each), the slot map by the second wave and the (scale, zero) pairs by the last D threads
   // (4 bytes each: the metadata's alignment is only that)
   // the planes are written once and read much later: non-temporal stores
   nt_store16(dst + tid * 16, *(const uint4*)(s_lo + ((tid * 16) ^ (((tid >> 4) & 15) << 4))));   // piece tid of the plane: row tid / 2, c8 = row / 8
-  if (tid < 2 * d_boost && (MODE != 0 || s_slot_used[tid >> 1])) nt_store16(dst + kLoBytes + tid * 16, ((const uint4*)s_hi)[tid]);
-  const int t1 = tid - 64, t2 = tid - 128;
-  if (t1 >= 0 && t1 < kD / 4) ((uint32_t*)(dst + kRowBytes * (kD + d_boost)))[t1] = ((const uint32_t*)s_idx)[t1];
+  if (tid < 2 * d_boost && (MODE != 0 || s_slot_used[tid >> 1])) nt_store16(dst + D * kRowBytes + tid * 16, ((const uint4*)s_hi)[tid]);
+  const int t1 = tid - 64, t2 = tid - D;
+  if (t1 >= 0 && t1 < D / 4) ((uint32_t*)(dst + kRowBytes * (D + d_boost)))[t1] = ((const uint32_t*)s_idx)[t1];
   if (t2 >= 0) ((uint32_t*)meta_dst)[t2] = s_meta[t2];
 }
 
-template <int MODE>
-__global__ __launch_bounds__(256) void quant_pack_k_kernel(
+template <int D, int MODE>
+__global__ __launch_bounds__(2 * D) void quant_pack_k_kernel(
     const uint8_t* __restrict__ key, int64_t stride_b, int64_t stride_h, int64_t stride_t,
     int t_offset, int d_boost,
     const uint8_t* __restrict__ slot_map_in, uint8_t* __restrict__ slot_map_out, int pages,
@@ -347,7 +377,7 @@ __global__ __launch_bounds__(256) void quant_pack_k_kernel(
     uint8_t* __restrict__ meta, int64_t meta_stride_page, int64_t cache_pages, int32_t* __restrict__ status) {
   const int p = blockIdx.x, h = blockIdx.y, b = blockIdx.z, H = gridDim.y;
   const uint8_t* src = key + (int64_t)b * stride_b + (int64_t)h * stride_h + (int64_t)(t_offset + p * kPage) * stride_t;
-  const int64_t slot_off = (((int64_t)b * H + h) * pages + p) * kD;
+  const int64_t slot_off = (((int64_t)b * H + h) * pages + p) * D;
   uint8_t* dst = nullptr;
   uint8_t* mdst = nullptr;
   if (MODE != 2) {
@@ -356,17 +386,17 @@ __global__ __launch_bounds__(256) void quant_pack_k_kernel(
       if (status && threadIdx.x == 0) status[b * KITTY_STATUS_FIELDS + KITTY_STATUS_BAD_PAGE_WRITE] = 1;
       return;
     }
-    dst = cache + pg * cache_stride_page + (int64_t)h * k_head_bytes(d_boost);
-    mdst = meta + pg * meta_stride_page + (int64_t)h * kD * 4;
+    dst = cache + pg * cache_stride_page + (int64_t)h * k_head_bytes_d(D, d_boost);
+    mdst = meta + pg * meta_stride_page + (int64_t)h * D * 4;
   }
-  quant_k_page<MODE>(StridedRows{src, stride_t}, d_boost, slot_map_in ? slot_map_in + slot_off : nullptr,
+  quant_k_page<D, MODE>(StridedRows{src, stride_t}, d_boost, slot_map_in ? slot_map_in + slot_off : nullptr,
                      slot_map_out ? slot_map_out + slot_off : nullptr, dst, mdst);
 }
 
 // The 16 codes (0..3) of one lane's 16 channels of a token - both halves of w[0..7], in the order low
 // half of w[0], high half of w[0], low half of w[1] .. - as bytes of four words: the two roundings of codes_of above, the exact division
 // where they disagree.
-__device__ __forceinline__ void codes_of_row(const uint32_t (&w)[8], float mn, float2 cab, Divisor k, uint32_t (&c)[4]) {
+__device__ __forceinline__ void codes_of_row(const uint32_t (&w)[8], float mn, float2 cab, Divisor k, bool exact, uint32_t (&c)[4]) {
   uint32_t b[4] = {0, 0, 0, 0};
 #pragma unroll
   for (int i = 0; i < 4; ++i) c[i] = 0;
@@ -376,7 +406,7 @@ __device__ __forceinline__ void codes_of_row(const uint32_t (&w)[8], float mn, f
     c[e >> 2] = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fmaf(x, k.r, cab.x), e & 3, c[e >> 2]);
     b[e >> 2] = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fmaf(x, k.r, cab.y), e & 3, b[e >> 2]);
   }
-  if (__any(!(cab.x == cab.x) || c[0] != b[0] || c[1] != b[1] || c[2] != b[2] || c[3] != b[3])) {
+  if (__any(exact || !(cab.x == cab.x) || c[0] != b[0] || c[1] != b[1] || c[2] != b[2] || c[3] != b[3])) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) c[i] = 0;
 #pragma unroll
@@ -385,54 +415,64 @@ __device__ __forceinline__ void codes_of_row(const uint32_t (&w)[8], float mn, f
   }
 }
 
-// One V page of one head: 256 threads, 8 consecutive lanes share a token, 4 tokens per thread.  A lane
-// holds channels 8 cg .. 8 cg + 7 and 64 + 8 cg .. 64 + 8 cg + 7 of its tokens: each load instruction
-// then reads whole 128-byte half rows, 16 bytes per lane.  row_of(t): the 256-byte row of token t of this head.
-template <class ROWS>
+// One V page of one head: 2 D threads, D / 16 consecutive lanes share a token, 4 tokens per thread.  A lane
+// holds channels 8 cg .. 8 cg + 7 and D / 2 + 8 cg .. D / 2 + 8 cg + 7 of its tokens: each load instruction
+// then reads whole half rows, 16 bytes per lane.  row_of(t): the 2 D-byte row of token t of this head.
+template <int D, class ROWS>
 __device__ __forceinline__ void quant_v_page(const ROWS row_of, uint8_t* __restrict__ dst, uint8_t* __restrict__ mdst) {
   const int tid = threadIdx.x;
-  const int cg = tid & 7;
+  constexpr int kCg = D / 16;
+  const int cg = tid & (kCg - 1);
   uint4 la[4], lc[4];   // all eight loads of the thread are in flight before the first is used
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const uint8_t* src = row_of((tid >> 3) + 32 * i) + cg * 16;
+    const uint8_t* src = row_of(tid / kCg + 32 * i) + cg * 16;
     la[i] = nt_load16(src);
-    lc[i] = nt_load16(src + kD);
+    lc[i] = nt_load16(src + D);
   }
-  // The lane's codes make bytes 2 cg, 2 cg + 1 and 16 + 2 cg, 17 + 2 cg of the token's 32-byte row.  Lanes
+  // The lane's codes make bytes 2 cg, 2 cg + 1 and D / 8 + 2 cg, D / 8 + 1 + 2 cg of the token's row.  Lanes
   // 2 m and 2 m + 1 swap one of the two pairs, so that the even lane has bytes 4 m .. 4 m + 3 and the odd
-  // lane bytes 16 + 4 m .. 19 + 4 m: one 4-byte store per lane.
+  // lane bytes D / 8 + 4 m ..: one 4-byte store per lane.
   const bool odd = cg & 1;
   const uint32_t pick = odd ? 0x03020706u : 0x05040100u;   // odd: (partner's upper pair, own upper pair); even: (own lower, partner's lower)
-  const int out_off = odd ? 14 + 2 * cg : 2 * cg;
+  const int out_off = odd ? D / 8 - 2 + 2 * cg : 2 * cg;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int t = (tid >> 3) + 32 * i;
+    const int t = tid / kCg + 32 * i;
     const uint4 a = la[i], c = lc[i];
     const uint32_t w[8] = {a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
     // The token's minimum and maximum in packed fp16 (exact): over the lane's 8 words, then with the
     // maximum negated beside the minimum in one word, so that one packed minimum per step serves both,
-    // over the word's own halves and over the 8 lanes that share the token.
+    // over the word's own halves and over the lanes that share the token.
     uint32_t mnw = w[0], mxw = w[0];
 #pragma unroll
     for (int k = 1; k < 8; ++k) {
       mnw = pk_min_f16(mnw, w[k]);
       mxw = pk_max_f16(mxw, w[k]);
     }
+    bool nan = false;
+    if constexpr (D != kD) {
+      const uint32_t one[1][8] = {{w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7]}};
+      nan = any_nan(one);
+      if (nan) range_without_nan(w, mnw, mxw);
+    }
     const uint32_t nmx = mxw ^ 0x80008000u;
     uint32_t m = pk_min_f16(__builtin_amdgcn_perm(nmx, mnw, 0x05040100u),    // (mnw.lo, nmx.lo)
                             __builtin_amdgcn_perm(nmx, mnw, 0x07060302u));   // (mnw.hi, nmx.hi)
-    // lanes l ^ 1, l ^ 2, then 7 - l of the group of 8 (whose quads agree by then): data-parallel moves,
-    // no trip through the LDS crossbar
+    // lanes l ^ 1, l ^ 2, then 7 - l of the group of 8 (whose quads agree by then), 15 - l of the group of 16:
+    // data-parallel moves, no trip through the LDS crossbar
     m = pk_min_f16(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0xB1 /* quad_perm [1,0,3,2] */, 0xf, 0xf, true));
     m = pk_min_f16(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0x4E /* quad_perm [2,3,0,1] */, 0xf, 0xf, true));
-    m = pk_min_f16(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0x141 /* row_half_mirror */, 0xf, 0xf, true));
+    if constexpr (D >= 128)
+      m = pk_min_f16(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0x141 /* row_half_mirror */, 0xf, 0xf, true));
+    if constexpr (D >= 256)
+      m = pk_min_f16(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0x140 /* row_mirror */, 0xf, 0xf, true));
     const float mn = widen_f16(m, 0), mx = -widen_f16(m, 1);
     float scale = (mx - mn) / 3.0f;
     scale = scale < 1e-6f ? 1e-6f : scale;
     const Divisor kd = make_divisor(scale);
     uint32_t code[4];
-    codes_of_row(w, mn, fast_offsets(mn, kd), kd, code);
+    codes_of_row(w, mn, fast_offsets(mn, kd), kd, nan, code);
     // 16 codes, 2 bits each: a dot product of four code bytes with (1, 4, 16, 64) is a byte of the row
     constexpr uint32_t kWeights = 0x40100401u;
     const uint32_t own = __builtin_amdgcn_udot4(code[0], kWeights, 0u, false) |
@@ -441,12 +481,13 @@ __device__ __forceinline__ void quant_v_page(const ROWS row_of, uint8_t* __restr
                          (__builtin_amdgcn_udot4(code[3], kWeights, 0u, false) << 24);
     const uint32_t partner = (uint32_t)__builtin_amdgcn_mov_dpp((int)own, 0xB1 /* quad_perm [1,0,3,2] */, 0xf, 0xf, true);
     const uint32_t packed = __builtin_amdgcn_perm(partner, own, pick);
-    __builtin_nontemporal_store(packed, (uint32_t*)(dst + t * kRowBytes + out_off));   // written once, read much later
+    __builtin_nontemporal_store(packed, (uint32_t*)(dst + t * (D / 4) + out_off));   // written once, read much later
     if (cg == 0) *(__half2*)(mdst + t * 4) = __halves2half2(__float2half_rn(scale), __float2half_rn(mn));
   }
 }
 
-__global__ __launch_bounds__(256) void quant_pack_v_kernel(
+template <int D>
+__global__ __launch_bounds__(2 * D) void quant_pack_v_kernel(
     const uint8_t* __restrict__ value, int64_t stride_b, int64_t stride_h, int64_t stride_t,
     int t_offset,
     const int64_t* __restrict__ page_table, int64_t pt_stride_b, int page_offset,
@@ -458,9 +499,9 @@ __global__ __launch_bounds__(256) void quant_pack_v_kernel(
     if (status && threadIdx.x == 0) status[b * KITTY_STATUS_FIELDS + KITTY_STATUS_BAD_PAGE_WRITE] = 1;
     return;
   }
-  quant_v_page(StridedRows{value + (int64_t)b * stride_b + (int64_t)h * stride_h + (int64_t)(t_offset + p * kPage) * stride_t,
+  quant_v_page<D>(StridedRows{value + (int64_t)b * stride_b + (int64_t)h * stride_h + (int64_t)(t_offset + p * kPage) * stride_t,
                            stride_t},
-               cache + pg * cache_stride_page + (int64_t)h * kVBytes,
+               cache + pg * cache_stride_page + (int64_t)h * v_head_bytes_d(D),
                meta + pg * meta_stride_page + (int64_t)h * kPage * 4);
 }
 
@@ -605,7 +646,7 @@ __global__ __launch_bounds__(256) void flush_full_kernel(kitty_kv_layer L) {
     if (cnt[KITTY_CNT_QBUF_K] != kPage || pk < 0 || pk >= L.MAX_PAGE) return;
     const int64_t pg = L.page_table_k[(int64_t)b * L.page_table_k_stride_b + pk];
     if (pg < 0 || pg >= L.cache_pages_k) return;
-    quant_k_page<1>(StridedRows{(const uint8_t*)L.qbuf_k + w, kD * 2}, L.D_BOOSTED, nullptr, nullptr,
+    quant_k_page<kD, 1>(StridedRows{(const uint8_t*)L.qbuf_k + w, kD * 2}, L.D_BOOSTED, nullptr, nullptr,
                     const_cast<uint8_t*>(L.key_cache) + pg * L.key_cache_stride_page + (int64_t)h * k_head_bytes(L.D_BOOSTED),
                     (uint8_t*)L.key_meta + pg * L.key_meta_stride_page + (int64_t)h * kD * 4);
   } else {
@@ -613,7 +654,7 @@ __global__ __launch_bounds__(256) void flush_full_kernel(kitty_kv_layer L) {
     if (cnt[KITTY_CNT_QBUF_V] != kPage || pv < 0 || pv >= L.MAX_PAGE) return;
     const int64_t pg = L.page_table_v[(int64_t)b * L.page_table_v_stride_b + pv];
     if (pg < 0 || pg >= L.cache_pages_v) return;
-    quant_v_page(StridedRows{(const uint8_t*)L.qbuf_v + w, kD * 2},
+    quant_v_page<kD>(StridedRows{(const uint8_t*)L.qbuf_v + w, kD * 2},
                  const_cast<uint8_t*>(L.value_cache) + pg * L.value_cache_stride_page + (int64_t)h * kVBytes,
                  (uint8_t*)L.value_meta + pg * L.value_meta_stride_page + (int64_t)h * kPage * 4);
   }
@@ -759,7 +800,7 @@ __global__ __launch_bounds__(256) void chunk_quant_kernel(kitty_kv_layer L, cons
       if (L.status && threadIdx.x == 0) L.status[b * KITTY_STATUS_FIELDS + KITTY_STATUS_BAD_PAGE_WRITE] = 1;
       return;
     }
-    quant_k_page<1>(KStreamRows{(const uint8_t*)L.qbuf_k + w, k_new + src, stride_t, c.rk, p * kPage}, L.D_BOOSTED,
+    quant_k_page<kD, 1>(KStreamRows{(const uint8_t*)L.qbuf_k + w, k_new + src, stride_t, c.rk, p * kPage}, L.D_BOOSTED,
                     nullptr, nullptr,
                     const_cast<uint8_t*>(L.key_cache) + pg * L.key_cache_stride_page + (int64_t)h * k_head_bytes(L.D_BOOSTED),
                     (uint8_t*)L.key_meta + pg * L.key_meta_stride_page + (int64_t)h * kD * 4);
@@ -769,7 +810,7 @@ __global__ __launch_bounds__(256) void chunk_quant_kernel(kitty_kv_layer L, cons
       if (L.status && threadIdx.x == 0) L.status[b * KITTY_STATUS_FIELDS + KITTY_STATUS_BAD_PAGE_WRITE] = 1;
       return;
     }
-    quant_v_page(VStreamRows{(const uint8_t*)L.qbuf_v + w, (const uint8_t*)L.local_v + w, v_new + src, stride_t, c.rv,
+    quant_v_page<kD>(VStreamRows{(const uint8_t*)L.qbuf_v + w, (const uint8_t*)L.local_v + w, v_new + src, stride_t, c.rv,
                              c.er, c.off, p * kPage},
                  const_cast<uint8_t*>(L.value_cache) + pg * L.value_cache_stride_page + (int64_t)h * kVBytes,
                  (uint8_t*)L.value_meta + pg * L.value_meta_stride_page + (int64_t)h * kPage * 4);
@@ -874,7 +915,6 @@ __global__ __launch_bounds__(64) void chunk_advance_kernel(kitty_kv_layer L, int
 // a layer with the host's part; 8.5 in one launch); a long one is memory bandwidth, where the K pages' arithmetic
 // and the V pages' streaming now overlap (B = 4, 32k tokens: quantizers of 60 and 53 us and the copies, 131 us;
 // 113 in one launch, 5.5 TB/s).
-// At D != 128 the quantizers stay launches of their own (npk = npv = 0 here).
 // ---------------------------------------------------------------------------------------------
 struct PromptRows {   // [first, first + n) of the prompt -> rows 0 .. n - 1 of a window
   int n, first;
@@ -896,7 +936,8 @@ __host__ __device__ inline PromptPlan prompt_plan(int S, int T) {
 }
 constexpr int kRowPieces = 1024;   // 16-byte pieces of fp16 rows per workgroup
 
-__global__ __launch_bounds__(256) void pack_prompt_kernel(kitty_kv_layer L, int first_row, const uint8_t* __restrict__ k_new,
+template <int D>
+__global__ __launch_bounds__(2 * D) void pack_prompt_kernel(kitty_kv_layer L, int first_row, const uint8_t* __restrict__ k_new,
                                                           int64_t k_sb, int64_t k_sh, int64_t k_st,
                                                           const uint8_t* __restrict__ v_new, int64_t v_sb, int64_t v_sh,
                                                           int64_t v_st, int T, int npk, int npv) {
@@ -911,9 +952,9 @@ __global__ __launch_bounds__(256) void pack_prompt_kernel(kitty_kv_layer L, int 
       if (L.status && threadIdx.x == 0) L.status[b * KITTY_STATUS_FIELDS + KITTY_STATUS_BAD_PAGE_WRITE] = 1;
       return;
     }
-    quant_k_page<1>(StridedRows{k + (int64_t)(sink + x * kPage) * k_st, k_st}, L.D_BOOSTED, nullptr, nullptr,
-                    const_cast<uint8_t*>(L.key_cache) + pg * L.key_cache_stride_page + (int64_t)h * k_head_bytes(L.D_BOOSTED),
-                    (uint8_t*)L.key_meta + pg * L.key_meta_stride_page + (int64_t)h * kD * 4);
+    quant_k_page<D, 1>(StridedRows{k + (int64_t)(sink + x * kPage) * k_st, k_st}, L.D_BOOSTED, nullptr, nullptr,
+                    const_cast<uint8_t*>(L.key_cache) + pg * L.key_cache_stride_page + (int64_t)h * k_head_bytes_d(D, L.D_BOOSTED),
+                    (uint8_t*)L.key_meta + pg * L.key_meta_stride_page + (int64_t)h * D * 4);
     return;
   }
   x -= npk;
@@ -923,15 +964,15 @@ __global__ __launch_bounds__(256) void pack_prompt_kernel(kitty_kv_layer L, int 
       if (L.status && threadIdx.x == 0) L.status[b * KITTY_STATUS_FIELDS + KITTY_STATUS_BAD_PAGE_WRITE] = 1;
       return;
     }
-    quant_v_page(StridedRows{v + (int64_t)(sink + x * kPage) * v_st, v_st},
-                 const_cast<uint8_t*>(L.value_cache) + pg * L.value_cache_stride_page + (int64_t)h * kVBytes,
+    quant_v_page<D>(StridedRows{v + (int64_t)(sink + x * kPage) * v_st, v_st},
+                 const_cast<uint8_t*>(L.value_cache) + pg * L.value_cache_stride_page + (int64_t)h * v_head_bytes_d(D),
                  (uint8_t*)L.value_meta + pg * L.value_meta_stride_page + (int64_t)h * kPage * 4);
     return;
   }
   x -= npv;
   const PromptPlan p = prompt_plan(L.S, T);
-  const int pieces = L.D >> 3;   // 16-byte pieces of a row: 8, 16 or 32
-  const int64_t row_bytes = (int64_t)L.D * 2;
+  constexpr int pieces = D / 8;   // 16-byte pieces of a row
+  const int64_t row_bytes = (int64_t)D * 2;
   const int64_t so = (int64_t)b * L.sink_stride_b + (int64_t)h * L.sink_stride_h;
   const int64_t wo = (int64_t)b * L.win_stride_b + (int64_t)h * L.win_stride_h;
   const struct { PromptRows r; uint8_t* dst; const uint8_t* src; int64_t st; } part[5] = {
@@ -939,8 +980,8 @@ __global__ __launch_bounds__(256) void pack_prompt_kernel(kitty_kv_layer L, int 
       {p.qk, (uint8_t*)L.qbuf_k + wo, k, k_st},   {p.qv, (uint8_t*)L.qbuf_v + wo, v, v_st},
       {p.ring, (uint8_t*)L.local_v + wo, v, v_st}};
 #pragma unroll
-  for (int j = 0; j < kRowPieces / 256; ++j) {
-    const int i = x * kRowPieces + j * 256 + threadIdx.x;
+  for (int j = 0; j < kRowPieces / (2 * D); ++j) {
+    const int i = x * kRowPieces + j * 2 * D + threadIdx.x;
     int row = i / pieces;
     const int off = (i - row * pieces) * 16;
 #pragma unroll
@@ -951,6 +992,14 @@ __global__ __launch_bounds__(256) void pack_prompt_kernel(kitty_kv_layer L, int 
       row -= part[s].r.n;
     }
   }
+}
+
+// f with the head dimension (64, 128 or 256) as a constant
+template <class F>
+void by_head_dim(int D, F f) {
+  if (D == 64) f(std::integral_constant<int, 64>{});
+  else if (D == kD) f(std::integral_constant<int, kD>{});
+  else f(std::integral_constant<int, 256>{});
 }
 
 int check_src(const void* p, int64_t sb, int64_t sh, int64_t st, int B, int H, int T, int D, int t_offset,
@@ -992,14 +1041,11 @@ extern "C" int kitty_select_boost_k(const void* key, int64_t stride_b, int64_t s
   KITTY_REQUIRE(d_boost >= 0 && d_boost <= D && d_boost <= 255, KITTY_E_SHAPE,
                 "d_boost must be in [0, %d] and fit the uint8 slot map, got %d", D, d_boost);
   if (B == 0 || pages == 0) return 0;
-  if (D != kD) {
-    launch_quant_k_any(D, 2, key, stride_b, stride_h, stride_t, B, H, t_offset, pages, d_boost, nullptr, slot_map,
-                       nullptr, 0, 0, nullptr, 0, nullptr, 0, 0, nullptr, (hipStream_t)stream);
-    return check_launch("kitty_select_boost_k");
-  }
-  hipLaunchKernelGGL(quant_pack_k_kernel<2>, dim3(pages, H, B), dim3(256), 0, (hipStream_t)stream,
-                     (const uint8_t*)key, stride_b, stride_h, stride_t, t_offset, d_boost, nullptr, slot_map,
-                     pages, nullptr, 0, 0, nullptr, 0, nullptr, 0, 0, nullptr);
+  by_head_dim(D, [&](auto dim) {
+    hipLaunchKernelGGL((quant_pack_k_kernel<dim.value, 2>), dim3(pages, H, B), dim3(2 * dim.value), 0, (hipStream_t)stream,
+                       (const uint8_t*)key, stride_b, stride_h, stride_t, t_offset, d_boost, nullptr, slot_map,
+                       pages, nullptr, 0, 0, nullptr, 0, nullptr, 0, 0, nullptr);
+  });
   return check_launch("kitty_select_boost_k");
 }
 
@@ -1022,23 +1068,13 @@ extern "C" int kitty_quant_pack_k(const void* key, int64_t stride_b, int64_t str
                          (int64_t)H * k_head_bytes_d(D, d_boost), (int64_t)H * D * 4))
     return rc;
   if (B == 0 || pages == 0) return 0;
-  if (D != kD) {
-    launch_quant_k_any(D, slot_map ? 0 : 1, key, stride_b, stride_h, stride_t, B, H, t_offset, pages, d_boost, slot_map,
-                       nullptr, page_table, page_table_stride_b, page_offset, cache, cache_stride_page, meta,
-                       meta_stride_page, cache_pages, status, (hipStream_t)stream);
-    return check_launch("kitty_quant_pack_k");
-  }
-  dim3 grid(pages, H, B), block(256);
-  if (slot_map)
-    hipLaunchKernelGGL(quant_pack_k_kernel<0>, grid, block, 0, (hipStream_t)stream, (const uint8_t*)key, stride_b,
+  by_head_dim(D, [&](auto dim) {
+    const auto kernel = slot_map ? quant_pack_k_kernel<dim.value, 0> : quant_pack_k_kernel<dim.value, 1>;
+    hipLaunchKernelGGL(kernel, dim3(pages, H, B), dim3(2 * dim.value), 0, (hipStream_t)stream, (const uint8_t*)key, stride_b,
                        stride_h, stride_t, t_offset, d_boost, slot_map, nullptr, pages, page_table,
                        page_table_stride_b, page_offset, cache, cache_stride_page, (uint8_t*)meta,
                        meta_stride_page, cache_pages, status);
-  else
-    hipLaunchKernelGGL(quant_pack_k_kernel<1>, grid, block, 0, (hipStream_t)stream, (const uint8_t*)key, stride_b,
-                       stride_h, stride_t, t_offset, d_boost, nullptr, nullptr, pages, page_table,
-                       page_table_stride_b, page_offset, cache, cache_stride_page, (uint8_t*)meta,
-                       meta_stride_page, cache_pages, status);
+  });
   return check_launch("kitty_quant_pack_k");
 }
 
@@ -1054,16 +1090,12 @@ extern "C" int kitty_quant_pack_v(const void* value, int64_t stride_b, int64_t s
                          (int64_t)H * v_head_bytes_d(D), (int64_t)H * kPage * 4))
     return rc;
   if (B == 0 || pages == 0) return 0;
-  if (D != kD) {
-    launch_quant_v_any(D, value, stride_b, stride_h, stride_t, B, H, t_offset, pages, page_table, page_table_stride_b,
-                       page_offset, cache, cache_stride_page, meta, meta_stride_page, cache_pages, status,
-                       (hipStream_t)stream);
-    return check_launch("kitty_quant_pack_v");
-  }
-  hipLaunchKernelGGL(quant_pack_v_kernel, dim3(pages, H, B), dim3(256), 0, (hipStream_t)stream,
-                     (const uint8_t*)value, stride_b, stride_h, stride_t, t_offset, page_table,
-                     page_table_stride_b, page_offset, cache, cache_stride_page, (uint8_t*)meta, meta_stride_page,
-                     cache_pages, status);
+  by_head_dim(D, [&](auto dim) {
+    hipLaunchKernelGGL((quant_pack_v_kernel<dim.value>), dim3(pages, H, B), dim3(2 * dim.value), 0, (hipStream_t)stream,
+                       (const uint8_t*)value, stride_b, stride_h, stride_t, t_offset, page_table,
+                       page_table_stride_b, page_offset, cache, cache_stride_page, (uint8_t*)meta, meta_stride_page,
+                       cache_pages, status);
+  });
   return check_launch("kitty_quant_pack_v");
 }
 
@@ -1234,22 +1266,10 @@ extern "C" int kitty_pack_prompt(const kitty_kv_layer* layer, int first_row, con
       return rc;
   const hipStream_t st = (hipStream_t)stream;
   const int pieces = (2 * p.sink.n + p.qk.n + p.qv.n + p.ring.n) * (L.D / 8), row_blocks = (pieces + kRowPieces - 1) / kRowPieces;
-  const int npk = L.D == kD ? p.npk : 0, npv = L.D == kD ? p.npv : 0;
-  hipLaunchKernelGGL(pack_prompt_kernel, dim3(npk + npv + row_blocks, L.H_KV, B), dim3(256), 0, st, L, first_row,
-                     (const uint8_t*)k_new, k_stride_b, k_stride_h, k_stride_t, (const uint8_t*)v_new, v_stride_b,
-                     v_stride_h, v_stride_t, T, npk, npv);
-  if (L.D != kD) {
-    int32_t* status = L.status ? L.status + (int64_t)first_row * KITTY_STATUS_FIELDS : nullptr;
-    if (p.npk > 0)
-      launch_quant_k_any(L.D, 1, k_new, k_stride_b, k_stride_h, k_stride_t, B, L.H_KV, p.sink.n, p.npk, L.D_BOOSTED,
-                         nullptr, nullptr, L.page_table_k + (int64_t)first_row * L.page_table_k_stride_b,
-                         L.page_table_k_stride_b, 0, const_cast<uint8_t*>(L.key_cache), L.key_cache_stride_page,
-                         const_cast<void*>(L.key_meta), L.key_meta_stride_page, L.cache_pages_k, status, st);
-    if (p.npv > 0)
-      launch_quant_v_any(L.D, v_new, v_stride_b, v_stride_h, v_stride_t, B, L.H_KV, p.sink.n, p.npv,
-                         L.page_table_v + (int64_t)first_row * L.page_table_v_stride_b, L.page_table_v_stride_b, 0,
-                         const_cast<uint8_t*>(L.value_cache), L.value_cache_stride_page,
-                         const_cast<void*>(L.value_meta), L.value_meta_stride_page, L.cache_pages_v, status, st);
-  }
+  by_head_dim(L.D, [&](auto dim) {
+    hipLaunchKernelGGL((pack_prompt_kernel<dim.value>), dim3(p.npk + p.npv + row_blocks, L.H_KV, B), dim3(2 * dim.value), 0, st,
+                       L, first_row, (const uint8_t*)k_new, k_stride_b, k_stride_h, k_stride_t, (const uint8_t*)v_new,
+                       v_stride_b, v_stride_h, v_stride_t, T, p.npk, p.npv);
+  });
   return check_launch("kitty_pack_prompt");
 }
