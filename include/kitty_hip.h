@@ -314,6 +314,9 @@ int kitty_append_chunk(const kitty_kv_layer* layer, const void* k_new, const voi
  */
 int kitty_append_chunk_host(const kitty_kv_layer* layer, const void* k_new, const void* v_new, int64_t stride_b,
                             int64_t stride_h, int64_t stride_t, int B, int T, void* stream);
+/* the same for any supported head dimension (kitty_append_chunk_host takes 128 alone) */
+int kitty_append_chunk_host_d(const kitty_kv_layer* layer, const void* k_new, const void* v_new, int64_t stride_b,
+                              int64_t stride_h, int64_t stride_t, int B, int T, void* stream);
 
 /*
  * A prompt into rows first_row .. first_row + B - 1 of a layer that hold nothing: what KittyCache.quantize_prefill

@@ -82,6 +82,8 @@ _SIGNATURES = {
                                    c_void_p]),
     "kitty_append_chunk_host": (c_int, [POINTER(KittyKVLayer), c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int,
                                         c_int, c_void_p]),
+    "kitty_append_chunk_host_d": (c_int, [POINTER(KittyKVLayer), c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int,
+                                          c_int, c_void_p]),
     "kitty_pack_prompt": (c_int, [POINTER(KittyKVLayer), c_int, c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int64,
                                   c_int64, c_int64, c_int, c_int, c_void_p]),
     "kitty_fake_quant_from": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int, c_int,

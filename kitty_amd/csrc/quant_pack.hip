@@ -761,20 +761,22 @@ struct ChunkSrc {
   int64_t stride_t;
 };
 // row s of the K stream / of the V stream of one (b, h)
+template <int D>
 struct KStreamRows {
   const uint8_t* qbuf; const uint8_t* chunk; int64_t stride_t; int rk, first;
   __device__ __forceinline__ const uint8_t* operator()(int t) const {
     const int s = first + t;
-    return s < rk ? qbuf + (int64_t)s * (kD * 2) : chunk + (int64_t)(s - rk) * stride_t;
+    return s < rk ? qbuf + (int64_t)s * (D * 2) : chunk + (int64_t)(s - rk) * stride_t;
   }
   __device__ __forceinline__ const uint8_t* operator()(int t0, int r) const { return (*this)(t0 + r); }
 };
+template <int D>
 struct VStreamRows {
   const uint8_t* qbuf; const uint8_t* ring; const uint8_t* chunk; int64_t stride_t; int rv, er, off, first;
   __device__ __forceinline__ const uint8_t* operator()(int t) const {
     const int s = first + t;
-    if (s < rv) return qbuf + (int64_t)s * (kD * 2);
-    if (s < rv + er) return ring + (int64_t)((off + s - rv) & (kPage - 1)) * (kD * 2);
+    if (s < rv) return qbuf + (int64_t)s * (D * 2);
+    if (s < rv + er) return ring + (int64_t)((off + s - rv) & (kPage - 1)) * (D * 2);
     return chunk + (int64_t)(s - rv - er) * stride_t;
   }
 };
@@ -782,8 +784,8 @@ struct VStreamRows {
 // grid (2 * max_pages, H_KV, B): blockIdx.x < max_pages: new K page blockIdx.x, else new V page.  With the
 // counters on the device a sequence takes the whole chunk or nothing; with host counters (HOST) a page whose id
 // is outside the cache is left out alone and recorded, as kitty_quant_pack_k / _v do it.
-template <bool HOST>
-__global__ __launch_bounds__(256) void chunk_quant_kernel(kitty_kv_layer L, const uint8_t* __restrict__ k_new,
+template <bool HOST, int D>
+__global__ __launch_bounds__(2 * D) void chunk_quant_kernel(kitty_kv_layer L, const uint8_t* __restrict__ k_new,
                                                           const uint8_t* __restrict__ v_new, int64_t stride_b,
                                                           int64_t stride_h, int64_t stride_t, int T, int max_pages) {
   const int h = blockIdx.y, b = blockIdx.z;
@@ -800,40 +802,43 @@ __global__ __launch_bounds__(256) void chunk_quant_kernel(kitty_kv_layer L, cons
       if (L.status && threadIdx.x == 0) L.status[b * KITTY_STATUS_FIELDS + KITTY_STATUS_BAD_PAGE_WRITE] = 1;
       return;
     }
-    quant_k_page<kD, 1>(KStreamRows{(const uint8_t*)L.qbuf_k + w, k_new + src, stride_t, c.rk, p * kPage}, L.D_BOOSTED,
+    quant_k_page<D, 1>(KStreamRows<D>{(const uint8_t*)L.qbuf_k + w, k_new + src, stride_t, c.rk, p * kPage}, L.D_BOOSTED,
                     nullptr, nullptr,
-                    const_cast<uint8_t*>(L.key_cache) + pg * L.key_cache_stride_page + (int64_t)h * k_head_bytes(L.D_BOOSTED),
-                    (uint8_t*)L.key_meta + pg * L.key_meta_stride_page + (int64_t)h * kD * 4);
+                    const_cast<uint8_t*>(L.key_cache) + pg * L.key_cache_stride_page + (int64_t)h * k_head_bytes_d(D, L.D_BOOSTED),
+                    (uint8_t*)L.key_meta + pg * L.key_meta_stride_page + (int64_t)h * D * 4);
   } else {
     const int64_t pg = L.page_table_v[(int64_t)b * L.page_table_v_stride_b + c.pv + p];
     if (HOST && (pg < 0 || pg >= L.cache_pages_v)) {
       if (L.status && threadIdx.x == 0) L.status[b * KITTY_STATUS_FIELDS + KITTY_STATUS_BAD_PAGE_WRITE] = 1;
       return;
     }
-    quant_v_page<kD>(VStreamRows{(const uint8_t*)L.qbuf_v + w, (const uint8_t*)L.local_v + w, v_new + src, stride_t, c.rv,
+    quant_v_page<D>(VStreamRows<D>{(const uint8_t*)L.qbuf_v + w, (const uint8_t*)L.local_v + w, v_new + src, stride_t, c.rv,
                              c.er, c.off, p * kPage},
-                 const_cast<uint8_t*>(L.value_cache) + pg * L.value_cache_stride_page + (int64_t)h * kVBytes,
+                 const_cast<uint8_t*>(L.value_cache) + pg * L.value_cache_stride_page + (int64_t)h * v_head_bytes_d(D),
                  (uint8_t*)L.value_meta + pg * L.value_meta_stride_page + (int64_t)h * kPage * 4);
   }
 }
 
 // grid (H_KV, B, 2): the fp16 rows of one (b, h) after the chunk - sink rows, what is left of the two
 // streams (the new Q-buffer contents) and the ring.  Runs after chunk_quant_kernel, which reads the
-// old Q-buffers and ring.  Rows are moved by 16 lanes x 16 bytes.
-// 64 rows at a time and the keys' rows beside the values' (blockIdx.z): the loops below wait for memory once per
+// old Q-buffers and ring.  Rows are moved by D / 8 lanes x 16 bytes.
+// (At D = 64 and 256 a chunk was up to nine launches of torch's copies and of the quantizers: 30 tokens over 300 in four
+// layers, attention included, 173 and 194 us a pass at 60 over 700; 106 and 164 in these two.)
+// 64 rows at a time (D = 128) and the keys' rows beside the values' (blockIdx.z): the loops below wait for memory once per
 // turn (with 16 rows at a time and both in one workgroup: 12.3 us for 200 tokens, 8 kv heads, half of what that append took).
-constexpr int kRowThreads = 1024, kRowStep = kRowThreads / 16;
-template <bool HOST>
+constexpr int kRowThreads = 1024;
+template <bool HOST, int D>
 __global__ __launch_bounds__(kRowThreads) void chunk_rows_kernel(kitty_kv_layer L, const uint8_t* __restrict__ k_new,
                                                          const uint8_t* __restrict__ v_new, int64_t stride_b,
                                                          int64_t stride_h, int64_t stride_t, int T) {
-  __shared__ uint4 s_stage[kPage][16];   // ring rows on their way to the V Q-buffer
+  constexpr int kPieces = D / 8, kRowStep = kRowThreads / kPieces;
+  __shared__ uint4 s_stage[kPage][kPieces];   // ring rows on their way to the V Q-buffer
   const int h = blockIdx.x, b = blockIdx.y;
   const bool values = blockIdx.z != 0;
   const ChunkPlan c = chunk_plan<HOST>(L, b, T);
   if (!c.active) return;
   if (!HOST && !chunk_pages_ok(L, b, c)) return;
-  const int piece = threadIdx.x & 15, r0 = threadIdx.x >> 4;
+  const int piece = threadIdx.x % kPieces, r0 = threadIdx.x / kPieces;
   const int64_t w = (int64_t)b * L.win_stride_b + (int64_t)h * L.win_stride_h;
   const uint8_t* ksrc = k_new + (int64_t)b * stride_b + (int64_t)h * stride_h;
   const uint8_t* vsrc = v_new + (int64_t)b * stride_b + (int64_t)h * stride_h;
@@ -843,7 +848,7 @@ __global__ __launch_bounds__(kRowThreads) void chunk_rows_kernel(kitty_kv_layer 
     const int64_t so = (int64_t)b * L.sink_stride_b + (int64_t)h * L.sink_stride_h;
     uint8_t* sink = (uint8_t*)(values ? L.sink_v : L.sink_k) + so;
     for (int i = r0; i < c.a; i += kRowStep)
-      ((uint4*)(sink + (int64_t)(c.sink + i) * (kD * 2)))[piece] = row16((values ? vsrc : ksrc) + (int64_t)i * stride_t);
+      ((uint4*)(sink + (int64_t)(c.sink + i) * (D * 2)))[piece] = row16((values ? vsrc : ksrc) + (int64_t)i * stride_t);
   }
   if (c.n == 0) return;
   ksrc += (int64_t)c.a * stride_t;
@@ -854,7 +859,7 @@ __global__ __launch_bounds__(kRowThreads) void chunk_rows_kernel(kitty_kv_layer 
     const int k_end = HOST && c.npk > 0 && c.rk > 0 ? kPage : c.rk2;
     for (int i = (c.npk ? 0 : c.rk) + r0; i < k_end; i += kRowStep) {
       const int s = i < c.rk2 ? c.npk * kPage + i : i;
-      if (s >= c.rk) ((uint4*)((uint8_t*)L.qbuf_k + w + (int64_t)i * (kD * 2)))[piece] = row16(ksrc + (int64_t)(s - c.rk) * stride_t);
+      if (s >= c.rk) ((uint4*)((uint8_t*)L.qbuf_k + w + (int64_t)i * (D * 2)))[piece] = row16(ksrc + (int64_t)(s - c.rk) * stride_t);
     }
     return;
   }
@@ -870,19 +875,19 @@ __global__ __launch_bounds__(kRowThreads) void chunk_rows_kernel(kitty_kv_layer 
   for (int i = lo + r0; i < v_end; i += kRowStep) {
     const int s = stream_row(i);
     if (s >= c.rv && s < waiting)
-      s_stage[i][piece] = row16((const uint8_t*)L.local_v + w + (int64_t)((c.off + s - c.rv) & (kPage - 1)) * (kD * 2));
+      s_stage[i][piece] = row16((const uint8_t*)L.local_v + w + (int64_t)((c.off + s - c.rv) & (kPage - 1)) * (D * 2));
   }
   __syncthreads();
   for (int i = lo + r0; i < v_end; i += kRowStep) {
     const int s = stream_row(i);
     if (s < c.rv) continue;   // lies there already
     const uint4 v = s < waiting ? s_stage[i][piece] : row16(vsrc + (int64_t)(s - waiting) * stride_t);
-    ((uint4*)((uint8_t*)L.qbuf_v + w + (int64_t)i * (kD * 2)))[piece] = v;
+    ((uint4*)((uint8_t*)L.qbuf_v + w + (int64_t)i * (D * 2)))[piece] = v;
   }
   // ring: the chunk rows that stay take the slots single steps would have given them
   const int base = c.lv < kPage ? c.lv : c.off;
   for (int j = c.e - c.er + r0; j < c.n; j += kRowStep)
-    ((uint4*)((uint8_t*)L.local_v + w + (int64_t)((base + j) & (kPage - 1)) * (kD * 2)))[piece] =
+    ((uint4*)((uint8_t*)L.local_v + w + (int64_t)((base + j) & (kPage - 1)) * (D * 2)))[piece] =
         row16(vsrc + (int64_t)j * stride_t);
 }
 
@@ -1100,17 +1105,18 @@ extern "C" int kitty_quant_pack_v(const void* value, int64_t stride_b, int64_t s
 }
 
 namespace {
-int check_append_layer(const kitty_kv_layer* layer, int B, bool device_counters = true) {
+int check_append_layer(const kitty_kv_layer* layer, int B, bool device_counters = true, bool any_head_dim = false) {
   KITTY_REQUIRE(layer != nullptr, KITTY_E_NULL, "layer is NULL");
   const kitty_kv_layer& L = *layer;
   KITTY_REQUIRE(!device_counters || L.seq_counts != nullptr, KITTY_E_NULL,
                 "this entry point needs per-sequence counters (seq_counts)");
-  KITTY_REQUIRE(L.D == kD && L.PAGE_SIZE == kPage, KITTY_E_SHAPE,
+  const int D = L.D;
+  KITTY_REQUIRE((D == kD || (any_head_dim && head_dim_supported(D))) && L.PAGE_SIZE == kPage, KITTY_E_SHAPE,
                 "the device-counter entry points are built for head_dim 128 and page_size 128 (other head dimensions "
                 "keep the counters on the host), got D=%d page_size=%d", L.D, L.PAGE_SIZE);
   KITTY_REQUIRE(L.H_KV >= 1 && L.H_KV <= 65535 && B >= 1 && B <= 65535, KITTY_E_RANGE, "bad H_KV=%d or B=%d", L.H_KV, B);
-  KITTY_REQUIRE(L.S >= 0 && L.S <= kPage && L.MAX_PAGE >= 0 && L.D_BOOSTED >= 0 && L.D_BOOSTED <= kD &&
-                    k_head_bytes(L.D_BOOSTED) % 16 == 0,
+  KITTY_REQUIRE(L.S >= 0 && L.S <= kPage && L.MAX_PAGE >= 0 && L.D_BOOSTED >= 0 && L.D_BOOSTED <= D && L.D_BOOSTED <= 255 &&
+                    k_head_bytes_d(D, L.D_BOOSTED) % 16 == 0,
                 KITTY_E_SHAPE, "bad S=%d, MAX_PAGE=%d or D_BOOSTED=%d", L.S, L.MAX_PAGE, L.D_BOOSTED);
   KITTY_REQUIRE(L.key_cache && L.key_meta && L.value_cache && L.value_meta && L.page_table_k && L.page_table_v &&
                     L.sink_k && L.sink_v && L.qbuf_k && L.qbuf_v && L.local_v,
@@ -1126,9 +1132,9 @@ int check_append_layer(const kitty_kv_layer* layer, int B, bool device_counters 
                     ((uintptr_t)L.status % 4) == 0,
                 KITTY_E_ALIGN, "cache tensors need 16-byte alignment");
   KITTY_REQUIRE(L.cache_pages_k >= 0 && L.cache_pages_v >= 0, KITTY_E_RANGE, "negative cache_pages_k / cache_pages_v");
-  KITTY_REQUIRE(L.key_cache_stride_page >= (int64_t)L.H_KV * k_head_bytes(L.D_BOOSTED) &&
-                    L.value_cache_stride_page >= (int64_t)L.H_KV * kVBytes &&
-                    L.key_meta_stride_page >= (int64_t)L.H_KV * kD * 4 &&
+  KITTY_REQUIRE(L.key_cache_stride_page >= (int64_t)L.H_KV * k_head_bytes_d(D, L.D_BOOSTED) &&
+                    L.value_cache_stride_page >= (int64_t)L.H_KV * v_head_bytes_d(D) &&
+                    L.key_meta_stride_page >= (int64_t)L.H_KV * D * 4 &&
                     L.value_meta_stride_page >= (int64_t)L.H_KV * kPage * 4,
                 KITTY_E_RANGE, "a page stride is smaller than one page");
   return 0;
@@ -1204,35 +1210,49 @@ extern "C" int kitty_append_chunk(const kitty_kv_layer* layer, const void* k_new
                 KITTY_E_ALIGN, "k_new / v_new need 16-byte aligned bases and strides with D contiguous");
   const int max_pages = (T + kPage - 1) / kPage;   // a stream holds at most 127 rows before the chunk
   const hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(chunk_quant_kernel<false>, dim3(2 * max_pages, layer->H_KV, B), dim3(256), 0, st, *layer,
+  hipLaunchKernelGGL((chunk_quant_kernel<false, kD>), dim3(2 * max_pages, layer->H_KV, B), dim3(256), 0, st, *layer,
                      (const uint8_t*)k_new, (const uint8_t*)v_new, stride_b, stride_h, stride_t, T, max_pages);
-  hipLaunchKernelGGL(chunk_rows_kernel<false>, dim3(layer->H_KV, B, 2), dim3(kRowThreads), 0, st, *layer, (const uint8_t*)k_new,
+  hipLaunchKernelGGL((chunk_rows_kernel<false, kD>), dim3(layer->H_KV, B, 2), dim3(kRowThreads), 0, st, *layer, (const uint8_t*)k_new,
                      (const uint8_t*)v_new, stride_b, stride_h, stride_t, T);
   hipLaunchKernelGGL(chunk_advance_kernel, dim3(B), dim3(64), 0, st, *layer, T);
   return check_launch("kitty_append_chunk");
 }
 
-extern "C" int kitty_append_chunk_host(const kitty_kv_layer* layer, const void* k_new, const void* v_new,
-                                       int64_t stride_b, int64_t stride_h, int64_t stride_t, int B, int T, void* stream) {
-  if (int rc = check_append_layer(layer, B, /* device_counters */ false)) return rc;
+namespace {
+int append_chunk_host(const kitty_kv_layer* layer, const void* k_new, const void* v_new, int64_t stride_b, int64_t stride_h,
+                      int64_t stride_t, int B, int T, bool any_head_dim, void* stream) {
+  if (int rc = check_append_layer(layer, B, /* device_counters */ false, any_head_dim)) return rc;
   KITTY_REQUIRE(layer->seq_counts == nullptr, KITTY_E_RANGE,
                 "the layer's counters live on the device (seq_counts): use kitty_append_chunk");
   KITTY_REQUIRE(k_new && v_new, KITTY_E_NULL, "k_new / v_new is NULL");
   KITTY_REQUIRE(T >= 1 && T <= (1 << 24), KITTY_E_RANGE, "T=%d out of range", T);
   KITTY_REQUIRE(((uintptr_t)k_new % 16) == 0 && ((uintptr_t)v_new % 16) == 0 && stride_b % 16 == 0 &&
-                    stride_h % 16 == 0 && stride_t % 16 == 0 && stride_t >= kD * 2,
+                    stride_h % 16 == 0 && stride_t % 16 == 0 && stride_t >= layer->D * 2,
                 KITTY_E_ALIGN, "k_new / v_new need 16-byte aligned bases and strides with D contiguous");
   const ChunkPlan c = chunk_plan<true>(*layer, 0, T);
   KITTY_REQUIRE(c.ok, KITTY_E_RANGE, "a cache counter is out of range, a Q-buffer is full, or the chunk exceeds MAX_PAGE=%d",
                 layer->MAX_PAGE);
   const int max_pages = c.npk > c.npv ? c.npk : c.npv;
   const hipStream_t st = (hipStream_t)stream;
-  if (max_pages > 0)
-    hipLaunchKernelGGL(chunk_quant_kernel<true>, dim3(2 * max_pages, layer->H_KV, B), dim3(256), 0, st, *layer,
-                       (const uint8_t*)k_new, (const uint8_t*)v_new, stride_b, stride_h, stride_t, T, max_pages);
-  hipLaunchKernelGGL(chunk_rows_kernel<true>, dim3(layer->H_KV, B, 2), dim3(kRowThreads), 0, st, *layer, (const uint8_t*)k_new,
-                     (const uint8_t*)v_new, stride_b, stride_h, stride_t, T);
+  by_head_dim(layer->D, [&](auto dim) {
+    if (max_pages > 0)
+      hipLaunchKernelGGL((chunk_quant_kernel<true, dim.value>), dim3(2 * max_pages, layer->H_KV, B), dim3(2 * dim.value), 0, st,
+                         *layer, (const uint8_t*)k_new, (const uint8_t*)v_new, stride_b, stride_h, stride_t, T, max_pages);
+    hipLaunchKernelGGL((chunk_rows_kernel<true, dim.value>), dim3(layer->H_KV, B, 2), dim3(kRowThreads), 0, st, *layer,
+                       (const uint8_t*)k_new, (const uint8_t*)v_new, stride_b, stride_h, stride_t, T);
+  });
   return check_launch("kitty_append_chunk_host");
+}
+}  // namespace
+
+extern "C" int kitty_append_chunk_host(const kitty_kv_layer* layer, const void* k_new, const void* v_new,
+                                       int64_t stride_b, int64_t stride_h, int64_t stride_t, int B, int T, void* stream) {
+  return append_chunk_host(layer, k_new, v_new, stride_b, stride_h, stride_t, B, T, /* any_head_dim */ false, stream);
+}
+
+extern "C" int kitty_append_chunk_host_d(const kitty_kv_layer* layer, const void* k_new, const void* v_new,
+                                         int64_t stride_b, int64_t stride_h, int64_t stride_t, int B, int T, void* stream) {
+  return append_chunk_host(layer, k_new, v_new, stride_b, stride_h, stride_t, B, T, /* any_head_dim */ true, stream);
 }
 
 extern "C" int kitty_pack_prompt(const kitty_kv_layer* layer, int first_row, const void* k_new, int64_t k_stride_b,

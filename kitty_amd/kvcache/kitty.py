@@ -400,13 +400,13 @@ class KittyCache(_HFCache):
         if L.PageCount_K + new_pk > L.MAX_PAGE or L.PageCount_V + new_pv > L.MAX_PAGE:
             raise ValueError(f"appending {T} tokens exceeds max_length={L.MAX_LEN}")
         # the whole batch in two launches (a part of it would leave what the rest's Q-buffers hold out of their pages)
-        if L.on_hip and L.seq_counts is None and L.D == 128 and self.select == "hip" and 1 <= T <= 1 << 24 and B == L.MAX_BS \
+        if L.on_hip and L.seq_counts is None and self.select == "hip" and 1 <= T <= 1 << 24 and B == L.MAX_BS \
                 and key_states.shape[1] == L.H_KV and key_states.shape[3] == L.D \
                 and L.Q_Buffer_Count_K < P and L.Q_Buffer_Count_V < P and key_states.stride() == value_states.stride() \
                 and _kernel_ready(L, key_states) and _kernel_ready(L, value_states) and _lib.launchable(key_states.device):
             ks = key_states.stride()
-            rc = _lib.lib().kitty_append_chunk_host(L.descriptor(), key_states.data_ptr(), value_states.data_ptr(), 2 * ks[0],
-                                                    2 * ks[1], 2 * ks[2], B, T, _lib.current_stream_ptr(key_states.device))
+            rc = _lib.lib().kitty_append_chunk_host_d(L.descriptor(), key_states.data_ptr(), value_states.data_ptr(), 2 * ks[0],
+                                                      2 * ks[1], 2 * ks[2], B, T, _lib.current_stream_ptr(key_states.device))
             if rc:
                 _lib.check(rc, "KittyCache.append")
             L.Sink_Count += a
