@@ -14,6 +14,7 @@
 // Wire format for general D (PAGE = 128 tokens): a K page-head is 32 D bytes of low plane (channel d at
 // 32 d), 32 d_boost bytes of high plane (slot s at 32 (D + s)) and D bytes of slot map; a V page-head is
 // 128 rows of D / 4 bytes; metadata as for D = 128 with D resp. 128 (scale, zero) pairs per head.
+#include <cmath>
 #include <type_traits>
 
 #include "any_dim.h"
@@ -24,8 +25,16 @@ void launch_rows_merge(int D, const float* ws_ml, const float* ws_acc, void* out
                        bool keep_nan, hipStream_t stream);
 namespace {
 
-// column tiles of 16 query rows per workgroup in chunked prefill: as many as the output's accumulators leave room for
-constexpr int kPrefillTiles64 = 4, kPrefillTiles256 = 2;
+// Column tiles of 16 query rows per workgroup in chunked prefill: what 256 registers, that is two workgroups on a compute unit,
+// leave room for.  (200 tokens over 8000 at D = 64, one share's worth of rounds each: 124 us with four, whose loop spills, 99
+// with three; with 512 registers and the accumulators copied between the paths' registers, 141.)
+// At D = 64 three, or two where blocks of 32 rows leave less of the chunk's edge empty; each block also costs what unpacking
+// a tile does, about 0.6 of a column tile.  (1000 rows of seven heads: 650 us with three, 730 with two; 16 of four: 19 and 16.)
+int prefill_tiles(int D, int G, int Tq) {
+  if (D != 64) return 1;
+  auto blocks = [&](int nt) { const int pb = 16 * nt / G > 0 ? 16 * nt / G : 1; return (Tq + pb - 1) / pb; };
+  return blocks(2) * 2.6f < blocks(3) * 3.6f ? 2 : 3;
+}
 
 // ---------------------------------------------------------------------------------------------
 // attention
@@ -69,7 +78,7 @@ struct AnyLds {
 // at most 2^-40 of the largest.
 // For decode, sharing a tile among four wavefronts pays where there are fewer tiles than compute units (any_decode.hip).
 template <int D, bool PREFILL, int NT>
-__global__ __launch_bounds__(256, PREFILL ? 1 : 2) void attn_any_kernel(
+__global__ __launch_bounds__(256, 2) void attn_any_kernel(
     kitty_kv_layer L, const uint8_t* __restrict__ q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
     const uint8_t* __restrict__ k_new, const uint8_t* __restrict__ v_new, int64_t new_stride_b,
     int64_t new_stride_h, int64_t new_stride_t, int H_Q, int Tq, float scaling, float* __restrict__ ws_ml,
@@ -143,6 +152,16 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : 2) void attn_any_kernel(
   uint4v pk[kKIter] = {}, pv[kVIter] = {}, pm = {};
   auto k_is_packed = [&](int tile) { return tile > 0 && tile < c.ntiles && tile - 1 < c.pk; };
   auto v_is_packed = [&](int tile) { return tile > 0 && tile < c.ntiles && tile - 1 < c.pv; };
+  // Whole packed tiles first, in a loop of their own: as branches of one loop the packed and the other paths have the
+  // accumulators copied from one set of registers to another at every tile (150 of 1270 instructions a tile at D = 64).
+  // (Decode has few tiles a workgroup: one loop, 9 KB of code less; 12000 tokens of one kv head at D = 256 20.7 us so, 22.0.)
+  const int full_begin = max(tile_begin, 1);
+  const int full_end = PREFILL ? max(full_begin, min(tile_end, 1 + min(min(c.pk, c.pv), c.nbody / kPage))) : full_begin;
+  auto next_of = [&](int tile) {   // full_begin .. full_end - 1, then the others
+    const bool full = tile >= full_begin && tile < full_end;
+    const int t = full && tile + 1 == full_end && tile_begin < full_begin ? tile_begin : tile + 1;
+    return !full && t >= full_begin && t < full_end ? full_end : t;
+  };
   int64_t id_k = 0, id_v = 0;   // of the tile fetched next, asked for one tile ahead: the load behind them waits for nothing
   auto ask = [&](int tile) {
     if (tile < tile_end && k_is_packed(tile)) id_k = page_id(L.page_table_k, (int64_t)b * L.page_table_k_stride_b + tile - 1);
@@ -167,7 +186,7 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : 2) void attn_any_kernel(
       if (tid >= 64 && tid < 96)
         pm = ((const uint4v*)((const uint8_t*)L.value_meta + pg * L.value_meta_stride_page + (int64_t)h * kPage * 4))[tid - 64];
     }
-    ask(tile + 1);
+    ask(next_of(tile));
   };
   auto stage = [&](int tile) {
     if (k_is_packed(tile)) {
@@ -184,19 +203,19 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : 2) void attn_any_kernel(
     }
   };
 
-  if (tile_begin < tile_end) ask(tile_begin), fetch(tile_begin);
-#pragma unroll 1
-  for (int tile = tile_begin; tile < tile_end; ++tile) {
-    const bool chunk = tile >= c.ntiles;                       // a tile of the new chunk (prefill only)
+  auto step = [&](auto full_, int tile) {
+    constexpr bool FULL = decltype(full_)::value;
+    const bool chunk = !FULL && tile >= c.ntiles;              // a tile of the new chunk (prefill only)
     const int chunk_t0 = chunk ? (tile - c.ntiles) * kPage : 0;
     const int body = tile - 1;                                  // -1 = sink
-    const int ntok = chunk ? min(kPage, kv_chunk - chunk_t0) : tile == 0 ? c.sink : min(kPage, c.nbody - body * kPage);
-    const bool k_packed = k_is_packed(tile), v_packed = v_is_packed(tile);
+    const int ntok = FULL ? kPage : chunk ? min(kPage, kv_chunk - chunk_t0) : tile == 0 ? c.sink : min(kPage, c.nbody - body * kPage);
+    const bool k_packed = FULL || k_is_packed(tile), v_packed = FULL || v_is_packed(tile);
     __syncthreads();   // everyone is done with the tile before
     stage(tile);
     __syncthreads();
-    if (tile + 1 < tile_end) fetch(tile + 1);
-    if (ntok <= 0) continue;   // an empty sink
+    const int after = next_of(tile);
+    if (after < tile_end) fetch(after);
+    if (ntok <= 0) return;   // an empty sink
 
     // ---- logits of tokens 8i + 2w + e: S[e][nt][j] is token 32 kg + 8 j + 2 w + e, row 16 nt + n -------------------
     float4v S[2][NT];
@@ -347,19 +366,23 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : 2) void attn_any_kernel(
         uint32_t X10[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) X10[j] = X[j] >> 10;
-        auto tile = [&](auto u_) {
+        auto piece = [&](auto u_, bool infinities) {
           constexpr int u = decltype(u_)::value;
           uint32_t a[4];
 #pragma unroll
           for (int j = 0; j < 4; ++j) a[j] = dequant_v<u>(X[j], X10[j], kCodeMagic, sc[j], zr[j]);
-          weigh(a, hf * kU + u, wild);
+          weigh(a, hf * kU + u, infinities);
         };
-        tile(std::integral_constant<int, 0>{}), tile(std::integral_constant<int, 1>{});
-        tile(std::integral_constant<int, 2>{}), tile(std::integral_constant<int, 3>{});
-        if constexpr (kU == 8) {
-          tile(std::integral_constant<int, 4>{}), tile(std::integral_constant<int, 5>{});
-          tile(std::integral_constant<int, 6>{}), tile(std::integral_constant<int, 7>{});
-        }
+        auto pieces = [&](bool infinities) {
+          piece(std::integral_constant<int, 0>{}, infinities), piece(std::integral_constant<int, 1>{}, infinities);
+          piece(std::integral_constant<int, 2>{}, infinities), piece(std::integral_constant<int, 3>{}, infinities);
+          if constexpr (kU == 8) {
+            piece(std::integral_constant<int, 4>{}, infinities), piece(std::integral_constant<int, 5>{}, infinities);
+            piece(std::integral_constant<int, 6>{}, infinities), piece(std::integral_constant<int, 7>{}, infinities);
+          }
+        };
+        if (wild) pieces(true);
+        else pieces(false);
       }
     } else {
       int first = t0;
@@ -398,7 +421,16 @@ __global__ __launch_bounds__(256, PREFILL ? 1 : 2) void attn_any_kernel(
         }
       }
     }
+  };
+  const int first = full_begin < full_end ? full_begin : tile_begin;
+  if (first < tile_end) ask(first), fetch(first);
+  if constexpr (PREFILL) {
+#pragma unroll 1
+    for (int tile = full_begin; tile < full_end; ++tile) step(std::true_type{}, tile);
   }
+#pragma unroll 1
+  for (int tile = full_begin < full_end && tile_begin >= full_begin ? full_end : tile_begin; tile < tile_end; tile = next_of(tile))
+    step(std::false_type{}, tile);
 
   if (tid == 0) report_bad_page(L, b, bad_page);
   // ---- the wavefronts' partials meet: a common maximum, then sums of four output tiles at a time ---------------
@@ -474,8 +506,8 @@ void launch_decode_by_tile(const kitty_kv_layer& L, const void* q, int B, int H_
 
 namespace {
 // chunk positions per workgroup
-int any_positions(int D, int G) {
-  const int rows = 16 * (D == 64 ? kPrefillTiles64 : kPrefillTiles256);
+int any_positions(int D, int G, int Tq) {   // chunk positions of a workgroup
+  const int rows = 16 * prefill_tiles(D, G, Tq);
   return rows / G > 0 ? rows / G : 1;
 }
 // Shares of ceil(tiles / s) tiles, as the kernel cuts them at D = 256, may leave the last of them empty: 65 tiles in 64 shares are
@@ -487,32 +519,35 @@ int without_empty_shares(int D, int tiles, int s) {
 }
 }  // namespace
 
-// Shares of a chunk's walk: enough workgroups for two on every compute unit (what their registers allow at
-// D = 256), of at least two tiles each.  `most`: shares the scratch allows.
+// Shares of a chunk's walk.  The device holds two workgroups per compute unit at a time (their registers); a share takes as
+// long as its tiles and one more (its start and its end), and rounds that are not full overlap with the next by about a half.
+// A share more also costs the merge its partials: a tile's time is some 4 us, in which it reads 12 MB.  At least two tiles
+// each.  200 tokens over 8000 at D = 64, 136 workgroups: 99 us with 7 shares (two rounds of 93 %), 105 with 3, 125 with 4;
+// 1000 over 30000 (334): 650 with 3, 968 with 1.  200 over 4000 at D = 256 (200): 121 with 5, 131 with 2, 140 with 3.
+// `most`: shares the scratch allows.
 int prefill_splits_any(int B, int H_Q, int H_KV, int D, int Tq, int tiles, int units, int most) {
-  const int PB = any_positions(D, H_Q / H_KV);
-  const int64_t wgs = (int64_t)((Tq + PB - 1) / PB) * H_KV * B;
-  int64_t s = 2 * units / wgs;
-  if (s > tiles / 2) s = tiles / 2;
-  if (s > most) s = most;
-  return without_empty_shares(D, tiles, s < 1 ? 1 : (int)s);
+  const int PB = any_positions(D, H_Q / H_KV, Tq);
+  const double wgs = (double)((Tq + PB - 1) / PB) * H_KV * B, merged = (double)B * Tq * H_Q * D * 4 / 12e6;
+  int best = 1;
+  double least = 0;
+  for (int s = 1; s <= most && s <= 64 && (s == 1 || 2 * s <= tiles); ++s) {
+    const double rounds = wgs * s / (2 * units), whole = ceil(rounds);
+    const double cost = (whole <= 1 ? 1 : (whole + rounds) / 2) * ((tiles + s - 1) / s + 1) + (s > 1 ? merged * s : 0);
+    if (s == 1 || cost < least) best = s, least = cost;
+  }
+  return without_empty_shares(D, tiles, best);
 }
 
 void launch_prefill_any(const kitty_kv_layer& L, const void* q, int64_t q_stride_b, int64_t q_stride_h,
                         int64_t q_stride_t, const void* k_new, const void* v_new, int64_t new_stride_b,
                         int64_t new_stride_h, int64_t new_stride_t, int B, int H_Q, int Tq, float scaling, void* out,
                         float* ws_ml, float* ws_acc, int num_splits, hipStream_t stream) {
-  const int PB = any_positions(L.D, H_Q / L.H_KV);
+  const int G = H_Q / L.H_KV, nt = prefill_tiles(L.D, G, Tq), PB = any_positions(L.D, G, Tq);
   const dim3 grid((Tq + PB - 1) / PB * num_splits, L.H_KV, B), block(256);
-  const int lds = AnyLds(L.D, L.D_BOOSTED).with_q(L.D, L.D == 64 ? kPrefillTiles64 : kPrefillTiles256);
-  if (L.D == 64)
-    hipLaunchKernelGGL((attn_any_kernel<64, true, kPrefillTiles64>), grid, block, lds, stream, L, (const uint8_t*)q, q_stride_b,
-                       q_stride_h, q_stride_t, (const uint8_t*)k_new, (const uint8_t*)v_new, new_stride_b,
-                       new_stride_h, new_stride_t, H_Q, Tq, scaling, ws_ml, ws_acc, num_splits, (__half*)out);
-  else
-    hipLaunchKernelGGL((attn_any_kernel<256, true, kPrefillTiles256>), grid, block, lds, stream, L, (const uint8_t*)q, q_stride_b,
-                       q_stride_h, q_stride_t, (const uint8_t*)k_new, (const uint8_t*)v_new, new_stride_b,
-                       new_stride_h, new_stride_t, H_Q, Tq, scaling, ws_ml, ws_acc, num_splits, (__half*)out);
+  const auto kernel = L.D == 256 ? attn_any_kernel<256, true, 1> : nt == 2 ? attn_any_kernel<64, true, 2> : attn_any_kernel<64, true, 3>;
+  hipLaunchKernelGGL(kernel, grid, block, AnyLds(L.D, L.D_BOOSTED).with_q(L.D, nt), stream, L, (const uint8_t*)q, q_stride_b,
+                     q_stride_h, q_stride_t, (const uint8_t*)k_new, (const uint8_t*)v_new, new_stride_b, new_stride_h,
+                     new_stride_t, H_Q, Tq, scaling, ws_ml, ws_acc, num_splits, (__half*)out);
   if (num_splits > 1)
     launch_rows_merge(L.D, ws_ml, ws_acc, out, (int64_t)B * Tq * H_Q, num_splits, /* keep_nan */ false, stream);
 }
