@@ -786,8 +786,10 @@ int prefill_lds_bytes() { return kLdsBytes; }
 // How many shares the walk over the tiles is cut into.  A workgroup has a compute unit to itself, so a launch
 // of W workgroups takes ceil(W / units) rounds of its longest walk; cutting the walk in s shortens the walk
 // and multiplies the workgroups.  What a share costs besides its tiles is about three tiles' time (filling
-// the pipeline, 128 KB of partials); the merge reads 512 bytes a row and share.  A tile takes 4.2 us with all
-// rows in use.  The smallest total wins; ties go to fewer shares.
+// the pipeline, 128 KB of partials); the merge reads 512 bytes a row and share.  A tile is priced at 5.4 us, what one of
+// fp16 rows takes with all rows in use (a whole page takes 4.2; priced so, short walks, which are mostly fp16 rows, get too
+// few shares: 300 tokens over 1000 three, 144 us, where four take 129; long ones the same).  The smallest total wins; ties go
+// to fewer shares.
 // `tiles`: 128-token tiles the layer holds (sink included) plus those of the chunk; `most`: shares the scratch allows.
 int prefill_splits(int B, int H_Q, int H_KV, int Tq, int tiles, int units, int most) {
   const int G = H_Q / H_KV;
@@ -798,7 +800,7 @@ int prefill_splits(int B, int H_Q, int H_KV, int Tq, int tiles, int units, int m
   float best_us = 0.f;
   for (int s = 1; s <= most && (s == 1 || 2 * s <= tiles); ++s) {
     const int64_t rounds = (wgs * s + units - 1) / units;
-    float us = 4.2f * (float)rounds * (float)(c_div_up(tiles, s) + 3);
+    float us = 5.4f * (float)rounds * (float)(c_div_up(tiles, s) + 3);
     if (s > 1) us += 4.f + rows * (float)s * 3.5e-4f;   // write + read of 1 KB at about 3 TB/s
     if (s == 1 || us < 0.98f * best_us) best = s, best_us = us;
   }
