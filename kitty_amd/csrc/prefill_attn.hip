@@ -786,10 +786,10 @@ int prefill_lds_bytes() { return kLdsBytes; }
 // How many shares the walk over the tiles is cut into.  A workgroup has a compute unit to itself, so a launch
 // of W workgroups takes ceil(W / units) rounds of its longest walk; cutting the walk in s shortens the walk
 // and multiplies the workgroups.  What a share costs besides its tiles is about three tiles' time (filling
-// the pipeline, 128 KB of partials); the merge reads 512 bytes a row and share.  A tile is priced at 5.4 us, what one of
-// fp16 rows takes with all rows in use (a whole page takes 4.2; priced so, short walks, which are mostly fp16 rows, get too
-// few shares: 300 tokens over 1000 three, 144 us, where four take 129; long ones the same).  The smallest total wins; ties go
-// to fewer shares.
+// the pipeline, 128 KB of partials); the merge reads 512 bytes a row and share.  A tile is priced at 5.4 us, between
+// a whole page (4.2 with all rows in use) and one of fp16 rows.  (At 4.2 short walks, which are mostly fp16 rows, get too few
+// shares: 300 tokens over 1000 three, 144 us, where four take 129; long ones the same.)  The smallest total wins; ties go to
+// fewer shares.
 // `tiles`: 128-token tiles the layer holds (sink included) plus those of the chunk; `most`: shares the scratch allows.
 int prefill_splits(int B, int H_Q, int H_KV, int Tq, int tiles, int units, int most) {
   const int G = H_Q / H_KV;
