@@ -47,13 +47,14 @@ template <int N>
 __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 __device__ __forceinline__ void wait_reads() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
-// 64 lanes x BYTES (4 or 16) from global memory to LDS; M0 reaches the instruction as an operand.  Every page is read once.
+// 64 lanes x BYTES (4 or 16) from global memory to LDS; M0 reaches the instruction as an operand.  The s_nop is the wait state that the
+// hardware needs between a scalar write of M0 and such a load, which the compiler does not put in front of assembly.  Every page is read once.
 template <int BYTES>
 __device__ __forceinline__ void to_lds(const uint8_t* src, uint32_t dst, int lane) {
   register uint32_t m0_lds asm("m0") = dst;
   const uint32_t off = lane * BYTES;
-  if (BYTES == 16) asm volatile("global_load_lds_dwordx4 %0, %1 nt" ::"v"(off), "s"(src), "s"(m0_lds) : "memory");
-  else asm volatile("global_load_lds_dword %0, %1 nt" ::"v"(off), "s"(src), "s"(m0_lds) : "memory");
+  if (BYTES == 16) asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(off), "s"(src), "s"(m0_lds) : "memory");
+  else asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1 nt" ::"v"(off), "s"(src), "s"(m0_lds) : "memory");
 }
 // `bytes` (a multiple of 16, at least 1024) in whole kilobytes, the last one ending with the data: bytes that two of them cover
 // are the same

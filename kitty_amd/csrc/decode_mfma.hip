@@ -288,27 +288,31 @@ __device__ __forceinline__ void k_load_regs(const Ctx& x, int page_index, KRegs&
 // lane l is M0 + instruction offset + l * BYTES, and the instruction offset advances the global
 // address as well.  N instructions of BYTES (4 or 16) per lane, 64 * BYTES apart.  M0 reaches the
 // instructions as an operand bound to that register (the compiler loads it and knows it is read),
-// not through a clobber.  Every tile is read exactly once, so the loads are marked non-temporal.
+// not through a clobber.  The s_nop is the wait state that the hardware needs between a scalar write of M0 and such a load; the
+// compiler puts it in front of its own builtin but not in front of assembly.  Every tile is read exactly once, so the loads are
+// marked non-temporal.
 template <int N, int BYTES>
 __device__ __forceinline__ void lds_dma(uint32_t lane_off, const uint8_t* base, uint32_t lds) {
   static_assert((BYTES == 16 && (N == 1 || N == 4)) || (BYTES == 4 && (N == 1 || N == 2)), "forms in use");
   register uint32_t m0_lds asm("m0") = lds;
   if constexpr (BYTES == 16 && N == 4)
     asm volatile(
+        "s_nop 0\n\t"
         "global_load_lds_dwordx4 %0, %1 nt\n\t"
         "global_load_lds_dwordx4 %0, %1 offset:1024 nt\n\t"
         "global_load_lds_dwordx4 %0, %1 offset:2048 nt\n\t"
         "global_load_lds_dwordx4 %0, %1 offset:3072 nt"
         :: "v"(lane_off), "s"(base), "s"(m0_lds) : "memory");
   else if constexpr (BYTES == 16)
-    asm volatile("global_load_lds_dwordx4 %0, %1 nt" :: "v"(lane_off), "s"(base), "s"(m0_lds) : "memory");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" :: "v"(lane_off), "s"(base), "s"(m0_lds) : "memory");
   else if constexpr (N == 2)
     asm volatile(
+        "s_nop 0\n\t"
         "global_load_lds_dword %0, %1 nt\n\t"
         "global_load_lds_dword %0, %1 offset:256 nt"
         :: "v"(lane_off), "s"(base), "s"(m0_lds) : "memory");
   else
-    asm volatile("global_load_lds_dword %0, %1 nt" :: "v"(lane_off), "s"(base), "s"(m0_lds) : "memory");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1 nt" :: "v"(lane_off), "s"(base), "s"(m0_lds) : "memory");
 }
 
 // Global -> LDS loads of one K page-head: 8 instructions with the high plane, 6 without
