@@ -620,7 +620,8 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void decode_any_kernel(kitty_
   for (int i = 0; i < 4; ++i)   // (a wavefront whose logits are all NaN has -inf for a maximum and NaN for a sum, which must stay)
     l += s_l[i][n] * (s_m[i][n] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s_m[i][n] - mm));
   const int64_t row = ((int64_t)b * H_Q + h * G + n) * num_splits + split;
-  if (n < G && w == 0 && kg == 0) *(float2*)(ws_ml + row * 2) = float2{mm, l};
+  // (a share of nothing but NaN counts: the merge passes over -inf)
+  if (n < G && w == 0 && kg == 0) *(float2*)(ws_ml + row * 2) = float2{l != l ? 0.f : mm, l};
 #pragma unroll
   for (int t4 = 0; t4 < kOT; t4 += 4) {
     __syncthreads();

@@ -466,8 +466,7 @@ __global__ __launch_bounds__(256, 2) void attn_any_kernel(
     else row = (int64_t)b * H_Q + h * G + qhead[nt];
     if (partial) row = row * num_splits + split;
     if (partial && qpos[nt] >= 0 && w == 0 && kg == 0) {
-      // a share of nothing but NaN counts in a chunk, whose walk may be one share or many (the merge passes over -inf)
-      if (PREFILL && l != l) mm = 0.f;
+      if (l != l) mm = 0.f;   // a share of nothing but NaN counts, whatever the number of shares (the merge passes over -inf)
       *(float2*)(ws_ml + row * 2) = float2{mm, l};
     }
 #pragma unroll
