@@ -103,6 +103,9 @@ def fake_quant_tokens_(x: torch.Tensor, t_offset: int, n_tokens: int, axis: int,
     return x
 
 
+_own_fake_quant_tokens = fake_quant_tokens_
+
+
 def fake_quant_groupwise_lastdim(data: torch.Tensor, group_size: int, bit: int,
                                  promote_mask: Optional[torch.Tensor] = None, promote_bit: int = 4) -> torch.Tensor:
     """The reference's signature: ``data`` fp16 [B, nh, M, N], groups of ``group_size`` along the
@@ -193,6 +196,12 @@ class KittyKVCache(_HFCache):
         n = query_length if isinstance(query_length, int) else int(query_length.shape[0])
         return self.get_seq_length(layer_idx) + n, 0
 
+    def _stock(self, *names: str) -> bool:
+        """Neither the module's quantizer nor any of these methods has been replaced, in the module, the class, a subclass or this
+        object: a launch may stand in for them."""
+        return fake_quant_tokens_ is _own_fake_quant_tokens \
+            and all(getattr(getattr(self, n), "__func__", None) is _own_methods[n] for n in names)
+
     # -- the three quantization steps of the reference, on [lo, hi) of a layer's buffers ----------
     def _quant_k(self, layer: int, lo: int, hi: int) -> None:
         c, K = self.cfg, self.key_cache[layer]
@@ -210,11 +219,11 @@ class KittyKVCache(_HFCache):
     def _quant_k_ranked(self, K: torch.Tensor, lo: int, hi: int, src: Optional[torch.Tensor]) -> bool:
         """The same with the top-k and its mask inside the quantizer's launch and, with ``src`` [B, nh, L, D], the keys' copy into
         the empty buffer.  False, and nothing done, where there is no top-k or nothing to quantize, where ``build_promote_mask``
-        has been replaced (it is then called), and for what tensor operations have to handle."""
+        or the quantizer has been replaced (they are then called), and for what tensor operations have to handle."""
         c, (B, nh, _, D) = self.cfg, K.shape
         k_chan = max(0, min(int(D * c.promote_ratio + 1e-6), D))
         if c.channel_selection == 0 or not 0 < k_chan < D or c.kbits >= 16 or build_promote_mask is not _own_promote_mask \
-                or not _rows_readable(K, K.device):
+                or not self._stock() or not _rows_readable(K, K.device):
             return False
         # (a variance is taken from the buffer's layout: the order of torch's sums)
         if src is not None and not (c.channel_selection == 1 and src.shape[2] <= 1 << 24 and _rows_readable(src, K.device)):
@@ -287,9 +296,10 @@ class KittyKVCache(_HFCache):
             for store, x in ((self.key_cache, key_states), (self.value_cache, value_states)):
                 buf = torch.empty((B, nh, cap, D), dtype=torch.float16, device=key_states.device)
                 store.append(buf)
-                if store is self.key_cache and jobs and self._quant_k_ranked(buf, jobs[0][1], jobs[0][2], x):
+                if store is self.key_cache and jobs and self._stock("_run", "_quant_k") and self._quant_k_ranked(buf, jobs[0][1], jobs[0][2], x):
                     jobs.pop()                                  # quantized on their way in
-                elif store is self.value_cache and v_to > v_from and self._values_from(x, buf, v_from, v_to):
+                elif store is self.value_cache and v_to > v_from and self._stock("_run", "_quant_v") \
+                        and self._values_from(x, buf, v_from, v_to):
                     v_to = v_from                               # quantized on their way in
                 else:
                     buf[:, :, :L].copy_(x)
@@ -303,9 +313,13 @@ class KittyKVCache(_HFCache):
         # decode
         L = self._len[layer_idx]
         T_new = key_states.shape[-2]
+        if not self._stock("flush_pending", "_run", "_quant_v"):
+            self.flush_pending(layer_idx)
         pending, self._pending[layer_idx] = self._pending[layer_idx], []
         # one token's values that the last step left are quantized by the launch that appends this step's rows
-        single = pending.pop() if pending and pending[-1][0] == "v" and pending[-1][2] == pending[-1][1] + 1 else None
+        single = None
+        if pending and pending[-1][0] == "v" and pending[-1][2] == pending[-1][1] + 1:
+            single = pending.pop()
         self._run(layer_idx, pending)
         try:
             assert T_new == 1, "decode appends one token per step"
@@ -356,3 +370,6 @@ class KittyKVCache(_HFCache):
                                          c.vbits if quant >= 0 else 1, _lib.current_stream_ptr(K.device))
         _lib.check(rc, "KittyKVCache.update")
         return True
+
+
+_own_methods = {n: getattr(KittyKVCache, n) for n in ("_run", "_quant_k", "_quant_v", "flush_pending")}
