@@ -293,16 +293,18 @@ class KittyKVCache(_HFCache):
                 nq = n - n % c.buffer_length
                 jobs.append(("k", c.sink_length, c.sink_length + nq))
                 v_to = c.sink_length + (nq if c.VCache_BitDecoding else n - c.buffer_length)
-            for store, x in ((self.key_cache, key_states), (self.value_cache, value_states)):
+            bufs = []
+            for keys, x in ((True, key_states), (False, value_states)):
                 buf = torch.empty((B, nh, cap, D), dtype=torch.float16, device=key_states.device)
-                store.append(buf)
-                if store is self.key_cache and jobs and self._stock("_run", "_quant_k") and self._quant_k_ranked(buf, jobs[0][1], jobs[0][2], x):
+                if keys and jobs and self._stock("_run", "_quant_k") and self._quant_k_ranked(buf, jobs[0][1], jobs[0][2], x):
                     jobs.pop()                                  # quantized on their way in
-                elif store is self.value_cache and v_to > v_from and self._stock("_run", "_quant_v") \
-                        and self._values_from(x, buf, v_from, v_to):
+                elif not keys and v_to > v_from and self._stock("_run", "_quant_v") and self._values_from(x, buf, v_from, v_to):
                     v_to = v_from                               # quantized on their way in
                 else:
                     buf[:, :, :L].copy_(x)
+                bufs.append(buf)
+            self.key_cache.append(bufs[0])                      # (both or, after an exception, neither)
+            self.value_cache.append(bufs[1])
             self._len.append(L)
             self._pending.append([])
             jobs.append(("v", v_from, v_to))
@@ -313,14 +315,14 @@ class KittyKVCache(_HFCache):
         # decode
         L = self._len[layer_idx]
         T_new = key_states.shape[-2]
-        if not self._stock("flush_pending", "_run", "_quant_v"):
+        # one token's values that the last step left are quantized by the launch that appends this step's rows (a job leaves the
+        # list once it is done)
+        pending, single = self._pending[layer_idx], None
+        if pending and pending[-1][0] == "v" and pending[-1][2] == pending[-1][1] + 1 and self._stock("flush_pending", "_run", "_quant_v"):
+            self._run(layer_idx, pending[:-1])
+            single, self._pending[layer_idx] = pending[-1], pending[-1:]
+        else:
             self.flush_pending(layer_idx)
-        pending, self._pending[layer_idx] = self._pending[layer_idx], []
-        # one token's values that the last step left are quantized by the launch that appends this step's rows
-        single = None
-        if pending and pending[-1][0] == "v" and pending[-1][2] == pending[-1][1] + 1:
-            single = pending.pop()
-        self._run(layer_idx, pending)
         try:
             assert T_new == 1, "decode appends one token per step"
             if self.max_length is not None and L + 1 > self.max_length:
@@ -334,13 +336,13 @@ class KittyKVCache(_HFCache):
                     store[layer_idx] = buf
             K, V = self.key_cache[layer_idx], self.value_cache[layer_idx]
             if self._append_step(K, V, key_states, value_states, L, single):
-                single = None
+                single, self._pending[layer_idx] = None, []
             else:
                 K[:, :, L:L + 1].copy_(key_states)
                 V[:, :, L:L + 1].copy_(value_states)
         finally:
             if single is not None:
-                self._run(layer_idx, [single])
+                self.flush_pending(layer_idx)
         L += 1
         self._len[layer_idx] = L
         n = L - c.sink_length - c.buffer_length
