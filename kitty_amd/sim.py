@@ -236,6 +236,8 @@ class KittyKVCache(_HFCache):
         else:
             blocks = blocks.transpose(-1, -2)
             score = (blocks - blocks.mean(dim=-1, keepdim=True)).pow(2).mean(dim=-1)
+        if score.dtype != torch.float16:      # autocast takes the power in fp32
+            return False
         score = score.contiguous()
         ks, ss = K.stride(), (0, 0, 0) if src is None else src.stride()
         rc = _lib.lib().kitty_fake_quant_topk(None if src is None else src.data_ptr(), ss[0] * 2, ss[1] * 2, ss[2] * 2, K.data_ptr(),
