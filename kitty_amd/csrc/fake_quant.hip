@@ -383,8 +383,8 @@ extern "C" int kitty_fake_quant_topk(const void* src, int64_t src_stride_b, int6
   KITTY_REQUIRE(bit >= 1 && bit <= 8 && promote_bit >= 1 && promote_bit <= 8, KITTY_E_SHAPE,
                 "bit widths must be in [1, 8], got %d / %d", bit, promote_bit);
   KITTY_REQUIRE(k_promote >= 0 && k_promote <= kD, KITTY_E_RANGE, "k_promote=%d out of range", k_promote);
-  KITTY_REQUIRE(B >= 0 && H >= 1 && B <= 65535 && H <= 65535 && t_offset >= 0 && n_tokens >= 0 && T >= 0 && T <= (1 << 24) &&
-                    (int64_t)t_offset + n_tokens <= (int64_t)T,
+  KITTY_REQUIRE(B >= 0 && H >= 1 && B <= 65535 && H <= 65535 && t_offset >= 0 && n_tokens >= 0 && T >= 0 &&
+                    (!src || T <= (1 << 24)) && (int64_t)t_offset + n_tokens <= (int64_t)T,
                 KITTY_E_RANGE, "bad B=%d H=%d or tokens [%d, %d) outside the %d of the tensor", B, H, t_offset,
                 t_offset + n_tokens, T);
   KITTY_REQUIRE(n_tokens % group_size == 0, KITTY_E_RANGE, "%d tokens are not a whole number of groups of %d", n_tokens, group_size);

@@ -364,8 +364,9 @@ class KittyKVCache(_HFCache):
         """A decode step's rows, and ``job``'s one token of values (or None), in one launch.  False, and nothing done, for
         what tensor operations have to handle."""
         c, (B, nh, T, D) = self.cfg, K.shape
-        if k.shape != (B, nh, 1, D) or v.shape != k.shape or K.stride() != V.stride() or not _rows_readable(k, K.device) \
-                or not _rows_readable(v, K.device) or not _rows_readable(K, K.device) or not _rows_readable(V, K.device):
+        if k.shape != (B, nh, 1, D) or v.shape != k.shape or K.stride() != V.stride() or not (1 <= B <= 65535 and 1 <= nh <= 65535) \
+                or not _rows_readable(k, K.device) or not _rows_readable(v, K.device) or not _rows_readable(K, K.device) \
+                or not _rows_readable(V, K.device):
             return False
         quant = job[1] if job is not None and c.vbits < 16 else -1
         ks, vs, st = k.stride(), v.stride(), K.stride()
