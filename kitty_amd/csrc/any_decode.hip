@@ -61,7 +61,7 @@ __device__ __forceinline__ void to_lds(const uint8_t* src, uint32_t dst, int lan
 __device__ __forceinline__ void block_to_lds(const uint8_t* src, uint32_t dst, int bytes, int lane) {
 #pragma unroll 1
   for (int at = 0; at < bytes; at += 1024) {
-    const int from = min(at, bytes - 1024);
+    const int from = __builtin_amdgcn_readfirstlane(min(at, bytes - 1024));
     to_lds<16>(src + from, dst + from, lane);
   }
 }
@@ -175,8 +175,10 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void decode_any_kernel(kitty_
 
   extern __shared__ __attribute__((aligned(16))) uint8_t lds_all[];
   __shared__ float s_m[4][16], s_l[4][16];
+  __shared__ int s_left[4];
   const WaveLds at(D, DB);
   uint8_t* const lds = lds_all + w * at.bytes;
+  const uint8_t* page_lds = lds;   // where a page's bytes are read
   const uint32_t lds_at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds);
   if (lane < 2) ((uint4*)(lds + at.zero_row))[lane] = uint4{0u, 0u, 0u, 0u};
 
@@ -247,17 +249,17 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void decode_any_kernel(kitty_
     return k;
   };
   auto slots = [&](int kc, const Corner& at_) {
-    const uint8_t* idx = lds + at_.slot + 32 * kc;
+    const uint8_t* idx = page_lds + at_.slot + 32 * kc;
     return (int)idx[0] | (int)idx[16] << 8;
   };
   auto read_k = [&](int kc, int slot, Chunk& k, const Corner& at_) {
     const int s0 = slot & 255, s1 = slot >> 8;
-    const uint8_t* p = lds + at_.plane + 32 * kc * kRowBytes;
+    const uint8_t* p = page_lds + at_.plane + 32 * kc * kRowBytes;
     lds_tr(p, k.X[0], k.X[1]);
     lds_tr(p + 16 * kRowBytes, k.X[2], k.X[3]);
-    lds_tr(lds + (s0 < DB ? (D + s0) * kRowBytes : at.zero_row) + at_.quarter, k.H[0], k.H[1]);
-    lds_tr(lds + (s1 < DB ? (D + s1) * kRowBytes : at.zero_row) + at_.quarter, k.H[2], k.H[3]);
-    const uint8_t* m = lds + at_.meta + 128 * kc;
+    lds_tr(page_lds + (s0 < DB ? (D + s0) * kRowBytes : at.zero_row) + at_.quarter, k.H[0], k.H[1]);
+    lds_tr(page_lds + (s1 < DB ? (D + s1) * kRowBytes : at.zero_row) + at_.quarter, k.H[2], k.H[3]);
+    const uint8_t* m = page_lds + at_.meta + 128 * kc;
     k.m0 = *(const uint4*)m;
     k.m1 = *(const uint4*)(m + 64);
   };
@@ -307,8 +309,8 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void decode_any_kernel(kitty_
     // take its lower and upper four codes
     uint32_t rows_at = at.v_raw + (32 * kg + (n >> 2)) * (D / 4) + (D == 64 ? n & 1 : n & 3) * 8, metas_at = at.v_meta + 32 * kg * 4;
     asm volatile("" : "+v"(rows_at), "+v"(metas_at));
-    const uint8_t* const rows = lds + rows_at;
-    const uint8_t* const metas = lds + metas_at;
+    const uint8_t* const rows = page_lds + rows_at;
+    const uint8_t* const metas = page_lds + metas_at;
     uint4 mm[2];
     uint32_t Y[4];
     auto read_meta = [&](int cj) { mm[0] = *(const uint4*)(metas + 32 * cj), mm[1] = *(const uint4*)(metas + 32 * cj + 16); };
@@ -378,7 +380,8 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void decode_any_kernel(kitty_
   };
 
   // ---- any tile: tokens 8i + 2w + e, e = 0, 1 -------------------------------------------------------------------------------
-  auto special = [&](int tile, int w) {
+  // there: its page lies at page_lds already
+  auto special = [&](int tile, int w, bool there) {
     int id = lane;
     asm volatile("" : "+v"(id));   // as above
     const int kg = id >> 4, n = id & 15;
@@ -389,8 +392,8 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void decode_any_kernel(kitty_
     const int64_t win_base = (int64_t)b * L.win_stride_b + (int64_t)h * L.win_stride_h;
     const int t0 = 32 * kg + 2 * w;   // operand register j of the second product: tokens t0 + 8 j, t0 + 8 j + 1
     uint32_t qq[kKC][4];
-    if (k_packed) fetch_k(body);
-    if (v_packed) fetch_v(body);
+    if (k_packed && !there) fetch_k(body);
+    if (v_packed && !there) fetch_v(body);
     load_query(qq);
     // fp16 values: rows u < lows of one tensor, then the ring's (the end of the sequence only); asked for before the logits
     typedef uint32_t words __attribute__((ext_vector_type(kU / 2)));
@@ -468,7 +471,7 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void decode_any_kernel(kitty_
       uint32_t sc[4], zr[4], big = 0u;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        uint2 mm = *(const uint2*)(lds + at.v_meta + (t0 + 8 * j) * 4);
+        uint2 mm = *(const uint2*)(page_lds + at.v_meta + (t0 + 8 * j) * 4);
         if (t0 + 8 * j >= ntok) mm.x = 0u;   // a token that does not count is 0, whatever its bytes say
         if (t0 + 8 * j + 1 >= ntok) mm.y = 0u;
         sc[j] = low_halves(mm.x, mm.y), zr[j] = high_halves(mm.x, mm.y);
@@ -479,7 +482,7 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void decode_any_kernel(kitty_
         constexpr bool WILD = decltype(wild_)::value;
 #pragma unroll
         for (int hf = 0; hf < kHalves; ++hf) {
-          const uint8_t* p = lds + at.v_raw + tok * (D / 4) + hf * kRowBytes + (D == 64 ? n & 1 : n & 3) * 8;
+          const uint8_t* p = page_lds + at.v_raw + tok * (D / 4) + hf * kRowBytes + (D == 64 ? n & 1 : n & 3) * 8;
           uint32_t X[4], X10[4];
           lds_tr(p, X[0], X[1]);
           lds_tr(p + 16 * (D / 4), X[2], X[3]);
@@ -537,7 +540,7 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void decode_any_kernel(kitty_
   const int dealt = num_splits >= 3 * n_special ? num_splits - n_special : num_splits;
   const int first_page = split < dealt ? split + dealt * w : n_full;
   int page = first_page;
-  bool missed = false;   // a page had a scale or zero out of dequant_fast's range
+  const auto wide = [](uint32_t big) { return __any((big & 0x80008000u) != 0u); };
   uint32_t qq[kKC][4];
   if (page < n_full) fetch_k(page), fetch_v(page), load_query(qq);
 #pragma unroll 1
@@ -554,54 +557,59 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void decode_any_kernel(kitty_
     wait_loads<0>();
     const uint2 mm = ((const uint2*)(lds + at.v_meta))[lane];
     big |= out_of_range(mm.x) | out_of_range(mm.y);
+    if (wide(big)) break;
     if (next < n_full) fetch_k(next);
-    if (!__any((big & 0x80008000u) != 0u)) {
-      float mx = vmax3(S[0][0], S[0][1], S[0][2]);
-      mx = vmax(mx, S[0][3]);
+    float mx = vmax3(S[0][0], S[0][1], S[0][2]);
+    mx = vmax(mx, S[0][3]);
 #pragma unroll
-      for (int u = 1; u < 8; ++u) mx = vmax3(mx, S[u][0], vmax3(S[u][1], S[u][2], S[u][3]));
-      A.settle(mx * sc2);
-      const float shift = A.shift();
-      float sum = 0.f;
+    for (int u = 1; u < 8; ++u) mx = vmax3(mx, S[u][0], vmax3(S[u][1], S[u][2], S[u][3]));
+    A.settle(mx * sc2);
+    const float shift = A.shift();
+    float sum = 0.f;
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
+    for (int u = 0; u < 8; ++u)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          S[u][j] = __builtin_amdgcn_exp2f(__builtin_fmaf(S[u][j], sc2, shift));
-          sum += S[u][j];
-        }
-      A.l += sum;
-      values(S);
-    } else {
-      missed = true;
-    }
+      for (int j = 0; j < 4; ++j) {
+        S[u][j] = __builtin_amdgcn_exp2f(__builtin_fmaf(S[u][j], sc2, shift));
+        sum += S[u][j];
+      }
+    A.l += sum;
+    values(S);
     if (next < n_full) fetch_v(next);
     page = next;
   }
+  // A page with a scale or zero out of dequant_fast's range ends a wavefront's walk (a channel of large numbers is one in every page): that
+  // page and those behind it are left to the four.  A decode layer with such a page per head / with nothing else (walking on and then
+  // fetching every page again to find those passed over, four times the one found: in brackets; no such page: third): D = 64, B = 8, 6100
+  // tokens, 32 / 8 heads: 25 / 33 us (29 / 36; 22); D = 256, B = 2, 9000 tokens, 16 / 8: 33 / 44 (49 / 69; 28); B = 4, 30000: 108 / 138 (107 /
+  // 293; 74).
+  if (lane == 0) s_left[w] = page;
 
-  // then what is left, a quarter of a tile's tokens at a time: the special tiles, shared by the wavefronts, and the pages this
-  // wavefront passed over, found again by their metadata
-  int r = num_splits - 1 - split, again = missed ? first_page : n_full, tile = 0, from = 0, to = 0;
+  // then what is left, a quarter of a tile's tokens per wavefront: the special tiles, and the pages left, of which each wavefront
+  // fetches one at a time
+  int r = num_splits - 1 - split, owner = 3, ahead = -4 * dealt;
 #pragma unroll 1
   while (true) {
-    if (from == to) {
-      if (r < n_special) {
-        tile = r < has_sink ? 0 : n_full + 1 + r - has_sink;
-        from = w, to = w + 1, r += num_splits;
-      } else if (again < n_full) {
-        fetch_k(again), fetch_v(again);
+    const bool there = r >= n_special;
+    int tile;
+    if (!there) {
+      tile = r < has_sink ? 0 : n_full + 1 + r - has_sink;
+      r += num_splits;
+    } else {
+      if (++owner == 4) {
+        owner = 0, ahead += 4 * dealt;
+        __syncthreads();   // everyone is done with the pages before
+        const int first = min(min(s_left[0], s_left[1]), min(s_left[2], s_left[3]));
+        if (__builtin_amdgcn_readfirstlane(first) + ahead >= n_full) break;
+        if (page + ahead < n_full) fetch_k(page + ahead), fetch_v(page + ahead);
         wait_loads<0>();
-        const uint2 mm = ((const uint2*)(lds + at.v_meta))[lane];
-        uint32_t big = out_of_range(mm.x) | out_of_range(mm.y);
-        for (int i = 0; i < D / 64; ++i) big |= out_of_range(((const uint32_t*)(lds + at.k_meta))[64 * i + lane]);
-        if (__any((big & 0x80008000u) != 0u)) tile = again + 1, from = 0, to = 4;
-        again += 4 * dealt;
-        continue;
-      } else {
-        break;
+        __syncthreads();
       }
+      tile = __builtin_amdgcn_readfirstlane(s_left[owner]) + ahead + 1;
+      if (tile > n_full) continue;
+      page_lds = lds_all + owner * at.bytes;
     }
-    special(tile, from++);
+    special(tile, w, there);
   }
 
   if (lane == 0) report_bad_page(L, b, bad_page);
