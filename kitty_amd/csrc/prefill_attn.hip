@@ -449,8 +449,10 @@ struct TileAttend {
   }
 
   __device__ __forceinline__ void run_masked(int ntok, int limit) const {
+    int sub = 0;
 #pragma unroll 1
-    for (int sub = 0; 32 * sub < ntok; ++sub) group<1, true>(sub, limit);
+    for (; 32 * (sub + 1) < ntok; sub += 2) group<2, true>(sub, limit);
+    if (32 * sub < ntok) group<1, true>(sub, limit);
   }
   // a whole tile that every row sees
   __device__ __forceinline__ void run_full() const {
