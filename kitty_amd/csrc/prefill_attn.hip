@@ -226,6 +226,22 @@ struct Prefill {
     const int64_t win = (int64_t)b * L.win_stride_b + (int64_t)h * L.win_stride_h;
     const int64_t sink = (int64_t)b * L.sink_stride_b + (int64_t)h * L.sink_stride_h;
     const bool in_sink = t < first_body, in_chunk = t >= first_chunk;
+    // The values' fp16 rows, asked for in front of the keys' stores: one way to memory in a tile's chain, not two (10 tokens over 150 cached,
+    // four layers: 117 -> 106 us; 300 over 1000, eight sequences: 623 -> 586; whole pages are not affected)
+    uint4 rows_v[4];
+    if (!FULL && !v_packed(t)) {   // dead rows must be finite
+      int e = value_token();
+      asm volatile("" : "+v"(e));
+      const bool ok = e < tokens(t);
+      const uint8_t* row = nullptr;
+      if (ok)
+        row = in_chunk ? v_new + (int64_t)(chunk_pos(t) + e) * new_stride_t
+              : in_sink ? (const uint8_t*)L.sink_v + sink + (int64_t)e * (kD * 2)
+                        : (const uint8_t*)v_tail_row(L, c, b, h, (body(t) - c.pv) * kPage + e);
+      const uint4* src = (const uint4*)(row + part() * 64);
+#pragma unroll
+      for (int w = 0; w < 4; ++w) rows_v[w] = ok ? src[w] : uint4{0u, 0u, 0u, 0u};
+    }
     if (FULL || k_packed(t)) {
       // thread = one channel, 32 tokens: plane words of 16 tokens each
       const half2v m2 = __builtin_bit_cast(half2v, g.kmeta);
@@ -306,20 +322,10 @@ struct Prefill {
         *(uint4*)(vrow + w * 32 + 16) = uint4{o[4], o[5], o[6], o[7]};
       }
     } else {
-      // 16 channels at a time: slot 2u + e' takes channel u + 8e'; dead rows must be finite
-      int e = value_token();
-      asm volatile("" : "+v"(e));
-      const bool ok = e < tokens(t);
-      const uint8_t* row = nullptr;
-      if (ok)
-        row = in_chunk ? v_new + (int64_t)(chunk_pos(t) + e) * new_stride_t
-              : in_sink ? (const uint8_t*)L.sink_v + sink + (int64_t)e * (kD * 2)
-                        : (const uint8_t*)v_tail_row(L, c, b, h, (body(t) - c.pv) * kPage + e);
-      const uint4* src = (const uint4*)(row + part() * 64);
-      const uint4 zero4 = uint4{0u, 0u, 0u, 0u};
 #pragma unroll
       for (int w = 0; w < 2; ++w) {
-        const uint4 a = ok ? src[2 * w] : zero4, bb = ok ? src[2 * w + 1] : zero4;   // channels 0..7, 8..15
+        // 16 channels at a time: slot 2u + e' takes channel u + 8e'
+        const uint4 a = rows_v[2 * w], bb = rows_v[2 * w + 1];   // channels 0..7, 8..15
         const uint32_t a4[4] = {a.x, a.y, a.z, a.w}, b4[4] = {bb.x, bb.y, bb.z, bb.w};
         uint32_t o[8];
 #pragma unroll
