@@ -151,13 +151,13 @@ struct Step {
 };
 
 // One workgroup of 4 wavefronts per (split, kv head, batch row).  Whole pages are dealt in turn: page i belongs to split
-// i % dealt, wavefront i / dealt % 4; with share_pages there are so few that four wavefronts share one.  The tiles with fp16 rows (sink, the end of the sequence) go to the splits from
+// i % dealt, wavefront i / dealt % 4.  The tiles with fp16 rows (sink, the end of the sequence) go to the splits from
 // the last on, one each, and all four wavefronts share its tokens: wavefront w takes 8i + 2w and 8i + 2w + 1.  The partial
 // (running maximum in log2 units, sum, un-normalised output) goes to the split-K workspace.
 template <int D, bool COLS>
 __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void decode_any_kernel(kitty_kv_layer L, const uint8_t* __restrict__ q,
                                                                           int H_Q, float scaling, float* __restrict__ ws_ml,
-                                                                          float* __restrict__ ws_acc, int num_splits, int share_pages) {
+                                                                          float* __restrict__ ws_acc, int num_splits) {
   static_assert(D == 64 || D == 256, "128 has kernels of its own");
   typedef Step<D, COLS> State;
   constexpr int kU = State::kU, kHalves = State::kHalves, kOT = State::kOT, kKC = D / 32;
@@ -169,7 +169,7 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void decode_any_kernel(kitty_
   SeqCounts c = load_counts(L, b);
   for (int* x : {&c.sink, &c.pk, &c.rk, &c.pv, &c.rv, &c.lv, &c.off, &c.nbody, &c.ntiles})   // the same in every lane
     *x = __builtin_amdgcn_readfirstlane(*x);
-  const int n_full = share_pages ? 0 : min(min(c.pk, c.pv), c.nbody / kPage);
+  const int n_full = min(min(c.pk, c.pv), c.nbody / kPage);
   const int has_sink = c.sink > 0 ? 1 : 0, n_special = has_sink + c.ntiles - 1 - n_full;
   int bad_page = 0;
 
@@ -654,7 +654,7 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void decode_any_kernel(kitty_
 
 template <int D>
 void launch(const kitty_kv_layer& L, const void* q, int B, int H_Q, float scaling, float* ws_ml, float* ws_acc, int num_splits,
-            int share_pages, hipStream_t stream) {
+            hipStream_t stream) {
   const dim3 grid(num_splits, L.H_KV, B), block(256);
   const int lds = 4 * WaveLds(D, L.D_BOOSTED).bytes;
 #define KITTY_LAUNCH(COLS)                                                                                                        \
@@ -662,7 +662,7 @@ void launch(const kitty_kv_layer& L, const void* q, int B, int H_Q, float scalin
     /* more LDS than the default per-workgroup limit; per device, so set on every launch */                                      \
     if (lds > 65536) (void)hipFuncSetAttribute((const void*)decode_any_kernel<D, COLS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds); \
     hipLaunchKernelGGL((decode_any_kernel<D, COLS>), grid, block, lds, stream, L, (const uint8_t*)q, H_Q, scaling, ws_ml, ws_acc, \
-                       num_splits, share_pages);                                                                                  \
+                       num_splits);                                                                                               \
   } while (0)
   if (H_Q / L.H_KV <= 5) KITTY_LAUNCH(true);
   else KITTY_LAUNCH(false);
@@ -674,19 +674,22 @@ void launch(const kitty_kv_layer& L, const void* q, int B, int H_Q, float scalin
 namespace {
 // Workgroups that fit the device at once: four per compute unit at D = 64, two at D = 256 (registers, LDS).
 int64_t slots_any(int D, int units) { return (int64_t)(D == 64 ? 4 : 2) * units; }
-// Fewer tiles than compute units: four wavefronts share one, and a tile takes a third of the time that one wavefront needs for it
-// (8 us at D = 256, of which two are the way to memory).  At D = 256 the kernel that does only that holds its query
-// operands in LDS and needs no scratch (B = 1, 16 / 8 heads, 300 tokens: 13.3 us against 16.2 for both passes; 2000
-// tokens: 14.3 against 17.6); at D = 64 there is nothing between the two (10.4 and 10.3, 10.4 and 10.6).
-bool few_tiles(int64_t walks, int tiles, int units) { return walks * tiles <= units; }
+// Few tiles: four wavefronts share one, and a tile takes a third of the time that one wavefront needs for it (8 us at D = 256, of which
+// two are the way to memory).  The kernel that does only that holds its query operands in LDS.  It is the faster one with a tile or less
+// a compute unit, and with two while a walk has not so many of them that the merge reads more than decode_any_kernel's fewer splits
+// leave it.  Both passes in a graph, it and decode_any_kernel: D = 64, 8 walks of 4 tiles 7.8 and 8.4 us, 24 of 11 10.1 and 11.9, 16 of 32 10.7
+// and 12.3, 8 of 63 10.8 and 11.5, 4 of 80 11.4 and 11.2, 2 of 200 12.9 and 11.4; D = 256, 8 of 17 13.8 and 17.6, 32 of 10 16.3 and 19.7, 24 of 21 17.2 and
+// 21.9, 16 of 25 16.9 and 16.7, 16 of 32 19.1 and 16.4.
+bool few_tiles(int D, int64_t walks, int tiles, int units) {
+  return walks * tiles <= units || (walks * tiles <= 2 * units && tiles <= (D == 64 ? 64 : 24));
+}
 }  // namespace
 
 void launch_decode_any(const kitty_kv_layer& L, const void* q, int B, int H_Q, float scaling, float* ws_ml, float* ws_acc,
                        int num_splits, int max_tiles, int units, hipStream_t stream) {
-  const bool few = few_tiles((int64_t)B * L.H_KV, max_tiles, units);
-  if (L.D == 64) launch<64>(L, q, B, H_Q, scaling, ws_ml, ws_acc, num_splits, few, stream);
-  else if (few) launch_decode_by_tile(L, q, B, H_Q, scaling, ws_ml, ws_acc, num_splits, stream);
-  else launch<256>(L, q, B, H_Q, scaling, ws_ml, ws_acc, num_splits, 0, stream);
+  if (few_tiles(L.D, (int64_t)B * L.H_KV, max_tiles, units)) launch_decode_by_tile(L, q, B, H_Q, scaling, ws_ml, ws_acc, num_splits, stream);
+  else if (L.D == 64) launch<64>(L, q, B, H_Q, scaling, ws_ml, ws_acc, num_splits, stream);
+  else launch<256>(L, q, B, H_Q, scaling, ws_ml, ws_acc, num_splits, stream);
 }
 
 // Splits of a decode walk.  Few tiles: one each.  Otherwise as many as give every wavefront a page at most, and the tiles with
@@ -698,7 +701,7 @@ void launch_decode_any(const kitty_kv_layer& L, const void* q, int B, int H_Q, f
 int decode_splits_any(int B, int H_KV, int D, int tiles, int units) {
   const int64_t walks = (int64_t)B * H_KV, slots = slots_any(D, units);
   int64_t s = tiles;
-  if (!few_tiles(walks, tiles, units)) {
+  if (!few_tiles(D, walks, tiles, units)) {
     s = (tiles + 1) / 4 + 3;
     if (s > slots / walks) s = slots / walks;
     if (s > tiles) s = tiles;

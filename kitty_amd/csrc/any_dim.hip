@@ -6,7 +6,7 @@
 // size of every model the reference names.  The kernels here cover the other sizes with the same
 // arithmetic and the same storage format, one template parameter for D:
 //
-//   attn_any_kernel<256, false, 1>            decode attention over few tokens, split pass (the reference's order of
+//   attn_any_kernel<D, false, 1>              decode attention over few tokens, split pass (the reference's order of
 //                                             operations: fp16 dequantization with both roundings; matrix cores)
 //   attn_any_kernel<D, true, NT>              chunked-prefill attention, in one pass or in shares
 // Decode attention otherwise: any_decode.hip.
@@ -76,7 +76,7 @@ struct AnyLds {
 // Probabilities stay fp32 numbers: 32768 p is split into three fp16 numbers, each a matrix operand of its own.
 // Together they are the fp32 number itself from 2^-16 of the row's largest probability on; below that they miss it by
 // at most 2^-40 of the largest.
-// For decode, sharing a tile among four wavefronts pays where there are fewer tiles than compute units (any_decode.hip).
+// For decode, sharing a tile among four wavefronts pays where there are few tiles (few_tiles in any_decode.hip).
 template <int D, bool PREFILL, int NT>
 __global__ __launch_bounds__(256, 2) void attn_any_kernel(
     kitty_kv_layer L, const uint8_t* __restrict__ q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
@@ -101,7 +101,7 @@ __global__ __launch_bounds__(256, 2) void attn_any_kernel(
   const int kv_chunk = PREFILL ? min(Tq, p0 + PB) : 0;           // chunk tokens this workgroup can see
   const int n_tiles = c.ntiles + (kv_chunk + kPage - 1) / kPage;
   int tile_begin, tile_end;
-  if (D == 64) {   // shares that differ by at most one tile (B = 8, 6100 tokens: 24.1 -> 22.8 us)
+  if (D == 64) {   // shares that differ by at most one tile
     const int least = n_tiles / num_splits, longer = n_tiles - least * num_splits;
     tile_begin = split * least + min(split, longer), tile_end = tile_begin + least + (split < longer ? 1 : 0);
   } else {         // equal ones (the last shorter): at D = 256 the compiler's code for the above costs 5 %
@@ -494,18 +494,19 @@ __global__ __launch_bounds__(256, 2) void attn_any_kernel(
 
 }  // namespace
 
-// decode at D = 256
+// decode over few tiles
 void launch_decode_by_tile(const kitty_kv_layer& L, const void* q, int B, int H_Q, float scaling, float* ws_ml, float* ws_acc,
                            int num_splits, hipStream_t stream) {
   const dim3 grid(num_splits, L.H_KV, B), block(256);
-  hipLaunchKernelGGL((attn_any_kernel<256, false, 1>), grid, block, AnyLds(256, L.D_BOOSTED).with_q(256, 1), stream, L, (const uint8_t*)q,
-                     (int64_t)H_Q * 512, (int64_t)512, (int64_t)0, nullptr, nullptr, (int64_t)0, (int64_t)0, (int64_t)0, H_Q, 1, scaling,
-                     ws_ml, ws_acc, num_splits, nullptr);
+  const int64_t row = (int64_t)L.D * 2;
+  const auto kernel = L.D == 64 ? attn_any_kernel<64, false, 1> : attn_any_kernel<256, false, 1>;
+  hipLaunchKernelGGL(kernel, grid, block, AnyLds(L.D, L.D_BOOSTED).with_q(L.D, 1), stream, L, (const uint8_t*)q, H_Q * row, row, (int64_t)0,
+                     nullptr, nullptr, (int64_t)0, (int64_t)0, (int64_t)0, H_Q, 1, scaling, ws_ml, ws_acc, num_splits, nullptr);
 }
 
 namespace {
 // chunk positions per workgroup
-int any_positions(int D, int G, int Tq) {   // chunk positions of a workgroup
+int any_positions(int D, int G, int Tq) {
   const int rows = 16 * prefill_tiles(D, G, Tq);
   return rows / G > 0 ? rows / G : 1;
 }
