@@ -696,8 +696,10 @@ void launch_decode_any(const kitty_kv_layer& L, const void* q, int B, int H_Q, f
 // fp16 rows (three, as a rule) a split of their own, if the device holds them at once: D = 64, B = 8, 6100 tokens, 32 / 8
 // heads: 19.1 us with 15 or 16 splits, 21.2 with 13, 21.9 with 22; D = 64, B = 1, 30000 tokens, 14 / 2: 12.4 with 78, 14.4 with 60;
 // D = 256, B = 2, 9000 tokens, 16 / 8: 26.0 with 24, 32.6 with 18.  Else as many as fit (D = 64, B = 32, 8000 tokens, 24 / 8: 45.6
-// us with 4, 49.1 with 8; D = 256, B = 4, 30000 tokens: 77 with 17, 84 with 29).  At D = 256 a count whose equal shares would
-// leave one without a tile is moved to the next that does not.
+// us with 4, 49.1 with 8; D = 256, B = 4, 30000 tokens: 77 with 17, 84 with 29).  At D = 256 a count whose equal shares would leave one
+// without a tile is moved to the next that does not, as for the kernel that cuts equal shares.  decode_any_kernel deals pages in turn and
+// does not need that; it costs where the move leaves some wavefront a second page (B = 1, 49500 tokens, 8 / 4 heads: 35.2 us with 97, 29.5
+// with 100) and gains a little where it adds splits (B = 2, 9000 tokens: 24.6 with 24, 25.5 with 21).
 int decode_splits_any(int B, int H_KV, int D, int tiles, int units) {
   const int64_t walks = (int64_t)B * H_KV, slots = slots_any(D, units);
   int64_t s = tiles;
