@@ -1,5 +1,5 @@
-"""Decode attention at head dimensions 64 and 256 over more tiles than compute units: whole pages, one a wavefront, beside
-tiles with fp16 rows.  Group sizes on either side of the limit for parts in columns, walks cut into few and many splits (a
+"""Decode attention at head dimensions 64 and 256 over more tiles than compute units, on either side of the line between the
+two decode kernels (test_gpu_head_dims_few has more on the far side): whole pages beside tiles with fp16 rows.  Group sizes on either side of the limit for parts in columns, walks cut into few and many splits (a
 wavefront with none, one and several pages), scales and zeros out of the range of the short dequantization, a high plane
 of another size.  Beyond the output's own fp16 rounding only fp32 sums remain (test_gpu_head_dims_edges)."""
 import numpy as np
