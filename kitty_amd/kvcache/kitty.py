@@ -44,6 +44,9 @@ def _row_source(device: torch.device, x: torch.Tensor) -> torch.Tensor:
     return x
 
 
+_MAX_GRID = 65535    # sequences of one launch: a batch of more keeps tensor copies (attention refuses it)
+
+
 def _kernel_ready(L: KVCache_Layer, x: torch.Tensor) -> bool:
     """``x [B, H_KV, T, D]`` can be read by the packing kernels as it lies: what tensor copies would convert, move or
     track stays with them."""
@@ -98,7 +101,7 @@ class KittyCache(_HFCache):
             self._append_token_device(kvcache, key_states, value_states)
             return False
         # (per-sequence counters set by hand: the host ints still say where the rows go, the kernel would not look at them)
-        if kvcache.on_hip and kvcache.seq_counts is None and 1 <= B <= kvcache.MAX_BS \
+        if kvcache.on_hip and kvcache.seq_counts is None and 1 <= B <= min(kvcache.MAX_BS, _MAX_GRID) \
                 and key_states.shape == (B, kvcache.H_KV, 1, kvcache.D) == value_states.shape \
                 and _lib.launchable(kvcache.KeyCache.device):
             self._append_row(kvcache, key_states, value_states)
@@ -169,7 +172,8 @@ class KittyCache(_HFCache):
         len_local_v, len_qbuf_v, pages_v = n["local_v"], n["qbuf_v"], n["pages_v"]
         if pages_k > kvcache.MAX_PAGE:
             raise ValueError(f"prefill of {len_prefill} tokens exceeds max_length={kvcache.MAX_LEN}")
-        if kvcache.on_hip and self.select == "hip" and 1 <= len_prefill <= 1 << 24 and 1 <= B <= kvcache.MAX_BS - first_row \
+        if kvcache.on_hip and self.select == "hip" and 1 <= len_prefill <= 1 << 24 \
+                and 1 <= B <= min(kvcache.MAX_BS - first_row, _MAX_GRID) \
                 and K.shape == (B, kvcache.H_KV, len_prefill, kvcache.D) == V.shape \
                 and _kernel_ready(kvcache, K) and _kernel_ready(kvcache, V) and _lib.launchable(K.device):
             ks, vs = K.stride(), V.stride()
@@ -400,7 +404,7 @@ class KittyCache(_HFCache):
         if L.PageCount_K + new_pk > L.MAX_PAGE or L.PageCount_V + new_pv > L.MAX_PAGE:
             raise ValueError(f"appending {T} tokens exceeds max_length={L.MAX_LEN}")
         # the whole batch in two launches (a part of it would leave what the rest's Q-buffers hold out of their pages)
-        if L.on_hip and L.seq_counts is None and self.select == "hip" and 1 <= T <= 1 << 24 and B == L.MAX_BS \
+        if L.on_hip and L.seq_counts is None and self.select == "hip" and 1 <= T <= 1 << 24 and B == L.MAX_BS <= _MAX_GRID \
                 and key_states.shape[1] == L.H_KV and key_states.shape[3] == L.D \
                 and L.Q_Buffer_Count_K < P and L.Q_Buffer_Count_V < P and key_states.stride() == value_states.stride() \
                 and _kernel_ready(L, key_states) and _kernel_ready(L, value_states) and _lib.launchable(key_states.device):
