@@ -19,7 +19,7 @@
 // The version before it dealt every page's tokens to the four wavefronts, each of which took two of the 8 codes of a piece,
 // behind two barriers a page: 553 vector and 147 scalar instructions per wavefront and page at D = 64, 1465 and 238 at D = 256,
 // four times; now 880 (D = 64) and 2900 (D = 256) vector instructions a page in all.  A decode layer (append, this
-// kernel, merge): D = 64, B = 8, 6100 tokens, 32 / 8 heads: 26 -> 22 us; D = 256, B = 2, 9000 tokens, 16 / 8: 39 -> 29.5.  Both
+// kernel, merge): D = 64, B = 8, 6100 tokens, 32 / 8 heads: 26 -> 22 us; D = 256, B = 2, 9000 tokens, 16 / 8: 39 -> 28.5.  Both
 // passes alone: D = 64, B = 32, 8000 tokens, 24 / 8: 80 -> 45; D = 256, B = 4, 30000 tokens, 16 / 8: 110 -> 75.
 #include <type_traits>
 

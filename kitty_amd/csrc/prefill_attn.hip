@@ -30,8 +30,8 @@
 // masked with 0x00030003 << 2u: slot 2u + e of a 16-block is element u + 8e.  Keys and values use
 // the same token permutation, the output undoes the channel permutation.
 //
-// What bounds it: power and the vector unit, in turn.  B = 4, 32 / 8 heads, 2048 positions over 30720 cached tokens:
-// 5.13 -> 4.7 ms (830 -> 910 TFLOP/s; the matrix instructions alone, on the same frame, take 3.1).  Per wave and tile, against
+// What bounds it: power and the vector unit, in turn.  B = 4, 32 / 8 heads, 2048 positions over 30720 cached tokens: 4.4 to
+// 5.0 ms by box, the card's power setting it (855 to 970 TFLOP/s; 5.13 to 5.29 before; the matrix instructions alone, on the same frame, take 3.1).  Per wave and tile, against
 // v_mfma_f32_16x16x32 (two rows per lane, twice the matrix instructions) with 288-byte rows: 100 vector instructions,
 // 60 scalar ones and a dependent load (the boost slot) less, and a quarter of the bank conflicts.
 #include <type_traits>
@@ -477,7 +477,7 @@ __host__ __device__ inline int block_positions(int G, int Tq) {
 
 // SPLIT: blockIdx.x = block * num_splits + split; a workgroup walks its share of the tiles and leaves a
 // partial per row (running maximum, running sum, un-normalised output) for rows_merge_kernel.  One
-// workgroup fills a compute unit (147 KB of LDS), and a short chunk has few of them: 200 positions over
+// workgroup fills a compute unit (143 KB of LDS), and a short chunk has few of them: 200 positions over
 // 12k cached tokens, 32 / 8 heads, are 32 workgroups of 98 tiles on 256 units; in 8 shares they are 256 of 13
 // tiles, and a layer (attention and append) takes 96 us instead of 520 (see prefill_splits).
 template <bool BOOST, bool SPLIT>
