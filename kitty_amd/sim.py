@@ -196,11 +196,13 @@ class KittyKVCache(_HFCache):
         n = query_length if isinstance(query_length, int) else int(query_length.shape[0])
         return self.get_seq_length(layer_idx) + n, 0
 
-    def _stock(self, *names: str) -> bool:
-        """Neither the module's quantizer nor any of these methods has been replaced, in the module, the class, a subclass or this
-        object: a launch may stand in for them."""
-        return fake_quant_tokens_ is _own_fake_quant_tokens \
-            and all(getattr(getattr(self, n), "__func__", None) is _own_methods[n] for n in names)
+    def _stock(self) -> bool:
+        """Neither the module's quantizer nor a method that quantizes has been replaced, in the module, the class, a subclass or this
+        object: launches may stand in for them."""
+        cls = type(self)
+        return (fake_quant_tokens_ is _own_fake_quant_tokens and cls._run is _own_methods["_run"]
+                and cls._quant_k is _own_methods["_quant_k"] and cls._quant_v is _own_methods["_quant_v"]
+                and cls.flush_pending is _own_methods["flush_pending"] and _own_methods.keys().isdisjoint(self.__dict__))
 
     # -- the three quantization steps of the reference, on [lo, hi) of a layer's buffers ----------
     def _quant_k(self, layer: int, lo: int, hi: int) -> None:
@@ -223,7 +225,7 @@ class KittyKVCache(_HFCache):
         c, (B, nh, _, D) = self.cfg, K.shape
         k_chan = max(0, min(int(D * c.promote_ratio + 1e-6), D))
         if c.channel_selection == 0 or not 0 < k_chan < D or c.kbits >= 16 or build_promote_mask is not _own_promote_mask \
-                or not self._stock() or not _rows_readable(K, K.device):
+                or fake_quant_tokens_ is not _own_fake_quant_tokens or not _rows_readable(K, K.device):
             return False
         # (a variance is taken from the buffer's layout: the order of torch's sums)
         if src is not None and not (c.channel_selection == 1 and src.shape[2] <= 1 << 24 and _rows_readable(src, K.device)):
@@ -279,7 +281,7 @@ class KittyKVCache(_HFCache):
         c = self.cfg
         if len(self.key_cache) < layer_idx:
             raise ValueError("QuantizedCache does not support model usage where layers are skipped. Use DynamicCache.")
-        jobs = []
+        jobs, stock = [], self._stock()
         if len(self.key_cache) == layer_idx:                                   # prefill
             B, nh, L, D = key_states.shape
             _lib.require_hip(key_states, "key_states")
@@ -298,9 +300,9 @@ class KittyKVCache(_HFCache):
             bufs = []
             for keys, x in ((True, key_states), (False, value_states)):
                 buf = torch.empty((B, nh, cap, D), dtype=torch.float16, device=key_states.device)
-                if keys and jobs and self._stock("_run", "_quant_k") and self._quant_k_ranked(buf, jobs[0][1], jobs[0][2], x):
+                if keys and jobs and stock and self._quant_k_ranked(buf, jobs[0][1], jobs[0][2], x):
                     jobs.pop()                                  # quantized on their way in
-                elif not keys and v_to > v_from and self._stock("_run", "_quant_v") and self._values_from(x, buf, v_from, v_to):
+                elif not keys and v_to > v_from and stock and self._values_from(x, buf, v_from, v_to):
                     v_to = v_from                               # quantized on their way in
                 else:
                     buf[:, :, :L].copy_(x)
@@ -320,7 +322,7 @@ class KittyKVCache(_HFCache):
         # one token's values that the last step left are quantized by the launch that appends this step's rows (a job leaves the
         # list once it is done)
         pending, single = self._pending[layer_idx], None
-        if pending and pending[-1][0] == "v" and pending[-1][2] == pending[-1][1] + 1 and self._stock("flush_pending", "_run", "_quant_v"):
+        if stock and pending and pending[-1][0] == "v" and pending[-1][2] == pending[-1][1] + 1:
             self._run(layer_idx, pending[:-1])
             single, self._pending[layer_idx] = pending[-1], pending[-1:]
         else:
