@@ -208,7 +208,11 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void decode_any_kernel(kitty_
 #pragma unroll
   for (int i = 0; i < 5; ++i) asm volatile("" : "+v"(magic[i]));   // in registers: with the mask as the instruction's constant, masking and merging are one
 
+  // (a lane's offsets are formed here, not kept in registers from one fetch to the next: with more than five heads at D = 64 others then
+  // spill, and a reload inside the page loop waits for the pages under way: B = 42, 4904 tokens, 14 / 2 heads: 25.0 us, 22.8 so)
   auto fetch_k = [&](int page) {
+    int lane = tid & 63;
+    asm volatile("" : "+v"(lane));
     const int64_t pg = checked_page(page_id(L.page_table_k, (int64_t)b * L.page_table_k_stride_b + page), L.cache_pages_k, bad_page);
     const uint8_t* src = L.key_cache + pg * L.key_cache_stride_page + (int64_t)h * k_head_bytes_d(D, DB);
     const uint8_t* meta = (const uint8_t*)L.key_meta + pg * L.key_meta_stride_page + (int64_t)h * D * 4;
@@ -223,6 +227,8 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void decode_any_kernel(kitty_
     to_lds<D == 64 ? 4 : 16>(meta, lds_at + at.k_meta, lane);
   };
   auto fetch_v = [&](int page) {
+    int lane = tid & 63;
+    asm volatile("" : "+v"(lane));
     const int64_t pg = checked_page(page_id(L.page_table_v, (int64_t)b * L.page_table_v_stride_b + page), L.cache_pages_v, bad_page);
     const uint8_t* src = L.value_cache + pg * L.value_cache_stride_page + (int64_t)h * v_head_bytes_d(D);
     const uint8_t* meta = (const uint8_t*)L.value_meta + pg * L.value_meta_stride_page + (int64_t)h * kPage * 4;
